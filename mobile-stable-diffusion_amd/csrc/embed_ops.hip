@@ -213,6 +213,68 @@ __global__ __launch_bounds__(kSmThreads) void softmax_team_kernel(const T *x, T 
     }
 }
 
+// Rows too long for one wavefront's registers (a 768-pixel image has 9216 keys): the row lives in
+// the registers of a whole workgroup, VPL 16-byte vectors per lane, one read and one write per
+// element; the wavefronts' maxima and sums meet in LDS.  Bound by HBM: 147456 x 9216 fp16 runs at
+// 6.0 TB/s (a copy reaches 6.5) against 1.8 in the kernel below, which reads a row twice or three
+// times in 2-byte pieces.  x and y may be the same buffer: a lane stores only what it loaded itself.
+constexpr int kSmBlockMaxThreads = 1024;
+constexpr int kSmBlockMaxVpl = 8;
+
+template <typename T, int VPL>
+__global__ __launch_bounds__(kSmBlockMaxThreads, 4) void softmax_block_kernel(const T *x, T *y, uint32_t row_vecs,
+                                                                            int stable) {
+    constexpr int EPV = Store<T>::EPV;
+    __shared__ float slots_max[kSmBlockMaxThreads / kWave], slots_sum[kSmBlockMaxThreads / kWave];
+    const uint32_t tid = threadIdx.x, nt = blockDim.x;
+    const uint32_t lane = tid & (kWave - 1), wave = tid / kWave, waves = nt / kWave;
+    const size_t row_base = (size_t)blockIdx.x * row_vecs;
+    const u32x4 *in = reinterpret_cast<const u32x4 *>(x) + row_base;
+    u32x4 *out = reinterpret_cast<u32x4 *>(y) + row_base;
+    u32x4 raw[VPL];
+#pragma unroll
+    for (int v = 0; v < VPL; v++) raw[v] = load_stream(in + min(v * nt + tid, row_vecs - 1));
+    float f[VPL][EPV];
+    float mx = kNegInf;
+#pragma unroll
+    for (int v = 0; v < VPL; v++) {
+        Store<T>::unpack(raw[v], f[v]);
+        const bool have = v * nt + tid < row_vecs;
+#pragma unroll
+        for (int e = 0; e < EPV; e++) {
+            f[v][e] = have ? f[v][e] : kNegInf;  // padding: exp gives 0
+            mx = fmaxf(mx, f[v][e]);
+        }
+    }
+    float shift = 0.0f;
+    if (stable) {
+        mx = team_max<64>(mx);
+        if (lane == 0) slots_max[wave] = mx;
+        __syncthreads();
+        shift = team_max<64>(lane < waves ? slots_max[lane] : kNegInf);
+        shift = shift == kNegInf ? 0.0f : shift;  // a row of -inf: keep the reference's 0/0
+    }
+    const float bias = -shift * kLog2e;
+    float total = 0.0f;
+#pragma unroll
+    for (int v = 0; v < VPL; v++)
+#pragma unroll
+        for (int e = 0; e < EPV; e++) {
+            f[v][e] = __builtin_amdgcn_exp2f(fmaf(f[v][e], kLog2e, bias));
+            total += f[v][e];
+        }
+    total = wave_sum(total);
+    if (lane == 0) slots_sum[wave] = total;
+    __syncthreads();
+    const float inv = 1.0f / wave_sum(lane < waves ? slots_sum[lane] : 0.0f);
+#pragma unroll
+    for (int v = 0; v < VPL; v++) {
+#pragma unroll
+        for (int e = 0; e < EPV; e++) f[v][e] *= inv;
+        if (v * nt + tid < row_vecs) store_stream(out + v * nt + tid, Store<T>::pack(f[v]));
+    }
+}
+
 // Any row length / alignment: one wavefront per row, lane-strided elements, the row
 // re-read from cache for each of the (up to) three passes.
 template <typename T>
@@ -426,6 +488,24 @@ void softmax_team_launch(const T *x, T *y, uint32_t rows, uint32_t row_vecs, int
                        dim3(threads), 0, stream, x, y, rows, row_vecs, stable);
 }
 
+template <typename T>
+void softmax_block_launch(const T *x, T *y, uint32_t rows, uint32_t row_vecs, int stable, hipStream_t stream) {
+    // 2-byte rows take eight vectors per lane and few lanes, 4-byte rows few vectors and many lanes.
+    // Measured over 1.36 GB rows of 1 ... 8 vectors per lane, TB/s, not stable: fp16 16384 columns
+    // 5.68 (two) 5.60 (five) 6.18 (eight), 9216 5.80 / 5.81 / 6.02; fp32 5184 columns 6.27 / 5.82 /
+    // 5.90, 9216 (three is the least that fits 1024 lanes) 5.75 / 5.61 / 5.79.
+    uint32_t vpl = sizeof(T) == 2 ? kSmBlockMaxVpl : 2;
+    auto lanes = [&]() { return (((row_vecs + vpl - 1) / vpl + kWave - 1) / kWave) * kWave; };
+    while (lanes() > (uint32_t)kSmBlockMaxThreads) vpl += vpl < 4 ? 1 : 4;
+    const dim3 grid(rows), block(lanes());
+    switch (vpl) {
+        case 2: launch((softmax_block_kernel<float, 2>), grid, block, 0, stream, (const float *)x, (float *)y, row_vecs, stable); break;
+        case 3: launch((softmax_block_kernel<float, 3>), grid, block, 0, stream, (const float *)x, (float *)y, row_vecs, stable); break;
+        case 4: launch((softmax_block_kernel<float, 4>), grid, block, 0, stream, (const float *)x, (float *)y, row_vecs, stable); break;
+        default: launch((softmax_block_kernel<T, kSmBlockMaxVpl>), grid, block, 0, stream, x, y, row_vecs, stable); break;
+    }
+}
+
 }  // namespace
 
 template <typename T>
@@ -547,7 +627,8 @@ int softmax_dispatch(const void *xv, void *yv, size_t rows, size_t cols, int sta
     if (rows > 0x7FFFFFFFull || cols > 0x7FFFFFFFull) return MSD_ERR_INVALID_VALUE;
     const uint32_t r = (uint32_t)rows, c = (uint32_t)cols;
     const size_t row_vecs = cols / EPV;
-    const bool vec_ok = cols % EPV == 0 && aligned16(x) && aligned16(y) && row_vecs <= 1024;
+    const bool vec_ok = cols % EPV == 0 && aligned16(x) && aligned16(y) &&
+                        row_vecs <= (size_t)kSmBlockMaxThreads * kSmBlockMaxVpl;
     if (vec_ok) {
         const uint32_t rv = (uint32_t)row_vecs;
         // up to 64 vectors per row: one vector per lane on the smallest team that holds the row
@@ -562,7 +643,8 @@ int softmax_dispatch(const void *xv, void *yv, size_t rows, size_t cols, int sta
         else if (rv <= 128) softmax_team_launch<T, 2, 64>(x, y, r, rv, stable, stream);
         else if (rv <= 256) softmax_team_launch<T, 4, 64>(x, y, r, rv, stable, stream);
         else if (rv <= 512) softmax_team_launch<T, 8, 64>(x, y, r, rv, stable, stream);
-        else softmax_team_launch<T, 16, 64>(x, y, r, rv, stable, stream);
+        else if (rv <= 1024) softmax_team_launch<T, 16, 64>(x, y, r, rv, stable, stream);
+        else softmax_block_launch<T>(x, y, r, rv, stable, stream);
         return launch_status();
     }
     // The flat kernel pays two barriers and two LDS round trips; below about 12000 rows the

@@ -231,6 +231,16 @@ def test_softmax_edge_shapes(msd, orc, cuda, rows, cols):
             _softmax_case(msd, orc, cuda, rows, cols, 8100 + cols, half, stable, sigma=1.5)
 
 
+@pytest.mark.parametrize("cols,half", [
+    (8200, True), (9216, True), (12288, True), (65536, True), (65544, True),       # 192, 192, 192, 1024 lanes; too long
+    (4100, False), (8192, False), (8196, False), (12292, False), (16388, False), (32768, False), (32772, False)])
+def test_softmax_rows_of_a_whole_workgroup(msd, orc, cuda, cols, half):
+    """Rows longer than 1024 vectors: the shortest and the longest of each vectors-per-lane count
+    and the first row that no workgroup holds."""
+    for stable in (0, 1):
+        _softmax_case(msd, orc, cuda, 5, cols, 8600 + cols + stable, half, stable, sigma=1.5, inplace=bool(stable))
+
+
 @pytest.mark.parametrize("rb", [16, 32, 64])
 def test_softmax_short_rows_flat_kernel(msd, orc, cuda, rb):
     """Rows of 77 / 100 moved as flat 16-byte vectors, rb rows per workgroup, plus a ragged tail."""
