@@ -145,8 +145,9 @@ int msd_groupnorm_noalloc(const void *x, void *y, const float *gamma, const floa
  * *threads lanes each, *vectors_per_lane 16-byte vectors held per lane.  *writers > 1 (then
  * *split = 1): that many workgroups per (sample, group) each load and reduce all of it and store
  * one part; such a launch is only made when y does not overlap x, so in_place != 0 asks for the
- * plan of a call with y == x.  *split = 0 (the others too) means the general kernel: one 256-lane
- * workgroup per (sample, group), nothing held in registers.  Host arithmetic only: needs no GPU
+ * plan of a call with y == x.  *split = 0 (the others too) means a shape with hw not a multiple of
+ * a vector: its launch is not reported (the same kernels where units are whole vectors, otherwise
+ * the general one: one 256-lane workgroup per (sample, group), nothing in registers).  Host arithmetic only: needs no GPU
  * and launches nothing.  For diagnostics, tests and benchmark tables.  No counterpart in the
  * reference (its geometry is fixed, M/nn/GroupNorm.cpp:105-128).
  */

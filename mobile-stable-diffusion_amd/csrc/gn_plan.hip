@@ -259,16 +259,21 @@ uint32_t rule_split(const Chip &chip, size_t elt, size_t units, size_t vec_per_u
 // each holding its slice as `k` vectors per lane.  `elt` = bytes per element, `max_units` = units
 // the exchange scratch has room for.  `writers` > 1 (only where `may_share`: the output does
 // not overlap the input) means whole units with that many workgroups each, every one loading and
-// reducing the whole unit and storing its part of it.  Reads the tuning knobs.
+// reducing the whole unit and storing its part of it.  `ragged_too`: also plan for channels that are
+// no whole number of vectors (gn_slice_kernel<..., RAGGED>).  Reads the tuning knobs.
 GnDecision gn_decide(size_t elt, size_t batch, size_t channels, size_t hw, size_t groups, bool aligned,
-                     size_t max_units, bool may_share) {
+                     size_t max_units, bool may_share, bool ragged_too) {
     GnDecision d{0, 0, 0, 0, 1};
     const size_t epv = 16 / elt;
     const size_t cpg = channels / groups;
     const size_t unit_size = cpg * hw;
     const size_t units = batch * groups;
     // (the register kernel addresses a unit with 32-bit byte offsets)
-    if (!aligned || hw % epv != 0 || unit_size * elt >= (1ull << 32)) return d;
+    if (!aligned || unit_size * elt >= (1ull << 32)) return d;
+    // Channels that are no whole number of vectors (`ragged_too`): the units still are (every unit starts
+    // on a vector), and a vector touches two channels at most
+    const bool ragged = hw % epv != 0;
+    if (ragged && !(ragged_too && unit_size % epv == 0 && hw >= epv && unit_size <= 0x7FFFFFFFull)) return d;
     const size_t vec_per_unit = unit_size / epv;
     const Chip chip = chip_info();
 
@@ -277,8 +282,8 @@ GnDecision gn_decide(size_t elt, size_t batch, size_t channels, size_t hw, size_
     const int tune_writers = g_tuning.gn_writers.load(std::memory_order_relaxed);
     const bool rule_only = g_tuning.gn_plan_rule_only.load(std::memory_order_relaxed) != 0;
     const bool can_split = units <= max_units;
-    // gamma / beta of the group go through LDS from seven vectors per lane on
-    auto affine_fits = [&](int k) { return !(k > kGnPrefetchAffineK && cpg > kGnLdsChannels); };
+    // gamma / beta of the group go through LDS from seven vectors per lane on (ragged: always)
+    auto affine_fits = [&](int k) { return !((ragged || k > kGnPrefetchAffineK) && cpg > kGnLdsChannels); };
 
     // ---- a measured plan for exactly this shape, on the chip it was measured on.  (With the
     // writers knob at 1, "never share", a launch whose output lies apart is planned exactly like

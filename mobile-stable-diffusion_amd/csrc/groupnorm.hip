@@ -48,7 +48,7 @@ struct GnParams {
     uint32_t split_shift;    // log2(split)
     uint32_t groups;
     uint32_t ch_per_group;
-    FastDiv hw_vec;          // vectors per channel
+    FastDiv hw_vec;          // vectors per channel (RAGGED: elements per channel)
     float eps;
     float inv_count;         // 1 / elements per unit
     uint32_t spin_limit;     // polls before a slice stops waiting for a sibling's words
@@ -294,8 +294,27 @@ __device__ __forceinline__ void gn_slice_stats(u32x4 (&raw)[K], uint32_t n_valid
     }
 }
 
-// FULL: every lane owns exactly K vectors (no masking anywhere).
-template <typename T, int K, bool SILU, bool FULL, bool SHARED>
+// Where a vector that may cross from one channel into the next (hw not a multiple of a vector, but
+// at least one) lies: its first element's channel inside the group, and how many of its elements,
+// from the first on, belong to that channel (all of them: EPV or more).
+struct GnStraddle {
+    uint32_t channel, first;
+};
+template <int EPV>
+__device__ __forceinline__ GnStraddle gn_straddle(uint32_t v, const FastDiv &hw) {
+    const uint32_t c = fast_div(v * EPV, hw);
+    return GnStraddle{c, (c + 1) * hw.d - v * EPV};
+}
+
+// FULL: every lane owns exactly K vectors (no masking anywhere).  RAGGED: hw is not a multiple of a
+// vector (deeper UNet levels of images that are not square powers of two: 9 x 7, 18 x 14), so
+// a vector may hold the end of one channel and the start of the next; each element then picks one
+// of two affine pairs (two selects per element, hidden like the rest of the epilogue).  Such shapes
+// used to take the general kernel, whose three passes in single elements are a latency chain.  us
+// per launch, before and now: fp16 batch 2, 2560 channels at 9 x 7 10.1 -> 2.9, in place 14.1 -> 3.8;
+// 1280 at 18 x 14 17.9 -> 2.9, in place 25.3 -> 4.4; batch 16, 640 at 18 x 14 10.7 -> 4.7; fp32 batch 4,
+// 2560 at 11 x 9 15.9 -> 3.4.
+template <typename T, int K, bool SILU, bool FULL, bool SHARED, bool RAGGED>
 __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
                                         const float *__restrict__ gamma,
                                         const float *__restrict__ beta, const GnScratch &scratch,
@@ -340,20 +359,30 @@ __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
 #pragma unroll
     for (int k = 0; k < K; k++) raw[k] = load_stream(at(xin, k, tid));
     const uint32_t ch0 = (unit % p.groups) * p.ch_per_group;
+    // v plus its channels' addends, rounded to the storage type
+    auto with_chunk = [&](const u32x4 &raw_v, uint32_t v, const T *cb) {
+        float f[EPV];
+        Store<T>::unpack(raw_v, f);
+        if (RAGGED) {
+            const GnStraddle at_v = gn_straddle<EPV>(v, p.hw_vec);
+            const float c0 = Store<T>::load1(cb + ch0 + at_v.channel);
+            const float c1 = Store<T>::load1(cb + ch0 + min(at_v.channel + 1, p.ch_per_group - 1));
+#pragma unroll
+            for (int e = 0; e < EPV; e++) f[e] += (uint32_t)e < at_v.first ? c0 : c1;
+        } else {
+            const float cv = Store<T>::load1(cb + ch0 + fast_div(v, p.hw_vec));
+#pragma unroll
+            for (int e = 0; e < EPV; e++) f[e] += cv;
+        }
+        return Store<T>::pack(f);
+    };
     // optional per-(sample, channel) addend applied before the statistics (the reference's
     // chunkwise_add pass): the sum replaces the slice in registers, rounded to the storage
     // type exactly as a separate add kernel would have stored it
     if (chunk != nullptr) {  // uniform
         const T *cb = chunk + (size_t)(unit / p.groups) * (p.groups * p.ch_per_group);
 #pragma unroll
-        for (int k = 0; k < K; k++) {
-            const float cv = Store<T>::load1(cb + ch0 + fast_div(vidx(k, tid), p.hw_vec));
-            float f[EPV];
-            Store<T>::unpack(raw[k], f);
-#pragma unroll
-            for (int e = 0; e < EPV; e++) f[e] += cv;
-            raw[k] = Store<T>::pack(f);
-        }
+        for (int k = 0; k < K; k++) raw[k] = with_chunk(raw[k], vidx(k, tid), cb);
     }
     if (!FULL) {  // registers of lanes past the end of a ragged slice hold zeros from here on
 #pragma unroll
@@ -367,7 +396,7 @@ __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
     // while the data is in flight.  More: the group's gamma and beta go to LDS once (they are
     // there after the barrier of the statistics) and the epilogue reads each vector's pair one
     // vector ahead, so a lane's registers hold little besides its packed slice.
-    constexpr bool kPrefetchAffine = K <= kGnPrefetchAffineK;
+    constexpr bool kPrefetchAffine = !RAGGED && K <= kGnPrefetchAffineK;
     float ga[kPrefetchAffine ? K : 1], be[kPrefetchAffine ? K : 1];
     if (kPrefetchAffine) {
 #pragma unroll
@@ -396,13 +425,7 @@ __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
             const uint32_t v = l * p.vec_per_slice + i;
             u32x4 r = xin[v];
             if (chunk != nullptr) {
-                const T *cb = chunk + (size_t)(unit / p.groups) * (p.groups * p.ch_per_group);
-                const float cv = Store<T>::load1(cb + ch0 + fast_div(v, p.hw_vec));
-                float f[EPV];
-                Store<T>::unpack(r, f);
-#pragma unroll
-                for (int e = 0; e < EPV; e++) f[e] += cv;
-                r = Store<T>::pack(f);
+                r = with_chunk(r, v, chunk + (size_t)(unit / p.groups) * (p.groups * p.ch_per_group));
             }
             return r;
         };
@@ -419,7 +442,7 @@ __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
     auto epilogue = [&](auto fold_tag) {
         constexpr bool kFold = decltype(fold_tag)::value;
         float g_next = 0.0f, b_next = 0.0f;
-        if (!kPrefetchAffine) {
+        if (!kPrefetchAffine && !RAGGED) {
             const uint32_t c = fast_div(vidx(0, lane_again()), p.hw_vec);
             const float2 gb = aff[c];  // one 8-byte LDS read
             g_next = gb.x;
@@ -428,7 +451,9 @@ __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
 #pragma unroll
         for (int k = 0; k < K; k++) {
             float g_k, b_k;
-            if (kPrefetchAffine) {
+            if (RAGGED) {
+                g_k = b_k = 0.0f;  // (two pairs per vector, read below)
+            } else if (kPrefetchAffine) {
                 g_k = ga[kPrefetchAffine ? k : 0];
                 b_k = be[kPrefetchAffine ? k : 0];
             } else {
@@ -447,15 +472,31 @@ __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
                 const uint32_t first = __builtin_amdgcn_readfirstlane(vidx(k, lane_again()));
                 if (first - part * p.part_vecs >= p.part_vecs) continue;
             }
-            const float a = rstd * g_k;
-            const float b_fold = fmaf(-mean, a, b_k);
             float f[EPV];
-            forget(raw[k]);  // unpack here, one vector at a time
-            Store<T>::unpack(raw[k], f);
+            if (RAGGED) {
+                const GnStraddle at_v = gn_straddle<EPV>(vidx(k, lane_again()), p.hw_vec);
+                const float2 gb0 = aff[at_v.channel];
+                const float2 gb1 = aff[min(at_v.channel + 1, p.ch_per_group - 1)];
+                const float a0 = rstd * gb0.x, a1 = rstd * gb1.x;
+                const float b0 = kFold ? fmaf(-mean, a0, gb0.y) : gb0.y, b1 = kFold ? fmaf(-mean, a1, gb1.y) : gb1.y;
+                forget(raw[k]);  // unpack here, one vector at a time
+                Store<T>::unpack(raw[k], f);
 #pragma unroll
-            for (int e = 0; e < EPV; e++) {
-                const float t = kFold ? fmaf(f[e], a, b_fold) : fmaf(f[e] - mean, a, b_k);
-                f[e] = SILU ? silu_f(t) : t;
+                for (int e = 0; e < EPV; e++) {
+                    const bool in0 = (uint32_t)e < at_v.first;
+                    const float t = fmaf(kFold ? f[e] : f[e] - mean, in0 ? a0 : a1, in0 ? b0 : b1);
+                    f[e] = SILU ? silu_f(t) : t;
+                }
+            } else {
+                const float a = rstd * g_k;
+                const float b_fold = fmaf(-mean, a, b_k);
+                forget(raw[k]);  // unpack here, one vector at a time
+                Store<T>::unpack(raw[k], f);
+#pragma unroll
+                for (int e = 0; e < EPV; e++) {
+                    const float t = kFold ? fmaf(f[e], a, b_fold) : fmaf(f[e] - mean, a, b_k);
+                    f[e] = SILU ? silu_f(t) : t;
+                }
             }
             const u32x4 packed = Store<T>::pack(f);
             const uint32_t t = lane_again();
@@ -475,7 +516,7 @@ __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
 // Up to five vectors per lane (four for float storage) the kernel fits 64 registers: eight
 // wavefronts per SIMD, so two 1024-lane workgroups share a CU and one loads while the other
 // computes (what large batches need).
-template <typename T, int K, bool SILU, bool SHARED>
+template <typename T, int K, bool SILU, bool SHARED, bool RAGGED>
 __global__ __launch_bounds__(kGnMaxThreads, (K <= (sizeof(T) == 2 ? 5 : 4) ? 8 : 4)) void gn_slice_kernel(
     const T *x, const T *chunk, T *y, const float *__restrict__ gamma,
     const float *__restrict__ beta, GnScratch scratch, GnParams p) {
@@ -483,7 +524,7 @@ __global__ __launch_bounds__(kGnMaxThreads, (K <= (sizeof(T) == 2 ? 5 : 4) ? 8 :
     __shared__ float red_b[kGnMaxThreads / kWave];
     __shared__ float red_c[kGnMaxThreads / kWave];
     __shared__ float stats[2];
-    __shared__ float2 aff[K <= kGnPrefetchAffineK ? 1 : kGnLdsChannels];  // (gamma, beta) of the group's channels
+    __shared__ float2 aff[!RAGGED && K <= kGnPrefetchAffineK ? 1 : kGnLdsChannels];  // (gamma, beta) of the group's channels
     uint32_t unit, slice, part;
     if (SHARED) {  // whole units, `writers` workgroups each
         const uint32_t j = blockIdx.x >> p.xcd_shift;
@@ -499,15 +540,15 @@ __global__ __launch_bounds__(kGnMaxThreads, (K <= (sizeof(T) == 2 ? 5 : 4) ? 8 :
     const uint32_t v_end = min(p.vec_per_unit, v_begin + p.vec_per_slice);
     // uniform over the workgroup; the largest K is only launched on slices it fits exactly
     if (K == kGnMaxK || v_end - v_begin == K * blockDim.x)
-        gn_body<T, K, SILU, true, SHARED>(x, chunk, y, gamma, beta, scratch, p, unit, slice, part, v_begin, v_end,
+        gn_body<T, K, SILU, true, SHARED, RAGGED>(x, chunk, y, gamma, beta, scratch, p, unit, slice, part, v_begin, v_end,
                                           red_a, red_b, red_c, stats, aff);
     else
-        gn_body<T, K, SILU, false, SHARED>(x, chunk, y, gamma, beta, scratch, p, unit, slice, part, v_begin, v_end,
+        gn_body<T, K, SILU, false, SHARED, RAGGED>(x, chunk, y, gamma, beta, scratch, p, unit, slice, part, v_begin, v_end,
                                            red_a, red_b, red_c, stats, aff);
 }
 
-// Any shape or alignment: one workgroup per unit, three passes over global memory with
-// scalar accesses (the second and third pass hit in cache for UNet-sized units).
+// Any shape or alignment (units that are no whole number of vectors, channels of less than a
+// vector): one workgroup per unit, three passes over global memory with scalar accesses (the second and third pass hit in cache for UNet-sized units).
 template <typename T, bool SILU>
 __global__ __launch_bounds__(kGenericThreads) void gn_generic_kernel(
     const T *x, const T *chunk, T *y, const float *__restrict__ gamma,
@@ -728,25 +769,38 @@ inline uint32_t gn_xcd_shift(const Chip &chip, bool shared, size_t units) {
     return (uint32_t)__builtin_ctz(chip.xcds);
 }
 
-template <typename T, int K>
+template <typename T, int K, bool RAGGED>
 void gn_launch_k(bool silu, bool shared, uint32_t blocks, uint32_t threads, hipStream_t stream, const T *x,
                  const T *chunk, T *y, const float *gamma, const float *beta, const GnScratch &sc,
                  const GnParams &p) {
     if (K <= kGnSharedMaxK && shared) {
         constexpr int KS = K <= kGnSharedMaxK ? K : 1;  // (larger K never get here: no such instances)
-        if (silu)
-            launch((gn_slice_kernel<T, KS, true, true>), dim3(blocks), dim3(threads), 0, stream, x,
-                               chunk, y, gamma, beta, sc, p);
-        else
-            launch((gn_slice_kernel<T, KS, false, true>), dim3(blocks), dim3(threads), 0, stream,
-                               x, chunk, y, gamma, beta, sc, p);
-    } else if (silu) {
-        launch((gn_slice_kernel<T, K, true, false>), dim3(blocks), dim3(threads), 0, stream, x,
-                           chunk, y, gamma, beta, sc, p);
+        launch((silu ? gn_slice_kernel<T, KS, true, true, RAGGED> : gn_slice_kernel<T, KS, false, true, RAGGED>),
+               dim3(blocks), dim3(threads), 0, stream, x, chunk, y, gamma, beta, sc, p);
     } else {
-        launch((gn_slice_kernel<T, K, false, false>), dim3(blocks), dim3(threads), 0, stream,
-                           x, chunk, y, gamma, beta, sc, p);
+        launch((silu ? gn_slice_kernel<T, K, true, false, RAGGED> : gn_slice_kernel<T, K, false, false, RAGGED>),
+               dim3(blocks), dim3(threads), 0, stream, x, chunk, y, gamma, beta, sc, p);
     }
+}
+
+template <typename T, bool RAGGED>
+int gn_launch(uint32_t k, bool silu, bool shared, uint32_t blocks, uint32_t threads, hipStream_t stream, const T *x,
+              const T *chunk, T *y, const float *gamma, const float *beta, const GnScratch &sc, const GnParams &p) {
+    switch (k) {
+        case 1: gn_launch_k<T, 1, RAGGED>(silu, shared, blocks, threads, stream, x, chunk, y, gamma, beta, sc, p); break;
+        case 2: gn_launch_k<T, 2, RAGGED>(silu, shared, blocks, threads, stream, x, chunk, y, gamma, beta, sc, p); break;
+        case 3: gn_launch_k<T, 3, RAGGED>(silu, shared, blocks, threads, stream, x, chunk, y, gamma, beta, sc, p); break;
+        case 4: gn_launch_k<T, 4, RAGGED>(silu, shared, blocks, threads, stream, x, chunk, y, gamma, beta, sc, p); break;
+        case 5: gn_launch_k<T, 5, RAGGED>(silu, shared, blocks, threads, stream, x, chunk, y, gamma, beta, sc, p); break;
+        case 6: gn_launch_k<T, 6, RAGGED>(silu, shared, blocks, threads, stream, x, chunk, y, gamma, beta, sc, p); break;
+        case 8: gn_launch_k<T, 8, RAGGED>(silu, shared, blocks, threads, stream, x, chunk, y, gamma, beta, sc, p); break;
+        case 10: gn_launch_k<T, 10, RAGGED>(silu, shared, blocks, threads, stream, x, chunk, y, gamma, beta, sc, p); break;
+        case 12: gn_launch_k<T, 12, RAGGED>(silu, shared, blocks, threads, stream, x, chunk, y, gamma, beta, sc, p); break;
+        case 16: gn_launch_k<T, 16, RAGGED>(silu, shared, blocks, threads, stream, x, chunk, y, gamma, beta, sc, p); break;
+        case 20: gn_launch_k<T, 20, RAGGED>(silu, shared, blocks, threads, stream, x, chunk, y, gamma, beta, sc, p); break;
+        default: return MSD_ERR_INVALID_VALUE;  // not a K the kernels are built for: a planning error
+    }
+    return launch_status();
 }
 
 template <typename T>
@@ -781,8 +835,9 @@ int gn_dispatch(const void *xv, const void *chunkv, void *yv, const float *gamma
     const char *xb = reinterpret_cast<const char *>(x), *yb = reinterpret_cast<const char *>(y);
     const size_t bytes = units * unit_size * sizeof(T);
     const bool apart = xb + bytes <= yb || yb + bytes <= xb;
+    const bool ragged = hw % EPV != 0;
     const GnDecision d = gn_decide(sizeof(T), batch, channels, hw, groups, aligned16(x) && aligned16(y),
-                                   fixed != nullptr ? fixed->units : kGnMaxUnits, apart);
+                                   fixed != nullptr ? fixed->units : kGnMaxUnits, apart, true);
     if (d.split == 0)
         return gn_generic<T>(silu, x, chunk, y, gamma, beta, units, unit_size, hw, groups, cpg, eps, stream);
 
@@ -794,7 +849,7 @@ int gn_dispatch(const void *xv, const void *chunkv, void *yv, const float *gamma
     p.split_shift = (uint32_t)__builtin_ctz(split);
     p.groups = (uint32_t)groups;
     p.ch_per_group = (uint32_t)cpg;
-    p.hw_vec = make_fast_div((uint32_t)(hw / EPV));
+    p.hw_vec = make_fast_div((uint32_t)(ragged ? hw : hw / EPV));
     p.eps = eps;
     p.inv_count = 1.0f / (float)unit_size;
     p.spin_limit = tune_spin > 0 ? (uint32_t)tune_spin : kGnSpinLimit;
@@ -812,22 +867,9 @@ int gn_dispatch(const void *xv, const void *chunkv, void *yv, const float *gamma
         if (err != hipSuccess) return (int)err;
     }
     const uint32_t blocks = (uint32_t)(units * split * d.writers);
-    const uint32_t threads = d.threads;
-    switch (d.k) {
-        case 1: gn_launch_k<T, 1>(silu, shared, blocks, threads, stream, x, chunk, y, gamma, beta, sc, p); break;
-        case 2: gn_launch_k<T, 2>(silu, shared, blocks, threads, stream, x, chunk, y, gamma, beta, sc, p); break;
-        case 3: gn_launch_k<T, 3>(silu, shared, blocks, threads, stream, x, chunk, y, gamma, beta, sc, p); break;
-        case 4: gn_launch_k<T, 4>(silu, shared, blocks, threads, stream, x, chunk, y, gamma, beta, sc, p); break;
-        case 5: gn_launch_k<T, 5>(silu, shared, blocks, threads, stream, x, chunk, y, gamma, beta, sc, p); break;
-        case 6: gn_launch_k<T, 6>(silu, shared, blocks, threads, stream, x, chunk, y, gamma, beta, sc, p); break;
-        case 8: gn_launch_k<T, 8>(silu, shared, blocks, threads, stream, x, chunk, y, gamma, beta, sc, p); break;
-        case 10: gn_launch_k<T, 10>(silu, shared, blocks, threads, stream, x, chunk, y, gamma, beta, sc, p); break;
-        case 12: gn_launch_k<T, 12>(silu, shared, blocks, threads, stream, x, chunk, y, gamma, beta, sc, p); break;
-        case 16: gn_launch_k<T, 16>(silu, shared, blocks, threads, stream, x, chunk, y, gamma, beta, sc, p); break;
-        case 20: gn_launch_k<T, 20>(silu, shared, blocks, threads, stream, x, chunk, y, gamma, beta, sc, p); break;
-        default: return MSD_ERR_INVALID_VALUE;  // not a K the kernels are built for: a planning error
-    }
-    return launch_status();
+    if (ragged)
+        return gn_launch<T, true>(d.k, silu, shared, blocks, d.threads, stream, x, chunk, y, gamma, beta, sc, p);
+    return gn_launch<T, false>(d.k, silu, shared, blocks, d.threads, stream, x, chunk, y, gamma, beta, sc, p);
 }
 
 template int gn_dispatch<float>(const void *, const void *, void *, const float *, const float *,

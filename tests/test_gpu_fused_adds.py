@@ -80,6 +80,39 @@ def test_chunk_add_groupnorm_equals_two_launches(msd, orc, cuda, shape, groups, 
     assert msd.status() == 0
 
 
+@pytest.mark.parametrize("batch,channels,hw,groups,half", [
+    (2, 1280, 63, 32, True), (2, 2560, 63, 32, True), (1, 2560, 81, 32, False),   # the deepest level: odd sizes, shared units
+    (2, 640, 252, 32, True), (20, 1280, 252, 32, True),                           # multiples of four: shared, whole units
+    (2, 320, 4092, 32, True), (1, 320, 16380, 32, True), (1, 320, 16390, 32, False),  # slices, the last one shorter
+    (1, 80, 9, 2, True), (3, 32, 5, 4, False), (2, 64, 8 + 1, 8, True),           # barely a vector per channel
+    (1, 16, 7, 2, True), (1, 24, 63, 8, True),                                    # below it; units of no whole vectors
+    (2, 8, 40961, 1, True)])                                                      # slices that start inside a channel
+def test_groupnorm_channels_of_no_whole_vectors(msd, orc, cuda, batch, channels, hw, groups, half):
+    """Vectors that hold the end of one channel and the start of the next, with and without the
+    addend, SiLU and a large mean, apart and in place."""
+    import torch
+    x = orc.normal((batch, channels, hw), seed=channels + hw, sigma=1.5)
+    emb = orc.normal((batch, channels), seed=channels + hw + 1, sigma=0.7)
+    g, b = _affine(orc, channels, 11)
+    xin, ein = (orc.round_to_half(x), orc.round_to_half(emb)) if half else (x, emb)
+    gd, bd, ed = _dev(g, cuda), _dev(b, cuda), _dev(ein, cuda, half)
+    close = assert_close_f16 if half else assert_close_f32
+    for mean, silu in ((0.0, True), (9.0, False)):  # 9: the mean is not folded into the offset
+        shifted = orc.round_to_half(xin + mean) if half else (xin + mean).astype(np.float32)
+        ref = orc.groupnorm64(shifted, g, b, groups, 1e-5, silu).astype(np.float32)
+        for inplace in (False, True):
+            xd = _dev(shifted, cuda, half)
+            got = msd.groupnorm(xd, gd, bd, groups, 1e-5, silu, out=xd if inplace else None)
+            close(got.float().cpu().numpy(), ref, what="gn ragged")
+            xd = _dev(shifted, cuda, half)
+            apart = torch.empty_like(xd)
+            tmp = msd.chunkwise_add(xd, ed, hw)
+            two = msd.groupnorm(tmp, gd, bd, groups, 1e-5, silu, out=tmp if inplace else apart)
+            fused = msd.chunk_add_groupnorm(xd, ed, gd, bd, groups, 1e-5, silu, out=xd if inplace else None)
+            assert torch.equal(fused, two)
+    assert msd.status() == 0
+
+
 @pytest.mark.parametrize("half", [False, True], ids=["f32", "f16"])
 @pytest.mark.parametrize("rows,dim", [(8192, 320), (2048, 640), (512, 1280), (77, 1024), (5, 100), (9, 64)])
 def test_add_layernorm_equals_two_launches(msd, orc, cuda, rows, dim, half):
