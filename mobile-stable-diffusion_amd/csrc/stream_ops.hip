@@ -4,6 +4,7 @@
 // but a ragged last one run branch-free.
 #include "msd_device.h"
 #include "msd_internal.h"
+#include "tile_transpose.h"
 
 #include <cmath>
 #include <type_traits>
@@ -145,120 +146,22 @@ __global__ __launch_bounds__(kStreamThreads) void add_generic_kernel(const T *a,
 }
 
 // ---------------------------------------------------------------------------
-// [i, j, k] -> [i, k, j] through a 64 x 64 LDS tile: reads run along k, writes along j, both in
-// 4-element pieces (8 or 16 bytes), tile rows padded by one piece against bank conflicts.
+// [i, j, k] -> [i, k, j], a workgroup per 64 x 64-element tile (tile_transpose.h).
+// ES = bytes per element; JFAST: consecutive workgroups take consecutive tiles of one output row.
+// RAGGED: sizes that are no whole number of 16-byte pieces, or planes that are not 16-byte aligned
+// (the tokens of a 9 x 7 latent); unaligned 16-byte accesses, only the pieces that a row's end cuts go
+// in parts.  Against element-wise and 4-element accesses, us: fp16 32 x 63 x 1280 9.36 -> 3.37, 2 x 252 x
+// 1280 2.58 -> 2.24, fp32 4 x 99 x 1280 3.18 -> 2.65; a copy of the first takes about 3.4.
 // ---------------------------------------------------------------------------
-constexpr int kTile = 64;
-
-template <typename T>
-__global__ __launch_bounds__(256) void permute_021_kernel(const T *__restrict__ src,
-                                                          T *__restrict__ dst, uint32_t jsize,
-                                                          uint32_t ksize) {
-    typedef T vec4 __attribute__((ext_vector_type(4)));
-    __shared__ T tile[kTile][kTile + 4];
-    const uint32_t k0 = blockIdx.x * kTile, j0 = blockIdx.y * kTile, i = blockIdx.z;
-    const T *in = src + (size_t)i * jsize * ksize;
-    T *out = dst + (size_t)i * jsize * ksize;
-    const uint32_t lane4 = (threadIdx.x & 15) * 4, row = threadIdx.x >> 4;  // 16 rows per pass
-#pragma unroll
-    for (int pass = 0; pass < 4; pass++) {
-        const uint32_t j = j0 + row + pass * 16, k = k0 + lane4;
-        if (j < jsize && k < ksize) {  // jsize, ksize are multiples of 4: a piece is all in or out
-            const vec4 v = *reinterpret_cast<const vec4 *>(in + (size_t)j * ksize + k);
-#pragma unroll
-            for (int e = 0; e < 4; e++) tile[row + pass * 16][lane4 + e] = v[e];
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int pass = 0; pass < 4; pass++) {
-        const uint32_t k = k0 + row + pass * 16, j = j0 + lane4;
-        if (k < ksize && j < jsize) {
-            vec4 v;
-#pragma unroll
-            for (int e = 0; e < 4; e++) v[e] = tile[lane4 + e][row + pass * 16];
-            *reinterpret_cast<vec4 *>(out + (size_t)k * jsize + j) = v;
-        }
-    }
-}
-
-// The same permute with 16-byte accesses on both sides and an LDS tile of 32-bit words that is
-// written transposed: word w of tile row k belongs to output row k (one 4-byte element, or the
-// 2-byte elements of input rows 2w and 2w + 1 at column k, paired in registers after the load).
-// Inside a tile row the aligned groups of four words are permuted by an XOR with a number taken
-// from the row index, chosen so that the 32 lanes of a half wavefront, which write one column each
-// (8 rows a fixed distance apart x 4 adjacent words), fall on 32 different banks, while a lane's
-// four output words stay adjacent and aligned: the read side is one 16-byte LDS access per piece,
-// and the eight lanes that read one tile row together take eight different groups.
-// ES = bytes per element; a workgroup moves 64 x 64 elements; jsize and ksize are multiples of
-// 16 / ES (host), so a 16-byte piece is all inside the tensor or all outside.
-template <int ES, bool JFAST>
-__global__ __launch_bounds__(256) void permute_021_words_kernel(const void *__restrict__ srcv,
-                                                                void *__restrict__ dstv, uint32_t jsize,
-                                                                uint32_t ksize) {
-    constexpr uint32_t kWords = kTile * ES / 4;   // 32-bit words per output row of the tile: 32 or 64
-    constexpr uint32_t kRowShift = ES == 4 ? 2 : 3;  // tile rows one lane writes: 4 or 8
-    __shared__ u32x4 tile4[kTile * kWords / 4];
-    uint32_t *tile = reinterpret_cast<uint32_t *>(tile4);
-    // word `col` of tile row `row` lives at this index
-    auto at = [](uint32_t row, uint32_t col) { return row * kWords + (col ^ (((row >> kRowShift) & 7u) << 2)); };
-    // JFAST: consecutive workgroups take consecutive tiles of one output row
+template <int ES, bool JFAST, bool RAGGED>
+__global__ __launch_bounds__(kTileThreads) void permute_021_words_kernel(const void *__restrict__ src,
+                                                                         void *__restrict__ dst, uint32_t jsize,
+                                                                         uint32_t ksize) {
+    __shared__ u32x4 tile4[tile_lds_words<ES>()];
     const uint32_t k0 = (JFAST ? blockIdx.y : blockIdx.x) * kTile, j0 = (JFAST ? blockIdx.x : blockIdx.y) * kTile;
-    const uint32_t i = blockIdx.z;
-    const size_t plane = (size_t)i * jsize * ksize;  // in elements
-    const char *in = static_cast<const char *>(srcv) + plane * ES;
-    char *out = static_cast<char *>(dstv) + plane * ES;
-    const uint32_t t = threadIdx.x;
-    if (ES == 4) {
-        // a lane loads elements k .. k+3 of one input row, four times: 8 lanes cover 32 columns,
-        // the passes take the two column halves of the tile and the two halves of its rows.  All
-        // loads leave before the first LDS write (a piece outside the tensor re-reads the plane's
-        // first piece instead of sitting behind a branch).
-        const uint32_t kq = (t & 7) * 4, jr = t >> 3;
-        u32x4 v[4];
-#pragma unroll
-        for (int pass = 0; pass < 4; pass++) {
-            const uint32_t k = k0 + kq + 32 * (pass & 1), j = j0 + jr + 32 * (pass >> 1);
-            const size_t from = (j < jsize && k < ksize) ? ((size_t)j * ksize + k) * 4 : 0;
-            v[pass] = load_stream(reinterpret_cast<const u32x4 *>(in + from));
-        }
-#pragma unroll
-        for (int pass = 0; pass < 4; pass++) {
-            const uint32_t kl = kq + 32 * (pass & 1), jl = jr + 32 * (pass >> 1);
-            if (j0 + jl < jsize && k0 + kl < ksize) {
-#pragma unroll
-                for (int e = 0; e < 4; e++) tile[at(kl + e, jl)] = v[pass][e];
-            }
-        }
-    } else {
-        // a lane loads elements k .. k+7 of input rows j and j+1 and pairs them by column
-        const uint32_t kq = (t & 7) * 8, jw = t >> 3;  // jw: word of the output rows, 0 .. 31
-        const uint32_t j = j0 + 2 * jw, k = k0 + kq;
-        if (j < jsize && k < ksize) {  // (jsize is even: row j + 1 exists)
-            const u32x4 a = load_stream(reinterpret_cast<const u32x4 *>(in + ((size_t)j * ksize + k) * 2));
-            const u32x4 b = load_stream(reinterpret_cast<const u32x4 *>(in + ((size_t)(j + 1) * ksize + k) * 2));
-#pragma unroll
-            for (int w = 0; w < 4; w++) {
-                tile[at(kq + 2 * w, jw)] = (a[w] & 0xffffu) | (b[w] << 16);
-                tile[at(kq + 2 * w + 1, jw)] = (a[w] >> 16) | (b[w] & 0xffff0000u);
-            }
-        }
-    }
-    __syncthreads();
-    // a lane stores 16-byte pieces (four words) of output rows; all LDS reads come first
-    constexpr uint32_t kPieces = kWords / 4;          // pieces per output row of the tile: 8 or 16
-    constexpr uint32_t kRowsPerPass = 256 / kPieces;  // 32 or 16
-    constexpr uint32_t kPasses = kTile / kRowsPerPass;
-    const uint32_t wq = (t % kPieces) * 4, kr = t / kPieces;
-    u32x4 w[kPasses];
-#pragma unroll
-    for (uint32_t pass = 0; pass < kPasses; pass++)  // (pieces outside the tensor are read but never stored)
-        w[pass] = tile4[at(kr + pass * kRowsPerPass, wq) / 4];
-#pragma unroll
-    for (uint32_t pass = 0; pass < kPasses; pass++) {
-        const uint32_t k = k0 + kr + pass * kRowsPerPass, j = j0 + wq * (4 / ES);
-        if (k < ksize && j < jsize) store_stream(reinterpret_cast<u32x4 *>(out + ((size_t)k * jsize + j) * ES), w[pass]);
-    }
+    const size_t plane = (size_t)blockIdx.z * jsize * ksize * ES;
+    transpose_tile<ES, RAGGED>(static_cast<const char *>(src) + plane, static_cast<char *>(dst) + plane, jsize, ksize, j0,
+                               k0, tile4, [] {}, [](uint32_t, const u32x4 &v) { return v; });
 }
 
 template <typename T>
@@ -402,29 +305,21 @@ int permute_021_dispatch(const void *srcv, void *dstv, size_t isize, size_t jsiz
     const T *src = static_cast<const T *>(srcv);
     T *dst = static_cast<T *>(dstv);
     if (isize * jsize * ksize == 0) return MSD_OK;
-    const uintptr_t piece = 4 * sizeof(T);
-    const bool tiled = jsize % 4 == 0 && ksize % 4 == 0 && reinterpret_cast<uintptr_t>(src) % piece == 0 &&
-                       reinterpret_cast<uintptr_t>(dst) % piece == 0 && isize <= 65535 &&
-                       (jsize + kTile - 1) / kTile <= 65535 && ksize < 0x7FFFFFFFull && jsize < 0x7FFFFFFFull;
     const size_t epv = 16 / sizeof(T);
-    const bool words = tiled && jsize % epv == 0 && ksize % epv == 0 && aligned16(src) && aligned16(dst);
+    const bool ragged = jsize % epv != 0 || ksize % epv != 0 || !aligned16(src) || !aligned16(dst);
     const dim3 tiles((uint32_t)((ksize + kTile - 1) / kTile), (uint32_t)((jsize + kTile - 1) / kTile), (uint32_t)isize);
+    const bool tiled = isize <= 65535 && ksize < 0x7FFFFFFFull && jsize < 0x7FFFFFFFull && (tiles.x <= 65535 || tiles.y <= 65535);
     // Output rows shorter than input rows: consecutive workgroups take the tiles of one output
     // row, so that its 128-byte pieces are written at about the same time (batch 32, 320 x 4096
     // -> 4096 x 320, fp16: 29.9 us against 32.1 with consecutive tiles along the input rows; the
     // copy takes 29.1; the other way round nothing changes).
-    const bool jfast = jsize < ksize;
-    if (words && jfast && tiles.x <= 65535) {
-        launch((permute_021_words_kernel<(int)sizeof(T), true>), dim3(tiles.y, tiles.x, tiles.z), dim3(256), 0,
-                           stream, srcv, dstv, (uint32_t)jsize, (uint32_t)ksize);
-    } else if (words) {
-        launch((permute_021_words_kernel<(int)sizeof(T), false>), tiles, dim3(256), 0, stream, srcv, dstv,
-                           (uint32_t)jsize, (uint32_t)ksize);
-    } else if (tiled) {
-        launch((permute_021_kernel<T>),
-                           dim3((uint32_t)((ksize + kTile - 1) / kTile), (uint32_t)((jsize + kTile - 1) / kTile),
-                                (uint32_t)isize),
-                           dim3(256), 0, stream, src, dst, (uint32_t)jsize, (uint32_t)ksize);
+    const bool jfast = (jsize < ksize && tiles.x <= 65535) || tiles.y > 65535;
+    if (tiled) {
+        constexpr int ES = (int)sizeof(T);
+        auto *kernel = jfast ? (ragged ? permute_021_words_kernel<ES, true, true> : permute_021_words_kernel<ES, true, false>)
+                             : (ragged ? permute_021_words_kernel<ES, false, true> : permute_021_words_kernel<ES, false, false>);
+        launch(kernel, jfast ? dim3(tiles.y, tiles.x, tiles.z) : tiles, dim3(kTileThreads), 0, stream, srcv, dstv,
+               (uint32_t)jsize, (uint32_t)ksize);
     } else {
         const size_t want = (isize * jsize * ksize + kStreamThreads - 1) / kStreamThreads;
         launch((permute_021_generic_kernel<T>), dim3((uint32_t)(want < 65536 ? want : 65536)),

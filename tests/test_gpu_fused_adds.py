@@ -206,6 +206,27 @@ def test_permute_0_2_1(msd, orc, cuda, shape, half):
     assert torch.equal(msd.permute_0_2_1(got), _dev(xin, cuda, half))  # its own inverse
 
 
+@pytest.mark.parametrize("half", [False, True], ids=["f32", "f16"])
+@pytest.mark.parametrize("shape", [(2, 63, 1280), (2, 1280, 63), (1, 65, 127), (3, 1, 9), (2, 9, 1), (1, 130, 66)])
+def test_permute_0_2_1_ragged_and_unaligned(msd, orc, cuda, shape, half):
+    """Rows that start at any element and end inside a 16-byte piece, in tensors that start one
+    element past an aligned address, with nothing written around the output."""
+    import torch
+    n = int(np.prod(shape))
+    x = orc.normal(shape, seed=sum(shape))
+    x = orc.round_to_half(x) if half else x
+    src = torch.zeros(n + 2, dtype=torch.float16 if half else torch.float32, device=cuda)
+    src[1:n + 1] = _dev(x, cuda, half).reshape(-1)
+    dst = torch.full_like(src, 7.0)
+    elt = src.element_size()
+    assert msd.load_library().msd_permute_0_2_1(src.data_ptr() + elt, dst.data_ptr() + elt, *shape,
+                                                msd.DTYPE_F16 if half else msd.DTYPE_F32, None) == 0
+    torch.cuda.synchronize()
+    got = dst.float().cpu().numpy()
+    assert np.array_equal(got[1:n + 1], orc.permute_0_2_1(x).reshape(-1))
+    assert got[0] == 7.0 and got[n + 1] == 7.0
+
+
 def test_fused_argument_checks(msd, cuda):
     lib = msd.load_library()
     assert lib.msd_chunk_add_groupnorm(None, None, None, None, None, 1, 32, 16, 32, 1e-5, 0, 0, None) == 1
