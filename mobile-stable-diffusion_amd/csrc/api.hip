@@ -26,10 +26,11 @@ std::mutex g_scratch_mutex;
 std::unordered_map<ScratchKey, GnScratch, ScratchKeyHash> g_scratch;
 
 // Scratch for `units` (sample, group) pairs, carved out of one block:
-// [slot_mean | slot_m2 | epoch | done | fallbacks], every part 256-byte aligned.
+// [slot_mean | slot_m2 | epoch | done | fallbacks | partials], every part 256-byte aligned.
 constexpr size_t slot_bytes(size_t units) { return sizeof(unsigned long long) * units * kGnMaxSplit; }
 constexpr size_t word_bytes(size_t units) { return sizeof(uint32_t) * units; }
-constexpr size_t scratch_bytes(size_t units) { return 2 * slot_bytes(units) + 2 * word_bytes(units) + 256; }
+constexpr size_t partial_bytes(size_t units) { return sizeof(float2) * units * kGnStatSlices; }
+constexpr size_t scratch_bytes(size_t units) { return 2 * slot_bytes(units) + 2 * word_bytes(units) + 256 + partial_bytes(units); }
 
 GnScratch carve(char *base, size_t units) {
     GnScratch s;
@@ -38,6 +39,7 @@ GnScratch carve(char *base, size_t units) {
     s.epoch = reinterpret_cast<uint32_t *>(base + 2 * slot_bytes(units));
     s.done = reinterpret_cast<uint32_t *>(base + 2 * slot_bytes(units) + word_bytes(units));
     s.fallbacks = reinterpret_cast<uint32_t *>(base + 2 * slot_bytes(units) + 2 * word_bytes(units));
+    s.partials = reinterpret_cast<float2 *>(base + 2 * slot_bytes(units) + 2 * word_bytes(units) + 256);
     s.units = (uint32_t)units;
     return s;
 }
@@ -56,7 +58,7 @@ char *g_static_base[kMaxDevices] = {nullptr};  // device address of `scratch`, p
 
 // Scratch is private to a (device, stream) pair: launches on one stream are ordered, so a
 // unit's slots are never shared by two launches in flight.
-hipError_t get_scratch(hipStream_t stream, GnScratch *out) {
+hipError_t get_scratch(hipStream_t stream, GnScratch *out, bool *capturing) {
     // one handle that names a different stream in every thread cannot key a per-stream scratch
     if (stream == hipStreamPerThread) return hipErrorInvalidValue;
     int device = 0;
@@ -68,6 +70,11 @@ hipError_t get_scratch(hipStream_t stream, GnScratch *out) {
     if (it != g_scratch.end()) {
         *out = it->second;
         return hipSuccess;
+    }
+    if (capturing != nullptr) {
+        hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+        *capturing = hipStreamIsCapturing(stream, &status) == hipSuccess && status != hipStreamCaptureStatusNone;
+        if (*capturing) return hipSuccess;
     }
     char *base = nullptr;
     err = hipMalloc(reinterpret_cast<void **>(&base), scratch_bytes(kGnMaxUnits));

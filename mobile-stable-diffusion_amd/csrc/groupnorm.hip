@@ -29,10 +29,12 @@
 // sibling's part of the input, which no workgroup overwrites before it has
 // seen every word of its unit.  The output is the same either way; a counter
 // in the scratch records how often it happened.
+#include <mutex>
 #include <type_traits>
 
 #include "msd_device.h"
 #include "msd_internal.h"
+#include "tile_transpose.h"
 
 namespace msd {
 
@@ -759,6 +761,137 @@ __global__ __launch_bounds__(kGenericThreads) void gn_tokens_generic_kernel(
 }
 
 // ---------------------------------------------------------------------------
+// The same in two launches: gn_stats_kernel leaves (mean, M2) of every slice of every unit in the
+// scratch, gn_tokens_apply_kernel transposes 64 x 64 tiles (tile_transpose.h) and normalises them on
+// the way.  The second launch reads x again, from the caches.  Takes every unit that is a whole number of
+// vectors, whatever its rows are: fp16 batch 2, 1280 channels at 18 x 14 27.2 -> 5.8 us, at 9 x 7 7.9 -> 5.3, at
+// 22 x 18 44.1 -> 6.4 (before: one workgroup per unit, three passes in single elements).
+// ---------------------------------------------------------------------------
+constexpr int kStatsThreads = 256;
+constexpr int kStatsUnroll = 4;  // vectors per lane in flight
+
+struct GnStatsParams {
+    uint32_t vec_per_unit;
+    uint32_t vec_per_slice;
+    FastDiv slices;  // per unit, at most kGnStatSlices
+};
+
+// (mean, M2) of one slice per workgroup.  Bound by the read of x.  Plain loads: the next launch wants
+// the lines in the caches.
+template <typename T>
+__global__ __launch_bounds__(kStatsThreads) void gn_stats_kernel(const T *__restrict__ x, float2 *__restrict__ partials,
+                                                                 GnStatsParams p) {
+    constexpr int EPV = Store<T>::EPV;
+    __shared__ float red_a[kStatsThreads / kWave], red_b[kStatsThreads / kWave], red_c[kStatsThreads / kWave];
+    const uint32_t unit = fast_div(blockIdx.x, p.slices);
+    const uint32_t slice = blockIdx.x - unit * p.slices.d;
+    const uint32_t begin = slice * p.vec_per_slice;
+    const uint32_t n = min(p.vec_per_unit, begin + p.vec_per_slice) - begin;
+    const u32x4 *in = reinterpret_cast<const u32x4 *>(x) + (size_t)unit * p.vec_per_unit + begin;
+    // every vector of the slice that is this lane's, kStatsUnroll requested at a time; what lies past
+    // the end re-reads the last vector and counts as `past`
+    auto for_each = [&](const u32x4 &past, auto use) {
+        for (uint32_t base = threadIdx.x; base < n; base += kStatsThreads * kStatsUnroll) {
+            u32x4 raw[kStatsUnroll];
+#pragma unroll
+            for (int u = 0; u < kStatsUnroll; u++) raw[u] = in[min(base + u * kStatsThreads, n - 1)];
+#pragma unroll
+            for (int u = 0; u < kStatsUnroll; u++) use(base + u * kStatsThreads < n ? raw[u] : past);
+        }
+    };
+    float s[2] = {0.0f, 0.0f}, q[2] = {0.0f, 0.0f};
+    for_each(u32x4{0, 0, 0, 0}, [&](const u32x4 &v) { Moments<T>::add(v, s, q); });
+    const uint32_t lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    auto total = [&](float v, float *slots) {
+        const float w = wave_sum(v);
+        if (lane == 0) slots[wave] = w;
+        __syncthreads();
+        float t = 0.0f;
+#pragma unroll
+        for (int i = 0; i < kStatsThreads / kWave; i++) t += slots[i];
+        return t;
+    };
+    const float sum_x = total(s[0] + s[1], red_a);
+    const float sum_xx = total(q[0] + q[1], red_b);
+    const float mean = sum_x / (float)(n * EPV);
+    float m2 = sum_xx - sum_x * mean;
+    // as in gn_slice_stats: when the mean is large against the spread, a second pass about the mean
+    if (!(sum_x * mean <= kGnFastMoments * m2)) {  // uniform over the workgroup
+        float c = 0.0f;
+        for (uint32_t i = threadIdx.x; i < n; i += kStatsThreads) {
+            float f[EPV];
+            Store<T>::unpack(in[i], f);
+#pragma unroll
+            for (int e = 0; e < EPV; e++) {
+                const float d = f[e] - mean;
+                c = fmaf(d, d, c);
+            }
+        }
+        m2 = total(c, red_c);
+    }
+    if (threadIdx.x == 0) partials[(size_t)unit * kGnStatSlices + slice] = make_float2(mean, m2);
+}
+
+struct GnApplyParams {
+    GnStatsParams stats;
+    FastDiv ch_per_group;
+    uint32_t groups, channels, hw;
+    float eps, inv_count;
+};
+
+// JFAST, RAGGED: as in permute_021_words_kernel.
+template <typename T, bool JFAST, bool RAGGED>
+__global__ __launch_bounds__(kTileThreads) void gn_tokens_apply_kernel(
+    const T *__restrict__ x, T *__restrict__ y, const float *__restrict__ gamma, const float *__restrict__ beta,
+    const float2 *__restrict__ partials, GnApplyParams p) {
+    constexpr int ES = (int)sizeof(T), EPV = Store<T>::EPV;
+    constexpr uint32_t kTeam = kTileThreads / kTile;  // lanes that merge one channel's statistics
+    __shared__ u32x4 tile4[tile_lds_words<ES>()];
+    __shared__ float4 affine[kTile];  // (mean, rstd * gamma, beta) of the tile's channels
+    const uint32_t k0 = (JFAST ? blockIdx.y : blockIdx.x) * kTile, j0 = (JFAST ? blockIdx.x : blockIdx.y) * kTile;
+    const size_t plane = (size_t)blockIdx.z * p.channels * p.hw;
+    // Chan's formula over the unit's slices, by the four lanes of a channel
+    auto ready = [&]() {
+        const uint32_t j = threadIdx.x / kTeam, lane = threadIdx.x % kTeam;
+        const uint32_t c = min(j0 + j, p.channels - 1);
+        const float g = gamma[c], b = beta[c];
+        const float2 *of_unit = partials + (size_t)(blockIdx.z * p.groups + fast_div(c, p.ch_per_group)) * kGnStatSlices;
+        float n_l[kGnStatSlices / kTeam];
+        float2 part[kGnStatSlices / kTeam];
+        float weighted = 0.0f;
+#pragma unroll
+        for (uint32_t i = 0; i < kGnStatSlices / kTeam; i++) {
+            const uint32_t l = lane + i * kTeam;
+            const bool have = l < p.stats.slices.d;
+            part[i] = of_unit[have ? l : 0];
+            const uint32_t begin = l * p.stats.vec_per_slice;
+            n_l[i] = have ? (float)((min(p.stats.vec_per_unit, begin + p.stats.vec_per_slice) - begin) * EPV) : 0.0f;
+            weighted = have ? fmaf(part[i].x, n_l[i], weighted) : weighted;
+        }
+        const float mean = team_sum<kTeam>(weighted) * p.inv_count;
+        float m2 = 0.0f;
+#pragma unroll
+        for (uint32_t i = 0; i < kGnStatSlices / kTeam; i++) {
+            const float d = part[i].x - mean;
+            if (lane + i * kTeam < p.stats.slices.d) m2 += fmaf(n_l[i] * d, d, part[i].y);
+        }
+        const float rstd = __builtin_amdgcn_rsqf(team_sum<kTeam>(m2) * p.inv_count + p.eps);
+        if (lane == 0) affine[j] = make_float4(mean, rstd * g, b, 0.0f);
+        __syncthreads();
+    };
+    auto normalise = [&](uint32_t row, const u32x4 &v) {
+        const float4 a = affine[row];
+        float f[EPV];
+        Store<T>::unpack(v, f);
+#pragma unroll
+        for (int e = 0; e < EPV; e++) f[e] = fmaf(f[e] - a.x, a.y, a.z);
+        return Store<T>::pack(f);
+    };
+    transpose_tile<ES, RAGGED>(reinterpret_cast<const char *>(x + plane), reinterpret_cast<char *>(y + plane), p.channels,
+                               p.hw, j0, k0, tile4, ready, normalise);
+}
+
+// ---------------------------------------------------------------------------
 // Host: launches (the plan comes from gn_plan.hip)
 // ---------------------------------------------------------------------------
 // log2 of the distance between the block ids of a unit's writers: the XCD count when the
@@ -859,7 +992,7 @@ int gn_dispatch(const void *xv, const void *chunkv, void *yv, const float *gamma
     p.part_vecs = (uint32_t)((((p.vec_per_unit + d.writers - 1) / d.writers + kWave - 1) / kWave) * kWave);
     p.xcd_shift = gn_xcd_shift(chip_info(), shared, units);
 
-    GnScratch sc{nullptr, nullptr, nullptr, nullptr, nullptr, 0};
+    GnScratch sc{};
     if (fixed != nullptr) {
         sc = *fixed;
     } else if (split > 1) {
@@ -893,6 +1026,72 @@ void gn_tokens_launch(bool shared, uint32_t blocks, uint32_t threads, size_t lds
     }
 }
 
+// Where the one-launch kernel can run, two launches (1.5 - 2 us more for the smallest tensors) pay when
+//   - its stores are short runs (cpg elements, at most 40 bytes, that must meet in the L2) and its units
+//     are long enough to be cut (us, before and now: 320 channels at 64 x 64 fp16 batch 2 8.08 -> 7.48, 16
+//     35.7 -> 23.6; 640 at 40 x 40 batch 8 12.7 -> 11.4; at 32 x 32 the one launch keeps 9.2 against 9.8), or
+//     divide so badly that it gets less than half a workgroup per CU (320 at 40 x 40 batch 2 7.41 -> 6.13);
+//   - the tensor is large, so that LDS and registers leave it too few workgroups in flight (fp16 640 at
+//     32 x 32 batch 32 27.5 -> 23.4, fp32 320 at 64 x 64 batch 16 61.3 -> 42.7; a copy takes 15.7 and 29; below
+//     24 MiB the one launch wins, fp32 640 at 32 x 32 batch 8 12.6 against 13.4), except where rows are no
+//     whole number of lines, which tiles of 64 positions then share (fp16 640 at 36 x 28 batch 32 23.4
+//     against 30.0).
+inline bool gn_tokens_prefers_two(const Chip &chip, size_t elt, size_t unit_size, size_t units, size_t cpg, size_t hw,
+                                  size_t blocks) {
+    if (cpg * elt <= 40 && (unit_size > 20480 || (unit_size >= 8192 && blocks * 2 < chip.cus))) return true;
+    return units * unit_size * elt >= (size_t)24 << 20 && hw * elt % 128 == 0;
+}
+
+// The two launches; false where their preconditions do not hold (nothing has been launched then).
+// The launches of one stream share its partials: the lock keeps another thread's pair from coming between.
+template <typename T>
+bool gn_tokens_two_launches(const T *x, T *y, const float *gamma, const float *beta, size_t batch, size_t channels,
+                            size_t hw, size_t groups, float eps, hipStream_t stream, int *status) {
+    constexpr size_t EPV = Store<T>::EPV;
+    const size_t cpg = channels / groups, unit_size = cpg * hw, units = batch * groups;
+    const dim3 tiles((uint32_t)((hw + kTile - 1) / kTile), (uint32_t)((channels + kTile - 1) / kTile), (uint32_t)batch);
+    if (!aligned16(x) || unit_size % EPV != 0 || units > kGnMaxUnits || hw > 0x7FFFFFFFull || channels > 0x7FFFFFFFull ||
+        (tiles.x > 65535 && tiles.y > 65535))
+        return false;
+    GnScratch sc;
+    bool capturing = false;
+    const hipError_t err = get_scratch(stream, &sc, &capturing);
+    if (capturing) return false;
+    if (err != hipSuccess) {
+        *status = (int)err;
+        return true;
+    }
+    GnApplyParams p;
+    p.stats.vec_per_unit = (uint32_t)(unit_size / EPV);
+    const Chip chip = chip_info();
+    // slices of at most 2048 vectors, shorter (two per lane at least) while the chip has less than two
+    // workgroups per CU
+    uint32_t slices = 1;
+    while (slices < kGnStatSlices && ((units * slices < 2 * (size_t)chip.cus && p.stats.vec_per_unit >= slices * 2 * kStatsThreads) ||
+                                      p.stats.vec_per_unit > slices * 2048))
+        slices *= 2;
+    p.stats.vec_per_slice = (p.stats.vec_per_unit + slices - 1) / slices;
+    slices = (p.stats.vec_per_unit + p.stats.vec_per_slice - 1) / p.stats.vec_per_slice;  // (no empty slice)
+    p.stats.slices = make_fast_div(slices);
+    p.ch_per_group = make_fast_div((uint32_t)cpg);
+    p.groups = (uint32_t)groups;
+    p.channels = (uint32_t)channels;
+    p.hw = (uint32_t)hw;
+    p.eps = eps;
+    p.inv_count = 1.0f / (float)unit_size;
+    const bool ragged = channels % EPV != 0 || hw % EPV != 0 || !aligned16(y);
+    const bool jfast = (channels < hw && tiles.x <= 65535) || tiles.y > 65535;
+    auto *apply = jfast ? (ragged ? gn_tokens_apply_kernel<T, true, true> : gn_tokens_apply_kernel<T, true, false>)
+                        : (ragged ? gn_tokens_apply_kernel<T, false, true> : gn_tokens_apply_kernel<T, false, false>);
+    static std::mutex pair;
+    std::lock_guard<std::mutex> lock(pair);
+    launch((gn_stats_kernel<T>), dim3((uint32_t)(units * slices)), dim3(kStatsThreads), 0, stream, x, sc.partials, p.stats);
+    launch(apply, jfast ? dim3(tiles.y, tiles.x, tiles.z) : tiles, dim3(kTileThreads), 0, stream, x, y, gamma, beta,
+           sc.partials, p);
+    *status = launch_status();
+    return true;
+}
+
 }  // namespace
 
 template <typename T>
@@ -908,7 +1107,10 @@ int gn_tokens_dispatch(const void *xv, void *yv, const float *gamma, const float
     const size_t units = batch * groups;
     if (units == 0 || unit_size == 0) return MSD_OK;
     if (units > 0x7FFFFFFFull || unit_size > 0x7FFFFFFFull) return MSD_ERR_INVALID_VALUE;
+    // what the one-launch kernel below does not take: the two launches, or the scalar kernel
     auto generic = [&]() {
+        int status = MSD_OK;
+        if (gn_tokens_two_launches<T>(x, y, gamma, beta, batch, channels, hw, groups, eps, stream, &status)) return status;
         launch((gn_tokens_generic_kernel<T>), dim3((uint32_t)units), dim3(kGenericThreads), 0,
                            stream, x, y, gamma, beta, (uint32_t)unit_size, (uint32_t)hw, (uint32_t)groups,
                            (uint32_t)cpg, eps);
@@ -1004,12 +1206,16 @@ int gn_tokens_dispatch(const void *xv, void *yv, const float *gamma, const float
                                                  true, true)
                                 : gn_threads_for(chip, sizeof(T), (uint32_t)nvec, split, units * split, kMaxK, false, false);
     if (pl.k == 0) return generic();
-    GnScratch sc{nullptr, nullptr, nullptr, nullptr, nullptr, 0};
+    const uint32_t blocks = (uint32_t)(units * (shared ? writers : split));
+    if (tune_split == 0 && tune_writers == 0 && gn_tokens_prefers_two(chip, sizeof(T), unit_size, units, cpg, hw, blocks)) {
+        int status = MSD_OK;
+        if (gn_tokens_two_launches<T>(x, y, gamma, beta, batch, channels, hw, groups, eps, stream, &status)) return status;
+    }
+    GnScratch sc{};
     if (!shared && split > 1) {
         const hipError_t err = get_scratch(stream, &sc);
         if (err != hipSuccess) return (int)err;
     }
-    const uint32_t blocks = (uint32_t)(units * (shared ? writers : split));
     const uint32_t threads = pl.threads;
     switch (pl.k) {
         case 1: gn_tokens_launch<T, 1>(shared, blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q); break;

@@ -46,6 +46,7 @@ inline int launch_status() {
 // ---- GroupNorm scratch: what workgroups sharing one (sample, group) exchange ----
 constexpr uint32_t kGnMaxSplit = 64;    // workgroups per unit (one wavefront reads all slots)
 constexpr uint32_t kGnMaxUnits = 8192;  // units that own scratch slots; larger launches never split
+constexpr uint32_t kGnStatSlices = 16;  // slices per unit of the token-major norm's statistics launch
 
 // ---- what the GroupNorm register kernels are built for (kernels: groupnorm.hip, plan: gn_plan.hip) ----
 constexpr int kGnMaxThreads = 1024;
@@ -61,11 +62,13 @@ struct GnScratch {
     uint32_t *epoch;                // [kGnMaxUnits] launches completed on this unit
     uint32_t *done;                 // [kGnMaxUnits] slices finished in the running launch
     uint32_t *fallbacks;            // [1] slices that stopped waiting and computed a sibling's statistics themselves
+    float2 *partials;               // [kGnMaxUnits][kGnStatSlices] (mean, M2), written and read by one pair of launches
     uint32_t units;                 // units the arrays above have room for
 };
 
-// Per-(device, stream) scratch, created on first use (hipMalloc + hipMemset).
-hipError_t get_scratch(hipStream_t stream, GnScratch *out);
+// Per-(device, stream) scratch, created on first use (hipMalloc + hipMemset).  With `capturing`, a stream
+// that has none and is being captured, where nothing can be allocated, sets it instead.
+hipError_t get_scratch(hipStream_t stream, GnScratch *out, bool *capturing = nullptr);
 // The fixed scratch inside the code object (no allocation), shared by all streams of a device.
 hipError_t get_static_scratch(GnScratch *out);
 

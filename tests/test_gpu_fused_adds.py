@@ -193,6 +193,65 @@ def test_groupnorm_tokens_equals_norm_then_permute(msd, orc, cuda, shape, groups
 
 
 @pytest.mark.parametrize("half", [False, True], ids=["f32", "f16"])
+@pytest.mark.parametrize("mean", [0.4, 60.0], ids=["", "far-mean"])  # 60: the statistics take their second pass
+@pytest.mark.parametrize("shape,groups", [((2, 1280, 9, 7), 32),    # rows of 63: pieces that a row's end cuts
+                                          ((1, 1280, 22, 18), 32),  # several slices, the last shorter
+                                          ((3, 136, 2, 5), 17),     # one tile, 17 groups in 64 channels
+                                          ((2, 65, 8, 8), 65),      # a group per channel, a second tile of one channel
+                                          ((1, 8, 300, 300), 1),    # one unit in 16 slices
+                                          ((2, 320, 56, 48), 32)])
+def test_groupnorm_tokens_in_two_launches(msd, orc, cuda, shape, groups, mean, half):
+    """Statistics, then normalising tiles: against the oracle in 64 bits, eagerly and from a graph that was
+    recorded on a stream without scratch (which takes the kernels that need none)."""
+    import torch
+    batch, channels, hw = shape[0], shape[1], int(np.prod(shape[2:]))
+    x = orc.normal(shape, seed=sum(shape) + 5, sigma=1.5, mean=mean)
+    g, b = _affine(orc, channels, 21)
+    xin = orc.round_to_half(x) if half else x
+    ref = orc.groupnorm64(xin, g, b, groups, 1e-6, False).astype(np.float32).reshape(batch, channels, hw).transpose(0, 2, 1)
+    xd, gd, bd = _dev(xin, cuda, half), _dev(g, cuda), _dev(b, cuda)
+
+    def check(got, what):
+        (assert_close_f16 if half else assert_close_f32)(got.float().cpu().numpy(), ref, what=what)
+
+    check(msd.groupnorm_tokens(xd, gd, bd, groups, 1e-6), "gn tokens, two launches")
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    # (the kernels that need no scratch do not split units: a unit that only fits in slices is left out)
+    if hw * channels // groups <= 20480:
+        with torch.cuda.graph(graph, stream=stream):
+            recorded = msd.groupnorm_tokens(xd, gd, bd, groups, 1e-6)
+        for _ in range(3):
+            recorded.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            check(recorded, "gn tokens, recorded without scratch")
+
+
+def test_groupnorm_tokens_from_two_threads_on_one_stream(msd, orc, cuda):
+    """The two launches of a call stay together when another thread launches on the same stream."""
+    import threading
+
+    import torch
+    g, b = (_dev(t, cuda) for t in _affine(orc, 320, 22))
+    xs = [torch.empty((2, 320, 64, 64), dtype=torch.float16, device=cuda).normal_(float(i), 1.0 + i) for i in range(2)]
+    want = [msd.groupnorm_tokens(x, g, b, 32) for x in xs]
+    got = [[], []]
+
+    def work(i):
+        for _ in range(40):
+            got[i].append(msd.groupnorm_tokens(xs[i], g, b, 32))
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert all(len(got[i]) == 40 and all(torch.equal(o, want[i]) for o in got[i]) for i in range(2))
+
+
+@pytest.mark.parametrize("half", [False, True], ids=["f32", "f16"])
 @pytest.mark.parametrize("shape", [(2, 320, 4096), (2, 4096, 320), (1, 1280, 64), (3, 100, 36), (2, 7, 5),
                                    (1, 64, 64), (5, 68, 132), (1, 1, 8),
                                    # 16-byte pieces on both sides with ragged tiles, one tile, thin planes
