@@ -497,12 +497,19 @@ void softmax_block_launch(const T *x, T *y, uint32_t rows, uint32_t row_vecs, in
     uint32_t vpl = sizeof(T) == 2 ? kSmBlockMaxVpl : 2;
     auto lanes = [&]() { return (((row_vecs + vpl - 1) / vpl + kWave - 1) / kWave) * kWave; };
     while (lanes() > (uint32_t)kSmBlockMaxThreads) vpl += vpl < 4 ? 1 : 4;
-    const dim3 grid(rows), block(lanes());
-    switch (vpl) {
-        case 2: launch((softmax_block_kernel<float, 2>), grid, block, 0, stream, (const float *)x, (float *)y, row_vecs, stable); break;
-        case 3: launch((softmax_block_kernel<float, 3>), grid, block, 0, stream, (const float *)x, (float *)y, row_vecs, stable); break;
-        case 4: launch((softmax_block_kernel<float, 4>), grid, block, 0, stream, (const float *)x, (float *)y, row_vecs, stable); break;
-        default: launch((softmax_block_kernel<T, kSmBlockMaxVpl>), grid, block, 0, stream, x, y, row_vecs, stable); break;
+    const dim3 block(lanes());
+    constexpr uint32_t kMostRows = 0xFFFFFFFFu / kSmBlockMaxThreads;  // (a grid holds less than 2^32 lanes)
+    for (uint32_t done = 0; done < rows; done += kMostRows) {
+        const dim3 grid(min(rows - done, kMostRows));
+        const T *xs = x + (size_t)done * row_vecs * Store<T>::EPV;
+        T *ys = y + (size_t)done * row_vecs * Store<T>::EPV;
+        switch (vpl) {
+            case 2: launch((softmax_block_kernel<float, 2>), grid, block, 0, stream, (const float *)xs, (float *)ys, row_vecs, stable); break;
+            case 3: launch((softmax_block_kernel<float, 3>), grid, block, 0, stream, (const float *)xs, (float *)ys, row_vecs, stable); break;
+            case 4: launch((softmax_block_kernel<float, 4>), grid, block, 0, stream, (const float *)xs, (float *)ys, row_vecs, stable); break;
+            default: launch((softmax_block_kernel<T, kSmBlockMaxVpl>), grid, block, 0, stream, xs, ys, row_vecs, stable); break;
+        }
+        if (rows - done <= kMostRows) break;
     }
 }
 

@@ -995,6 +995,11 @@ int gn_dispatch(const void *xv, const void *chunkv, void *yv, const float *gamma
     GnScratch sc{};
     if (fixed != nullptr) {
         sc = *fixed;
+    } else if (split > 1 && ragged) {
+        // (the general kernel needs no scratch: it takes over on a stream that can have none)
+        bool capturing = false;
+        if (get_scratch(stream, &sc, &capturing) != hipSuccess || capturing)
+            return gn_generic<T>(silu, x, chunk, y, gamma, beta, units, unit_size, hw, groups, cpg, eps, stream);
     } else if (split > 1) {
         const hipError_t err = get_scratch(stream, &sc);
         if (err != hipSuccess) return (int)err;
@@ -1042,25 +1047,20 @@ inline bool gn_tokens_prefers_two(const Chip &chip, size_t elt, size_t unit_size
     return units * unit_size * elt >= (size_t)24 << 20 && hw * elt % 128 == 0;
 }
 
-// The two launches; false where their preconditions do not hold (nothing has been launched then).
-// The launches of one stream share its partials: the lock keeps another thread's pair from coming between.
+// The two launches; false where their preconditions do not hold or the stream can have no scratch
+// (nothing has been launched then: the other kernels take over).  The launches of one stream share its partials: the lock keeps another thread's pair from coming between.
 template <typename T>
 bool gn_tokens_two_launches(const T *x, T *y, const float *gamma, const float *beta, size_t batch, size_t channels,
                             size_t hw, size_t groups, float eps, hipStream_t stream, int *status) {
     constexpr size_t EPV = Store<T>::EPV;
     const size_t cpg = channels / groups, unit_size = cpg * hw, units = batch * groups;
     const dim3 tiles((uint32_t)((hw + kTile - 1) / kTile), (uint32_t)((channels + kTile - 1) / kTile), (uint32_t)batch);
-    if (!aligned16(x) || unit_size % EPV != 0 || units > kGnMaxUnits || hw > 0x7FFFFFFFull || channels > 0x7FFFFFFFull ||
+    if (!aligned16(x) || unit_size % EPV != 0 || units > kGnMaxUnits || hw >= 0x3FFFFFFFull || channels >= 0x3FFFFFFFull ||
         (tiles.x > 65535 && tiles.y > 65535))
         return false;
     GnScratch sc;
     bool capturing = false;
-    const hipError_t err = get_scratch(stream, &sc, &capturing);
-    if (capturing) return false;
-    if (err != hipSuccess) {
-        *status = (int)err;
-        return true;
-    }
+    if (get_scratch(stream, &sc, &capturing) != hipSuccess || capturing) return false;
     GnApplyParams p;
     p.stats.vec_per_unit = (uint32_t)(unit_size / EPV);
     const Chip chip = chip_info();

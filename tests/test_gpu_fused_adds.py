@@ -192,6 +192,25 @@ def test_groupnorm_tokens_equals_norm_then_permute(msd, orc, cuda, shape, groups
     assert msd.status() == 0
 
 
+@pytest.mark.parametrize("shape", [(2, 640, 63, 63), (1, 640, 127, 65)])  # units that are cut into slices
+def test_groupnorm_of_no_whole_vectors_is_recorded_without_scratch(msd, orc, cuda, shape):
+    """A stream that has no scratch and is being captured, where none can be made."""
+    import torch
+    x = orc.normal(shape, seed=sum(shape), sigma=1.5)
+    g, b = _affine(orc, shape[1], 31)
+    xd, gd, bd = _dev(x, cuda), _dev(g, cuda), _dev(b, cuda)
+    ref = orc.groupnorm64(x.reshape(shape[0], shape[1], -1), g, b, 32, 1e-5, True).astype(np.float32).reshape(shape)
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    assert msd.load_library().msd_release(stream.cuda_stream) == 0  # (an earlier stream may have had this handle)
+    with torch.cuda.graph(graph, stream=stream):
+        recorded = msd.groupnorm(xd, gd, bd, 32, 1e-5, True)
+    for _ in range(3):
+        recorded.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert_close_f32(recorded.cpu().numpy(), ref, what="gn ragged, recorded without scratch")
+
+
 @pytest.mark.parametrize("half", [False, True], ids=["f32", "f16"])
 @pytest.mark.parametrize("mean", [0.4, 60.0], ids=["", "far-mean"])  # 60: the statistics take their second pass
 @pytest.mark.parametrize("shape,groups", [((2, 1280, 9, 7), 32),    # rows of 63: pieces that a row's end cuts
