@@ -163,8 +163,9 @@ GnThreads gn_threads_for(const Chip &chip, size_t elt, uint32_t vecs, uint32_t s
         // workgroup, four per SIMD) - as long as short units still give every CU ten wavefronts to
         // hide latency with.  From eight workgroups per CU on, slices of cut units take the
         // smallest workgroup that holds them in at most five vectors per lane instead (eight
-        // wavefronts per SIMD).
-        if (split > 1 && blocks >= 8 * (size_t)chip.cus)
+        // wavefronts per SIMD), unless that is more than 768 lanes (slices of 4320 vectors, fp32 9 x 960 x
+        // 96 x 96: 512 lanes 108 us, 1024 112; fp16 10 x 960 x 96 x 96: 61.6 against 65.5).
+        if (split > 1 && blocks >= 8 * (size_t)chip.cus && vecs <= 5 * 768)
             for (uint32_t t = 256; t <= kGnMaxThreads && pl.threads == 0; t += kWave) {
                 const int k = k_of(t);
                 if (k != 0 && k <= 5) pl.threads = t;
@@ -252,6 +253,28 @@ uint32_t rule_split(const Chip &chip, size_t elt, size_t units, size_t vec_per_u
     return want;
 }
 
+// Slices of a launch with more workgroups than CUs that 512 lanes cannot hold (8192 vectors, or
+// exactly 10240) are cut once more.  768 and 1024 lanes with 10 and more vectors each leave a CU one workgroup:
+// all of them load, then all of them store; two of 512 lanes load and store at the same time.  us per launch, a copy
+// of the same bytes, before and now:
+//   fp32 1 x 128 x 512 x 512 50 57 -> 47     2 x 256 x 256 x 256 50 55 -> 46    2 x 128 x 512 x 512 100 111 -> 94
+//        8 x 640 x 96 x 96   73.5 -> 67.7    9 x 960 x 96 x 96 126 -> 108       8 x 320 x 96 x 96 37.3 -> 35.5
+//   fp16 1 x 128 x 512 x 512 26 28 -> 24.5   2 x 256 x 384 x 384 66 -> 57       10 x 960 x 96 x 96 70 -> 62
+// (exactly 10240, fp32 8 x 640 x 64 x 64, 28.7 against 32.4 cut; 2-byte units in halves at just two per CU,
+// 8 x 640 x 96 x 96, 36.6 against 37.9: these stay.)  At just one per CU it pays above 12288 vectors (16384, fp32
+// 1 x 256 x 256 x 256, 28.6 -> 22.9; 15360, 1 x 128 x 384 x 320, 23.4 -> 22.2; 9216, fp16 1 x 512 x 192 x 192,
+// 15.8 against 16.7).
+uint32_t shorten_slices(const Chip &chip, size_t elt, size_t units, size_t vec_per_unit, uint32_t split) {
+    constexpr size_t kHeld = 512 * kGnMaxRaggedK, kHeldExactly = 512 * kGnMaxK, kHeldAlone = 12288;
+    while (split > 1 && split < kGnMaxSplit && vec_per_unit > split * kHeld && vec_per_unit != split * kHeldExactly) {
+        const size_t blocks = units * split;
+        if (blocks < chip.cus || (blocks == chip.cus && vec_per_unit <= split * kHeldAlone)) break;
+        if (elt == 2 && split == 2 && blocks == 2 * (size_t)chip.cus) break;
+        split *= 2;
+    }
+    return split;
+}
+
 }  // namespace
 
 // What a GroupNorm launch looks like for a shape: split == 0 means the general kernel (one
@@ -334,6 +357,7 @@ GnDecision gn_decide(size_t elt, size_t batch, size_t channels, size_t hw, size_
     } else if (can_split) {
         const uint32_t want = (tuned && tuned->writers <= 1) ? tuned->split : rule_split(chip, elt, units, vec_per_unit);
         while (split < want && vec_per_unit >= (size_t)2 * split * 256) split *= 2;
+        if (!tuned) split = shorten_slices(chip, elt, units, vec_per_unit, split);
     }
 
     const size_t vec_per_slice = (vec_per_unit + split - 1) / split;

@@ -211,6 +211,26 @@ def test_groupnorm_of_no_whole_vectors_is_recorded_without_scratch(msd, orc, cud
         assert_close_f32(recorded.cpu().numpy(), ref, what="gn ragged, recorded without scratch")
 
 
+@pytest.mark.parametrize("shape,half,plan", [
+    ((1, 128, 512, 512), False, (32, 512, 16)), ((1, 128, 512, 512), True, (16, 512, 16)),  # the whole 512 lanes
+    ((1, 512, 192, 192), False, (32, 512, 10)),                                            # 4608 vectors a slice
+    ((1, 128, 320, 392), False, (16, 512, 16)),                                            # 7840: masked lanes
+    ((9, 64, 192, 384), True, (4, 512, 10)),                                               # halves, then quarters
+    ((1, 128, 384, 384), True, (8, 960, 10))])                                             # one per CU, not longer than 12288: stays
+def test_groupnorm_long_slices_are_cut_for_512_lanes(msd, orc, cuda, shape, half, plan):
+    x = orc.normal(shape, seed=sum(shape), sigma=1.5, mean=0.3)
+    g, b = _affine(orc, shape[1], 41)
+    got_plan = msd.groupnorm_plan(shape[0], shape[1], shape[2] * shape[3], 32, msd.DTYPE_F16 if half else msd.DTYPE_F32)
+    assert got_plan[:3] == plan and got_plan[3] == 1
+    xin = orc.round_to_half(x) if half else x
+    ref = orc.groupnorm64(xin, g, b, 32, 1e-6, True).astype(np.float32)
+    xd, gd, bd = _dev(xin, cuda, half), _dev(g, cuda), _dev(b, cuda)
+    apart = msd.groupnorm(xd, gd, bd, 32, 1e-6, True).float().cpu().numpy()
+    inplace = msd.groupnorm(xd, gd, bd, 32, 1e-6, True, out=xd).float().cpu().numpy()
+    (assert_close_f16 if half else assert_close_f32)(apart, ref, what="gn, long slices")
+    assert np.array_equal(apart, inplace)
+
+
 @pytest.mark.parametrize("half", [False, True], ids=["f32", "f16"])
 @pytest.mark.parametrize("mean", [0.4, 60.0], ids=["", "far-mean"])  # 60: the statistics take their second pass
 @pytest.mark.parametrize("shape,groups", [((2, 1280, 9, 7), 32),    # rows of 63: pieces that a row's end cuts
