@@ -4,6 +4,7 @@
 // of a team of lanes) and the DDIM latent update.
 #include "msd_device.h"
 #include "msd_internal.h"
+#include "tile_transpose.h"
 
 #include <cmath>
 
@@ -161,22 +162,32 @@ __global__ __launch_bounds__(kLinThreads) void linear_rows_generic_kernel(
 constexpr int kSmThreads = 256;
 constexpr float kNegInf = -__builtin_huge_valf();
 
-template <typename T, int VPL, int TL>
-__global__ __launch_bounds__(kSmThreads) void softmax_team_kernel(const T *x, T *y, uint32_t rows,
-                                                                  uint32_t row_vecs, int stable) {
-    constexpr int EPV = Store<T>::EPV;
+// RAGGED: rows that are no whole number of vectors or start at any element (the 18 x 14 = 252 positions of a
+// deeper UNet level): the last piece of a row is cut.Bound
+// like the others by one read and one write, which element by element were eight loads and stores a lane
+// (and three passes beyond 512 columns).  fp16, us, before and now: 16128 x 252 6.63 -> 4.66, 32256 x 252
+// 10.9 -> 7.1, 65536 x 140 17.9 -> 10.2, 4000 x 1023 9.5 -> 5.2; 16128 x 256, whole vectors, takes 4.1.
+template <typename T, int VPL, int TL, bool RAGGED>
+__global__ __launch_bounds__(kSmThreads) void softmax_team_kernel(const T *x, T *y, uint32_t rows, uint32_t cols,
+                                                                  int stable) {
+    constexpr int EPV = Store<T>::EPV, ES = (int)sizeof(T);
     constexpr int RPW = kWave / TL;
     const uint32_t lane = threadIdx.x & (kWave - 1);
     const uint32_t wave = blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave;
     const uint32_t row = wave * RPW + lane / TL;
     const uint32_t j = lane % TL;
     const bool live = row < rows;
-    const size_t row_base = (size_t)min(row, rows - 1) * row_vecs;
-    const u32x4 *in = reinterpret_cast<const u32x4 *>(x) + row_base;
-    u32x4 *out = reinterpret_cast<u32x4 *>(y) + row_base;
+    const uint32_t row_vecs = RAGGED ? (cols + EPV - 1) / EPV : cols / EPV;
+    const size_t row_base = (size_t)min(row, rows - 1) * cols * ES;
+    const char *in = reinterpret_cast<const char *>(x) + row_base;
+    char *out = reinterpret_cast<char *>(y) + row_base;
+    auto left = [&](uint32_t v) { return cols - v * EPV; };  // elements of the row from vector v on
     u32x4 raw[VPL];
 #pragma unroll
-    for (int v = 0; v < VPL; v++) raw[v] = load_stream(in + min(v * TL + j, row_vecs - 1));
+    for (int v = 0; v < VPL; v++) {
+        const uint32_t at = min(v * TL + j, row_vecs - 1);
+        raw[v] = tile_load<ES, RAGGED>(in + (size_t)at * 16, left(at));
+    }
     float f[VPL][EPV];
     float mx = kNegInf;
 #pragma unroll
@@ -185,7 +196,7 @@ __global__ __launch_bounds__(kSmThreads) void softmax_team_kernel(const T *x, T 
         const bool have = v * TL + j < row_vecs;
 #pragma unroll
         for (int e = 0; e < EPV; e++) {
-            f[v][e] = have ? f[v][e] : kNegInf;  // padding: exp gives 0
+            f[v][e] = (RAGGED ? (v * TL + j) * EPV + e < cols : have) ? f[v][e] : kNegInf;  // padding: exp gives 0
             mx = fmaxf(mx, f[v][e]);
         }
     }
@@ -209,7 +220,8 @@ __global__ __launch_bounds__(kSmThreads) void softmax_team_kernel(const T *x, T 
     for (int v = 0; v < VPL; v++) {
 #pragma unroll
         for (int e = 0; e < EPV; e++) f[v][e] *= inv;
-        if (live && v * TL + j < row_vecs) store_stream(out + v * TL + j, Store<T>::pack(f[v]));
+        const uint32_t at = v * TL + j;
+        if (live && at < row_vecs) tile_store<ES, RAGGED>(out + (size_t)at * 16, left(at), Store<T>::pack(f[v]));
     }
 }
 
@@ -477,15 +489,14 @@ void linear_launch(const T *x, const T *w, const float *bias, T *y, uint32_t m, 
                            k / EPV, act_in, act_out);
 }
 
-template <typename T, int VPL, int TL>
-void softmax_team_launch(const T *x, T *y, uint32_t rows, uint32_t row_vecs, int stable,
-                         hipStream_t stream) {
+template <typename T, int VPL, int TL, bool RAGGED>
+void softmax_team_launch(const T *x, T *y, uint32_t rows, uint32_t cols, int stable, hipStream_t stream) {
     // long rows (a wavefront per row, 8 or 16 vectors per lane) run as single-wavefront
     // workgroups: 3 % faster at 65536 x 4096; the shorter ones keep 256 lanes
     constexpr uint32_t threads = (TL == kWave && VPL >= 8) ? kWave : kSmThreads;
     constexpr uint32_t rows_per_block = (threads / kWave) * (kWave / TL);
-    launch((softmax_team_kernel<T, VPL, TL>), dim3((rows + rows_per_block - 1) / rows_per_block),
-                       dim3(threads), 0, stream, x, y, rows, row_vecs, stable);
+    launch((softmax_team_kernel<T, VPL, TL, RAGGED>), dim3((rows + rows_per_block - 1) / rows_per_block),
+                       dim3(threads), 0, stream, x, y, rows, cols, stable);
 }
 
 template <typename T>
@@ -642,15 +653,15 @@ int softmax_dispatch(const void *xv, void *yv, size_t rows, size_t cols, int sta
         // (measured against two or four vectors per lane on smaller teams at 4 ... 32 vectors per
         // row, 2048 ... 524288 rows of fp16: never slower, 25-vector rows 71 against 109 us, 4-vector
         // rows 12.9 against 17.1, 32-vector rows 2.4 against 2.7 us at 2048 rows)
-        if (rv <= 4) softmax_team_launch<T, 1, 4>(x, y, r, rv, stable, stream);
-        else if (rv <= 8) softmax_team_launch<T, 1, 8>(x, y, r, rv, stable, stream);
-        else if (rv <= 16) softmax_team_launch<T, 1, 16>(x, y, r, rv, stable, stream);
-        else if (rv <= 32) softmax_team_launch<T, 1, 32>(x, y, r, rv, stable, stream);
-        else if (rv <= 64) softmax_team_launch<T, 1, 64>(x, y, r, rv, stable, stream);
-        else if (rv <= 128) softmax_team_launch<T, 2, 64>(x, y, r, rv, stable, stream);
-        else if (rv <= 256) softmax_team_launch<T, 4, 64>(x, y, r, rv, stable, stream);
-        else if (rv <= 512) softmax_team_launch<T, 8, 64>(x, y, r, rv, stable, stream);
-        else if (rv <= 1024) softmax_team_launch<T, 16, 64>(x, y, r, rv, stable, stream);
+        if (rv <= 4) softmax_team_launch<T, 1, 4, false>(x, y, r, c, stable, stream);
+        else if (rv <= 8) softmax_team_launch<T, 1, 8, false>(x, y, r, c, stable, stream);
+        else if (rv <= 16) softmax_team_launch<T, 1, 16, false>(x, y, r, c, stable, stream);
+        else if (rv <= 32) softmax_team_launch<T, 1, 32, false>(x, y, r, c, stable, stream);
+        else if (rv <= 64) softmax_team_launch<T, 1, 64, false>(x, y, r, c, stable, stream);
+        else if (rv <= 128) softmax_team_launch<T, 2, 64, false>(x, y, r, c, stable, stream);
+        else if (rv <= 256) softmax_team_launch<T, 4, 64, false>(x, y, r, c, stable, stream);
+        else if (rv <= 512) softmax_team_launch<T, 8, 64, false>(x, y, r, c, stable, stream);
+        else if (rv <= 1024) softmax_team_launch<T, 16, 64, false>(x, y, r, c, stable, stream);
         else softmax_block_launch<T>(x, y, r, rv, stable, stream);
         return launch_status();
     }
@@ -689,10 +700,13 @@ int softmax_dispatch(const void *xv, void *yv, size_t rows, size_t cols, int sta
     }
     const uint32_t r_left = (uint32_t)rows;
     const dim3 grid((uint32_t)((rows + waves_per_block - 1) / waves_per_block));
-    if (cols <= 2 * kWave)
-        launch((softmax_short_kernel<T, 2>), grid, dim3(kSmThreads), 0, stream, x, y, r_left, c, stable);
-    else if (cols <= 8 * kWave)
-        launch((softmax_short_kernel<T, 8>), grid, dim3(kSmThreads), 0, stream, x, y, r_left, c, stable);
+    const size_t pieces = (cols + EPV - 1) / EPV;
+    if (cols <= 2 * kWave) launch((softmax_short_kernel<T, 2>), grid, dim3(kSmThreads), 0, stream, x, y, r_left, c, stable);
+    else if (pieces <= 32) softmax_team_launch<T, 1, 32, true>(x, y, r_left, c, stable, stream);
+    else if (pieces <= 64) softmax_team_launch<T, 1, 64, true>(x, y, r_left, c, stable, stream);
+    else if (pieces <= 128) softmax_team_launch<T, 2, 64, true>(x, y, r_left, c, stable, stream);
+    else if (pieces <= 256) softmax_team_launch<T, 4, 64, true>(x, y, r_left, c, stable, stream);
+    else if (pieces <= 512) softmax_team_launch<T, 8, 64, true>(x, y, r_left, c, stable, stream);
     else
         launch((softmax_generic_kernel<T>), grid, dim3(kSmThreads), 0, stream, x, y, r_left, c, stable);
     return launch_status();

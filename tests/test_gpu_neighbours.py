@@ -232,6 +232,17 @@ def test_softmax_edge_shapes(msd, orc, cuda, rows, cols):
 
 
 @pytest.mark.parametrize("cols,half", [
+    (129, True), (130, True), (252, True), (255, True), (257, True), (260, True), (324, True), (511, True), (513, True),
+    (1023, True), (1026, True), (2044, True), (4095, True), (4097, True),
+    (129, False), (130, False), (255, False), (257, False), (514, False), (1023, False), (2047, False), (2049, False)])
+def test_softmax_rows_of_no_whole_vectors(msd, orc, cuda, cols, half):
+    """Longer than the text scores, with every remainder of a vector around the steps of vectors per lane, up to
+    the first row that goes to the kernel for any length."""
+    for stable in (0, 1):
+        _softmax_case(msd, orc, cuda, 11, cols, 7300 + cols + stable, half, stable, sigma=1.5, inplace=bool(stable))
+
+
+@pytest.mark.parametrize("cols,half", [
     (8200, True), (9216, True), (12288, True), (65536, True), (65544, True),       # 192, 192, 192, 1024 lanes; too long
     (4100, False), (8192, False), (8196, False), (12292, False), (16388, False), (32768, False), (32772, False)])
 def test_softmax_rows_of_a_whole_workgroup(msd, orc, cuda, cols, half):
