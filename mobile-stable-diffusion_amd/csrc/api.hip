@@ -1,7 +1,6 @@
 // C ABI of libmsd_hip.so (declared in include/msd_hip.h): argument checks, dtype
 // dispatch and the per-(device, stream) GroupNorm scratch.
 #include <cmath>
-#include <mutex>
 #include <unordered_map>
 
 #include <hip/hip_fp16.h>
@@ -91,6 +90,14 @@ hipError_t get_scratch(hipStream_t stream, GnScratch *out, bool *capturing) {
     g_scratch.emplace(key, s);
     *out = s;
     return hipSuccess;
+}
+
+// A fixed set of locks, chosen by the scratch's address: the same one for every thread and element type
+// on a stream, almost always another one for another stream, and none that dies with its scratch.
+std::mutex &partials_lock(const GnScratch &scratch) {
+    constexpr size_t kLocks = 61;
+    static std::mutex locks[kLocks];
+    return locks[(reinterpret_cast<uintptr_t>(scratch.partials) >> 12) % kLocks];
 }
 
 // The device address of the static scratch on the current device, looked up once per device.

@@ -29,7 +29,6 @@
 // sibling's part of the input, which no workgroup overwrites before it has
 // seen every word of its unit.  The output is the same either way; a counter
 // in the scratch records how often it happened.
-#include <mutex>
 #include <type_traits>
 
 #include "msd_device.h"
@@ -1048,7 +1047,8 @@ inline bool gn_tokens_prefers_two(const Chip &chip, size_t elt, size_t unit_size
 }
 
 // The two launches; false where their preconditions do not hold or the stream can have no scratch
-// (nothing has been launched then: the other kernels take over).  The launches of one stream share its partials: the lock keeps another thread's pair from coming between.
+// (nothing has been launched then: the other kernels take over).  All launches on one stream, of either
+// element type, share its partials: the lock keeps another thread's pair from coming between.
 template <typename T>
 bool gn_tokens_two_launches(const T *x, T *y, const float *gamma, const float *beta, size_t batch, size_t channels,
                             size_t hw, size_t groups, float eps, hipStream_t stream, int *status) {
@@ -1083,8 +1083,7 @@ bool gn_tokens_two_launches(const T *x, T *y, const float *gamma, const float *b
     const bool jfast = (channels < hw && tiles.x <= 65535) || tiles.y > 65535;
     auto *apply = jfast ? (ragged ? gn_tokens_apply_kernel<T, true, true> : gn_tokens_apply_kernel<T, true, false>)
                         : (ragged ? gn_tokens_apply_kernel<T, false, true> : gn_tokens_apply_kernel<T, false, false>);
-    static std::mutex pair;
-    std::lock_guard<std::mutex> lock(pair);
+    std::lock_guard<std::mutex> lock(partials_lock(sc));
     launch((gn_stats_kernel<T>), dim3((uint32_t)(units * slices)), dim3(kStatsThreads), 0, stream, x, sc.partials, p.stats);
     launch(apply, jfast ? dim3(tiles.y, tiles.x, tiles.z) : tiles, dim3(kTileThreads), 0, stream, x, y, gamma, beta,
            sc.partials, p);

@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 #include <atomic>
+#include <mutex>
 #include <stddef.h>
 #include <stdint.h>
 #include <tuple>
@@ -69,6 +70,8 @@ struct GnScratch {
 // Per-(device, stream) scratch, created on first use (hipMalloc + hipMemset).  With `capturing`, a stream
 // that has none and is being captured, where nothing can be allocated, sets it instead.
 hipError_t get_scratch(hipStream_t stream, GnScratch *out, bool *capturing = nullptr);
+// Held while two launches that meet in the partials of `scratch` are made.
+std::mutex &partials_lock(const GnScratch &scratch);
 // The fixed scratch inside the code object (no allocation), shared by all streams of a device.
 hipError_t get_static_scratch(GnScratch *out);
 

@@ -268,18 +268,22 @@ def test_groupnorm_tokens_in_two_launches(msd, orc, cuda, shape, groups, mean, h
             check(recorded, "gn tokens, recorded without scratch")
 
 
-def test_groupnorm_tokens_from_two_threads_on_one_stream(msd, orc, cuda):
-    """The two launches of a call stay together when another thread launches on the same stream."""
+@pytest.mark.parametrize("halves", [(True, True), (True, False), (False, False)], ids=["f16", "f16-f32", "f32"])
+def test_groupnorm_tokens_from_two_threads_on_one_stream(msd, orc, cuda, halves):
+    """The two launches of a call stay together when another thread launches on the same stream, with
+    elements of its own type or of the other."""
     import threading
 
     import torch
     g, b = (_dev(t, cuda) for t in _affine(orc, 320, 22))
-    xs = [torch.empty((2, 320, 64, 64), dtype=torch.float16, device=cuda).normal_(float(i), 1.0 + i) for i in range(2)]
+    xs = [torch.empty((2, 320, 64, 64), dtype=torch.float16 if half else torch.float32, device=cuda)
+          .normal_(float(i), 1.0 + i) for i, half in enumerate(halves)]
     want = [msd.groupnorm_tokens(x, g, b, 32) for x in xs]
-    got = [[], []]
+    got, start = [[], []], threading.Barrier(2)
 
     def work(i):
-        for _ in range(40):
+        start.wait()
+        for _ in range(100):
             got[i].append(msd.groupnorm_tokens(xs[i], g, b, 32))
 
     threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
@@ -287,7 +291,7 @@ def test_groupnorm_tokens_from_two_threads_on_one_stream(msd, orc, cuda):
         t.start()
     for t in threads:
         t.join()
-    assert all(len(got[i]) == 40 and all(torch.equal(o, want[i]) for o in got[i]) for i in range(2))
+    assert all(len(got[i]) == 100 and all(torch.equal(o, want[i]) for o in got[i]) for i in range(2))
 
 
 @pytest.mark.parametrize("half", [False, True], ids=["f32", "f16"])
