@@ -48,7 +48,10 @@ const char *msd_error_string(int code);
  * stream capture.  A graph captured on a stream keeps using that stream's
  * scratch: GroupNorm launches that share scratch must not run concurrently
  * (do not replay such a graph on a second stream while the first is busy with
- * GroupNorms).  Also looks up the device address of msd_groupnorm_noalloc's fixed
+ * GroupNorms, nor two graphs captured on one stream at the same time).  Channels of no
+ * whole 16-byte vectors are recorded without it: such a GroupNorm works on whole units then,
+ * or through the general kernel, and may differ from the same call outside a capture in the
+ * last bit, as it may where no scratch can be allocated.  Also looks up the device address of msd_groupnorm_noalloc's fixed
  * scratch on the current device.  hipStreamPerThread is refused (one handle, a
  * different stream in every thread) - here and by msd_groupnorm, msd_chunk_add_groupnorm
  * and msd_groupnorm_tokens for every shape, whether or not that launch would need the
@@ -117,7 +120,8 @@ int msd_set_tuning(int knob, int value);
  * (msd_groupnorm_plan tells); the statistics are then summed in another order than for the
  * call in place, so the two results can differ in the last bit.  A given call is
  * reproducible bit for bit as long as msd_gn_fallbacks() stays 0: a workgroup that stopped
- * waiting for a sibling sums that sibling's part in another order (same accuracy).
+ * waiting for a sibling sums that sibling's part in another order (same accuracy).  (hw of no
+ * whole 16-byte vectors: inside a capture and outside it may differ, see msd_init.)
  */
 int msd_groupnorm(const void *x, void *y, const float *gamma, const float *beta,
                   size_t batch, size_t channels, size_t hw, size_t groups, float eps,
@@ -158,13 +162,27 @@ int msd_groupnorm_plan(size_t batch, size_t channels, size_t hw, size_t groups, 
  * GroupNorm whose result is stored token-major: x is [batch, channels, hw], y is
  * [batch, hw, channels], y[b, p, c] = GroupNorm(x)[b, c, p].  Replaces GroupNorm::forward
  * followed by the permute3D_0_2_1 enqueue of SpatialTransformer::forward
- * (M/nn/SpatialTransformer.cpp:127-139; K/util.cl:47-64) in one launch; equal to
- * msd_groupnorm + that permute up to the summation order of the statistics (a few float
- * ulps).  No SiLU (the reference has none there; its eps is 1e-6).  y must not overlap x.
+ * (M/nn/SpatialTransformer.cpp:127-139; K/util.cl:47-64) in one launch or, where that is
+ * faster, in two that meet in the stream's scratch; equal to msd_groupnorm + that permute up to
+ * the summation order of the statistics (a few float ulps).  No SiLU (the reference has none there;
+ * its eps is 1e-6).  y must not overlap x.  While the stream is being captured, and where it can have
+ * no scratch, two launches are not made: slower for hw of no whole 16-byte vectors, and another
+ * summation order (msd_groupnorm_tokens_workspace has neither).
  */
 int msd_groupnorm_tokens(const void *x, void *y, const float *gamma, const float *beta, size_t batch,
                          size_t channels, size_t hw, size_t groups, float eps, int dtype,
                          void *stream);
+
+/*
+ * msd_groupnorm_tokens with memory of the caller's for what its two launches exchange: inside a
+ * capture and outside it the same launches and, bit for bit, the same result.  workspace: 8-byte aligned device
+ * memory of at least MSD_TOKENS_WORKSPACE_BYTES * batch * groups bytes, apart from x and y; its contents need
+ * not be set, are left undefined, and belong to this call until it (or every replay of it) is done.
+ */
+#define MSD_TOKENS_WORKSPACE_BYTES 128
+int msd_groupnorm_tokens_workspace(const void *x, void *y, const float *gamma, const float *beta, size_t batch,
+                                   size_t channels, size_t hw, size_t groups, float eps, int dtype, void *workspace,
+                                   size_t workspace_bytes, void *stream);
 
 /*
  * dst[i, k, j] = src[i, j, k]: the permute3D_0_2_1 kernel (K/util.cl:47-64) that

@@ -21,6 +21,7 @@ TUNE_GN_SPLIT, TUNE_GN_THREADS, TUNE_LN_CHUNK, TUNE_LN_THREADS, TUNE_GEGLU_VECTO
     TUNE_SOFTMAX_ROWS, TUNE_GN_SPIN_LIMIT, TUNE_GN_WRITERS, TUNE_DEVICE_CUS, TUNE_DEVICE_XCDS, \
     TUNE_GN_PLAN_RULE_ONLY = range(12)
 ERR_SCRATCH_LIMIT = -2
+TOKENS_WORKSPACE_BYTES = 128  # per (sample, group): MSD_TOKENS_WORKSPACE_BYTES of include/msd_hip.h
 
 # every symbol include/msd_hip.h declares
 C_ABI_SYMBOLS = (
@@ -28,7 +29,7 @@ C_ABI_SYMBOLS = (
     "msd_gn_fallbacks", "msd_set_tuning", "msd_groupnorm", "msd_groupnorm_noalloc", "msd_groupnorm_plan", "msd_layernorm", "msd_geglu",
     "msd_silu", "msd_gelu", "msd_quick_gelu", "msd_timestep_embedding", "msd_ddim_timesteps",
     "msd_elemwise_add", "msd_chunkwise_add", "msd_chunk_add_groupnorm", "msd_add_layernorm", "msd_copy",
-    "msd_groupnorm_tokens", "msd_permute_0_2_1",
+    "msd_groupnorm_tokens", "msd_groupnorm_tokens_workspace", "msd_permute_0_2_1",
     "msd_linear_rows", "msd_linear_rows_grouped", "msd_softmax", "msd_alphas_cumprod", "msd_ddim_schedule", "msd_ddim_update",
 )
 ACT_NONE, ACT_SILU = 0, 1
@@ -69,6 +70,7 @@ def load_library(path=None):
     lib.msd_copy.argtypes = [vp, vp, sz, vp]
     lib.msd_permute_0_2_1.argtypes = [vp, vp, sz, sz, sz, it, vp]
     lib.msd_groupnorm_tokens.argtypes = [vp, vp, vp, vp, sz, sz, sz, sz, fl, it, vp]
+    lib.msd_groupnorm_tokens_workspace.argtypes = [vp, vp, vp, vp, sz, sz, sz, sz, fl, it, vp, sz, vp]
     lib.msd_elemwise_add.argtypes = [vp, vp, vp, sz, it, vp]
     lib.msd_chunkwise_add.argtypes = [vp, vp, vp, sz, sz, it, vp]
     lib.msd_chunk_add_groupnorm.argtypes = [vp, vp, vp, vp, vp, sz, sz, sz, sz, fl, it, it, vp]
@@ -221,9 +223,14 @@ def groupnorm_tokens(x, gamma, beta, groups, eps=1e-6):
     batch, channels, hw = _planes(x)
     xp = _dev(x)
     out = x.new_empty((batch, hw, channels))
-    check(lib.msd_groupnorm_tokens(xp, out.data_ptr(), _affine(gamma, channels, x, "gamma"),
-                                   _affine(beta, channels, x, "beta"), batch, channels, hw, groups, eps,
-                                   _dtype_code(x), _stream()))
+    args = (xp, out.data_ptr(), _affine(gamma, channels, x, "gamma"), _affine(beta, channels, x, "beta"), batch, channels,
+            hw, groups, eps, _dtype_code(x))
+    if _torch.cuda.is_current_stream_capturing():  # (the graph keeps the workspace in its pool, apart from other graphs')
+        size = TOKENS_WORKSPACE_BYTES * batch * groups
+        workspace = x.new_empty(size, dtype=_torch.uint8)
+        check(lib.msd_groupnorm_tokens_workspace(*args, workspace.data_ptr(), size, _stream()))
+    else:
+        check(lib.msd_groupnorm_tokens(*args, _stream()))
     return out
 
 

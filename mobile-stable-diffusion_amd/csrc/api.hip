@@ -57,7 +57,7 @@ char *g_static_base[kMaxDevices] = {nullptr};  // device address of `scratch`, p
 
 // Scratch is private to a (device, stream) pair: launches on one stream are ordered, so a
 // unit's slots are never shared by two launches in flight.
-hipError_t get_scratch(hipStream_t stream, GnScratch *out, bool *capturing) {
+hipError_t get_scratch(hipStream_t stream, GnScratch *out) {
     // one handle that names a different stream in every thread cannot key a per-stream scratch
     if (stream == hipStreamPerThread) return hipErrorInvalidValue;
     int device = 0;
@@ -69,11 +69,6 @@ hipError_t get_scratch(hipStream_t stream, GnScratch *out, bool *capturing) {
     if (it != g_scratch.end()) {
         *out = it->second;
         return hipSuccess;
-    }
-    if (capturing != nullptr) {
-        hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-        *capturing = hipStreamIsCapturing(stream, &status) == hipSuccess && status != hipStreamCaptureStatusNone;
-        if (*capturing) return hipSuccess;
     }
     char *base = nullptr;
     err = hipMalloc(reinterpret_cast<void **>(&base), scratch_bytes(kGnMaxUnits));
@@ -90,6 +85,12 @@ hipError_t get_scratch(hipStream_t stream, GnScratch *out, bool *capturing) {
     g_scratch.emplace(key, s);
     *out = s;
     return hipSuccess;
+}
+
+bool optional_scratch(hipStream_t stream, GnScratch *out) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(stream, &status) == hipSuccess && status == hipStreamCaptureStatusNone &&
+           get_scratch(stream, out) == hipSuccess;
 }
 
 // A fixed set of locks, chosen by the scratch's address: the same one for every thread and element type
@@ -343,9 +344,9 @@ int msd_chunk_add_groupnorm(const void *x, const void *chunk, void *y, const flo
                            dtype, nullptr, stream);
 }
 
-int msd_groupnorm_tokens(const void *x, void *y, const float *gamma, const float *beta, size_t batch,
-                         size_t channels, size_t hw, size_t groups, float eps, int dtype,
-                         void *stream) {
+static int groupnorm_tokens_entry(const void *x, void *y, const float *gamma, const float *beta, size_t batch,
+                                  size_t channels, size_t hw, size_t groups, float eps, int dtype, float2 *partials,
+                                  void *stream) {
     if (groups == 0 || channels == 0 || channels % groups != 0) return MSD_ERR_INVALID_VALUE;
     if (dtype != MSD_DTYPE_F32 && dtype != MSD_DTYPE_F16) return MSD_ERR_INVALID_VALUE;
     if (batch * hw != 0 && (!x || !y || !gamma || !beta)) return MSD_ERR_INVALID_VALUE;
@@ -357,8 +358,31 @@ int msd_groupnorm_tokens(const void *x, void *y, const float *gamma, const float
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (s == hipStreamPerThread) return MSD_ERR_INVALID_VALUE;  // as for msd_groupnorm: may need the per-stream scratch
     if (dtype == MSD_DTYPE_F32)
-        return gn_tokens_dispatch<float>(x, y, gamma, beta, batch, channels, hw, groups, eps, s);
-    return gn_tokens_dispatch<__half>(x, y, gamma, beta, batch, channels, hw, groups, eps, s);
+        return gn_tokens_dispatch<float>(x, y, gamma, beta, batch, channels, hw, groups, eps, partials, s);
+    return gn_tokens_dispatch<__half>(x, y, gamma, beta, batch, channels, hw, groups, eps, partials, s);
+}
+
+int msd_groupnorm_tokens(const void *x, void *y, const float *gamma, const float *beta, size_t batch,
+                         size_t channels, size_t hw, size_t groups, float eps, int dtype,
+                         void *stream) {
+    return groupnorm_tokens_entry(x, y, gamma, beta, batch, channels, hw, groups, eps, dtype, nullptr, stream);
+}
+
+static_assert(MSD_TOKENS_WORKSPACE_BYTES == sizeof(float2) * kGnStatSlices, "the header's figure");
+
+int msd_groupnorm_tokens_workspace(const void *x, void *y, const float *gamma, const float *beta, size_t batch,
+                                   size_t channels, size_t hw, size_t groups, float eps, int dtype, void *workspace,
+                                   size_t workspace_bytes, void *stream) {
+    size_t need, count;
+    if (__builtin_mul_overflow(batch, groups, &need) || __builtin_mul_overflow(need, (size_t)MSD_TOKENS_WORKSPACE_BYTES, &need) ||
+        __builtin_mul_overflow(batch, channels, &count) || __builtin_mul_overflow(count, hw, &count) || count > (SIZE_MAX >> 3))
+        return MSD_ERR_INVALID_VALUE;
+    if (need != 0 && (workspace == nullptr || (reinterpret_cast<uintptr_t>(workspace) & 7u) != 0 || workspace_bytes < need))
+        return MSD_ERR_INVALID_VALUE;
+    if (ranges_overlap(workspace, need, x, count * elt_bytes(dtype)) || ranges_overlap(workspace, need, y, count * elt_bytes(dtype)))
+        return MSD_ERR_INVALID_VALUE;
+    return groupnorm_tokens_entry(x, y, gamma, beta, batch, channels, hw, groups, eps, dtype,
+                                  static_cast<float2 *>(workspace), stream);
 }
 
 static int layernorm_entry(const void *x, const void *res, void *sum, void *y, const float *gamma,

@@ -968,8 +968,14 @@ int gn_dispatch(const void *xv, const void *chunkv, void *yv, const float *gamma
     const size_t bytes = units * unit_size * sizeof(T);
     const bool apart = xb + bytes <= yb || yb + bytes <= xb;
     const bool ragged = hw % EPV != 0;
-    const GnDecision d = gn_decide(sizeof(T), batch, channels, hw, groups, aligned16(x) && aligned16(y),
-                                   fixed != nullptr ? fixed->units : kGnMaxUnits, apart, true);
+    auto decide = [&](size_t max_units) {
+        return gn_decide(sizeof(T), batch, channels, hw, groups, aligned16(x) && aligned16(y), max_units, apart, true);
+    };
+    GnDecision d = decide(fixed != nullptr ? fixed->units : kGnMaxUnits);
+    GnScratch sc{};
+    // Channels of no whole vectors go without scratch where there is none to take: in whole units, or
+    // (units that no workgroup holds) through the general kernel
+    if (ragged && fixed == nullptr && d.split > 1 && !optional_scratch(stream, &sc)) d = decide(0);
     if (d.split == 0)
         return gn_generic<T>(silu, x, chunk, y, gamma, beta, units, unit_size, hw, groups, cpg, eps, stream);
 
@@ -991,15 +997,9 @@ int gn_dispatch(const void *xv, const void *chunkv, void *yv, const float *gamma
     p.part_vecs = (uint32_t)((((p.vec_per_unit + d.writers - 1) / d.writers + kWave - 1) / kWave) * kWave);
     p.xcd_shift = gn_xcd_shift(chip_info(), shared, units);
 
-    GnScratch sc{};
     if (fixed != nullptr) {
         sc = *fixed;
-    } else if (split > 1 && ragged) {
-        // (the general kernel needs no scratch: it takes over on a stream that can have none)
-        bool capturing = false;
-        if (get_scratch(stream, &sc, &capturing) != hipSuccess || capturing)
-            return gn_generic<T>(silu, x, chunk, y, gamma, beta, units, unit_size, hw, groups, cpg, eps, stream);
-    } else if (split > 1) {
+    } else if (split > 1 && !ragged) {
         const hipError_t err = get_scratch(stream, &sc);
         if (err != hipSuccess) return (int)err;
     }
@@ -1046,21 +1046,26 @@ inline bool gn_tokens_prefers_two(const Chip &chip, size_t elt, size_t unit_size
     return units * unit_size * elt >= (size_t)24 << 20 && hw * elt % 128 == 0;
 }
 
-// The two launches; false where their preconditions do not hold or the stream can have no scratch
-// (nothing has been launched then: the other kernels take over).  All launches on one stream, of either
-// element type, share its partials: the lock keeps another thread's pair from coming between.
+// The two launches; false where their preconditions do not hold or there is no memory for the partials,
+// neither the caller's nor scratch of the stream (nothing has been launched then: the other kernels take
+// over).  All launches on one stream, of either element type, share its scratch: the lock keeps another
+// thread's pair from coming between.
 template <typename T>
 bool gn_tokens_two_launches(const T *x, T *y, const float *gamma, const float *beta, size_t batch, size_t channels,
-                            size_t hw, size_t groups, float eps, hipStream_t stream, int *status) {
+                            size_t hw, size_t groups, float eps, float2 *partials, hipStream_t stream, int *status) {
     constexpr size_t EPV = Store<T>::EPV;
     const size_t cpg = channels / groups, unit_size = cpg * hw, units = batch * groups;
     const dim3 tiles((uint32_t)((hw + kTile - 1) / kTile), (uint32_t)((channels + kTile - 1) / kTile), (uint32_t)batch);
     if (!aligned16(x) || unit_size % EPV != 0 || units > kGnMaxUnits || hw >= 0x3FFFFFFFull || channels >= 0x3FFFFFFFull ||
         (tiles.x > 65535 && tiles.y > 65535))
         return false;
-    GnScratch sc;
-    bool capturing = false;
-    if (get_scratch(stream, &sc, &capturing) != hipSuccess || capturing) return false;
+    std::unique_lock<std::mutex> lock;
+    if (partials == nullptr) {
+        GnScratch sc;
+        if (!optional_scratch(stream, &sc)) return false;
+        partials = sc.partials;
+        lock = std::unique_lock<std::mutex>(partials_lock(sc));
+    }
     GnApplyParams p;
     p.stats.vec_per_unit = (uint32_t)(unit_size / EPV);
     const Chip chip = chip_info();
@@ -1083,10 +1088,9 @@ bool gn_tokens_two_launches(const T *x, T *y, const float *gamma, const float *b
     const bool jfast = (channels < hw && tiles.x <= 65535) || tiles.y > 65535;
     auto *apply = jfast ? (ragged ? gn_tokens_apply_kernel<T, true, true> : gn_tokens_apply_kernel<T, true, false>)
                         : (ragged ? gn_tokens_apply_kernel<T, false, true> : gn_tokens_apply_kernel<T, false, false>);
-    std::lock_guard<std::mutex> lock(partials_lock(sc));
-    launch((gn_stats_kernel<T>), dim3((uint32_t)(units * slices)), dim3(kStatsThreads), 0, stream, x, sc.partials, p.stats);
+    launch((gn_stats_kernel<T>), dim3((uint32_t)(units * slices)), dim3(kStatsThreads), 0, stream, x, partials, p.stats);
     launch(apply, jfast ? dim3(tiles.y, tiles.x, tiles.z) : tiles, dim3(kTileThreads), 0, stream, x, y, gamma, beta,
-           sc.partials, p);
+           partials, p);
     *status = launch_status();
     return true;
 }
@@ -1095,7 +1099,7 @@ bool gn_tokens_two_launches(const T *x, T *y, const float *gamma, const float *b
 
 template <typename T>
 int gn_tokens_dispatch(const void *xv, void *yv, const float *gamma, const float *beta, size_t batch,
-                       size_t channels, size_t hw, size_t groups, float eps, hipStream_t stream) {
+                       size_t channels, size_t hw, size_t groups, float eps, float2 *partials, hipStream_t stream) {
     constexpr int EPV = Store<T>::EPV;
     constexpr uint32_t kMaxK = sizeof(T) == 4 ? 10 : kGnMaxRaggedK;
     constexpr size_t kMaxLds = 60 * 1024;
@@ -1109,7 +1113,7 @@ int gn_tokens_dispatch(const void *xv, void *yv, const float *gamma, const float
     // what the one-launch kernel below does not take: the two launches, or the scalar kernel
     auto generic = [&]() {
         int status = MSD_OK;
-        if (gn_tokens_two_launches<T>(x, y, gamma, beta, batch, channels, hw, groups, eps, stream, &status)) return status;
+        if (gn_tokens_two_launches<T>(x, y, gamma, beta, batch, channels, hw, groups, eps, partials, stream, &status)) return status;
         launch((gn_tokens_generic_kernel<T>), dim3((uint32_t)units), dim3(kGenericThreads), 0,
                            stream, x, y, gamma, beta, (uint32_t)unit_size, (uint32_t)hw, (uint32_t)groups,
                            (uint32_t)cpg, eps);
@@ -1208,7 +1212,7 @@ int gn_tokens_dispatch(const void *xv, void *yv, const float *gamma, const float
     const uint32_t blocks = (uint32_t)(units * (shared ? writers : split));
     if (tune_split == 0 && tune_writers == 0 && gn_tokens_prefers_two(chip, sizeof(T), unit_size, units, cpg, hw, blocks)) {
         int status = MSD_OK;
-        if (gn_tokens_two_launches<T>(x, y, gamma, beta, batch, channels, hw, groups, eps, stream, &status)) return status;
+        if (gn_tokens_two_launches<T>(x, y, gamma, beta, batch, channels, hw, groups, eps, partials, stream, &status)) return status;
     }
     GnScratch sc{};
     if (!shared && split > 1) {
@@ -1232,8 +1236,8 @@ int gn_tokens_dispatch(const void *xv, void *yv, const float *gamma, const float
 }
 
 template int gn_tokens_dispatch<float>(const void *, void *, const float *, const float *, size_t, size_t,
-                                       size_t, size_t, float, hipStream_t);
+                                       size_t, size_t, float, float2 *, hipStream_t);
 template int gn_tokens_dispatch<__half>(const void *, void *, const float *, const float *, size_t, size_t,
-                                        size_t, size_t, float, hipStream_t);
+                                        size_t, size_t, float, float2 *, hipStream_t);
 
 }  // namespace msd

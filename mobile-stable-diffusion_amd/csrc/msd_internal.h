@@ -67,9 +67,11 @@ struct GnScratch {
     uint32_t units;                 // units the arrays above have room for
 };
 
-// Per-(device, stream) scratch, created on first use (hipMalloc + hipMemset).  With `capturing`, a stream
-// that has none and is being captured, where nothing can be allocated, sets it instead.
-hipError_t get_scratch(hipStream_t stream, GnScratch *out, bool *capturing = nullptr);
+// Per-(device, stream) scratch, created on first use (hipMalloc + hipMemset).
+hipError_t get_scratch(hipStream_t stream, GnScratch *out);
+// The same for a launch that can do without: false where none can be made, and while `stream` is being
+// captured, so that what is recorded shares no memory with the stream's later launches or other graphs.
+bool optional_scratch(hipStream_t stream, GnScratch *out);
 // Held while two launches that meet in the partials of `scratch` are made.
 std::mutex &partials_lock(const GnScratch &scratch);
 // The fixed scratch inside the code object (no allocation), shared by all streams of a device.
@@ -128,10 +130,11 @@ template <typename T>
 int gn_dispatch(const void *x, const void *chunk, void *y, const float *gamma, const float *beta,
                 size_t batch, size_t channels, size_t hw, size_t groups, float eps, bool silu,
                 const GnScratch *fixed, hipStream_t stream);
-// y is token-major [batch, hw, channels]; must not overlap x
+// y is token-major [batch, hw, channels]; must not overlap x.  `partials`: the caller's memory for the
+// statistics of two launches, [batch * groups][kGnStatSlices]; null: the stream's scratch
 template <typename T>
 int gn_tokens_dispatch(const void *x, void *y, const float *gamma, const float *beta, size_t batch,
-                       size_t channels, size_t hw, size_t groups, float eps, hipStream_t stream);
+                       size_t channels, size_t hw, size_t groups, float eps, float2 *partials, hipStream_t stream);
 // res / sum may be null (plain LayerNorm); otherwise sum = x + res is written and normalised
 template <typename T>
 int ln_dispatch(const void *x, const void *res, void *sum, void *y, const float *gamma,

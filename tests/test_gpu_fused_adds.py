@@ -192,7 +192,8 @@ def test_groupnorm_tokens_equals_norm_then_permute(msd, orc, cuda, shape, groups
     assert msd.status() == 0
 
 
-@pytest.mark.parametrize("shape", [(2, 640, 63, 63), (1, 640, 127, 65)])  # units that are cut into slices
+@pytest.mark.parametrize("shape", [(2, 320, 71, 70),                        # cut into slices outside a capture; whole in it
+                                   (2, 640, 63, 63), (1, 640, 127, 65)])    # longer than one workgroup holds
 def test_groupnorm_of_no_whole_vectors_is_recorded_without_scratch(msd, orc, cuda, shape):
     """A stream that has no scratch and is being captured, where none can be made."""
     import torch
@@ -240,8 +241,8 @@ def test_groupnorm_long_slices_are_cut_for_512_lanes(msd, orc, cuda, shape, half
                                           ((1, 8, 300, 300), 1),    # one unit in 16 slices
                                           ((2, 320, 56, 48), 32)])
 def test_groupnorm_tokens_in_two_launches(msd, orc, cuda, shape, groups, mean, half):
-    """Statistics, then normalising tiles: against the oracle in 64 bits, eagerly and from a graph that was
-    recorded on a stream without scratch (which takes the kernels that need none)."""
+    """Statistics, then normalising tiles: against the oracle in 64 bits, eagerly and from graphs recorded on
+    a stream without scratch, with a workspace (the same bits) and without (the kernels that need neither)."""
     import torch
     batch, channels, hw = shape[0], shape[1], int(np.prod(shape[2:]))
     x = orc.normal(shape, seed=sum(shape) + 5, sigma=1.5, mean=mean)
@@ -253,19 +254,86 @@ def test_groupnorm_tokens_in_two_launches(msd, orc, cuda, shape, groups, mean, h
     def check(got, what):
         (assert_close_f16 if half else assert_close_f32)(got.float().cpu().numpy(), ref, what=what)
 
-    check(msd.groupnorm_tokens(xd, gd, bd, groups, 1e-6), "gn tokens, two launches")
-    stream = torch.cuda.Stream()
+    eager = msd.groupnorm_tokens(xd, gd, bd, groups, 1e-6)
+    check(eager, "gn tokens, two launches")
+    stream, lib = torch.cuda.Stream(), msd.load_library()
+    assert lib.msd_release(stream.cuda_stream) == 0  # (an earlier stream may have had this handle)
     stream.wait_stream(torch.cuda.current_stream())
-    graph = torch.cuda.CUDAGraph()
     # (the kernels that need no scratch do not split units: a unit that only fits in slices is left out)
-    if hw * channels // groups <= 20480:
-        with torch.cuda.graph(graph, stream=stream):
-            recorded = msd.groupnorm_tokens(xd, gd, bd, groups, 1e-6)
-        for _ in range(3):
-            recorded.zero_()
-            graph.replay()
+    scratch_free = hw * channels // groups <= 20480
+    with_workspace, without = torch.cuda.CUDAGraph(), torch.cuda.CUDAGraph()
+    with torch.cuda.graph(with_workspace, stream=stream):
+        recorded = msd.groupnorm_tokens(xd, gd, bd, groups, 1e-6)
+    plain = torch.empty_like(recorded)
+    with torch.cuda.graph(without, stream=stream):
+        assert not scratch_free or lib.msd_groupnorm_tokens(xd.data_ptr(), plain.data_ptr(), gd.data_ptr(), bd.data_ptr(), batch, channels, hw,
+                                        groups, 1e-6, msd.DTYPE_F16 if half else msd.DTYPE_F32, stream.cuda_stream) == 0
+    for _ in range(3):
+        recorded.zero_()
+        with_workspace.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(recorded, eager)
+        if scratch_free:
+            plain.zero_()
+            without.replay()
             torch.cuda.synchronize()
-            check(recorded, "gn tokens, recorded without scratch")
+            check(plain, "gn tokens, recorded without scratch")
+
+
+def test_graphs_of_one_capture_stream_run_at_the_same_time(msd, orc, cuda):
+    """Two graphs recorded on one stream, replayed on two: token norms in two launches, and norms in place of
+    channels of no whole vectors, which outside a capture go through the stream's scratch."""
+    import torch
+    g, b = (_dev(t, cuda) for t in _affine(orc, 320, 23))
+    capture = torch.cuda.Stream()
+    graphs, inputs, wants, gots = [], [], [], []
+    for i in range(2):
+        x = torch.empty((2, 320, 64, 64), dtype=torch.float16, device=cuda).normal_(float(i), 1.0 + i)
+        z = torch.empty((2, 320, 62, 66), dtype=torch.float16, device=cuda).normal_(float(2 * i), 1.0 + i)
+        inputs.append((x, z))
+        with torch.cuda.stream(capture):
+            msd.init()
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=capture):
+            tokens = [msd.groupnorm_tokens(x, g, b, 32) for _ in range(20)]
+            inplace = [z.clone() for _ in range(20)]
+            for t in inplace:
+                msd.groupnorm(t, g, b, 32, out=t)
+        graph.replay()
+        torch.cuda.synchronize()
+        wants.append([t.clone() for t in tokens + inplace])
+        gots.append(tokens + inplace)
+        graphs.append(graph)
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    for _ in range(5):
+        for t in gots[0] + gots[1]:
+            t.zero_()
+        torch.cuda.synchronize()
+        for graph, stream in zip(graphs, streams):
+            with torch.cuda.stream(stream):
+                graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(t, w) for i in range(2) for t, w in zip(gots[i], wants[i]))
+    assert torch.equal(wants[0][0], wants[0][19]) and torch.equal(wants[0][20], wants[0][39])
+
+
+def test_groupnorm_tokens_workspace_arguments(msd, cuda):
+    import torch
+    lib = msd.load_library()
+    x, y = (torch.empty((2, 64, 16), dtype=torch.float16, device=cuda) for _ in range(2))
+    w = torch.ones(64, device=cuda)
+    ws = torch.empty(2 * 32 * msd.TOKENS_WORKSPACE_BYTES, dtype=torch.uint8, device=cuda)
+
+    def call(workspace, size, groups=32):
+        return lib.msd_groupnorm_tokens_workspace(x.data_ptr(), y.data_ptr(), w.data_ptr(), w.data_ptr(), 2, 64, 16, groups, 1e-6,
+                                                  msd.DTYPE_F16, workspace, size, None)
+
+    assert call(ws.data_ptr(), ws.numel()) == 0
+    for bad in (call(None, ws.numel()), call(ws.data_ptr(), ws.numel() - 1), call(ws.data_ptr() + 4, ws.numel()),
+                call(x.data_ptr(), ws.numel()), call(y.data_ptr(), ws.numel()), call(ws.data_ptr(), ws.numel(), 0)):
+        assert bad == 1
+    assert msd.status() == 0
 
 
 @pytest.mark.parametrize("halves", [(True, True), (True, False), (False, False)], ids=["f16", "f16-f32", "f32"])
