@@ -57,7 +57,7 @@ char *g_static_base[kMaxDevices] = {nullptr};  // device address of `scratch`, p
 
 // Scratch is private to a (device, stream) pair: launches on one stream are ordered, so a
 // unit's slots are never shared by two launches in flight.
-hipError_t get_scratch(hipStream_t stream, GnScratch *out) {
+hipError_t get_scratch(hipStream_t stream, GnScratch *out, bool clear_on_stream) {
     // one handle that names a different stream in every thread cannot key a per-stream scratch
     if (stream == hipStreamPerThread) return hipErrorInvalidValue;
     int device = 0;
@@ -73,10 +73,15 @@ hipError_t get_scratch(hipStream_t stream, GnScratch *out) {
     char *base = nullptr;
     err = hipMalloc(reinterpret_cast<void **>(&base), scratch_bytes(kGnMaxUnits));
     if (err != hipSuccess) return err;
-    err = hipMemset(base, 0, scratch_bytes(kGnMaxUnits));  // tags, epochs and counters start at zero
-    // the fill runs on the null stream: it must have finished before a launch on `stream`
-    // (which may not synchronise with the null stream) reads the scratch
-    if (err == hipSuccess) err = hipStreamSynchronize(nullptr);
+    // tags, epochs and counters start at zero
+    if (clear_on_stream) {
+        err = hipMemsetAsync(base, 0, scratch_bytes(kGnMaxUnits), stream);
+    } else {
+        err = hipMemset(base, 0, scratch_bytes(kGnMaxUnits));
+        // this fill runs on the null stream: it must have finished before a launch on `stream`
+        // (which may not synchronise with the null stream) reads the scratch
+        if (err == hipSuccess) err = hipStreamSynchronize(nullptr);
+    }
     if (err != hipSuccess) {
         (void)hipFree(base);
         return err;
@@ -88,9 +93,19 @@ hipError_t get_scratch(hipStream_t stream, GnScratch *out) {
 }
 
 bool optional_scratch(hipStream_t stream, GnScratch *out) {
+    // The caller goes on without an error, so none may stay behind as the thread's last one; and the capture
+    // of another stream is not to be spoiled: neither by the allocation (relaxed: captures are not looked
+    // at) nor by work on the null stream.
+    const bool clean = hipPeekAtLastError() == hipSuccess;
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
     hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-    return hipStreamIsCapturing(stream, &status) == hipSuccess && status == hipStreamCaptureStatusNone &&
-           get_scratch(stream, out) == hipSuccess;
+    bool ok = hipStreamIsCapturing(stream, &status) == hipSuccess && status == hipStreamCaptureStatusNone;
+    if (ok && hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess) {
+        ok = get_scratch(stream, out, true) == hipSuccess;
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
+    }
+    if (!ok && clean) (void)hipGetLastError();
+    return ok;
 }
 
 // A fixed set of locks, chosen by the scratch's address: the same one for every thread and element type

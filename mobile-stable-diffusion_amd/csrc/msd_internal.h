@@ -67,8 +67,9 @@ struct GnScratch {
     uint32_t units;                 // units the arrays above have room for
 };
 
-// Per-(device, stream) scratch, created on first use (hipMalloc + hipMemset).
-hipError_t get_scratch(hipStream_t stream, GnScratch *out);
+// Per-(device, stream) scratch, created on first use: allocated and cleared, with `clear_on_stream`
+// (only on a stream that is not being captured) in stream order instead of at once.
+hipError_t get_scratch(hipStream_t stream, GnScratch *out, bool clear_on_stream = false);
 // The same for a launch that can do without: false where none can be made, and while `stream` is being
 // captured, so that what is recorded shares no memory with the stream's later launches or other graphs.
 bool optional_scratch(hipStream_t stream, GnScratch *out);

@@ -318,6 +318,36 @@ def test_graphs_of_one_capture_stream_run_at_the_same_time(msd, orc, cuda):
     assert torch.equal(wants[0][0], wants[0][19]) and torch.equal(wants[0][20], wants[0][39])
 
 
+def test_scratch_made_while_another_stream_is_captured(msd, orc, cuda):
+    """Channels of no whole vectors on a stream that has no scratch yet, launched while another stream is being
+    captured: the results are right, the capture is whole and no HIP error is left behind."""
+    import ctypes
+
+    import torch
+    lib, hip = msd.load_library(), ctypes.CDLL("libamdhip64.so")
+    shape = (2, 320, 62, 66)
+    x = orc.round_to_half(orc.normal(shape, seed=77, sigma=1.5))
+    g, b = _affine(orc, 320, 26)
+    ref = orc.groupnorm64(x, g, b, 32, 1e-6, False).astype(np.float32).reshape(2, 320, -1)
+    xd, zd, gd, bd = _dev(x, cuda, True), _dev(x, cuda, True), _dev(g, cuda), _dev(b, cuda)
+    tokens = torch.empty((2, 62 * 66, 320), dtype=torch.float16, device=cuda)
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    assert lib.msd_release(stream.cuda_stream) == 0
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=torch.cuda.Stream()):
+        recorded = gd * 2
+        assert lib.msd_groupnorm_tokens(xd.data_ptr(), tokens.data_ptr(), gd.data_ptr(), bd.data_ptr(), 2, 320, 62 * 66, 32,
+                                        1e-6, msd.DTYPE_F16, stream.cuda_stream) == 0
+        assert lib.msd_groupnorm(zd.data_ptr(), zd.data_ptr(), gd.data_ptr(), bd.data_ptr(), 2, 320, 62 * 66, 32, 1e-6, 0,
+                                 msd.DTYPE_F16, stream.cuda_stream) == 0
+        assert hip.hipPeekAtLastError() == 0
+    graph.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(recorded, gd * 2)
+    assert_close_f16(tokens.float().cpu().numpy(), ref.transpose(0, 2, 1), what="gn tokens, capture elsewhere")
+    assert_close_f16(zd.float().cpu().numpy(), ref.reshape(shape), what="gn ragged, capture elsewhere")
+
+
 def test_groupnorm_tokens_workspace_arguments(msd, cuda):
     import torch
     lib = msd.load_library()
