@@ -149,11 +149,10 @@ int msd_groupnorm_noalloc(const void *x, void *y, const float *gamma, const floa
  * *threads lanes each, *vectors_per_lane 16-byte vectors held per lane.  *writers > 1 (then
  * *split = 1): that many workgroups per (sample, group) each load and reduce all of it and store
  * one part; such a launch is only made when y does not overlap x, so in_place != 0 asks for the
- * plan of a call with y == x.  *split = 0 (the others too) means a shape with hw not a multiple of
- * a vector: its launch is not reported (the same kernels where units are whole vectors, otherwise
- * the general one: one 256-lane workgroup per (sample, group), nothing in registers).  Host arithmetic only: needs no GPU
- * and launches nothing.  For diagnostics, tests and benchmark tables.  No counterpart in the
- * reference (its geometry is fixed, M/nn/GroupNorm.cpp:105-128).
+ * plan of a call with y == x.  *split = 0 (the others too) means the general kernel: one 256-lane
+ * workgroup per (sample, group), nothing in registers.  (hw of no whole vectors: where this says
+ * *split > 1, a call that can use no scratch, see msd_init, has another launch.)  Host arithmetic only: needs no GPU and launches nothing.  For
+ * diagnostics, tests and benchmark tables.  No counterpart in the reference (its geometry is fixed, M/nn/GroupNorm.cpp:105-128).
  */
 int msd_groupnorm_plan(size_t batch, size_t channels, size_t hw, size_t groups, int dtype, int noalloc,
                        int in_place, int *split, int *threads, int *vectors_per_lane, int *writers);

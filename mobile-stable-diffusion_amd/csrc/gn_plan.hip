@@ -282,10 +282,9 @@ uint32_t shorten_slices(const Chip &chip, size_t elt, size_t units, size_t vec_p
 // each holding its slice as `k` vectors per lane.  `elt` = bytes per element, `max_units` = units
 // the exchange scratch has room for.  `writers` > 1 (only where `may_share`: the output does
 // not overlap the input) means whole units with that many workgroups each, every one loading and
-// reducing the whole unit and storing its part of it.  `ragged_too`: also plan for channels that are
-// no whole number of vectors (gn_slice_kernel<..., RAGGED>).  Reads the tuning knobs.
+// reducing the whole unit and storing its part of it.  Reads the tuning knobs.
 GnDecision gn_decide(size_t elt, size_t batch, size_t channels, size_t hw, size_t groups, bool aligned,
-                     size_t max_units, bool may_share, bool ragged_too) {
+                     size_t max_units, bool may_share) {
     GnDecision d{0, 0, 0, 0, 1};
     const size_t epv = 16 / elt;
     const size_t cpg = channels / groups;
@@ -293,10 +292,10 @@ GnDecision gn_decide(size_t elt, size_t batch, size_t channels, size_t hw, size_
     const size_t units = batch * groups;
     // (the register kernel addresses a unit with 32-bit byte offsets)
     if (!aligned || unit_size * elt >= (1ull << 32)) return d;
-    // Channels that are no whole number of vectors (`ragged_too`): the units still are (every unit starts
-    // on a vector), and a vector touches two channels at most
+    // Channels that are no whole number of vectors (gn_slice_kernel<..., RAGGED>): the units still are (every
+    // unit starts on a vector), and a vector touches two channels at most
     const bool ragged = hw % epv != 0;
-    if (ragged && !(ragged_too && unit_size % epv == 0 && hw >= epv && unit_size <= 0x7FFFFFFFull)) return d;
+    if (ragged && !(unit_size % epv == 0 && hw >= epv && unit_size <= 0x7FFFFFFFull)) return d;
     const size_t vec_per_unit = unit_size / epv;
     const Chip chip = chip_info();
 

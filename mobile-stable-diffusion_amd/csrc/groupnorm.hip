@@ -969,7 +969,7 @@ int gn_dispatch(const void *xv, const void *chunkv, void *yv, const float *gamma
     const bool apart = xb + bytes <= yb || yb + bytes <= xb;
     const bool ragged = hw % EPV != 0;
     auto decide = [&](size_t max_units) {
-        return gn_decide(sizeof(T), batch, channels, hw, groups, aligned16(x) && aligned16(y), max_units, apart, true);
+        return gn_decide(sizeof(T), batch, channels, hw, groups, aligned16(x) && aligned16(y), max_units, apart);
     };
     GnDecision d = decide(fixed != nullptr ? fixed->units : kGnMaxUnits);
     GnScratch sc{};

@@ -107,7 +107,7 @@ struct GnDecision {
     uint32_t writers;  // workgroups per whole unit that each store a part of it (1: the usual launch)
 };
 GnDecision gn_decide(size_t elt, size_t batch, size_t channels, size_t hw, size_t groups, bool aligned,
-                     size_t max_units, bool may_share, bool ragged_too = false);
+                     size_t max_units, bool may_share);
 
 // Compute units and XCDs of the current device (gn_plan.hip; the knobs can replace them).
 struct Chip {

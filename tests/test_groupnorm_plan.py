@@ -25,7 +25,10 @@ def _check(batch, channels, hw, groups, code, noalloc=False, in_place=False):
     if split == 0:
         assert threads == 0 and k == 0 and writers == 1
         return split, threads, k, writers
-    assert hw % epv == 0 and unit * elt < 2 ** 32          # what the register kernel assumes
+    assert unit % epv == 0 and unit * elt < 2 ** 32        # what the register kernel assumes
+    ragged = hw % epv != 0
+    if ragged:                                             # a vector touches two channels at most, 32-bit division
+        assert hw >= epv and unit < 2 ** 31
     vecs = unit // epv
     assert split & (split - 1) == 0 and 1 <= split <= MAX_SPLIT
     if split > 1:
@@ -38,7 +41,7 @@ def _check(batch, channels, hw, groups, code, noalloc=False, in_place=False):
     assert (k - 1) * threads < per_slice or k == min(v for v in K_VALUES if v * threads >= per_slice)
     if k == 20:                                            # no masked code for the largest K
         assert per_slice * split == vecs and per_slice == 20 * threads
-    if k > 6:                                              # gamma / beta of the group go through LDS
+    if k > 6 or ragged:                                    # gamma / beta of the group go through LDS
         assert channels // groups <= 1024
     assert writers in (1, 2, 4, 8, 16)
     if writers > 1:                                        # whole units, kernels built up to K = 10,
@@ -140,9 +143,24 @@ def test_plans_of_the_unet_shapes_at_batch_2_and_32():
     assert _check(3, 24, 4096, 3, f16)[3] == 1    # 9 units: not in whole rows of 8, the writers would sit on different XCDs
 
 
+def test_channels_of_no_whole_vectors_get_a_plan_of_the_register_kernel():
+    """The sizes of the deeper levels of images that are no power of two, and units that only slices hold."""
+    f16, f32 = msd.DTYPE_F16, msd.DTYPE_F32
+    for batch, channels, hw, code in ((2, 1280, 63, f16), (2, 2560, 63, f16), (1, 2560, 121, f32), (16, 640, 252, f16),
+                                      (2, 640, 3969, f32), (2, 320, 4092, f16), (32, 2560, 252, f16), (1, 256, 65532, f16)):
+        apart, in_place = (_check(batch, channels, hw, 32, code, in_place=p) for p in (False, True))
+        assert apart[0] >= 1 and in_place[0] >= 1
+    assert _check(2, 640, 3969, 32, f32)[0] >= 2                # 19845 vectors: more than a workgroup holds
+    assert _check(2, 1280, 252, 32, f16)[3] > 1 and _check(2, 1280, 252, 32, f16, in_place=True)[3] == 1
+
+
 def test_shapes_the_register_kernel_cannot_take_go_to_the_general_kernel():
-    assert msd.groupnorm_plan(2, 320, 4090, 32, msd.DTYPE_F16) == (0, 0, 0, 1)   # hw not in whole vectors
-    assert msd.groupnorm_plan(2, 320, 4094, 32, msd.DTYPE_F32) == (0, 0, 0, 1)
+    assert msd.groupnorm_plan(2, 320, 4090, 32, msd.DTYPE_F16) == (0, 0, 0, 1)   # units of no whole vectors
+    assert msd.groupnorm_plan(2, 320, 4093, 32, msd.DTYPE_F32) == (0, 0, 0, 1)
+    assert msd.groupnorm_plan(2, 320, 4, 32, msd.DTYPE_F16) == (0, 0, 0, 1)        # channels shorter than a vector
+    assert msd.groupnorm_plan(1, 32 * 1100, 66, 32, msd.DTYPE_F16) == (0, 0, 0, 1)   # ragged, and too many channels for the LDS
+    assert msd.groupnorm_plan(1, 35200, 4096, 32, msd.DTYPE_F32) == (0, 0, 0, 1)
+    assert _check(2, 320, 4094, 32, msd.DTYPE_F32)[0] == 1                         # channels of no whole vectors are taken
     assert msd.groupnorm_plan(1, 32 * 1100, 32, 32, msd.DTYPE_F16)[2] <= 6         # wide groups: no LDS affine
     assert msd.groupnorm_plan(0, 320, 4096, 32, msd.DTYPE_F16) == (0, 0, 0, 1)     # nothing to do
     lib = msd.load_library()
@@ -170,7 +188,8 @@ def test_random_shapes_always_get_a_launch_that_fits(seed):
             for _ in range(1500):
                 groups = rng.choice([1, 2, 8, 32, 32, 32, 64])
                 cpg = rng.choice([1, 2, 3, 5, 10, 20, 30, 40, 60, 80, 128, 1100])
-                hw = rng.choice([8, 16, 24, 64, 72, 256, 1000, 1024, 4096, 4104, 16384, 65536, 262144])
+                hw = rng.choice([8, 16, 24, 64, 72, 256, 1000, 1024, 4096, 4104, 16384, 65536, 262144,
+                                 1, 3, 4, 5, 7, 9, 63, 99, 252, 1023, 4092, 16390, 40961, 65532])
                 batch = rng.choice([1, 2, 2, 3, 8, 16, 32, 64, 300])
                 code = rng.choice([msd.DTYPE_F16, msd.DTYPE_F32])
                 if cpg * hw > 0x7FFFFFFF or batch * groups > 0x7FFFFFFF:
