@@ -1056,7 +1056,7 @@ bool gn_tokens_two_launches(const T *x, T *y, const float *gamma, const float *b
     constexpr size_t EPV = Store<T>::EPV;
     const size_t cpg = channels / groups, unit_size = cpg * hw, units = batch * groups;
     const dim3 tiles((uint32_t)((hw + kTile - 1) / kTile), (uint32_t)((channels + kTile - 1) / kTile), (uint32_t)batch);
-    if (!aligned16(x) || unit_size % EPV != 0 || units > kGnMaxUnits || hw >= 0x3FFFFFFFull || channels >= 0x3FFFFFFFull ||
+    if (!aligned16(x) || unit_size % EPV != 0 || units > kGnMaxUnits || hw > kTileMaxSide || channels > kTileMaxSide ||
         (tiles.x > 65535 && tiles.y > 65535))
         return false;
     std::unique_lock<std::mutex> lock;

@@ -308,8 +308,7 @@ int permute_021_dispatch(const void *srcv, void *dstv, size_t isize, size_t jsiz
     const size_t epv = 16 / sizeof(T);
     const bool ragged = jsize % epv != 0 || ksize % epv != 0 || !aligned16(src) || !aligned16(dst);
     const dim3 tiles((uint32_t)((ksize + kTile - 1) / kTile), (uint32_t)((jsize + kTile - 1) / kTile), (uint32_t)isize);
-    // (a grid holds less than 2^32 lanes)
-    const bool tiled = isize <= 65535 && ksize < 0x3FFFFFFFull && jsize < 0x3FFFFFFFull && (tiles.x <= 65535 || tiles.y <= 65535);
+    const bool tiled = isize <= 65535 && ksize <= kTileMaxSide && jsize <= kTileMaxSide && (tiles.x <= 65535 || tiles.y <= 65535);
     // Output rows shorter than input rows: consecutive workgroups take the tiles of one output
     // row, so that its 128-byte pieces are written at about the same time (batch 32, 320 x 4096
     // -> 4096 x 320, fp16: 29.9 us against 32.1 with consecutive tiles along the input rows; the

@@ -17,6 +17,8 @@ namespace msd {
 
 constexpr int kTile = 64;
 constexpr int kTileThreads = 256;
+// Most positions along a side: a grid holds less than 2^32 lanes in a dimension.
+constexpr size_t kTileMaxSide = 0xFFFFFFFFull / kTileThreads * kTile;
 
 // LDS of a tile, in 16-byte words.
 template <int ES>

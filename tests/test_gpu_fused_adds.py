@@ -427,6 +427,15 @@ def test_permute_0_2_1_ragged_and_unaligned(msd, orc, cuda, shape, half):
     assert got[0] == 7.0 and got[n + 1] == 7.0
 
 
+def test_permute_0_2_1_of_a_row_beyond_the_tiles_of_a_grid(msd, cuda):
+    """The first length whose tiles of 256 lanes are 2^32 lanes, which no launch takes."""
+    import torch
+    j, k = 5, 2 ** 30 - 63
+    x = torch.randint(-2 ** 15, 2 ** 15, (1, j, k), dtype=torch.int16, device=cuda)
+    got = msd.permute_0_2_1(x.view(torch.float16)).view(torch.int16)
+    assert got.shape == (1, k, j) and all(torch.equal(got[0, :, i], x[0, i]) for i in range(j))
+
+
 def test_fused_argument_checks(msd, cuda):
     lib = msd.load_library()
     assert lib.msd_chunk_add_groupnorm(None, None, None, None, None, 1, 32, 16, 32, 1e-5, 0, 0, None) == 1
