@@ -151,7 +151,7 @@ __global__ __launch_bounds__(kStreamThreads) void add_generic_kernel(const T *a,
 // RAGGED: sizes that are no whole number of 16-byte pieces, or planes that are not 16-byte aligned
 // (the tokens of a 9 x 7 latent); unaligned 16-byte accesses, only the pieces that a row's end cuts go
 // in parts.  Against element-wise and 4-element accesses, us: fp16 32 x 63 x 1280 9.36 -> 3.37, 2 x 252 x
-// 1280 2.58 -> 2.24, fp32 4 x 99 x 1280 3.18 -> 2.65; a copy of the first takes about 3.4.
+// 1280 2.58 -> 2.24, fp32 3 x 99 x 1280 4.56 -> 3.14; a copy of the first takes about 3.4.
 // ---------------------------------------------------------------------------
 template <int ES, bool JFAST, bool RAGGED>
 __global__ __launch_bounds__(kTileThreads) void permute_021_words_kernel(const void *__restrict__ src,
@@ -308,7 +308,22 @@ int permute_021_dispatch(const void *srcv, void *dstv, size_t isize, size_t jsiz
     const size_t epv = 16 / sizeof(T);
     const bool ragged = jsize % epv != 0 || ksize % epv != 0 || !aligned16(src) || !aligned16(dst);
     const dim3 tiles((uint32_t)((ksize + kTile - 1) / kTile), (uint32_t)((jsize + kTile - 1) / kTile), (uint32_t)isize);
-    const bool tiled = isize <= 65535 && ksize <= kTileMaxSide && jsize <= kTileMaxSide && (tiles.x <= 65535 || tiles.y <= 65535);
+    // A tile costs its workgroup, its barrier and, ragged, a chain of loads for each cut piece, however little
+    // of it lies in the tensor: planes and rows that fill few of its 4096 elements, and small tensors, move
+    // faster element by element.  us, tile against elements (elements per tile):
+    //   whole pieces   fp32 400 x 4 x 1000 (250) 10.1 / 7.1     31250 x 16 x 16 (256) 27.2 / 28.7
+    //   ragged fp16    65535 x 2 x 2 (4) 30.5 / 3.0    1778 x 3 x 300 (180) 8.2 / 6.7   6275 x 17 x 15 (255) 8.8 / 6.7
+    //                  400 x 4 x 1000 (250, a cut piece is 8 bytes) 6.2 / 6.8           5000 x 5 x 64 (320) 5.6 / 6.8
+    //          fp32    5000 x 5 x 64 (320) 7.8 / 7.2   714 x 7 x 320 (448) 7.6 / 7.2, transposed 6.5 / 9.2
+    //   small  fp16    30 x 77 x 77 2.86 / 2.79, 37 of them 2.88 / 3.31   2 x 768 x 77 2.81 / 2.92, 3 of them 2.81 / 3.13
+    //          fp32    15 x 77 x 77 3.07 / 2.67, 19 of them 3.07 / 3.20   1 x 768 x 77 2.90 / 2.74, 2 of them 2.93 / 3.39
+    const size_t n = isize * jsize * ksize;
+    const size_t per_tile = jsize * ksize / (((jsize + kTile - 1) / kTile) * ((ksize + kTile - 1) / kTile));
+    const bool tile_pays = !ragged ? per_tile >= 256
+                           : sizeof(T) == 2 ? per_tile >= ((jsize | ksize) % 4 == 0 ? 240 : 300) && n >= 192 * 1024
+                                            : per_tile >= 400 && n >= 112 * 1024;
+    const bool tiled = tile_pays && isize <= 65535 && ksize <= kTileMaxSide && jsize <= kTileMaxSide &&
+                       (tiles.x <= 65535 || tiles.y <= 65535);
     // Output rows shorter than input rows: consecutive workgroups take the tiles of one output
     // row, so that its 128-byte pieces are written at about the same time (batch 32, 320 x 4096
     // -> 4096 x 320, fp16: 29.9 us against 32.1 with consecutive tiles along the input rows; the
@@ -321,7 +336,7 @@ int permute_021_dispatch(const void *srcv, void *dstv, size_t isize, size_t jsiz
         launch(kernel, jfast ? dim3(tiles.y, tiles.x, tiles.z) : tiles, dim3(kTileThreads), 0, stream, srcv, dstv,
                (uint32_t)jsize, (uint32_t)ksize);
     } else {
-        const size_t want = (isize * jsize * ksize + kStreamThreads - 1) / kStreamThreads;
+        const size_t want = (n + kStreamThreads - 1) / kStreamThreads;
         launch((permute_021_generic_kernel<T>), dim3((uint32_t)(want < 65536 ? want : 65536)),
                            dim3(kStreamThreads), 0, stream, src, dst, isize, jsize, ksize);
     }
