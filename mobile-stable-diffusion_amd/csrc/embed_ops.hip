@@ -701,8 +701,21 @@ int softmax_dispatch(const void *xv, void *yv, size_t rows, size_t cols, int sta
     const uint32_t r_left = (uint32_t)rows;
     const dim3 grid((uint32_t)((rows + waves_per_block - 1) / waves_per_block));
     const size_t pieces = (cols + EPV - 1) / EPV;
+    // Up to 512 columns, element by element or in 16-byte pieces: what the pieces save in accesses they pay in
+    // latency (a cut piece is a chain of loads, and pieces that start at any element touch more lines), so they need
+    // rows enough, and more of them the less their starts are aligned.  Over random shapes, pieces against elements:
+    // fp16 up to 256 columns and 1000 / 4000 / 8000 / 32000 rows, odd 1.14 / 1.03 / 0.93 / 0.79, even 1.09 / 0.95 /
+    // 0.86 / 0.70; fp16 beyond 256, odd and even 1.02 - 1.17 at any number of rows, multiples of four 1.04 below
+    // 8000 rows and 0.96 from there on; fp32 up to 256, odd 0.99 - 1.07, even 1.03 below 6000 rows and 0.93 above,
+    // beyond 256 1.01 - 1.14.
+    bool pieces_pay = cols > 8 * kWave;
+    if (sizeof(T) == 2)
+        pieces_pay = pieces_pay || (cols <= 256 ? rows >= (cols % 2 ? 5120u : 3072u) : cols % 4 == 0 && rows >= 8192);
+    else
+        pieces_pay = pieces_pay || (cols <= 256 && cols % 2 == 0 && rows >= 6144);
     if (cols <= 2 * kWave) launch((softmax_short_kernel<T, 2>), grid, dim3(kSmThreads), 0, stream, x, y, r_left, c, stable);
-    else if (pieces <= 32) softmax_team_launch<T, 1, 32, true>(x, y, r_left, c, stable, stream);
+    else if (!pieces_pay) launch((softmax_short_kernel<T, 8>), grid, dim3(kSmThreads), 0, stream, x, y, r_left, c, stable);
+    else if (pieces <= 32) softmax_team_launch<T, 1, EPV == 8 ? 32 : 64, true>(x, y, r_left, c, stable, stream);  // (fp32: no such row)
     else if (pieces <= 64) softmax_team_launch<T, 1, 64, true>(x, y, r_left, c, stable, stream);
     else if (pieces <= 128) softmax_team_launch<T, 2, 64, true>(x, y, r_left, c, stable, stream);
     else if (pieces <= 256) softmax_team_launch<T, 4, 64, true>(x, y, r_left, c, stable, stream);

@@ -242,6 +242,14 @@ def test_softmax_rows_of_no_whole_vectors(msd, orc, cuda, cols, half):
         _softmax_case(msd, orc, cuda, 11, cols, 7300 + cols + stable, half, stable, sigma=1.5, inplace=bool(stable))
 
 
+@pytest.mark.parametrize("rows,cols,half", [
+    (3071, 130, True), (3072, 130, True), (5119, 255, True), (5120, 255, True), (3075, 252, True), (8191, 260, True),
+    (8195, 260, True), (8197, 511, True), (6143, 130, False), (8195, 254, False), (8195, 255, False), (8195, 510, False)])
+def test_softmax_rows_of_no_whole_vectors_by_their_number(msd, orc, cuda, rows, cols, half):
+    """On both sides of the numbers of rows from which 16-byte pieces replace single elements."""
+    _softmax_case(msd, orc, cuda, rows, cols, 7500 + cols, half, rows % 2, sigma=1.5, inplace=True)
+
+
 @pytest.mark.parametrize("cols,half", [
     (8200, True), (9216, True), (12288, True), (65536, True), (65544, True),       # 192, 192, 192, 1024 lanes; too long
     (4100, False), (8192, False), (8196, False), (12292, False), (16388, False), (32768, False), (32772, False)])
