@@ -308,27 +308,28 @@ int permute_021_dispatch(const void *srcv, void *dstv, size_t isize, size_t jsiz
     const size_t epv = 16 / sizeof(T);
     const bool ragged = jsize % epv != 0 || ksize % epv != 0 || !aligned16(src) || !aligned16(dst);
     const dim3 tiles((uint32_t)((ksize + kTile - 1) / kTile), (uint32_t)((jsize + kTile - 1) / kTile), (uint32_t)isize);
-    // A tile costs its workgroup, its barrier and, ragged, a chain of loads for each cut piece, however little
-    // of it lies in the tensor: planes and rows that fill few of its 4096 elements, and small tensors, move
-    // faster element by element.  us, tile against elements (elements per tile):
-    //   whole pieces   fp32 400 x 4 x 1000 (250) 10.1 / 7.1     31250 x 16 x 16 (256) 27.2 / 28.7
-    //   ragged fp16    65535 x 2 x 2 (4) 30.5 / 3.0    1778 x 3 x 300 (180) 8.2 / 6.7   6275 x 17 x 15 (255) 8.8 / 6.7
-    //                  400 x 4 x 1000 (250, a cut piece is 8 bytes) 6.2 / 6.8           5000 x 5 x 64 (320) 5.6 / 6.8
-    //          fp32    5000 x 5 x 64 (320) 7.8 / 7.2   714 x 7 x 320 (448) 7.6 / 7.2, transposed 6.5 / 9.2
-    //   small  fp16    30 x 77 x 77 2.86 / 2.79, 37 of them 2.88 / 3.31   2 x 768 x 77 2.81 / 2.92, 3 of them 2.81 / 3.13
-    //          fp32    15 x 77 x 77 3.07 / 2.67, 19 of them 3.07 / 3.20   1 x 768 x 77 2.90 / 2.74, 2 of them 2.93 / 3.39
+    // Ragged, a tile costs its workgroup, its barrier and a chain of loads for each cut piece, however little of it
+    // lies in the tensor: planes and rows that fill few of its 4096 elements, and small tensors, move faster element
+    // by element.  us, tile against elements (elements per tile):
+    //   fp16  65535 x 2 x 2 (4) 30.5 / 3.0    1778 x 3 x 300 (180) 8.2 / 6.7    6275 x 17 x 15 (255) 8.8 / 6.7
+    //   fp32  5000 x 5 x 64 (320) 7.8 / 7.2   714 x 7 x 320 (448) 7.6 / 7.2, transposed 6.5 / 9.2   15 x 77 x 77 3.07 / 2.67
+    // (by elements per tile from 256 Ki in all, tile against elements: fp16 128 - 200 1.2, 200 - 300 0.96, 350 - 400 0.82;
+    // fp32 input rows longer than output rows 300 - 400 1.15, 400 - 450 1.03, 450 - 600 0.88, shorter 250 - 300 1.13,
+    // 300 - 350 1.03, 350 - 400 0.92.)  In pieces that nothing cuts, or only in halves (2-byte sides in multiples of
+    // four), the tile is within 5 % of the better one or ahead at every size.
     const size_t n = isize * jsize * ksize;
     const size_t per_tile = jsize * ksize / (((jsize + kTile - 1) / kTile) * ((ksize + kTile - 1) / kTile));
-    const bool tile_pays = !ragged ? per_tile >= 256
-                           : sizeof(T) == 2 ? per_tile >= ((jsize | ksize) % 4 == 0 ? 240 : 300) && n >= 192 * 1024
-                                            : per_tile >= 400 && n >= 112 * 1024;
+    const bool halves = ragged && sizeof(T) == 2 && (jsize | ksize) % 4 == 0 &&
+                        ((reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(dst)) & 7u) == 0;
+    const bool tile_pays = !ragged || halves || (per_tile >= (sizeof(T) == 2 ? 250u : jsize > ksize ? 350u : 450u) && n >= 256 * 1024);
     const bool tiled = tile_pays && isize <= 65535 && ksize <= kTileMaxSide && jsize <= kTileMaxSide &&
                        (tiles.x <= 65535 || tiles.y <= 65535);
     // Output rows shorter than input rows: consecutive workgroups take the tiles of one output
     // row, so that its 128-byte pieces are written at about the same time (batch 32, 320 x 4096
     // -> 4096 x 320, fp16: 29.9 us against 32.1 with consecutive tiles along the input rows; the
-    // copy takes 29.1; the other way round nothing changes).
-    const bool jfast = (jsize < ksize && tiles.x <= 65535) || tiles.y > 65535;
+    // copy takes 29.1; the other way round nothing changes; in halves it costs up to 15 %, 695 x 368 x 452 fp16
+    // 136 against 117, and gains 2 % at most).
+    const bool jfast = (jsize < ksize && !halves && tiles.x <= 65535) || tiles.y > 65535;
     if (tiled) {
         constexpr int ES = (int)sizeof(T);
         auto *kernel = jfast ? (ragged ? permute_021_words_kernel<ES, true, true> : permute_021_words_kernel<ES, true, false>)

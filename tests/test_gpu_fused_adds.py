@@ -409,6 +409,7 @@ def test_permute_0_2_1(msd, orc, cuda, shape, half):
 @pytest.mark.parametrize("half", [False, True], ids=["f32", "f16"])
 @pytest.mark.parametrize("shape", [(2, 63, 1280), (2, 1280, 63), (1, 65, 127), (3, 1, 9), (2, 9, 1), (1, 130, 66),
                                    (4, 63, 1280), (4, 1280, 63), (24, 65, 127), (23, 130, 66), (1, 5, 40000), (1, 40000, 7),
+                                   (33, 65, 127), (31, 130, 66),
                                    (700, 17, 17), (650, 20, 17), (3000, 3, 64)])   # tiles; planes that fill too few of them
 def test_permute_0_2_1_ragged_and_unaligned(msd, orc, cuda, shape, half):
     """Rows that start at any element and end inside a 16-byte piece, in tensors that start one
@@ -427,6 +428,25 @@ def test_permute_0_2_1_ragged_and_unaligned(msd, orc, cuda, shape, half):
     got = dst.float().cpu().numpy()
     assert np.array_equal(got[1:n + 1], orc.permute_0_2_1(x).reshape(-1))
     assert got[0] == 7.0 and got[n + 1] == 7.0
+
+
+@pytest.mark.parametrize("shape", [(3, 4, 12), (300, 12, 4), (2, 20, 36), (1, 68, 132), (2, 252, 1280), (2, 1280, 252)])
+def test_permute_0_2_1_in_halves_of_a_piece(msd, orc, cuda, shape):
+    """2-byte sides in multiples of four, and of eight in planes that start in the middle of a piece."""
+    import torch
+    for scale, offset in ((1, 0), (1, 4), (2, 4)):
+        i, j, k = shape[0], shape[1] * scale, shape[2] * scale
+        n = i * j * k
+        x = orc.round_to_half(orc.normal((i, j, k), seed=sum(shape) + scale))
+        src = torch.zeros(n + 16, dtype=torch.float16, device=cuda)
+        src[offset:n + offset] = _dev(x, cuda, True).reshape(-1)
+        dst = torch.full_like(src, 7.0)
+        assert msd.load_library().msd_permute_0_2_1(src.data_ptr() + 2 * offset, dst.data_ptr() + 2 * offset, i, j, k,
+                                                    msd.DTYPE_F16, None) == 0
+        torch.cuda.synchronize()
+        got = dst.float().cpu().numpy()
+        assert np.array_equal(got[offset:n + offset], orc.permute_0_2_1(x).reshape(-1))
+        assert (got[:offset] == 7.0).all() and (got[n + offset:] == 7.0).all()
 
 
 def test_permute_0_2_1_of_a_row_beyond_the_tiles_of_a_grid(msd, cuda):
