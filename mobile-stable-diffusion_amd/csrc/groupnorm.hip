@@ -1111,9 +1111,16 @@ int gn_tokens_dispatch(const void *xv, void *yv, const float *gamma, const float
     if (units == 0 || unit_size == 0) return MSD_OK;
     if (units > 0x7FFFFFFFull || unit_size > 0x7FFFFFFFull) return MSD_ERR_INVALID_VALUE;
     // what the one-launch kernel below does not take: the two launches, or the scalar kernel
+    // (short units of small tensors, or of planes much narrower than a tile: one short launch instead of two.  us, one
+    // and two: fp16 1 x 320 x 36 3.4 / 5.1, 64 x 2560 x 4 4.5 / 8.3, 22 x 2560 x 10 4.8 / 6.4, 8 x 960 x 28
+    // 4.3 / 5.1, 166 x 256 x 79 22.8 / 10.6, 2 x 1280 x 63 7.9 / 5.3.  Over 3100 random shapes 6 are more than 1.1
+    // times the one launch, none more than 1.2.)
     auto generic = [&]() {
         int status = MSD_OK;
-        if (gn_tokens_two_launches<T>(x, y, gamma, beta, batch, channels, hw, groups, eps, partials, stream, &status)) return status;
+        const bool pays = unit_size >= 1280 || (unit_size >= 256 && hw >= 24 && units * unit_size >= 400000);
+        if (pays &&
+            gn_tokens_two_launches<T>(x, y, gamma, beta, batch, channels, hw, groups, eps, partials, stream, &status))
+            return status;
         launch((gn_tokens_generic_kernel<T>), dim3((uint32_t)units), dim3(kGenericThreads), 0,
                            stream, x, y, gamma, beta, (uint32_t)unit_size, (uint32_t)hw, (uint32_t)groups,
                            (uint32_t)cpg, eps);

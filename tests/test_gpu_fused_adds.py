@@ -232,15 +232,32 @@ def test_groupnorm_long_slices_are_cut_for_512_lanes(msd, orc, cuda, shape, half
     assert np.array_equal(apart, inplace)
 
 
-@pytest.mark.parametrize("half", [False, True], ids=["f32", "f16"])
+def _takes_two_launches(msd, xd, gd, bd, groups):
+    """Only two launches leave anything in the workspace."""
+    import torch
+    batch, channels = xd.shape[:2]
+    workspace = torch.zeros(batch * groups * msd.TOKENS_WORKSPACE_BYTES, dtype=torch.uint8, device=xd.device)
+    out = torch.empty_like(xd)
+    assert msd.load_library().msd_groupnorm_tokens_workspace(
+        xd.data_ptr(), out.data_ptr(), gd.data_ptr(), bd.data_ptr(), batch, channels, xd.numel() // (batch * channels), groups,
+        1e-6, msd.DTYPE_F16 if xd.dtype == torch.float16 else msd.DTYPE_F32, workspace.data_ptr(), workspace.numel(),
+        torch.cuda.current_stream().cuda_stream) == 0
+    return bool(workspace.any())
+
+
 @pytest.mark.parametrize("mean", [0.4, 60.0], ids=["", "far-mean"])  # 60: the statistics take their second pass
-@pytest.mark.parametrize("shape,groups", [((2, 1280, 9, 7), 32),    # rows of 63: pieces that a row's end cuts
-                                          ((1, 1280, 22, 18), 32),  # several slices, the last shorter
-                                          ((3, 136, 2, 5), 17),     # one tile, 17 groups in 64 channels
-                                          ((2, 65, 8, 8), 65),      # a group per channel, a second tile of one channel
-                                          ((1, 8, 300, 300), 1),    # one unit in 16 slices
-                                          ((2, 320, 56, 48), 32)])
-def test_groupnorm_tokens_in_two_launches(msd, orc, cuda, shape, groups, mean, half):
+@pytest.mark.parametrize("shape,groups,half,two", [
+    ((2, 1280, 9, 7), 32, True, True), ((2, 1280, 9, 7), 32, False, True),     # rows of 63: pieces that a row's end cuts
+    ((1, 1280, 21, 19), 32, True, True), ((1, 1280, 21, 19), 32, False, True),  # several slices, the last shorter
+    ((3, 136, 7, 23), 17, True, True), ((3, 136, 7, 23), 17, False, True),     # 17 groups, a last tile of 8 channels
+    ((2, 65, 8, 161), 65, True, True), ((2, 65, 10, 129), 65, False, False),   # a group per channel; no whole vectors
+    ((1, 8, 300, 300), 1, True, True), ((1, 8, 300, 300), 1, False, True),     # one unit in 16 slices
+    ((2, 320, 56, 48), 32, True, True), ((2, 320, 56, 48), 32, False, True),   # short runs, long units
+    ((1, 2560, 34, 32), 128, True, True),                                      # ... and more channels than positions
+    ((20, 640, 2, 13), 32, False, False), ((40, 640, 2, 13), 32, False, True),  # units of 520: few of them, many
+    ((40, 640, 2, 13), 32, True, True), ((60, 640, 1, 22), 32, False, False),   # planes much narrower than a tile
+    ((16, 2560, 4, 4), 32, True, False), ((3, 136, 2, 5), 17, True, False)])   # short units
+def test_groupnorm_tokens_in_two_launches(msd, orc, cuda, shape, groups, mean, half, two):
     """Statistics, then normalising tiles: against the oracle in 64 bits, eagerly and from graphs recorded on
     a stream without scratch, with a workspace (the same bits) and without (the kernels that need neither)."""
     import torch
@@ -257,6 +274,7 @@ def test_groupnorm_tokens_in_two_launches(msd, orc, cuda, shape, groups, mean, h
     eager = msd.groupnorm_tokens(xd, gd, bd, groups, 1e-6)
     check(eager, "gn tokens, two launches")
     stream, lib = torch.cuda.Stream(), msd.load_library()
+    assert _takes_two_launches(msd, xd, gd, bd, groups) == two
     assert lib.msd_release(stream.cuda_stream) == 0  # (an earlier stream may have had this handle)
     stream.wait_stream(torch.cuda.current_stream())
     # (the kernels that need no scratch do not split units: a unit that only fits in slices is left out)
