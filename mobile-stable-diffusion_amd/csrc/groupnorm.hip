@@ -1034,16 +1034,28 @@ void gn_tokens_launch(bool shared, uint32_t blocks, uint32_t threads, size_t lds
 //   - its stores are short runs (cpg elements, at most 40 bytes, that must meet in the L2) and its units
 //     are long enough to be cut (us, before and now: 320 channels at 64 x 64 fp16 batch 2 8.08 -> 7.48, 16
 //     35.7 -> 23.6; 640 at 40 x 40 batch 8 12.7 -> 11.4; at 32 x 32 the one launch keeps 9.2 against 9.8), or
-//     divide so badly that it gets less than half a workgroup per CU (320 at 40 x 40 batch 2 7.41 -> 6.13);
+//     divide so badly that it gets less than half a workgroup per CU (320 at 40 x 40 batch 2 7.41 -> 6.13; shorter
+//     ones keep the one launch: 640 at 432 positions batch 1 3.95 against 4.89);
 //   - the tensor is large, so that LDS and registers leave it too few workgroups in flight (fp16 640 at
 //     32 x 32 batch 32 27.5 -> 23.4, fp32 320 at 64 x 64 batch 16 61.3 -> 42.7; a copy takes 15.7 and 29; below
-//     24 MiB the one launch wins, fp32 640 at 32 x 32 batch 8 12.6 against 13.4), except where rows are no
-//     whole number of lines, which tiles of 64 positions then share (fp16 640 at 36 x 28 batch 32 23.4
-//     against 30.0).
+//     24 MiB the one launch wins, fp32 640 at 32 x 32 batch 8 12.6 against 13.4).  Not where its workgroups are a
+//     whole number per CU, few enough to be in flight at once (fp16 1280 at 2560 positions batch 6, three per CU,
+//     19.3 against 24.6; fp32 2560 at 640 batch 6, 16.8 against 21.2) and cut the rows at whole 32 bytes (fp16 1920
+//     at 4032 batch 2 in parts of 504 positions 33.1, two launches 18.0), nor where rows are no whole number of
+//     lines, which tiles of 64 positions then share (fp16 640 at 36 x 28 batch 32 23.4 against 30.0).
+// Both need positions that fill the tiles (fp32 1280 at 288 positions, 4.5 tiles, batch 23 14.2 against 20.7).
+// Over 2800 random shapes of 1280 and more elements per unit what this takes is 0.955 of the one launch on average;
+// 23 are more than 1.1 times it (to 1.29: fp16 640 at 1232 batch 16 18.9 against 14.6).
 inline bool gn_tokens_prefers_two(const Chip &chip, size_t elt, size_t unit_size, size_t units, size_t cpg, size_t hw,
-                                  size_t blocks) {
-    if (cpg * elt <= 40 && (unit_size > 20480 || (unit_size >= 8192 && blocks * 2 < chip.cus))) return true;
-    return units * unit_size * elt >= (size_t)24 << 20 && hw * elt % 128 == 0;
+                                  size_t blocks, size_t part_vecs) {
+    const size_t tiled = (hw + kTile - 1) / kTile * kTile, bytes = units * unit_size * elt;
+    if (hw * 16 < tiled * 15) return false;
+    if (cpg * elt <= 40)
+        return unit_size > 20480 || (unit_size >= 12288 && blocks * 2 < chip.cus) || bytes >= (size_t)24 << 20;
+    if (bytes < (size_t)24 << 20 || hw * elt % 128 != 0) return false;
+    const size_t rounds = (blocks + chip.cus - 1) / chip.cus;
+    return rounds * 2 > 3 * elt || blocks * 100 <= rounds * chip.cus * 97 || part_vecs % 2 != 0 ||
+           (elt == 4 && unit_size > 160000);
 }
 
 // The two launches; false where their preconditions do not hold or there is no memory for the partials,
@@ -1217,7 +1229,7 @@ int gn_tokens_dispatch(const void *xv, void *yv, const float *gamma, const float
                                 : gn_threads_for(chip, sizeof(T), (uint32_t)nvec, split, units * split, kMaxK, false, false);
     if (pl.k == 0) return generic();
     const uint32_t blocks = (uint32_t)(units * (shared ? writers : split));
-    if (tune_split == 0 && tune_writers == 0 && gn_tokens_prefers_two(chip, sizeof(T), unit_size, units, cpg, hw, blocks)) {
+    if (tune_split == 0 && tune_writers == 0 && gn_tokens_prefers_two(chip, sizeof(T), unit_size, units, cpg, hw, blocks, pvs)) {
         int status = MSD_OK;
         if (gn_tokens_two_launches<T>(x, y, gamma, beta, batch, channels, hw, groups, eps, partials, stream, &status)) return status;
     }

@@ -298,6 +298,23 @@ def test_groupnorm_tokens_in_two_launches(msd, orc, cuda, shape, groups, mean, h
             check(plain, "gn tokens, recorded without scratch")
 
 
+@pytest.mark.parametrize("shape,half,two", [
+    ((39, 1280, 16, 16), True, True), ((38, 1280, 16, 16), True, False),       # 24 MiB; more channels than positions
+    ((20, 1280, 16, 16), False, True), ((24, 1280, 16, 16), False, False),     # a whole number of workgroups per CU
+    ((16, 640, 36, 36), False, False)])                                        # positions that leave a tile half empty
+def test_groupnorm_tokens_of_large_tensors(msd, orc, cuda, shape, half, two):
+    import torch
+    batch, channels, hw = shape[0], shape[1], shape[2] * shape[3]
+    xd = torch.empty(shape, dtype=torch.float16 if half else torch.float32, device=cuda).normal_(0.4, 1.5)
+    g, b = _affine(orc, channels, 24)
+    gd, bd = _dev(g, cuda), _dev(b, cuda)
+    assert _takes_two_launches(msd, xd, gd, bd, 32) == two
+    got = msd.groupnorm_tokens(xd, gd, bd, 32, 1e-6)[::7].float().cpu().numpy()
+    ref = orc.groupnorm64(xd[::7].float().cpu().numpy(), g, b, 32, 1e-6, False).astype(np.float32)
+    ref = ref.reshape(-1, channels, hw).transpose(0, 2, 1)
+    (assert_close_f16 if half else assert_close_f32)(got, ref, what="gn tokens, large")
+
+
 def test_graphs_of_one_capture_stream_run_at_the_same_time(msd, orc, cuda):
     """Two graphs recorded on one stream, replayed on two: token norms in two launches, and norms in place of
     channels of no whole vectors, which outside a capture go through the stream's scratch."""
