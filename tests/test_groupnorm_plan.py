@@ -158,6 +158,8 @@ def test_shapes_the_register_kernel_cannot_take_go_to_the_general_kernel():
     assert msd.groupnorm_plan(2, 320, 4090, 32, msd.DTYPE_F16) == (0, 0, 0, 1)   # units of no whole vectors
     assert msd.groupnorm_plan(2, 320, 4093, 32, msd.DTYPE_F32) == (0, 0, 0, 1)
     assert msd.groupnorm_plan(2, 320, 4, 32, msd.DTYPE_F16) == (0, 0, 0, 1)        # channels shorter than a vector
+    assert msd.groupnorm_plan(9, 128, 30, 32, msd.DTYPE_F16) == (0, 0, 0, 1)       # ragged, many units of 15 vectors
+    assert _check(8, 128, 30, 32, msd.DTYPE_F16)[0] == 1 and _check(9, 128, 34, 32, msd.DTYPE_F16) == (1, 256, 1, 1)
     assert msd.groupnorm_plan(1, 32 * 1100, 66, 32, msd.DTYPE_F16) == (0, 0, 0, 1)   # ragged, and too many channels for the LDS
     assert msd.groupnorm_plan(1, 35200, 4096, 32, msd.DTYPE_F32) == (0, 0, 0, 1)
     assert _check(2, 320, 4094, 32, msd.DTYPE_F32)[0] == 1                         # channels of no whole vectors are taken
