@@ -260,16 +260,21 @@ uint32_t rule_split(const Chip &chip, size_t elt, size_t units, size_t vec_per_u
 //   fp32 1 x 128 x 512 x 512 50 57 -> 47     2 x 256 x 256 x 256 50 55 -> 46    2 x 128 x 512 x 512 100 111 -> 94
 //        8 x 640 x 96 x 96   73.5 -> 67.7    9 x 960 x 96 x 96 126 -> 108       8 x 320 x 96 x 96 37.3 -> 35.5
 //   fp16 1 x 128 x 512 x 512 26 28 -> 24.5   2 x 256 x 384 x 384 66 -> 57       10 x 960 x 96 x 96 70 -> 62
-// (exactly 10240, fp32 8 x 640 x 64 x 64, 28.7 against 32.4 cut; 2-byte units in halves at just two per CU,
-// 8 x 640 x 96 x 96, 36.6 against 37.9: these stay.)  At just one per CU it pays above 12288 vectors (16384, fp32
-// 1 x 256 x 256 x 256, 28.6 -> 22.9; 15360, 1 x 128 x 384 x 320, 23.4 -> 22.2; 9216, fp16 1 x 512 x 192 x 192,
-// 15.8 against 16.7).
-uint32_t shorten_slices(const Chip &chip, size_t elt, size_t units, size_t vec_per_unit, uint32_t split) {
-    constexpr size_t kHeld = 512 * kGnMaxRaggedK, kHeldExactly = 512 * kGnMaxK, kHeldAlone = 12288;
+// (exactly 10240, fp32 8 x 640 x 64 x 64, 28.7 against 32.4 cut, stays.)  It does not pay where the launch is in
+// balance as it is and the halves would fill 512 lanes badly.  Over 4000 random shapes, cut against not cut:
+//   one workgroup per CU    fp32 slices of 14336 vectors and more 0.97, shorter 1.01 (to 1.08); fp16 of 16320 and
+//                           16384 0.77 - 0.92, shorter 1.01 (to 1.07)
+//   two, three per CU, fp16 slices of 10240 ... 15872 vectors: output apart 1.02 (to 1.11); in place at two 0.99, as
+//                           many above as below 1, at three 0.97; beyond 15872 0.91 - 0.94
+//   anything else           0.85 - 0.98
+uint32_t shorten_slices(const Chip &chip, size_t elt, size_t units, size_t vec_per_unit, uint32_t split, bool apart) {
+    constexpr size_t kHeld = 512 * kGnMaxRaggedK, kHeldExactly = 512 * kGnMaxK;
     while (split > 1 && split < kGnMaxSplit && vec_per_unit > split * kHeld && vec_per_unit != split * kHeldExactly) {
         const size_t blocks = units * split;
-        if (blocks < chip.cus || (blocks == chip.cus && vec_per_unit <= split * kHeldAlone)) break;
-        if (elt == 2 && split == 2 && blocks == 2 * (size_t)chip.cus) break;
+        if (blocks < chip.cus || (blocks == chip.cus && vec_per_unit < split * (elt == 4 ? 14336u : 16256u))) break;
+        if (elt == 2 && (blocks == 2 * (size_t)chip.cus || (apart && blocks == 3 * (size_t)chip.cus)) &&
+            vec_per_unit > split * kHeldExactly && vec_per_unit <= split * 15872u)
+            break;
         split *= 2;
     }
     return split;
@@ -359,7 +364,7 @@ GnDecision gn_decide(size_t elt, size_t batch, size_t channels, size_t hw, size_
     } else if (can_split) {
         const uint32_t want = (tuned && tuned->writers <= 1) ? tuned->split : rule_split(chip, elt, units, vec_per_unit);
         while (split < want && vec_per_unit >= (size_t)2 * split * 256) split *= 2;
-        if (!tuned) split = shorten_slices(chip, elt, units, vec_per_unit, split);
+        if (!tuned) split = shorten_slices(chip, elt, units, vec_per_unit, split, may_share);
     }
 
     const size_t vec_per_slice = (vec_per_unit + split - 1) / split;

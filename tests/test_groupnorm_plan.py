@@ -154,6 +154,18 @@ def test_channels_of_no_whole_vectors_get_a_plan_of_the_register_kernel():
     assert _check(2, 1280, 252, 32, f16)[3] > 1 and _check(2, 1280, 252, 32, f16, in_place=True)[3] == 1
 
 
+def test_slices_that_would_fill_512_lanes_badly_stay_where_a_launch_is_in_balance():
+    f16, f32 = msd.DTYPE_F16, msd.DTYPE_F32
+    for shape, code, in_place, split in (
+            ((8, 640, 9216), f16, False, 2), ((4, 960, 13440), f16, False, 4),            # two per CU, 11520 and 12600 vectors
+            ((3, 320, 78848), f16, False, 8), ((3, 320, 78848), f16, True, 16),            # three: in place they are cut
+            ((5, 320, 78848), f16, False, 16),                                           # five are cut
+            ((2, 256, 65280), f16, False, 8), ((2, 256, 65280), f32, False, 16),          # 16320 vectors, 32 bits cut
+            ((1, 128, 98368), f32, True, 8), ((1, 128, 122880), f32, True, 16),           # one per CU: from 14336 on
+            ((1, 128, 253952), f16, True, 8), ((1, 128, 261120), f16, True, 16)):          # 16-bit: 16256
+        assert _check(*shape, 32, code, in_place=in_place)[0] == split, (shape, code, in_place)
+
+
 def test_shapes_the_register_kernel_cannot_take_go_to_the_general_kernel():
     assert msd.groupnorm_plan(2, 320, 4090, 32, msd.DTYPE_F16) == (0, 0, 0, 1)   # units of no whole vectors
     assert msd.groupnorm_plan(2, 320, 4093, 32, msd.DTYPE_F32) == (0, 0, 0, 1)
