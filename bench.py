@@ -8,11 +8,11 @@ each layer on its own HBM-resident buffers, launched back to back on one stream.
 `value` = algorithmic bytes of one step / time per step.
 
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--mode graph|eager] [--no-cpu] [--no-shapes]
-                    [--tables shapes,gn_split,fusions,neighbours,large_batch,gn_plan_sweep]
+                    [--tables all | shapes,gn_split,fusions,neighbours,large_batch,gn_plan_sweep]
     python bench.py --sweep-summary OUT.json[,...]               (no GPU: markdown of gn_plan_sweep rows)
     python bench.py --trace-summary TRACE.csv --bench-json OUT [--plain-json OUT2]   (no GPU: shapes rows next to a kernel trace)
 
-Prints ONE JSON line (see the keys below).  The CPU oracle is used only for the
+Prints ONE JSON line (see the keys below), of a few KB without the per-kernel tables.  The CPU oracle is used only for the
 `cpu_baseline` leg.
 """
 import argparse
@@ -1295,9 +1295,10 @@ def main():
     ap.add_argument("--mode", choices=["graph", "eager"], default="graph")
     ap.add_argument("--no-cpu", action="store_true")
     ap.add_argument("--no-shapes", action="store_true", help="skip the per-kernel tables")
-    ap.add_argument("--tables", default="shapes,gn_split,fusions,neighbours,large_batch",
-                    help="comma list of the per-kernel tables to measure (also: gn_plan_sweep, the automatic "
-                         "GroupNorm launch plan against every forced one at --sweep-batches; minutes per batch)")
+    ap.add_argument("--tables", default="",
+                    help="comma list of the per-kernel tables to measure as well (they make the line tens of KB long): "
+                         "shapes, gn_split, fusions, neighbours, large_batch, or all of these; also gn_plan_sweep, the "
+                         "automatic GroupNorm launch plan against every forced one at --sweep-batches (minutes per batch)")
     ap.add_argument("--sweep-batches", default="1,2,4,8,16,32", help="batches of the gn_plan_sweep table")
     ap.add_argument("--sweep-summary", default=None, metavar="JSON[,JSON...]",
                     help="no GPU: print the markdown summary of gn_plan_sweep rows in these bench.py outputs")
@@ -1439,6 +1440,8 @@ def main():
     out["config"]["launch_floor_us"] = round(floor_us, 3)
     out["config"]["graph_launch_us"] = round(graph_us, 2)
     tables = set() if args.no_shapes else set(t for t in args.tables.split(",") if t)
+    if "all" in tables:
+        tables |= {"shapes", "gn_split", "fusions", "neighbours", "large_batch"}
     if "shapes" in tables:
         markers = TraceMarkers(torch, msd, dev)
         out["shapes"] = shape_table(torch, msd, dev, stream, floor_us, markers)
