@@ -51,8 +51,8 @@ const char *msd_error_string(int code);
  * GroupNorms, nor two graphs captured on one stream at the same time).  Channels of no
  * whole 16-byte vectors are recorded without it: such a GroupNorm works on whole units then,
  * or through the general kernel, and may differ from the same call outside a capture in the
- * last bit, as it may where no scratch can be allocated.  Also looks up the device address of msd_groupnorm_noalloc's fixed
- * scratch on the current device.  hipStreamPerThread is refused (one handle, a
+ * last bit, as it may where no scratch can be allocated.  Also looks up the device address of
+ * msd_groupnorm_noalloc's fixed scratch on the current device.  hipStreamPerThread is refused (one handle, a
  * different stream in every thread) - here and by msd_groupnorm, msd_chunk_add_groupnorm
  * and msd_groupnorm_tokens for every shape, whether or not that launch would need the
  * scratch; msd_groupnorm_noalloc, which has its own, takes it.  No reference counterpart
@@ -130,9 +130,9 @@ int msd_groupnorm(const void *x, void *y, const float *gamma, const float *beta,
 /*
  * msd_groupnorm for callers that cannot allocate (code under stream capture, tight serving
  * loops, harnesses that forbid hipMalloc): same arguments, same kernels, same result bit for
- * bit (while msd_gn_fallbacks() stays 0, see msd_groupnorm), but the workgroups' exchange
- * area is a fixed 1 MiB array inside the library's code
- * object instead of a per-stream allocation, so the call never allocates or frees (its first
+ * bit (while msd_gn_fallbacks() stays 0, see msd_groupnorm; hw of no whole 16-byte vectors: as
+ * msd_groupnorm outside a capture, inside one too), but the workgroups' exchange area is a fixed
+ * 1 MiB array inside the library's code object instead of a per-stream allocation, so the call never allocates or frees (its first
  * call on a device looks the array's address up; msd_init does that ahead of time).  Limit:
  * batch * groups <= 1024, otherwise MSD_ERR_SCRATCH_LIMIT.  Every stream of a device shares
  * the one array: calls that overlap in time on one GPU race (their results are undefined);
@@ -151,8 +151,9 @@ int msd_groupnorm_noalloc(const void *x, void *y, const float *gamma, const floa
  * one part; such a launch is only made when y does not overlap x, so in_place != 0 asks for the
  * plan of a call with y == x.  *split = 0 (the others too) means the general kernel: one 256-lane
  * workgroup per (sample, group), nothing in registers.  (hw of no whole vectors: where this says
- * *split > 1, a call that can use no scratch, see msd_init, has another launch.)  Host arithmetic only: needs no GPU and launches nothing.  For
- * diagnostics, tests and benchmark tables.  No counterpart in the reference (its geometry is fixed, M/nn/GroupNorm.cpp:105-128).
+ * *split > 1, a call that can use no scratch, see msd_init, has another launch.)  Host arithmetic
+ * only: needs no GPU and launches nothing.  For diagnostics, tests and benchmark tables.  No
+ * counterpart in the reference (its geometry is fixed, M/nn/GroupNorm.cpp:105-128).
  */
 int msd_groupnorm_plan(size_t batch, size_t channels, size_t hw, size_t groups, int dtype, int noalloc,
                        int in_place, int *split, int *threads, int *vectors_per_lane, int *writers);
@@ -174,9 +175,10 @@ int msd_groupnorm_tokens(const void *x, void *y, const float *gamma, const float
 
 /*
  * msd_groupnorm_tokens with memory of the caller's for what its two launches exchange: inside a
- * capture and outside it the same launches and, bit for bit, the same result.  workspace: 8-byte aligned device
- * memory of at least MSD_TOKENS_WORKSPACE_BYTES * batch * groups bytes, apart from x and y; its contents need
- * not be set, are left undefined, and belong to this call until it (or every replay of it) is done.
+ * capture and outside it the same launches and, bit for bit, the same result.  workspace: 8-byte
+ * aligned device memory of at least MSD_TOKENS_WORKSPACE_BYTES * batch * groups bytes, apart from
+ * x and y; its contents need not be set, are left undefined, and belong to this call until it (or
+ * every replay of it) is done.
  */
 #define MSD_TOKENS_WORKSPACE_BYTES 128
 int msd_groupnorm_tokens_workspace(const void *x, void *y, const float *gamma, const float *beta, size_t batch,

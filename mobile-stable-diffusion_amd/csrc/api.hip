@@ -25,20 +25,21 @@ std::mutex g_scratch_mutex;
 std::unordered_map<ScratchKey, GnScratch, ScratchKeyHash> g_scratch;
 
 // Scratch for `units` (sample, group) pairs, carved out of one block:
-// [slot_mean | slot_m2 | epoch | done | fallbacks | partials], every part 256-byte aligned.
+// [slot_mean | slot_m2 | epoch | done | fallbacks] and, in an allocated one, [partials], every part 256-byte aligned.
 constexpr size_t slot_bytes(size_t units) { return sizeof(unsigned long long) * units * kGnMaxSplit; }
 constexpr size_t word_bytes(size_t units) { return sizeof(uint32_t) * units; }
 constexpr size_t partial_bytes(size_t units) { return sizeof(float2) * units * kGnStatSlices; }
-constexpr size_t scratch_bytes(size_t units) { return 2 * slot_bytes(units) + 2 * word_bytes(units) + 256 + partial_bytes(units); }
+constexpr size_t exchange_bytes(size_t units) { return 2 * slot_bytes(units) + 2 * word_bytes(units) + 256; }
+constexpr size_t kAllocatedBytes = exchange_bytes(kGnMaxUnits) + partial_bytes(kGnMaxUnits);
 
-GnScratch carve(char *base, size_t units) {
+GnScratch carve(char *base, size_t units, bool with_partials) {
     GnScratch s;
     s.slot_mean = reinterpret_cast<unsigned long long *>(base);
     s.slot_m2 = reinterpret_cast<unsigned long long *>(base + slot_bytes(units));
     s.epoch = reinterpret_cast<uint32_t *>(base + 2 * slot_bytes(units));
     s.done = reinterpret_cast<uint32_t *>(base + 2 * slot_bytes(units) + word_bytes(units));
     s.fallbacks = reinterpret_cast<uint32_t *>(base + 2 * slot_bytes(units) + 2 * word_bytes(units));
-    s.partials = reinterpret_cast<float2 *>(base + 2 * slot_bytes(units) + 2 * word_bytes(units) + 256);
+    s.partials = with_partials ? reinterpret_cast<float2 *>(base + exchange_bytes(units)) : nullptr;
     s.units = (uint32_t)units;
     return s;
 }
@@ -48,7 +49,7 @@ GnScratch carve(char *base, size_t units) {
 // are never reset: see groupnorm.hip).  In host code this name is only a handle for
 // hipGetSymbolAddress; kernels get the device address that call returns.
 constexpr uint32_t kStaticUnits = 1024;
-static __device__ __align__(256) unsigned char scratch[scratch_bytes(kStaticUnits)];
+static __device__ __align__(256) unsigned char scratch[exchange_bytes(kStaticUnits)];
 
 constexpr int kMaxDevices = 64;
 char *g_static_base[kMaxDevices] = {nullptr};  // device address of `scratch`, per device
@@ -71,13 +72,13 @@ hipError_t get_scratch(hipStream_t stream, GnScratch *out, bool clear_on_stream)
         return hipSuccess;
     }
     char *base = nullptr;
-    err = hipMalloc(reinterpret_cast<void **>(&base), scratch_bytes(kGnMaxUnits));
+    err = hipMalloc(reinterpret_cast<void **>(&base), kAllocatedBytes);
     if (err != hipSuccess) return err;
     // tags, epochs and counters start at zero
     if (clear_on_stream) {
-        err = hipMemsetAsync(base, 0, scratch_bytes(kGnMaxUnits), stream);
+        err = hipMemsetAsync(base, 0, kAllocatedBytes, stream);
     } else {
-        err = hipMemset(base, 0, scratch_bytes(kGnMaxUnits));
+        err = hipMemset(base, 0, kAllocatedBytes);
         // this fill runs on the null stream: it must have finished before a launch on `stream`
         // (which may not synchronise with the null stream) reads the scratch
         if (err == hipSuccess) err = hipStreamSynchronize(nullptr);
@@ -86,7 +87,7 @@ hipError_t get_scratch(hipStream_t stream, GnScratch *out, bool clear_on_stream)
         (void)hipFree(base);
         return err;
     }
-    const GnScratch s = carve(base, kGnMaxUnits);
+    const GnScratch s = carve(base, kGnMaxUnits, true);
     g_scratch.emplace(key, s);
     *out = s;
     return hipSuccess;
@@ -130,7 +131,7 @@ hipError_t get_static_scratch(GnScratch *out) {
         if (ptr == nullptr) return hipErrorInvalidSymbol;
         g_static_base[device] = static_cast<char *>(ptr);
     }
-    *out = carve(g_static_base[device], kStaticUnits);
+    *out = carve(g_static_base[device], kStaticUnits, false);
     return hipSuccess;
 }
 
@@ -203,7 +204,7 @@ int msd_gn_fallbacks(void *stream, unsigned int *count, int reset) {
         auto it = g_scratch.find(ScratchKey{device, s});
         if (it != g_scratch.end()) counters[0] = it->second.fallbacks;
         if (device >= 0 && device < kMaxDevices && g_static_base[device])
-            counters[1] = carve(g_static_base[device], kStaticUnits).fallbacks;
+            counters[1] = carve(g_static_base[device], kStaticUnits, false).fallbacks;
     }
     for (uint32_t *c : counters) {
         if (!c) continue;

@@ -163,9 +163,9 @@ constexpr int kSmThreads = 256;
 constexpr float kNegInf = -__builtin_huge_valf();
 
 // RAGGED: rows that are no whole number of vectors or start at any element (the 18 x 14 = 252 positions of a
-// deeper UNet level): the last piece of a row is cut.Bound
-// like the others by one read and one write, which element by element were eight loads and stores a lane
-// (and three passes beyond 512 columns).  fp16, us, before and now: 16128 x 252 6.63 -> 4.66, 32256 x 252
+// deeper UNet level): the last piece of a row is cut.  Bound like the others by one read and one write, which element
+// by element are eight loads and stores a lane (and three passes beyond 512 columns); softmax_dispatch says from how
+// many rows on that is slower.  fp16, us, element by element and so: 16128 x 252 6.63 -> 4.66, 32256 x 252
 // 10.9 -> 7.1, 65536 x 140 17.9 -> 10.2, 4000 x 1023 9.5 -> 5.2; 16128 x 256, whole vectors, takes 4.1.
 template <typename T, int VPL, int TL, bool RAGGED>
 __global__ __launch_bounds__(kSmThreads) void softmax_team_kernel(const T *x, T *y, uint32_t rows, uint32_t cols,

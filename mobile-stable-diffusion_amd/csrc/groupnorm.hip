@@ -548,8 +548,9 @@ __global__ __launch_bounds__(kGnMaxThreads, (K <= (sizeof(T) == 2 ? 5 : 4) ? 8 :
                                            red_a, red_b, red_c, stats, aff);
 }
 
-// Any shape or alignment (units that are no whole number of vectors, channels of less than a
-// vector): one workgroup per unit, three passes over global memory with scalar accesses (the second and third pass hit in cache for UNet-sized units).
+// Any shape or alignment (units that are no whole number of vectors, channels of less than a vector, many
+// units of a few vectors): one workgroup per unit, three passes over global memory with scalar accesses (the
+// second and third pass hit in cache for UNet-sized units).
 template <typename T, bool SILU>
 __global__ __launch_bounds__(kGenericThreads) void gn_generic_kernel(
     const T *x, const T *chunk, T *y, const float *__restrict__ gamma,

@@ -63,7 +63,7 @@ struct GnScratch {
     uint32_t *epoch;                // [kGnMaxUnits] launches completed on this unit
     uint32_t *done;                 // [kGnMaxUnits] slices finished in the running launch
     uint32_t *fallbacks;            // [1] slices that stopped waiting and computed a sibling's statistics themselves
-    float2 *partials;               // [kGnMaxUnits][kGnStatSlices] (mean, M2), written and read by one pair of launches
+    float2 *partials;               // [kGnMaxUnits][kGnStatSlices] (mean, M2) for one pair of launches; null in the fixed scratch
     uint32_t units;                 // units the arrays above have room for
 };
 

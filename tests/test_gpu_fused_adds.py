@@ -284,8 +284,9 @@ def test_groupnorm_tokens_in_two_launches(msd, orc, cuda, shape, groups, mean, h
         recorded = msd.groupnorm_tokens(xd, gd, bd, groups, 1e-6)
     plain = torch.empty_like(recorded)
     with torch.cuda.graph(without, stream=stream):
-        assert not scratch_free or lib.msd_groupnorm_tokens(xd.data_ptr(), plain.data_ptr(), gd.data_ptr(), bd.data_ptr(), batch, channels, hw,
-                                        groups, 1e-6, msd.DTYPE_F16 if half else msd.DTYPE_F32, stream.cuda_stream) == 0
+        assert not scratch_free or lib.msd_groupnorm_tokens(
+            xd.data_ptr(), plain.data_ptr(), gd.data_ptr(), bd.data_ptr(), batch, channels, hw, groups, 1e-6,
+            msd.DTYPE_F16 if half else msd.DTYPE_F32, stream.cuda_stream) == 0
     for _ in range(3):
         recorded.zero_()
         with_workspace.replay()

@@ -382,3 +382,54 @@ def test_ddim_sampling_loop_is_bit_exact(msd, orc, cuda):
         x = orc.ddim_update(x, e, a[index], ap[index], s1m[index])
         msd.ddim_update(xd, ed, float(a[index]), float(ap[index]), float(s1m[index]), out=xd)
     assert np.array_equal(xd.cpu().numpy(), x)
+
+
+@pytest.mark.parametrize("rows,cols,half", [(70, 256, True), (3075, 256, True), (9, 1024, True), (70, 256, False), (9, 1024, False),
+                                            (5, 2048, False)])
+def test_softmax_rows_that_start_at_any_element(msd, orc, cuda, rows, cols, half):
+    """Whole vectors in length, one element past an aligned address; nothing is written around the output."""
+    torch = _torch()
+    n = rows * cols
+    x = orc.normal((rows, cols), seed=8700 + cols, sigma=1.5)
+    x = orc.round_to_half(x) if half else x
+    buf = torch.full((n + 2,), 7.0, dtype=torch.float16 if half else torch.float32, device=cuda)
+    buf[1:n + 1] = _to_dev(x, cuda, half).reshape(-1)
+    at = buf.data_ptr() + buf.element_size()
+    assert msd.load_library().msd_softmax(at, at, rows, cols, 1, msd.DTYPE_F16 if half else msd.DTYPE_F32, None) == 0
+    torch.cuda.synchronize()
+    got = buf.float().cpu().numpy()
+    assert got[0] == 7.0 and got[n + 1] == 7.0
+    got = got[1:n + 1].reshape(rows, cols)
+    if half:
+        assert assert_close_f16(got, orc.softmax(x), "softmax, unaligned rows", rel_floor=0.0)[1] > 0.99
+    else:
+        np.testing.assert_allclose(got, orc.softmax64(x), rtol=1e-5, atol=1e-9)
+
+
+@pytest.mark.parametrize("cols,rows,half", [(9216, 8, True), (8196, 8, False),              # a workgroup's registers
+                                            (252, 3080, True), (514, 8, True), (1023, 8, False),   # pieces, cut ones too
+                                            (147, 8, True), (255, 8, False)])                    # single elements
+def test_softmax_rows_with_infinities_and_nan(msd, cuda, cols, rows, half):
+    """Masked positions are 0; a row of -inf, or with +inf or NaN, is NaN throughout where the maximum is taken
+    first (0 / 0 and inf - inf), and never touches its neighbours."""
+    torch = _torch()
+    x = torch.empty((rows, cols), device=cuda).normal_(0.0, 1.5)
+    x = (x.half() if half else x)
+    x[0, cols // 2:] = -float("inf")
+    x[1] = -float("inf")
+    x[2, cols - 1] = float("inf")
+    x[3, 0] = float("nan")
+    x[4, 1:] = torch.finfo(x.dtype).min
+    x[5] = -65504.0
+    ref = torch.softmax(x.double().cpu(), -1)
+    for inplace in (False, True):
+        y = x.clone()
+        got = msd.softmax(y, stable=True, out=y if inplace else None).double().cpu()
+        for i in range(rows):
+            assert torch.equal(torch.isnan(got[i]), torch.isnan(ref[i])), (i, inplace)
+        ok = ~torch.isnan(ref)
+        assert (got[0, cols // 2:] == 0).all()
+        # half an ulp of the stored value (2^-11 of it in fp16, 2^-25 below the normal range) and 1e-5 of it
+        torch.testing.assert_close(got[ok], ref[ok], rtol=1e-5 + (2.0 ** -11 if half else 0.0), atol=2.0 ** -25 if half else 1e-9)
+    with_mask = msd.softmax(x[:1].clone(), stable=False).double().cpu()
+    torch.testing.assert_close(with_mask, ref[:1], rtol=1e-5 + (2.0 ** -11 if half else 0.0), atol=2.0 ** -25 if half else 1e-9)

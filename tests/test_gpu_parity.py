@@ -276,6 +276,40 @@ def test_groupnorm_slice_that_stops_waiting_computes_its_siblings_statistics(msd
     assert msd.status() == 0
 
 
+@pytest.mark.parametrize("shape", [(2, 640, 63, 63), (2, 320, 62, 66)])  # vectors of one or two channels, fp16 and fp32
+def test_groupnorm_of_no_whole_vectors_gives_up_on_a_sibling(msd, orc, cuda, shape):
+    """The same on channels of no whole vectors, with and without the embedding's addend, which the workgroup adds to
+    what it reads of a sibling's part."""
+    lib = msd.load_library()
+    x = orc.normal(shape, seed=98, sigma=2.0, mean=1.0)
+    g, b = _affine(orc, shape[1], 98)
+    chunk = orc.round_to_half(orc.normal(shape[:2], seed=99))
+    msd.gn_fallbacks(reset=True)
+    try:
+        assert lib.msd_set_tuning(msd.TUNE_GN_SPLIT, 8) == 0
+        assert lib.msd_set_tuning(msd.TUNE_GN_SPIN_LIMIT, 1) == 0
+        for half in (False, True):
+            if shape[1] // 32 * shape[2] * shape[3] % (8 if half else 4):
+                continue  # (units of no whole vectors either: the general kernel)
+            xin = orc.round_to_half(x) if half else x
+            summed = xin + chunk[:, :, None, None]
+            summed = orc.round_to_half(summed) if half else summed
+            gd, bd, cd = _to_dev(g, cuda), _to_dev(b, cuda), _to_dev(chunk, cuda, half)
+            for inplace in (False, True):
+                xd, yd = _to_dev(xin, cuda, half), _to_dev(xin, cuda, half)
+                plain = msd.groupnorm(xd, gd, bd, 32, 1e-5, True, out=xd if inplace else None)
+                added = msd.chunk_add_groupnorm(yd, cd, gd, bd, 32, 1e-5, True, out=yd if inplace else None)
+                for got, of in ((plain, xin), (added, summed)):
+                    ref = orc.groupnorm64(of, g, b, 32, 1e-5, True).astype(np.float32).reshape(shape)
+                    (assert_close_f16 if half else assert_close_f32)(got.float().cpu().numpy(), ref,
+                                                                     what="gn ragged, forced give-up")
+    finally:
+        lib.msd_set_tuning(msd.TUNE_GN_SPLIT, 0)
+        lib.msd_set_tuning(msd.TUNE_GN_SPIN_LIMIT, 0)
+    assert msd.gn_fallbacks() > 0  # the path was really taken
+    assert msd.status() == 0
+
+
 def test_groupnorm_repeated_launches_reuse_scratch(msd, orc, cuda):
     # the arrival counters are never reset: many launches with changing split factors
     lib = msd.load_library()

@@ -67,6 +67,41 @@ def test_noalloc_groupnorm_matches_allocating_entry_point_twice(msd, orc, cuda, 
     assert _call(lib.msd_groupnorm_noalloc, xd, got, gd, bd, 40, channels, hw, True, code, stream) == msd.ERR_SCRATCH_LIMIT
 
 
+@pytest.mark.parametrize("half", [True, False], ids=["f16", "f32"])
+@pytest.mark.parametrize("batch,channels,hw", [(2, 320, 4092), (2, 1280, 252), (1, 640, 8198)])
+def test_noalloc_groupnorm_of_no_whole_vectors(msd, orc, cuda, batch, channels, hw, half):
+    """The same bits as msd_groupnorm, apart and in place, and recorded into a graph as outside of one."""
+    import torch
+    from tolerances import assert_close_f16, assert_close_f32
+    lib, code = msd.load_library(), msd.DTYPE_F16 if half else msd.DTYPE_F32
+    msd.init()
+    msd.gn_fallbacks(reset=True)
+    x = orc.normal((batch, channels, hw), seed=hw, sigma=2.0, mean=0.3)
+    x = orc.round_to_half(x) if half else x
+    g, b = orc.normal((channels,), seed=31, mean=1.0, sigma=0.1), orc.normal((channels,), seed=32, sigma=0.1)
+    xd = torch.from_numpy(x).to(cuda)
+    xd = xd.half() if half else xd
+    gd, bd = torch.from_numpy(g).to(cuda), torch.from_numpy(b).to(cuda)
+    sp = torch.cuda.current_stream().cuda_stream
+    want, want_in, got, got_in = torch.empty_like(xd), xd.clone(), torch.empty_like(xd), xd.clone()
+    for fn, apart, inplace in ((lib.msd_groupnorm, want, want_in), (lib.msd_groupnorm_noalloc, got, got_in)):
+        assert _call(fn, xd, apart, gd, bd, batch, channels, hw, True, code, sp) == 0
+        assert _call(fn, inplace, inplace, gd, bd, batch, channels, hw, True, code, sp) == 0
+    graph, recorded = torch.cuda.CUDAGraph(), torch.empty_like(xd)
+    with torch.cuda.graph(graph):
+        assert _call(lib.msd_groupnorm_noalloc, xd, recorded, gd, bd, batch, channels, hw, True, code,
+                     torch.cuda.current_stream().cuda_stream) == 0
+    for _ in range(3):
+        recorded.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(recorded, want)
+    assert msd.gn_fallbacks() == 0
+    assert torch.equal(got, want) and torch.equal(got_in, want_in)
+    ref = orc.groupnorm64(x, g, b, 32, 1e-5, True).astype(np.float32).reshape(x.shape)
+    (assert_close_f16 if half else assert_close_f32)(got.float().cpu().numpy(), ref, what="noalloc, ragged")
+
+
 def test_noalloc_groupnorm_runs_under_stream_capture_and_allocates_nothing(msd, orc, cuda):
     """The callers the entry point is for: two calls of different shapes, both cut into slices
     that exchange through the fixed array, are recorded into one HIP graph (an allocation under
