@@ -107,14 +107,15 @@ def check(code):
 # transformer block 81.6 -> 52.8, 22 grouped projections 70.4 -> 52.2.
 _torch = None
 _dtype_codes = {}
-_raw_stream = _current_device = None
+_raw_stream = _current_device = _capturing = None
 
 
 def _bind_torch():
     """torch, imported by the first call that takes tensors (the host-only calls do without)."""
-    global _torch
+    global _torch, _capturing
     if _torch is None:
         import torch
+        _capturing = torch.cuda.is_current_stream_capturing
         _dtype_codes.update({torch.float32: DTYPE_F32, torch.float16: DTYPE_F16})
         _torch = torch
     return _torch
@@ -226,14 +227,15 @@ def groupnorm_tokens(x, gamma, beta, groups, eps=1e-6):
     batch, channels, hw = _planes(x)
     xp = _dev(x)
     out = x.new_empty((batch, hw, channels))
-    args = (xp, out.data_ptr(), _affine(gamma, channels, x, "gamma"), _affine(beta, channels, x, "beta"), batch, channels,
-            hw, groups, eps, _dtype_code(x))
-    if _torch.cuda.is_current_stream_capturing():  # (the graph keeps the workspace in its pool, apart from other graphs')
-        size = TOKENS_WORKSPACE_BYTES * batch * groups
-        workspace = x.new_empty(size, dtype=_torch.uint8)
-        check(lib.msd_groupnorm_tokens_workspace(*args, workspace.data_ptr(), size, _stream()))
-    else:
-        check(lib.msd_groupnorm_tokens(*args, _stream()))
+    gp, bp = _affine(gamma, channels, x, "gamma"), _affine(beta, channels, x, "beta")
+    if not _capturing():
+        check(lib.msd_groupnorm_tokens(xp, out.data_ptr(), gp, bp, batch, channels, hw, groups, eps, _dtype_code(x),
+                                       _stream()))
+        return out
+    size = TOKENS_WORKSPACE_BYTES * batch * groups
+    workspace = x.new_empty(size, dtype=_torch.uint8)  # (the graph keeps it in its pool, apart from other graphs')
+    check(lib.msd_groupnorm_tokens_workspace(xp, out.data_ptr(), gp, bp, batch, channels, hw, groups, eps, _dtype_code(x),
+                                             workspace.data_ptr(), size, _stream()))
     return out
 
 
