@@ -1409,7 +1409,7 @@ def main():
     # geglu_kernel<__half, 1>; the GroupNorm family as a whole takes more of the step and sits
     # furthest below the roofline, which `roofline.families` shows.
     traffic = measured_traffic()
-    kernel_names = {"gn_silu": "gn_slice_kernel<__half, K, true, SHARED>", "ln": "ln_team_kernel<__half, NW, VPL, TL, EARLY>",
+    kernel_names = {"gn_silu": "gn_slice_kernel<__half, K, true, SHARED, RAGGED>", "ln": "ln_team_kernel<__half, NW, VPL, TL, EARLY>",
                     "geglu": "geglu_kernel<__half, 1>"}
     roofline_families = {}
     for kind, fam in families.items():
