@@ -313,15 +313,17 @@ int permute_021_dispatch(const void *srcv, void *dstv, size_t isize, size_t jsiz
     // by element.  us, tile against elements (elements per tile):
     //   fp16  65535 x 2 x 2 (4) 30.5 / 3.0    1778 x 3 x 300 (180) 8.2 / 6.7    6275 x 17 x 15 (255) 8.8 / 6.7
     //   fp32  5000 x 5 x 64 (320) 7.8 / 7.2   714 x 7 x 320 (448) 7.6 / 7.2, transposed 6.5 / 9.2   15 x 77 x 77 3.07 / 2.67
-    // (by elements per tile from 256 Ki in all, tile against elements: fp16 128 - 200 1.2, 200 - 300 0.96, 350 - 400 0.82;
-    // fp32 input rows longer than output rows 300 - 400 1.15, 400 - 450 1.03, 450 - 600 0.88, shorter 250 - 300 1.13,
-    // 300 - 350 1.03, 350 - 400 0.92.)  In pieces that nothing cuts, or only in halves (2-byte sides in multiples of
+    // (by elements per tile, 256 Ki and more in all, tile against elements: fp16 128 - 200 1.2, 200 - 300 0.96, 350 - 400
+    // 0.82; fp32 input rows longer than output rows 300 - 400 1.15, 400 - 450 1.03, 450 - 600 0.88, shorter 250 - 300
+    // 1.13, 300 - 350 1.03, 350 - 400 0.92; by elements in all, 1500 and more per tile: fp16 140 - 180 Ki 0.98, 180 - 256 Ki
+    // 0.90, fp32 180 - 220 Ki 1.02, 220 - 256 Ki 0.94.)  In pieces that nothing cuts, or only in halves (2-byte sides in multiples of
     // four), the tile is within 5 % of the better one or ahead at every size.
     const size_t n = isize * jsize * ksize;
     const size_t per_tile = jsize * ksize / (((jsize + kTile - 1) / kTile) * ((ksize + kTile - 1) / kTile));
     const bool halves = ragged && sizeof(T) == 2 && (jsize | ksize) % 4 == 0 &&
                         ((reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(dst)) & 7u) == 0;
-    const bool tile_pays = !ragged || halves || (per_tile >= (sizeof(T) == 2 ? 250u : jsize > ksize ? 350u : 450u) && n >= 256 * 1024);
+    const size_t least = sizeof(T) == 2 ? 250 : jsize > ksize ? 350 : 450, least_in_all = (sizeof(T) == 2 ? 192 : 256) * 1024;
+    const bool tile_pays = !ragged || halves || (per_tile >= least && n >= least_in_all);
     const bool tiled = tile_pays && isize <= 65535 && ksize <= kTileMaxSide && jsize <= kTileMaxSide &&
                        (tiles.x <= 65535 || tiles.y <= 65535);
     // Output rows shorter than input rows: consecutive workgroups take the tiles of one output

@@ -445,7 +445,7 @@ def test_permute_0_2_1(msd, orc, cuda, shape, half):
 @pytest.mark.parametrize("half", [False, True], ids=["f32", "f16"])
 @pytest.mark.parametrize("shape", [(2, 63, 1280), (2, 1280, 63), (1, 65, 127), (3, 1, 9), (2, 9, 1), (1, 130, 66),
                                    (4, 63, 1280), (4, 1280, 63), (24, 65, 127), (23, 130, 66), (1, 5, 40000), (1, 40000, 7),
-                                   (33, 65, 127), (31, 130, 66),
+                                   (33, 65, 127), (31, 130, 66), (23, 65, 127),
                                    (700, 17, 17), (650, 20, 17), (3000, 3, 64)])   # tiles; planes that fill too few of them
 def test_permute_0_2_1_ragged_and_unaligned(msd, orc, cuda, shape, half):
     """Rows that start at any element and end inside a 16-byte piece, in tensors that start one
