@@ -6,6 +6,7 @@
 #include "msd_internal.h"
 #include "tile_transpose.h"
 
+#include <algorithm>
 #include <cmath>
 
 namespace msd {
@@ -225,11 +226,16 @@ __global__ __launch_bounds__(kSmThreads) void softmax_team_kernel(const T *x, T 
     }
 }
 
-// Rows too long for one wavefront's registers (a 768-pixel image has 9216 keys): the row lives in
-// the registers of a whole workgroup, VPL 16-byte vectors per lane, one read and one write per
-// element; the wavefronts' maxima and sums meet in LDS.  Bound by HBM: 147456 x 9216 fp16 runs at
-// 6.0 TB/s (a copy reaches 6.5) against 1.8 in the kernel below, which reads a row twice or three
-// times in 2-byte pieces.  x and y may be the same buffer: a lane stores only what it loaded itself.
+// Rows of more than 256 vectors: the row lives in the registers of a workgroup, VPL 16-byte vectors per lane,
+// one read and one write per element; the wavefronts' maxima and sums meet in LDS.  Bound by HBM, and by how many
+// rows are open at once: what the CUs hold between a row's read and its write is a window on memory that moves
+// through x and y, and beyond about 48 KB a CU a wider window only costs (rows scattered over more pages, reads among
+// writes).  The launch therefore asks for LDS it does not use, which is what keeps workgroups off a CU
+// (softmax_block_launch).  A wavefront per row with 8 - 16 vectors a lane and workgroups of 8 a lane, both as many
+// as fit, before, and so; us, TB/s: fp16 65536 x 4096 170 -> 167 (6.4), 102400 x 6400 437 -> 420 (6.2), 123904 x 7744
+// 661 -> 630 (6.1), 135168 x 8448 796 -> 748 (6.1), 147456 x 9216 917 -> 899 (6.0); fp32 65536 x 4096 351 -> 335 (6.4),
+// 102400 x 6400 905 -> 862 (6.1), 73728 x 9216 967 -> 906 (6.0).  A copy takes 6.4 to 6.5.
+// x and y may be the same buffer: a lane stores only what it loaded itself.
 constexpr int kSmBlockMaxThreads = 1024;
 constexpr int kSmBlockMaxVpl = 8;
 
@@ -499,29 +505,48 @@ void softmax_team_launch(const T *x, T *y, uint32_t rows, uint32_t cols, int sta
                        dim3(threads), 0, stream, x, y, rows, cols, stable);
 }
 
+// How many rows are open at once: 48 KB of them a CU as soon as the launch fills the chip many times (us with 2, 3, 4, 5,
+// 6 rows a CU: fp16 82944 x 5184 329 285 275 274 273, 147456 x 9216 899 932 929; fp32 65536 x 4096 343 335 334 336,
+// 102400 x 6400 862 906); fewer rows are better served all at once (fp16 1000 x 9216, two rows a CU 10.4, no limit 7.8).
+// Vectors per lane: with the limit enough wavefronts for the exponentials and no more (2 / 4 / 8 us: fp16 36864 x 2304
+// 55.0 / 55.7, 82944 x 5184 275 / 275 / 493, fp32 49152 x 3072 190 / 191 / 188, 102400 x 6400 900 / 896 / 862); without,
+// many short lanes (2 / 4 / 8: fp16 4096 x 4096 12.8 / 12.9 / 13.4, 1024 x 9216 8.8 / 7.4 / 10.6, 16 x 9216 2.8 / 3.0 / 4.6,
+// fp32 4096 x 6400 33.7 / 35.3 / 34.8, 16 x 6400 2.5 / 2.5 / 2.7).
+constexpr size_t kSmOpenBytes = 48 * 1024;
+constexpr size_t kLdsPerCu = 160 * 1024, kSmMostLds = 60 * 1024;
+constexpr size_t kSmLimitRounds = 16;  // the limit holds for launches of this many times the rows then in flight
+
 template <typename T>
 void softmax_block_launch(const T *x, T *y, uint32_t rows, uint32_t row_vecs, int stable, hipStream_t stream) {
-    // 2-byte rows take eight vectors per lane and few lanes, 4-byte rows few vectors and many lanes.
-    // Measured over 1.36 GB rows of 1 ... 8 vectors per lane, TB/s, not stable: fp16 16384 columns
-    // 5.68 (two) 5.60 (five) 6.18 (eight), 9216 5.80 / 5.81 / 6.02; fp32 5184 columns 6.27 / 5.82 /
-    // 5.90, 9216 (three is the least that fits 1024 lanes) 5.75 / 5.61 / 5.79.
-    uint32_t vpl = sizeof(T) == 2 ? kSmBlockMaxVpl : 2;
-    auto lanes = [&]() { return (((row_vecs + vpl - 1) / vpl + kWave - 1) / kWave) * kWave; };
-    while (lanes() > (uint32_t)kSmBlockMaxThreads) vpl += vpl < 4 ? 1 : 4;
+    const size_t open = std::max<size_t>(kSmOpenBytes / (row_vecs * 16), 2);  // rows a CU holds: at most 11
+    const bool limit = row_vecs <= 4096 && rows >= kSmLimitRounds * open * chip_info().cus;
+    // one workgroup's share of the LDS, less what it has anyway: `open` of them fit a CU, one more does not
+    const size_t lds = limit ? std::min(kLdsPerCu / open - 1024, kSmMostLds) : 0;
+    uint32_t vpl = sizeof(T) == 2 ? (row_vecs <= (limit ? 320u : 512u) ? 2 : 4) : !limit ? 2 : row_vecs <= 1344 ? 4 : 8;
+    auto lanes = [&]() { return ((row_vecs + vpl - 1) / vpl + kWave - 1) / kWave * kWave; };
+    while (lanes() > (uint32_t)kSmBlockMaxThreads) vpl = vpl == 2 && sizeof(T) == 4 ? 3 : vpl < 4 ? 4 : 8;
     const dim3 block(lanes());
+    auto *kernel = vpl == 8 ? softmax_block_kernel<T, 8> : vpl == 4 ? softmax_block_kernel<T, 4> : softmax_block_kernel<T, 2>;
+    if (vpl == 3) kernel = softmax_block_kernel<T, sizeof(T) == 4 ? 3 : 2>;
     constexpr uint32_t kMostRows = 0xFFFFFFFFu / kSmBlockMaxThreads;  // (a grid holds less than 2^32 lanes)
     for (uint32_t done = 0; done < rows; done += kMostRows) {
         const dim3 grid(min(rows - done, kMostRows));
         const T *xs = x + (size_t)done * row_vecs * Store<T>::EPV;
         T *ys = y + (size_t)done * row_vecs * Store<T>::EPV;
-        switch (vpl) {
-            case 2: launch((softmax_block_kernel<float, 2>), grid, block, 0, stream, (const float *)xs, (float *)ys, row_vecs, stable); break;
-            case 3: launch((softmax_block_kernel<float, 3>), grid, block, 0, stream, (const float *)xs, (float *)ys, row_vecs, stable); break;
-            case 4: launch((softmax_block_kernel<float, 4>), grid, block, 0, stream, (const float *)xs, (float *)ys, row_vecs, stable); break;
-            default: launch((softmax_block_kernel<T, kSmBlockMaxVpl>), grid, block, 0, stream, xs, ys, row_vecs, stable); break;
-        }
+        launch(kernel, grid, block, lds, stream, xs, ys, row_vecs, stable);
         if (rows - done <= kMostRows) break;
     }
+}
+
+// A row of 257 vectors up to what a wavefront's registers hold (512 of 2-byte storage, whose floats take twice the
+// room, 1024 of 4-byte): a workgroup per row where the rows leave CUs idle or fill the chip many times, a wavefront per
+// row between.  us, wavefront and workgroup: fp16 16 x 3072 2.67 / 2.38, 256 x 4096 3.20 / 2.91, 1024 x 3072 stable 4.15 /
+// 4.32, 4096 x 2304 stable 8.88 / 9.32, 8192 x 4096 23.5 / 22.8, 49152 x 3072 97.2 / 94.4; fp32 16 x 3072 2.58 / 2.03,
+// 2048 x 4096 11.2 / 12.7, 2048 x 2304 7.14 / 8.4, 3072 x 3072 14.6 / 13.9, 8192 x 4096 44.8 / 42.1.
+template <typename T>
+bool softmax_wave_per_row(uint32_t rows, uint32_t row_vecs) {
+    const uint32_t cus = chip_info().cus;
+    return row_vecs <= 256 || (row_vecs <= (sizeof(T) == 2 ? 512u : 1024u) && rows > cus && rows < (sizeof(T) == 2 ? 32u : 12u) * cus);
 }
 
 }  // namespace
@@ -653,7 +678,8 @@ int softmax_dispatch(const void *xv, void *yv, size_t rows, size_t cols, int sta
         // (measured against two or four vectors per lane on smaller teams at 4 ... 32 vectors per
         // row, 2048 ... 524288 rows of fp16: never slower, 25-vector rows 71 against 109 us, 4-vector
         // rows 12.9 against 17.1, 32-vector rows 2.4 against 2.7 us at 2048 rows)
-        if (rv <= 4) softmax_team_launch<T, 1, 4, false>(x, y, r, c, stable, stream);
+        if (!softmax_wave_per_row<T>(r, rv)) softmax_block_launch<T>(x, y, r, rv, stable, stream);
+        else if (rv <= 4) softmax_team_launch<T, 1, 4, false>(x, y, r, c, stable, stream);
         else if (rv <= 8) softmax_team_launch<T, 1, 8, false>(x, y, r, c, stable, stream);
         else if (rv <= 16) softmax_team_launch<T, 1, 16, false>(x, y, r, c, stable, stream);
         else if (rv <= 32) softmax_team_launch<T, 1, 32, false>(x, y, r, c, stable, stream);
@@ -661,8 +687,7 @@ int softmax_dispatch(const void *xv, void *yv, size_t rows, size_t cols, int sta
         else if (rv <= 128) softmax_team_launch<T, 2, 64, false>(x, y, r, c, stable, stream);
         else if (rv <= 256) softmax_team_launch<T, 4, 64, false>(x, y, r, c, stable, stream);
         else if (rv <= 512) softmax_team_launch<T, 8, 64, false>(x, y, r, c, stable, stream);
-        else if (rv <= 1024) softmax_team_launch<T, 16, 64, false>(x, y, r, c, stable, stream);
-        else softmax_block_launch<T>(x, y, r, rv, stable, stream);
+        else softmax_team_launch<T, sizeof(T) == 4 ? 16 : 8, 64, false>(x, y, r, c, stable, stream);  // (fp16: no such row)
         return launch_status();
     }
     // The flat kernel pays two barriers and two LDS round trips; below about 12000 rows the

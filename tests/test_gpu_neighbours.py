@@ -260,6 +260,33 @@ def test_softmax_rows_of_a_whole_workgroup(msd, orc, cuda, cols, half):
         _softmax_case(msd, orc, cuda, 5, cols, 8600 + cols + stable, half, stable, sigma=1.5, inplace=bool(stable))
 
 
+@pytest.mark.parametrize("rows,cols,half", [
+    (256, 2056, True), (257, 2056, True), (8191, 2056, True), (8192, 2560, True), (36864, 2568, True),   # wavefront or workgroup
+    (45056, 2056, True), (40960, 4096, True), (16384, 4104, True), (8191, 8448, True), (8192, 9216, True),  # few rows open
+    (256, 1028, False), (257, 4096, False), (3071, 1284, False), (3072, 1284, False), (45056, 1028, False),
+    (8191, 5376, False), (8192, 5380, False), (8192, 8196, False)])
+def test_softmax_long_rows_by_their_number(msd, orc, cuda, rows, cols, half):
+    """On both sides of the numbers of rows at which a row gets a workgroup and the rows in flight are limited, with a
+    vector more than each count of lanes holds; some rows of each launch, the first and the last among them."""
+    torch = _torch()
+    g = torch.Generator(device=cuda).manual_seed(rows + cols)
+    x = torch.randn((rows, cols), device=cuda, dtype=torch.float16 if half else torch.float32, generator=g) * 1.5
+    some = torch.tensor(sorted({0, 1, rows // 3, rows // 2 + 1, rows - 2, rows - 1}), device=cuda)
+    ref = orc.softmax(x[some].float().cpu().numpy())
+    for stable in (False, True):
+        y = msd.softmax(x, stable=stable)
+        got = y[some].float().cpu().numpy()
+        if half:
+            assert assert_close_f16(got, ref, "softmax, long rows", rel_floor=0.0)[1] > 0.99
+        else:
+            np.testing.assert_allclose(got, ref, rtol=1e-5, atol=1e-9)
+        # every row was written: cols results of at most half an ulp of their size off (2^-11, and in 16-bit
+        # storage the subnormal spacing 2^-25 each), and the sum's own rounding
+        sums = y.sum(dim=-1, dtype=torch.float64)
+        assert float((sums - 1.0).abs().max()) <= (2.0 ** -11 + cols * 2.0 ** -25 if half else 1e-5)
+        del y, sums
+
+
 @pytest.mark.parametrize("rb", [16, 32, 64])
 def test_softmax_short_rows_flat_kernel(msd, orc, cuda, rb):
     """Rows of 77 / 100 moved as flat 16-byte vectors, rb rows per workgroup, plus a ragged tail."""
