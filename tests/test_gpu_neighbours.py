@@ -124,6 +124,70 @@ def test_grouped_linear_runs_the_22_resblock_projections_in_one_launch(msd, orc,
             assert_close_f32(o.cpu().numpy(), ref, what="grouped linear %d" % i)
 
 
+@pytest.mark.parametrize("m", [3, 4, 5, 8])
+@pytest.mark.parametrize("n,k", [(1, 640), (16, 648), (17, 704), (33, 1280), (15, 2568), (130, 4096), (7, 632)])
+def test_linear_several_half_rows_on_the_matrix_cores(msd, orc, cuda, m, n, k):
+    """Tiles of 16 columns with columns and rows left over; k of whole runs, of runs cut after each number of
+    pieces, of more than one round; the last k is the longest that goes a column per wavefront."""
+    torch = _torch()
+    for act_in, act_out, bias in ((0, 1, True), (1, 0, False), (1, 1, True)):
+        _linear_case(msd, orc, cuda, m, n, k, 7950 + m + n + k, True, act_in, act_out, bias)
+    x = orc.round_to_half(orc.normal((m, k), seed=7960 + k))
+    w = orc.round_to_half(orc.normal((n, k), seed=7961 + k, sigma=k ** -0.5))
+    xd, wd = _to_dev(x, cuda, True), _to_dev(w, cuda, True)
+    single = msd.linear_rows(xd, wd, act_in=msd.ACT_SILU)
+    other = _to_dev(orc.normal((9, k), seed=7962), cuda, True)
+    for grouped in (msd.linear_rows_grouped(xd, [wd, other], act_in=msd.ACT_SILU)[0],
+                    msd.linear_rows_grouped(xd, [other, wd], act_in=msd.ACT_SILU)[1]):
+        assert torch.equal(grouped, single)
+
+
+def test_linear_matrix_core_rows_with_infinities_nan_and_subnormals(msd, cuda):
+    """An infinity or a NaN reaches the outputs it reaches in a sum of products, and no others; halves below the normal
+    range count, in x, in the weights and in what SiLU leaves."""
+    torch = _torch()
+    g = torch.Generator(device=cuda).manual_seed(17)
+    x = torch.randn((5, 1280), device=cuda, dtype=torch.float16, generator=g) + 0.25  # (no zeros: inf * 0)
+    w = torch.randn((40, 1280), device=cuda, dtype=torch.float16, generator=g) * 0.03
+    w[w == 0] = 0.01
+    x[1, 700], x[2, 3], x[3, 1279] = float("inf"), float("nan"), -float("inf")
+    w[5, 0], w[21, 650], w[39, 1279] = float("inf"), -float("inf"), float("nan")
+    for act in (msd.ACT_NONE, msd.ACT_SILU):
+        got = msd.linear_rows(x, w, act_in=act).double().cpu()
+        xd, wd = x.double().cpu(), w.double().cpu()
+        xd = xd / (1 + torch.exp(-xd)) if act else xd  # (-inf: NaN, as the product with 1 / (1 + inf))
+        want = (xd[:, None, :] * wd[None]).sum(-1)
+        assert torch.equal(torch.isnan(got), torch.isnan(want))
+        assert torch.equal(torch.isinf(got), torch.isinf(want))
+        assert torch.equal(got[torch.isinf(got)], want[torch.isinf(want)])
+        fine = torch.isfinite(want)
+        # half an ulp of the 16-bit result, and 1280 products' float32 sums
+        assert float(((got - want)[fine].abs() / want[fine].abs().clamp(min=1.0)).max()) <= 2.0 ** -11 + 1e-5
+    tiny = 2.0 ** -20  # x * w of halves below the normal range, against weights that bring the sum back
+    xs = torch.full((4, 640), tiny, device=cuda, dtype=torch.float16)
+    ws = torch.full((16, 640), 512.0, device=cuda, dtype=torch.float16)
+    assert float((msd.linear_rows(xs, ws).double() - 640 * tiny * 512).abs().max()) <= 640 * tiny * 512 * 2.0 ** -11
+    half_sum = 640 * 512 * (tiny / (1 + np.exp(-tiny)))
+    assert float((msd.linear_rows(xs, ws, act_in=msd.ACT_SILU).double() - half_sum).abs().max()) <= half_sum * (2.0 ** -11 + 1e-5)
+    assert float((msd.linear_rows(ws[:4], xs[:1]).double() - 640 * tiny * 512).abs().max()) <= 640 * tiny * 512 * 2.0 ** -11
+
+
+@pytest.mark.parametrize("m", [2, 3, 4, 5, 8])
+@pytest.mark.parametrize("k", [4, 1280, 1284, 2564])
+def test_large_grouped_linear_of_floats_is_each_layers_own(msd, cuda, m, k):
+    """8192 columns and more of 4-byte weights share the rows in LDS: bit for bit what a column or two per wavefront
+    give, with columns left over and k of one and of several chunks."""
+    torch = _torch()
+    g = torch.Generator(device=cuda).manual_seed(m * 10000 + k)
+    x = torch.randn((m, k), device=cuda, generator=g)
+    ws = [torch.randn((n, k), device=cuda, generator=g) * k ** -0.5 for n in (3, 8170, 1, 18)]
+    bs = [torch.randn((w.shape[0],), device=cuda, generator=g) for w in ws]
+    bs[2] = None
+    for act_in, act_out in ((msd.ACT_SILU, msd.ACT_NONE), (msd.ACT_NONE, msd.ACT_SILU)):
+        for out, w, b in zip(msd.linear_rows_grouped(x, ws, bs, act_in=act_in, act_out=act_out), ws, bs):
+            assert torch.equal(out, msd.linear_rows(x, w, b, act_in=act_in, act_out=act_out))
+
+
 def test_grouped_linear_edge_cases(msd, orc, cuda):
     torch = _torch()
     # more problems than one launch's table holds, empty problems, missing biases, no activation
