@@ -29,6 +29,7 @@
 // sibling's part of the input, which no workgroup overwrites before it has
 // seen every word of its unit.  The output is the same either way; a counter
 // in the scratch records how often it happened.
+#include <algorithm>
 #include <type_traits>
 
 #include "msd_device.h"
@@ -602,15 +603,9 @@ struct GnTokParams {
     uint32_t channels;
     uint32_t pitch;       // LDS elements between channels: positions per slice + 16 bytes
     FastDiv combos;       // batch * split: (sample, slice) pairs, the fastest part of the block id
-    FastDiv part_len;     // SHARED: vectors of one part, ch_per_group * pos_vecs.d (a multiple of 64)
 };
 
-// SHARED: `writers` workgroups per whole unit (output apart from the input by construction).  Each
-// loads and reduces the whole unit, enumerated part by part (a part = all channels over a range of
-// positions, what a slice is above), and normalises, transposes and stores its own part; nothing
-// is exchanged.  The writers of a unit have block ids one XCD count apart (one XCD: their loads meet in
-// its L2).
-template <typename T, int K, bool SHARED>
+template <typename T, int K>
 __global__ __launch_bounds__(kGnMaxThreads) void gn_tokens_kernel(
     const T *__restrict__ x, T *__restrict__ y, const float *__restrict__ gamma,
     const float *__restrict__ beta, GnScratch scratch, GnTokParams q) {
@@ -628,39 +623,27 @@ __global__ __launch_bounds__(kGnMaxThreads) void gn_tokens_kernel(
     // that differ by multiples of batch * split, so with workgroups dealt round-robin to the
     // 8 XCDs they meet in one L2 when that product is a multiple of 8 (batch 2 x 4 slices);
     // the slices of a unit stay adjacent
-    uint32_t unit, slice;  // SHARED: `slice` is the part this workgroup stores
-    if (SHARED) {
-        const uint32_t j = blockIdx.x >> p.xcd_shift;
-        slice = j & (p.writers - 1);
-        unit = ((j >> p.writers_shift) << p.xcd_shift) + (blockIdx.x & ((1u << p.xcd_shift) - 1u));
-    } else {
-        const uint32_t group = fast_div(blockIdx.x, q.combos);
-        const uint32_t combo = blockIdx.x - group * q.combos.d;
-        unit = (combo >> p.split_shift) * p.groups + group;
-        slice = combo & (p.split - 1);
-    }
-    const uint32_t nvec = SHARED ? p.vec_per_unit : p.vec_per_slice;  // vectors this workgroup holds
+    const uint32_t group = fast_div(blockIdx.x, q.combos);
+    const uint32_t combo = blockIdx.x - group * q.combos.d;
+    const uint32_t unit = (combo >> p.split_shift) * p.groups + group;
+    const uint32_t slice = combo & (p.split - 1);
+    const uint32_t nvec = p.vec_per_slice;
     const uint32_t pvs = q.pos_vecs.d;
     const u32x4 *xin = reinterpret_cast<const u32x4 *>(x) + (size_t)unit * p.vec_per_unit;
 
     uint32_t epoch = 0;
-    if (!SHARED && p.split > 1 && tid == 0)
+    if (p.split > 1 && tid == 0)
         epoch = __hip_atomic_load(scratch.epoch + unit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 
-    // lane-local vector -> (part, channel of the group, position vector of the part / slice)
+    // lane-local vector -> (channel of the group, position vector of the slice)
     u32x4 raw[K];
     uint32_t cl[K], pv[K];
 #pragma unroll
     for (int k = 0; k < K; k++) {
-        uint32_t vl = min(k * nt + tid, nvec - 1);  // ragged tail re-reads the last vector
-        uint32_t part_of = slice;
-        if (SHARED) {
-            part_of = fast_div(vl, q.part_len);
-            vl -= part_of * q.part_len.d;
-        }
+        const uint32_t vl = min(k * nt + tid, nvec - 1);  // ragged tail re-reads the last vector
         cl[k] = fast_div(vl, q.pos_vecs);
         pv[k] = vl - cl[k] * pvs;
-        raw[k] = load_stream(xin + (size_t)cl[k] * p.hw_vec.d + part_of * pvs + pv[k]);
+        raw[k] = load_stream(xin + (size_t)cl[k] * p.hw_vec.d + slice * pvs + pv[k]);
         const bool have = k * nt + tid < nvec;  // lanes past the end hold zeros (the statistics rely on it)
 #pragma unroll
         for (int i = 0; i < 4; i++) raw[k][i] = have ? raw[k][i] : 0u;
@@ -671,7 +654,7 @@ __global__ __launch_bounds__(kGnMaxThreads) void gn_tokens_kernel(
     gn_slice_stats<T, K, false>(raw, nvec, red_a, red_b, red_c, slice_mean, slice_m2);
 
     float mean, rstd;
-    if (SHARED || p.split == 1) {
+    if (p.split == 1) {
         mean = slice_mean;
         rstd = __builtin_amdgcn_rsqf(slice_m2 * p.inv_count + p.eps);
     } else {
@@ -689,10 +672,6 @@ __global__ __launch_bounds__(kGnMaxThreads) void gn_tokens_kernel(
     T *lds = reinterpret_cast<T *>(lds_vec);
 #pragma unroll
     for (int k = 0; k < K; k++) {
-        if (SHARED) {  // a wavefront lies inside one part (part_len is a multiple of 64): a scalar branch
-            const uint32_t first = __builtin_amdgcn_readfirstlane(min(k * nt + tid, nvec - 1));
-            if (first - slice * q.part_len.d >= q.part_len.d) continue;
-        }
         if (k * nt + tid < nvec) {
             const float a = rstd * gamma[ch0 + cl[k]];
             const float b = beta[ch0 + cl[k]];
@@ -706,7 +685,7 @@ __global__ __launch_bounds__(kGnMaxThreads) void gn_tokens_kernel(
     __syncthreads();
     // the slice counts itself done here, behind the last barrier: nothing waits for the answer
     uint32_t arrived_before = 0;
-    if (!SHARED && p.split > 1 && tid == 0) arrived_before = gn_exchange_arrive(scratch, unit);
+    if (p.split > 1 && tid == 0) arrived_before = gn_exchange_arrive(scratch, unit);
 
     // ---- token-major store: for each position of the slice one run of ch_per_group values
     const uint32_t rows = pvs * EPV;                         // positions in the slice
@@ -728,7 +707,101 @@ __global__ __launch_bounds__(kGnMaxThreads) void gn_tokens_kernel(
         }
         out[(size_t)r * row_stride + c] = w;
     }
-    if (!SHARED && p.split > 1 && tid == 0) gn_exchange_close(scratch, p, unit, epoch, arrived_before);
+    if (p.split > 1 && tid == 0) gn_exchange_close(scratch, p, unit, epoch, arrived_before);
+}
+
+// The token-major norm for units that stay whole: `writers` workgroups (one or several) per unit, each of which loads
+// and reduces all of it and stores its own part, all channels of the group over a range of positions (several writers: as
+// in gn_slice_kernel<..., SHARED>, nothing is exchanged).  What a part needs goes to LDS as it was loaded, before the
+// statistics are there, so one barrier covers both; it is normalised on the way out, by lanes that keep to their channels.
+// An XCD takes units_per_xcd units in a row: what the writers of a unit load meets in its L2, and so do the pieces of an
+// output line (ch_per_group elements each) that neighbouring groups store; with units dealt to the XCDs in turn every line
+// was put together in memory from several.
+// RAGGED: hw is no whole number of vectors, a vector may cross from one channel into the next; LDS then holds the whole unit
+// as it lies in memory.
+struct GnTokUnitParams {
+    uint32_t vec_per_unit;
+    uint32_t groups, ch_per_group, channels, hw;
+    uint32_t writers, writers_shift, xcd_shift;
+    uint32_t units_per_xcd;  // units >> xcd_shift
+    uint32_t part_pos;       // positions of a part; of the last one what is left
+    uint32_t pitch;          // LDS elements between channels
+    uint32_t row_step;       // positions that the workgroup stores at a time
+    FastDiv hw_vec;          // vectors per channel (not RAGGED)
+    FastDiv row_dwords;      // 4-byte words per output run: ch_per_group * sizeof(T) / 4
+    float eps, inv_count;
+};
+
+// Stores of 4 bytes: 8 and 16 bytes at a time read LDS with more bank conflicts (us with 16 / 8 / 4 bytes, fp16 batch 2: 1280
+// channels at 16 x 16 4.2 / - / 3.7, 640 at 32 x 32 - / 4.9 / 4.7).
+template <typename T>
+__device__ __forceinline__ void gn_tokens_store(const T *lds, T *y, uint32_t unit, uint32_t pos0, uint32_t rows, float mean,
+                                                float rstd, const float *gamma, const float *beta, const GnTokUnitParams &q) {
+    constexpr int N = 4 / (int)sizeof(T);  // channels per store
+    const uint32_t row0 = fast_div(threadIdx.x, q.row_dwords), c0 = (threadIdx.x - row0 * q.row_dwords.d) * N;
+    if (row0 >= q.row_step) return;
+    const uint32_t ch0 = (unit % q.groups) * q.ch_per_group + c0;
+    float a[N], b[N];
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        a[i] = rstd * gamma[ch0 + i];
+        b[i] = beta[ch0 + i];
+    }
+    T *out = y + ((size_t)(unit / q.groups) * q.hw + pos0) * q.channels + ch0;
+    const T *in = lds + c0 * q.pitch;
+#pragma unroll 4
+    for (uint32_t r = row0; r < rows; r += q.row_step) {
+        float f[N];
+#pragma unroll
+        for (int i = 0; i < N; i++) f[i] = fmaf(Store<T>::load1(in + i * q.pitch + r) - mean, a[i], b[i]);
+        uint32_t w;
+        if constexpr (sizeof(T) == 2) {
+            const __half2 h = __floats2half2_rn(f[0], f[N - 1]);
+            w = *reinterpret_cast<const uint32_t *>(&h);
+        } else {
+            w = __float_as_uint(f[0]);
+        }
+        *reinterpret_cast<uint32_t *>(out + (size_t)r * q.channels) = w;
+    }
+}
+
+template <typename T, int K, bool RAGGED>
+__global__ __launch_bounds__(kGnMaxThreads) void gn_tokens_unit_kernel(
+    const T *__restrict__ x, T *__restrict__ y, const float *__restrict__ gamma, const float *__restrict__ beta,
+    GnTokUnitParams q) {
+    constexpr int EPV = Store<T>::EPV;
+    extern __shared__ u32x4 lds_vec[];
+    __shared__ float red_a[kGnMaxThreads / kWave];
+    __shared__ float red_b[kGnMaxThreads / kWave];
+    __shared__ float red_c[kGnMaxThreads / kWave];
+    const uint32_t tid = threadIdx.x, nt = blockDim.x;
+    const uint32_t of_xcd = blockIdx.x >> q.xcd_shift;
+    const uint32_t part = of_xcd & (q.writers - 1);
+    const uint32_t unit = (blockIdx.x & ((1u << q.xcd_shift) - 1u)) * q.units_per_xcd + (of_xcd >> q.writers_shift);
+    const uint32_t nvec = q.vec_per_unit;
+    const uint32_t pos0 = part * q.part_pos, rows = min(q.part_pos, q.hw - pos0);
+    const u32x4 *xin = reinterpret_cast<const u32x4 *>(x) + (size_t)unit * nvec;
+    T *lds = reinterpret_cast<T *>(lds_vec);
+    u32x4 raw[K];
+#pragma unroll
+    for (int k = 0; k < K; k++) raw[k] = load_stream(xin + min(k * nt + tid, nvec - 1));  // ragged tail: the last vector again
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+        const uint32_t v = k * nt + tid;
+        const bool have = v < nvec;
+        if (RAGGED) {
+            if (have) lds_vec[v] = raw[k];
+        } else {
+            const uint32_t c = fast_div(v, q.hw_vec), p = (v - c * q.hw_vec.d) * EPV - pos0;
+            if (have && p < rows) *reinterpret_cast<u32x4 *>(lds + c * q.pitch + p) = raw[k];
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) raw[k][i] = have ? raw[k][i] : 0u;  // (the statistics rely on it)
+    }
+    float mean, m2;
+    gn_slice_stats<T, K, false>(raw, nvec, red_a, red_b, red_c, mean, m2);  // (its barrier covers the tile)
+    const float rstd = __builtin_amdgcn_rsqf(m2 * q.inv_count + q.eps);
+    gn_tokens_store<T>(RAGGED ? lds + pos0 : lds, y, unit, pos0, rows, mean, rstd, gamma, beta, q);
 }
 
 // Any shape: one workgroup per unit, three passes, element-wise scattered stores.
@@ -1017,18 +1090,118 @@ template int gn_dispatch<__half>(const void *, const void *, void *, const float
 
 namespace {
 
+// How gn_tokens_unit_kernel takes a shape (k == 0: not at all).
+struct GnTokUnitPlan {
+    uint32_t writers, threads, k;
+    bool ragged;
+    uint32_t part_pos, pitch;
+    size_t lds;
+};
+
+constexpr size_t kGnTokMaxLds = 60 * 1024;
+
+template <typename T>
+GnTokUnitPlan gn_tokens_unit_plan(const Chip &chip, size_t units, size_t cpg, size_t hw, int tune_writers) {
+    constexpr size_t EPV = Store<T>::EPV;
+    const size_t unit_size = cpg * hw, run = cpg * sizeof(T);
+    GnTokUnitPlan pl{1, 0, 0, hw % EPV != 0, 0, 0, 0};
+    if (unit_size % EPV != 0 || run % 4 != 0 || units > 0x7FFFFFFFull / 16) return pl;
+    // as many writers as give the chip a workgroup per CU; they must share an XCD (gn_auto_writers)
+    const bool may_share = (chip.xcds & (chip.xcds - 1)) == 0 && units % chip.xcds == 0;
+    uint32_t w = tune_writers > 0 ? (uint32_t)tune_writers : 1;
+    if (tune_writers == 0 && may_share)
+        while (w < 8 && units * w * 2 <= chip.cus) w *= 2;
+    for (bool more = true; more; w *= 2) {
+        pl.writers = w;
+        const size_t vecs = (hw / EPV + w - 1) / w;  // per channel and part
+        pl.part_pos = (uint32_t)(pl.ragged ? (hw + w - 1) / w : vecs * EPV);
+        pl.pitch = (uint32_t)(pl.ragged ? hw : vecs * EPV + EPV);
+        pl.lds = (cpg * pl.pitch * sizeof(T) + 15) / 16 * 16;
+        // (a part more where one is too much for the LDS)
+        more = !pl.ragged && tune_writers == 0 && may_share && pl.lds > kGnTokMaxLds && w < 8;
+    }
+    while (pl.writers > 1 && (size_t)(pl.writers - 1) * pl.part_pos >= hw) {  // no empty part
+        pl.writers /= 2;
+        const size_t vecs = (hw / EPV + pl.writers - 1) / pl.writers;
+        pl.part_pos = (uint32_t)(pl.ragged ? (hw + pl.writers - 1) / pl.writers : vecs * EPV);
+        if (!pl.ragged) pl.pitch = (uint32_t)(vecs * EPV + EPV);
+        pl.lds = (cpg * pl.pitch * sizeof(T) + 15) / 16 * 16;
+    }
+    if (pl.lds > kGnTokMaxLds) return pl;
+    const uint32_t max_k = sizeof(T) == 4 ? 10 : kGnMaxRaggedK;
+    // (writers that a knob asks for get the lanes of a launch with a workgroup per CU)
+    const size_t blocks = tune_writers > 0 ? std::min(units * pl.writers, (size_t)chip.cus) : units * pl.writers;
+    const GnThreads t = gn_threads_for(chip, sizeof(T), (uint32_t)(unit_size / EPV), 1, blocks, max_k, false, pl.writers > 1);
+    pl.threads = t.threads;
+    pl.k = t.threads < run / 4 ? 0 : (uint32_t)t.k;  // (a lane per word of an output run)
+    return pl;
+}
+
 template <typename T, int K>
-void gn_tokens_launch(bool shared, uint32_t blocks, uint32_t threads, size_t lds_bytes, hipStream_t stream,
+void gn_tokens_unit_launch(const GnTokUnitPlan &pl, uint32_t blocks, hipStream_t stream, const T *x, T *y, const float *gamma,
+                           const float *beta, const GnTokUnitParams &q) {
+    launch((pl.ragged ? gn_tokens_unit_kernel<T, K, true> : gn_tokens_unit_kernel<T, K, false>), dim3(blocks),
+           dim3(pl.threads), pl.lds, stream, x, y, gamma, beta, q);
+}
+
+template <typename T>
+int gn_tokens_unit(const GnTokUnitPlan &pl, const Chip &chip, const T *x, T *y, const float *gamma, const float *beta,
+                   size_t units, size_t channels, size_t hw, size_t groups, float eps, hipStream_t stream) {
+    constexpr uint32_t EPV = Store<T>::EPV;
+    const size_t cpg = channels / groups, unit_size = cpg * hw;
+    GnTokUnitParams q;
+    q.vec_per_unit = (uint32_t)(unit_size / EPV);
+    q.groups = (uint32_t)groups;
+    q.ch_per_group = (uint32_t)cpg;
+    q.channels = (uint32_t)channels;
+    q.hw = (uint32_t)hw;
+    q.writers = pl.writers;
+    q.writers_shift = (uint32_t)__builtin_ctz(pl.writers);
+    q.xcd_shift = gn_xcd_shift(chip, true, units);
+    q.units_per_xcd = (uint32_t)(units >> q.xcd_shift);
+    q.part_pos = pl.part_pos;
+    q.pitch = pl.pitch;
+    q.hw_vec = make_fast_div(pl.ragged ? 1u : (uint32_t)hw / EPV);
+    q.row_dwords = make_fast_div((uint32_t)(cpg * sizeof(T) / 4));
+    q.row_step = pl.threads / q.row_dwords.d;
+    q.eps = eps;
+    q.inv_count = 1.0f / (float)unit_size;
+    const uint32_t blocks = (uint32_t)(units * pl.writers);
+    switch (pl.k) {
+        case 1: gn_tokens_unit_launch<T, 1>(pl, blocks, stream, x, y, gamma, beta, q); break;
+        case 2: gn_tokens_unit_launch<T, 2>(pl, blocks, stream, x, y, gamma, beta, q); break;
+        case 3: gn_tokens_unit_launch<T, 3>(pl, blocks, stream, x, y, gamma, beta, q); break;
+        case 4: gn_tokens_unit_launch<T, 4>(pl, blocks, stream, x, y, gamma, beta, q); break;
+        case 5: gn_tokens_unit_launch<T, 5>(pl, blocks, stream, x, y, gamma, beta, q); break;
+        case 6: gn_tokens_unit_launch<T, 6>(pl, blocks, stream, x, y, gamma, beta, q); break;
+        case 8: gn_tokens_unit_launch<T, 8>(pl, blocks, stream, x, y, gamma, beta, q); break;
+        case 10: gn_tokens_unit_launch<T, 10>(pl, blocks, stream, x, y, gamma, beta, q); break;
+        case 12: gn_tokens_unit_launch<T, 12>(pl, blocks, stream, x, y, gamma, beta, q); break;
+        default: gn_tokens_unit_launch<T, 16>(pl, blocks, stream, x, y, gamma, beta, q); break;
+    }
+    return launch_status();
+}
+
+template <typename T, int K>
+void gn_tokens_launch(uint32_t blocks, uint32_t threads, size_t lds_bytes, hipStream_t stream,
                       const T *x, T *y, const float *gamma, const float *beta, const GnScratch &sc,
                       const GnTokParams &q) {
-    if (K <= kGnSharedMaxK && shared) {
-        constexpr int KS = K <= kGnSharedMaxK ? K : 1;  // (no instances with several writers beyond that)
-        launch((gn_tokens_kernel<T, KS, true>), dim3(blocks), dim3(threads), lds_bytes, stream, x, y,
-                           gamma, beta, sc, q);
-    } else {
-        launch((gn_tokens_kernel<T, K, false>), dim3(blocks), dim3(threads), lds_bytes, stream, x, y,
-                           gamma, beta, sc, q);
-    }
+    launch((gn_tokens_kernel<T, K>), dim3(blocks), dim3(threads), lds_bytes, stream, x, y, gamma, beta, sc, q);
+}
+
+// Whether gn_tokens_unit_kernel is the better one launch for a shape it can take: its units are loaded once per writer and
+// held by one workgroup, so they may be the longer the fewer there are.  us, the kernels below (slices with an exchange, or
+// one workgroup per unit and 4 K positions; two launches for `halves`) and this one: fp16 640 channels, batch 2, at 24 x 24
+// 4.9 / 3.8, 36 x 28 7.2 / 4.6, 40 x 40 6.8 / 5.5, batch 8 at 32 x 32 8.9 / 7.9; 1280 at 18 x 14 batch 2 5.6 / 3.7, 8 8.0 / 5.3, at
+// 24 x 24 batch 2 6.4 / 5.0; fp32 640 at 32 x 32 batch 2 6.5 / 5.7, 16 24.3 / 22.6, 1280 at 18 x 14 batch 2 7.8 / 4.4.
+// Above the limits (ratio of this one to the others over 8000 random shapes, by KB a unit): up to half a unit per CU 128: 0.96,
+// 136: 1.01, 152: 1.03; up to one 104: 0.83, 112: 0.88, 120: 1.1 - 1.3; more 64: 0.95, 72: 1.0, 80: 1.0, 88: 1.1.
+// Ragged planes: the 2-byte ones whose rows are whole halves of a vector (others keep the two launches, though 2 x 1280 x 63
+// would take 2.7 us instead of 5.1), short runs of many units not (128 channels at 5732 batch 10 13.9 / 18.6).
+inline bool gn_tokens_stays_whole(const Chip &chip, size_t elt, size_t units, size_t unit_size, size_t cpg, size_t hw) {
+    if (hw * elt % 16 != 0 && (elt != 2 || hw % 4 != 0 || (cpg * elt < 40 && units > chip.cus))) return false;
+    const size_t limit = units * 2 <= chip.cus ? 128 : units <= chip.cus ? 112 : 72;
+    return unit_size * elt <= limit * 1024;
 }
 
 // Where the one-launch kernel can run, two launches (1.5 - 2 us more for the smallest tensors) pay when
@@ -1048,11 +1221,11 @@ void gn_tokens_launch(bool shared, uint32_t blocks, uint32_t threads, size_t lds
 // Over 2800 random shapes of 1280 and more elements per unit what this takes is 0.955 of the one launch on average;
 // 23 are more than 1.1 times it (to 1.29: fp16 640 at 1232 batch 16 18.9 against 14.6).
 inline bool gn_tokens_prefers_two(const Chip &chip, size_t elt, size_t unit_size, size_t units, size_t cpg, size_t hw,
-                                  size_t blocks, size_t part_vecs) {
+                                  size_t blocks, size_t part_vecs, bool whole) {
     const size_t tiled = (hw + kTile - 1) / kTile * kTile, bytes = units * unit_size * elt;
     if (hw * 16 < tiled * 15) return false;
     if (cpg * elt <= 40)
-        return unit_size > 20480 || (unit_size >= 12288 && blocks * 2 < chip.cus) || bytes >= (size_t)24 << 20;
+        return unit_size > 20480 || (!whole && unit_size >= 12288 && blocks * 2 < chip.cus) || bytes >= (size_t)24 << 20;
     if (bytes < (size_t)24 << 20 || hw * elt % 128 != 0) return false;
     const size_t rounds = (blocks + chip.cus - 1) / chip.cus;
     return rounds * 2 > 3 * elt || blocks * 100 <= rounds * chip.cus * 97 || part_vecs % 2 != 0 ||
@@ -1115,7 +1288,6 @@ int gn_tokens_dispatch(const void *xv, void *yv, const float *gamma, const float
                        size_t channels, size_t hw, size_t groups, float eps, float2 *partials, hipStream_t stream) {
     constexpr int EPV = Store<T>::EPV;
     constexpr uint32_t kMaxK = sizeof(T) == 4 ? 10 : kGnMaxRaggedK;
-    constexpr size_t kMaxLds = 60 * 1024;
     const T *x = static_cast<const T *>(xv);
     T *y = static_cast<T *>(yv);
     const size_t cpg = channels / groups;
@@ -1139,8 +1311,17 @@ int gn_tokens_dispatch(const void *xv, void *yv, const float *gamma, const float
                            (uint32_t)cpg, eps);
         return launch_status();
     };
-    const bool vector_ok = aligned16(x) && (reinterpret_cast<uintptr_t>(y) & 3u) == 0 && hw % EPV == 0 &&
-                           (cpg * sizeof(T)) % 4 == 0 && (channels * sizeof(T)) % 4 == 0;
+    const Chip chip = chip_info();
+    const int tune_split = g_tuning.gn_split.load(std::memory_order_relaxed);
+    const int tune_writers = g_tuning.gn_writers.load(std::memory_order_relaxed);
+    const bool words_ok = aligned16(x) && (reinterpret_cast<uintptr_t>(y) & 3u) == 0;
+    // whole units, unless a knob asks for slices (or for what one writer does without sharing: slices)
+    GnTokUnitPlan unit{};
+    if (words_ok && tune_split <= 1 && tune_writers != 1) unit = gn_tokens_unit_plan<T>(chip, units, cpg, hw, tune_writers);
+    const bool whole = unit.k != 0 && (tune_writers > 1 || tune_split == 1 || gn_tokens_stays_whole(chip, sizeof(T), units, unit_size, cpg, hw));
+    auto in_one = [&]() { return gn_tokens_unit<T>(unit, chip, x, y, gamma, beta, units, channels, hw, groups, eps, stream); };
+    const bool vector_ok = words_ok && hw % EPV == 0 && (cpg * sizeof(T)) % 4 == 0 && (channels * sizeof(T)) % 4 == 0;
+    if (whole && (!vector_ok || tune_writers > 1 || tune_split == 1)) return in_one();
     if (!vector_ok) return generic();
     const size_t hw_vec = hw / EPV;
     // slices cut the positions: the split must divide them, fit the registers and the LDS.
@@ -1149,13 +1330,11 @@ int gn_tokens_dispatch(const void *xv, void *yv, const float *gamma, const float
     // is worth more than the exchange costs from 16 Ki elements on.  With half a workgroup per CU
     // or more, units stay whole or (exactly half) go in two; four slices otherwise, eight when
     // even that leaves a quarter of the chip idle and a slice keeps 4 Ki elements.
-    const Chip chip = chip_info();
     uint32_t want = 1;
     if (unit_size > 16384) {
         want = units * 2 > chip.cus ? 1 : units * 2 == chip.cus ? 2 : 4;
         if (units * 16 < 3 * (size_t)chip.cus && unit_size >= 32768) want = 8;
     }
-    const int tune_split = g_tuning.gn_split.load(std::memory_order_relaxed);
     const int tune_spin = g_tuning.gn_spin_limit.load(std::memory_order_relaxed);
     if (tune_split > 0) want = (uint32_t)tune_split;
     uint32_t split = 0;
@@ -1163,53 +1342,23 @@ int gn_tokens_dispatch(const void *xv, void *yv, const float *gamma, const float
         if (hw_vec % s != 0) break;
         const size_t nvec = cpg * (hw_vec / s);
         const size_t lds = cpg * (hw / s + 16 / sizeof(T)) * sizeof(T);
-        if (nvec > (size_t)kGnMaxThreads * kMaxK || lds > kMaxLds) continue;
+        if (nvec > (size_t)kGnMaxThreads * kMaxK || lds > kGnTokMaxLds) continue;
         split = s;
         if (s >= want) break;
     }
-    // Several writers per whole unit instead of slices with an exchange (see gn_auto_writers): the
-    // parts cut the positions like slices do, must divide them, hold whole wavefronts' vectors
-    // and fit the LDS; the whole unit must fit the registers of one workgroup.
-    const int tune_writers = g_tuning.gn_writers.load(std::memory_order_relaxed);
-    uint32_t writers = 1;
-    const size_t vec_per_unit = cpg * hw_vec;
-    const char *xb = reinterpret_cast<const char *>(x), *yb = reinterpret_cast<const char *>(y);
-    const size_t bytes = units * unit_size * sizeof(T);
-    const bool apart = xb + bytes <= yb || yb + bytes <= xb;
-    if (apart && tune_split <= 1 && tune_writers != 1 && vec_per_unit <= (size_t)kGnMaxThreads * kGnSharedMaxK) {
-        uint32_t w = tune_writers > 1 ? (uint32_t)tune_writers : gn_auto_writers(chip, sizeof(T), units, vec_per_unit);
-        // Here the limit is lower than for the channel-major store: the slices of a cut unit
-        // also keep the writers of an output line on one XCD, which the writers of a unit give
-        // up.  Measured, batch 2 fp16, several writers against slices: 1280 channels at 16 x 16
-        // 4.03 against 4.64 us, 640 at 32 x 32 5.79 against 6.11, 320 at 64 x 64 9.14 against
-        // 7.90; batch 4 (two writers): 4.72 against 5.13, 7.45 against 7.07.
-        if (tune_writers <= 1 && unit_size > (w >= 4 ? 20480u : 10240u)) w = 1;
-        for (; w > 1; w /= 2) {
-            if (hw_vec % w != 0) continue;
-            const size_t part_len = cpg * (hw_vec / w);
-            const size_t lds = cpg * (hw / w + 16 / sizeof(T)) * sizeof(T);
-            if (part_len % kWave == 0 && lds <= kMaxLds) break;
-        }
-        writers = (w < 1 || units * w > 0x7FFFFFFFull) ? 1 : w;  // (the grid is units * writers blocks)
-        if (writers > 1 &&
-            gn_threads_for(chip, sizeof(T), (uint32_t)vec_per_unit, 1, units * writers, kGnSharedMaxK, true, true).k == 0)
-            writers = 1;  // (the whole unit does not fit one workgroup's registers: slices as below)
-    }
-    const bool shared = writers > 1;
-    if (!shared && (split == 0 || (split > 1 && units > kGnMaxUnits))) return generic();
-    if (shared) split = 1;
+    if (split == 0 || (split > 1 && units > kGnMaxUnits)) return whole ? in_one() : generic();
 
     GnTokParams q;
-    const size_t pvs = hw_vec / (shared ? writers : split);  // position vectors of a part / slice
+    const size_t pvs = hw_vec / split;  // position vectors of a slice
     const size_t nvec = cpg * pvs;
-    q.base.vec_per_unit = (uint32_t)vec_per_unit;
+    q.base.vec_per_unit = (uint32_t)(cpg * hw_vec);
     q.base.vec_per_slice = (uint32_t)nvec;
     q.base.split = split;
     q.base.split_shift = (uint32_t)__builtin_ctz(split);
-    q.base.writers = writers;
-    q.base.writers_shift = (uint32_t)__builtin_ctz(writers);
+    q.base.writers = 1;
+    q.base.writers_shift = 0;
     q.base.part_vecs = (uint32_t)nvec;
-    q.base.xcd_shift = gn_xcd_shift(chip, shared, units);
+    q.base.xcd_shift = 0;
     q.base.groups = (uint32_t)groups;
     q.base.ch_per_group = (uint32_t)cpg;
     q.base.hw_vec = make_fast_div((uint32_t)hw_vec);
@@ -1222,35 +1371,33 @@ int gn_tokens_dispatch(const void *xv, void *yv, const float *gamma, const float
     q.channels = (uint32_t)channels;
     q.pitch = (uint32_t)(pvs * EPV + 16 / sizeof(T));
     q.combos = make_fast_div((uint32_t)(batch * split));
-    q.part_len = make_fast_div((uint32_t)nvec);
     const size_t lds_bytes = cpg * q.pitch * sizeof(T);
-    // a workgroup holds its slice, or with several writers the whole unit
-    const GnThreads pl = shared ? gn_threads_for(chip, sizeof(T), (uint32_t)vec_per_unit, 1, units * writers, kGnSharedMaxK,
-                                                 true, true)
-                                : gn_threads_for(chip, sizeof(T), (uint32_t)nvec, split, units * split, kMaxK, false, false);
-    if (pl.k == 0) return generic();
-    const uint32_t blocks = (uint32_t)(units * (shared ? writers : split));
-    if (tune_split == 0 && tune_writers == 0 && gn_tokens_prefers_two(chip, sizeof(T), unit_size, units, cpg, hw, blocks, pvs)) {
+    const GnThreads pl = gn_threads_for(chip, sizeof(T), (uint32_t)nvec, split, units * split, kMaxK, false, false);
+    if (pl.k == 0) return whole ? in_one() : generic();
+    const uint32_t blocks = (uint32_t)(units * split);
+    if (tune_split == 0 && tune_writers == 0 &&
+        gn_tokens_prefers_two(chip, sizeof(T), unit_size, units, cpg, hw, blocks, pvs, whole)) {
         int status = MSD_OK;
         if (gn_tokens_two_launches<T>(x, y, gamma, beta, batch, channels, hw, groups, eps, partials, stream, &status)) return status;
     }
+    if (whole) return in_one();
     GnScratch sc{};
-    if (!shared && split > 1) {
+    if (split > 1) {
         const hipError_t err = get_scratch(stream, &sc);
         if (err != hipSuccess) return (int)err;
     }
     const uint32_t threads = pl.threads;
     switch (pl.k) {
-        case 1: gn_tokens_launch<T, 1>(shared, blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q); break;
-        case 2: gn_tokens_launch<T, 2>(shared, blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q); break;
-        case 3: gn_tokens_launch<T, 3>(shared, blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q); break;
-        case 4: gn_tokens_launch<T, 4>(shared, blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q); break;
-        case 5: gn_tokens_launch<T, 5>(shared, blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q); break;
-        case 6: gn_tokens_launch<T, 6>(shared, blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q); break;
-        case 8: gn_tokens_launch<T, 8>(shared, blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q); break;
-        case 10: gn_tokens_launch<T, 10>(shared, blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q); break;
-        case 12: gn_tokens_launch<T, 12>(shared, blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q); break;
-        default: gn_tokens_launch<T, 16>(shared, blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q); break;
+        case 1: gn_tokens_launch<T, 1>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q); break;
+        case 2: gn_tokens_launch<T, 2>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q); break;
+        case 3: gn_tokens_launch<T, 3>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q); break;
+        case 4: gn_tokens_launch<T, 4>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q); break;
+        case 5: gn_tokens_launch<T, 5>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q); break;
+        case 6: gn_tokens_launch<T, 6>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q); break;
+        case 8: gn_tokens_launch<T, 8>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q); break;
+        case 10: gn_tokens_launch<T, 10>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q); break;
+        case 12: gn_tokens_launch<T, 12>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q); break;
+        default: gn_tokens_launch<T, 16>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q); break;
     }
     return launch_status();
 }

@@ -192,6 +192,37 @@ def test_groupnorm_tokens_equals_norm_then_permute(msd, orc, cuda, shape, groups
     assert msd.status() == 0
 
 
+@pytest.mark.parametrize("mean", [0.4, 60.0], ids=["", "far-mean"])  # 60: the statistics take their second pass
+@pytest.mark.parametrize("shape,groups,half", [
+    ((2, 640, 36, 28), 32, True), ((2, 640, 24, 24), 32, True), ((1, 1280, 24, 24), 32, True),  # parts of unequal length
+    ((2, 640, 32, 32), 32, False), ((3, 320, 10, 8), 32, False), ((1, 1280, 16, 8), 32, False),
+    ((2, 1280, 18, 14), 32, True), ((5, 1280, 18, 22), 32, True), ((9, 640, 6, 10), 32, True),  # vectors across channels
+    ((1, 1280, 2, 2), 32, True), ((3, 136, 6, 6), 17, True), ((3, 136, 6, 6), 17, False),       # rows of half a vector; 17 groups
+    ((16, 64, 16, 16), 32, True), ((7, 96, 4, 4), 96, False), ((33, 64, 8, 8), 32, True),       # one word per position; odd batches
+    ((5, 1280, 28, 28), 32, True), ((1, 1280, 40, 40), 32, True)])                              # a part more for the LDS; long units
+def test_groupnorm_tokens_of_whole_units(msd, orc, cuda, shape, groups, half, mean):
+    """One launch in which every workgroup reduces whole units: against the oracle in 64 bits, eagerly and recorded."""
+    import torch
+    batch, channels, hw = shape[0], shape[1], shape[2] * shape[3]
+    x = orc.normal(shape, seed=sum(shape) + 9, sigma=1.5, mean=mean)
+    g, b = _affine(orc, channels, 27)
+    xin = orc.round_to_half(x) if half else x
+    ref = orc.groupnorm64(xin, g, b, groups, 1e-6, False).astype(np.float32).reshape(batch, channels, hw).transpose(0, 2, 1)
+    xd, gd, bd = _dev(xin, cuda, half), _dev(g, cuda), _dev(b, cuda)
+    assert not _takes_two_launches(msd, xd, gd, bd, groups)
+    eager = msd.groupnorm_tokens(xd, gd, bd, groups, 1e-6)
+    (assert_close_f16 if half else assert_close_f32)(eager.float().cpu().numpy(), ref, what="gn tokens, whole units")
+    graph, stream = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.graph(graph, stream=stream):
+        recorded = msd.groupnorm_tokens(xd, gd, bd, groups, 1e-6)
+    for _ in range(3):
+        recorded.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(recorded, eager)
+
+
 @pytest.mark.parametrize("shape", [(2, 320, 71, 70),                        # cut into slices outside a capture; whole in it
                                    (2, 640, 63, 63), (1, 640, 127, 65)])    # longer than one workgroup holds
 def test_groupnorm_of_no_whole_vectors_is_recorded_without_scratch(msd, orc, cuda, shape):
