@@ -8,12 +8,14 @@ streams, nothing else.  There is no fallback: if the library was not built
 the loader raises.
 """
 import ctypes
+import importlib.util
 import os
 
 _PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 CSRC_DIR = os.path.join(_PKG_DIR, "csrc")
 LIB_HIP_PATH = os.path.join(CSRC_DIR, "libmsd_hip.so")
 LIB_NN_PATH = os.path.join(CSRC_DIR, "libmsd_nn.so")
+TORCH_CALLS_PATH = os.path.join(CSRC_DIR, "msd_torch_calls.so")
 
 DTYPE_F32 = 0
 DTYPE_F16 = 1
@@ -91,6 +93,8 @@ def load_library(path=None):
         if name != "msd_error_string":
             getattr(lib, name).restype = it
     _lib = lib
+    if not isinstance(_native, _Unbound):
+        _bind_addresses(_native)
     return lib
 
 
@@ -100,11 +104,41 @@ def check(code):
                        % (code, load_library().msd_error_string(code).decode()))
 
 
-# What a call does on the host is most of a small call's time (a LayerNorm of 154 rows: 8 us of host work
-# around a kernel of 2.5), so it is kept short: torch and its raw-stream query are looked up once, pointers
-# and streams are passed as plain numbers, an output made here from a checked input is not checked again.
-# Eager passes, us, before and now: the 49 calls of a text encoder 486 -> 304, the 8 calls of a 640-channel
-# transformer block 81.6 -> 52.8, 22 grouped projections 70.4 -> 52.2.
+# What a call does on the host is most of a small call's time (a LayerNorm of 154 rows: a kernel of 2.2 us behind 2.5 to
+# 3.5 us of the runtime's launch), so plain calls (dense device tensors that fit each other, no mode or transform around
+# them) go through csrc/torch_calls.cpp, which checks them, makes the outputs and calls the C ABI; it returns None for any
+# other, which the general path below it then makes or refuses.  Eager passes, us, from Python and so: four calls of a
+# sampler's tick 24.8 -> 16.4, the 49 of a text encoder 322 -> 237, 22 grouped projections 53 -> 19.5, the 8 of a
+# 640-channel transformer block 53.5 -> 38.
+class _Unbound:
+    """Stands for the native calls until the first one."""
+
+    def __getattr__(self, name):
+        return getattr(_bind_native(), name)
+
+
+_native = _Unbound()
+
+
+def _bind_addresses(native):
+    native.bind({name: ctypes.cast(getattr(_lib, name), ctypes.c_void_p).value for name in native.names()}, check)
+
+
+def _bind_native():
+    global _native
+    load_library()
+    _bind_torch()  # the extension's symbols are torch's
+    if isinstance(_native, _Unbound):
+        if not os.path.exists(TORCH_CALLS_PATH):
+            raise MsdError("native library %s is missing: run __graft_entry__.build()" % TORCH_CALLS_PATH)
+        spec = importlib.util.spec_from_file_location("msd_torch_calls", TORCH_CALLS_PATH)
+        native = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(native)
+        _bind_addresses(native)
+        _native = native
+    return _native
+
+
 _torch = None
 _dtype_codes = {}
 _raw_stream = _current_device = _capturing = None
@@ -200,6 +234,9 @@ def _planes(x):
 def groupnorm(x, gamma, beta, groups, eps=1e-5, fuse_silu=False, out=None, noalloc=False):
     """x: [batch, C, ...] device tensor; gamma/beta float32 [C]; out may be x (in place).
     noalloc: go through msd_groupnorm_noalloc (fixed scratch, batch * groups <= 1024)."""
+    done = _native.groupnorm(x, gamma, beta, groups, eps, fuse_silu, out, noalloc)
+    if done is not None:
+        return done
     lib = _lib or load_library()
     batch, channels, hw = _planes(x)
     xp = _dev(x)
@@ -223,6 +260,9 @@ def groupnorm_plan(batch, channels, hw, groups=32, dtype_code=DTYPE_F16, noalloc
 
 def groupnorm_tokens(x, gamma, beta, groups, eps=1e-6):
     """x: [batch, C, ...] -> [batch, H*W, C] = GroupNorm(x) with channels last (no SiLU)."""
+    done = _native.groupnorm_tokens(x, gamma, beta, groups, eps)
+    if done is not None:
+        return done
     lib = _lib or load_library()
     batch, channels, hw = _planes(x)
     xp = _dev(x)
@@ -241,6 +281,9 @@ def groupnorm_tokens(x, gamma, beta, groups, eps=1e-6):
 
 def permute_0_2_1(x):
     """[i, j, k] -> [i, k, j] (new tensor)."""
+    done = _native.permute_0_2_1(x)
+    if done is not None:
+        return done
     lib = _lib or load_library()
     i, j, k = x.shape
     xp = _dev(x)
@@ -251,6 +294,9 @@ def permute_0_2_1(x):
 
 def chunk_add_groupnorm(x, chunk, gamma, beta, groups, eps=1e-5, fuse_silu=False, out=None):
     """GroupNorm(x + chunk[:, :, None]) (+ SiLU); chunk: [batch, C] in x's dtype."""
+    done = _native.chunk_add_groupnorm(x, chunk, gamma, beta, groups, eps, fuse_silu, out)
+    if done is not None:
+        return done
     lib = _lib or load_library()
     batch, channels, hw = _planes(x)
     xp = _dev(x)
@@ -263,6 +309,9 @@ def chunk_add_groupnorm(x, chunk, gamma, beta, groups, eps=1e-5, fuse_silu=False
 
 def add_layernorm(a, b, gamma, beta, eps=1e-5, sum_out=None, out=None):
     """Returns (a + b, LayerNorm(a + b)); sum_out may be a or b."""
+    done = _native.add_layernorm(a, b, gamma, beta, eps, sum_out, out)
+    if done is not None:
+        return done
     lib = _lib or load_library()
     n, dim = a.numel(), a.shape[-1]
     rows = n // dim if dim else 0
@@ -275,6 +324,9 @@ def add_layernorm(a, b, gamma, beta, eps=1e-5, sum_out=None, out=None):
 
 
 def elemwise_add(a, b, out=None):
+    done = _native.elemwise_add(a, b, out)
+    if done is not None:
+        return done
     lib = _lib or load_library()
     n = a.numel()
     ap, bp = _dev(a), _same(b, a, n, "b")
@@ -284,6 +336,9 @@ def elemwise_add(a, b, out=None):
 
 
 def chunkwise_add(a, chunk, chunk_size, out=None):
+    done = _native.chunkwise_add(a, chunk, chunk_size, out)
+    if done is not None:
+        return done
     lib = _lib or load_library()
     n = a.numel()
     if chunk_size <= 0 or n % chunk_size:
@@ -295,6 +350,9 @@ def chunkwise_add(a, chunk, chunk_size, out=None):
 
 
 def layernorm(x, gamma, beta, eps=1e-5, out=None):
+    done = _native.layernorm(x, gamma, beta, eps, out)
+    if done is not None:
+        return done
     lib = _lib or load_library()
     dim = x.shape[-1]
     rows = x.numel() // dim if dim else 0
@@ -307,6 +365,9 @@ def layernorm(x, gamma, beta, eps=1e-5, out=None):
 
 def geglu(proj, out=None):
     """proj: [..., 2*inner] (value | gate) -> [..., inner]."""
+    done = _native.geglu(proj, out)
+    if done is not None:
+        return done
     lib = _lib or load_library()
     shape = proj.shape
     inner = shape[-1] // 2
@@ -327,22 +388,30 @@ def _act(name, x, out):
 
 
 def silu(x, out=None):
-    return _act("msd_silu", x, out)
+    done = _native.silu(x, out)
+    return done if done is not None else _act("msd_silu", x, out)
 
 
 def gelu(x, out=None):
-    return _act("msd_gelu", x, out)
+    done = _native.gelu(x, out)
+    return done if done is not None else _act("msd_gelu", x, out)
 
 
 def quick_gelu(x, out=None):
-    return _act("msd_quick_gelu", x, out)
+    done = _native.quick_gelu(x, out)
+    return done if done is not None else _act("msd_quick_gelu", x, out)
 
 
 def timestep_embedding(timesteps, dim, max_period=10000.0, dtype=None):
     """timesteps: int64 device tensor [batch] -> [batch, dim] as [cos | sin]."""
+    torch = _torch or _bind_torch()
+    if dtype is None or dtype is torch.float32 or dtype is torch.float16:
+        done = _native.timestep_embedding(timesteps, dim, max_period, dtype is torch.float16)
+        if done is not None:
+            return done
     lib = _lib or load_library()
     n = timesteps.numel()
-    out = timesteps.new_empty((n, dim), dtype=dtype or (_torch or _bind_torch()).float32)
+    out = timesteps.new_empty((n, dim), dtype=dtype or torch.float32)
     check(lib.msd_timestep_embedding(_dev(timesteps), _dev(out), n, dim, max_period, _dtype_code(out), _stream()))
     return out
 
@@ -360,6 +429,9 @@ def ddim_timesteps(steps):
 
 def linear_rows(x, weight, bias=None, act_in=ACT_NONE, act_out=ACT_NONE, out=None):
     """x [m <= 8, k], weight [n, k] (x's dtype), bias float32 [n] or None -> [m, n]."""
+    done = _native.linear_rows(x, weight, bias, act_in, act_out, out)
+    if done is not None:
+        return done
     lib = _lib or load_library()
     m, k = x.shape
     n = weight.shape[0]
@@ -377,6 +449,9 @@ def linear_rows(x, weight, bias=None, act_in=ACT_NONE, act_out=ACT_NONE, out=Non
 def linear_rows_grouped(x, weights, biases=None, act_in=ACT_NONE, act_out=ACT_NONE):
     """One launch for several Linear layers on the same x [m <= 8, k]: weights[i] is [n_i, k] in
     x's dtype, biases[i] float32 [n_i] or None -> list of [m, n_i] tensors."""
+    done = _native.linear_rows_grouped(x, weights, biases, act_in, act_out)
+    if done is not None:
+        return done
     lib = _lib or load_library()
     m, k = x.shape
     xp, dtype, device, new = _dev(x), x.dtype, x.get_device(), x.new_empty
@@ -404,6 +479,9 @@ def linear_rows_grouped(x, weights, biases=None, act_in=ACT_NONE, act_out=ACT_NO
 
 def softmax(x, stable=False, out=None):
     """Softmax over the last axis; out may be x (in place)."""
+    done = _native.softmax(x, stable, out)
+    if done is not None:
+        return done
     lib = _lib or load_library()
     cols = x.shape[-1]
     rows = x.numel() // cols if cols else 0
@@ -434,6 +512,9 @@ def ddim_schedule(steps):
 
 def ddim_update(x, e_t, a_t, a_prev, sqrt_one_minus_at, out=None):
     """One DDIM step (eta 0) on device tensors; out may be x."""
+    done = _native.ddim_update(x, e_t, a_t, a_prev, sqrt_one_minus_at, out)
+    if done is not None:
+        return done
     lib = _lib or load_library()
     n = x.numel()
     xp, ep = _dev(x), _same(e_t, x, n, "e_t")

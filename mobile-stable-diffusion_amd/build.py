@@ -2,6 +2,7 @@
 
     libmsd_hip.so   HIP kernels + the C ABI declared in include/msd_hip.h
     libmsd_nn.so    C++ host layer objects (GroupNorm / LayerNorm / GEGLU / ...) on top of it
+    msd_torch_calls.so  the package's calls for plain torch tensors (a CPython extension, host only)
     cli/msd_compare golden-file comparison tool (host only)
     cli/msd_layer_check  runs the layer objects against golden .npy files (needs a GPU)
 
@@ -27,6 +28,7 @@ DEVICE_FLAGS = [
 
 LIB_HIP = os.path.join(CSRC, "libmsd_hip.so")
 LIB_NN = os.path.join(CSRC, "libmsd_nn.so")
+TORCH_CALLS = os.path.join(CSRC, "msd_torch_calls.so")
 CLI_COMPARE = os.path.join(CSRC, "cli", "msd_compare")
 CLI_LAYER_CHECK = os.path.join(CSRC, "cli", "msd_layer_check")
 
@@ -74,6 +76,19 @@ def build_nn():
     return LIB_NN
 
 
+def build_torch_calls():
+    """msd_torch_calls.so: host C++ against the headers and libraries of the torch that will import it."""
+    import importlib.util
+    import sysconfig
+    torch_dir = importlib.util.find_spec("torch").submodule_search_locations[0]
+    _run([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__",
+          "-Wall", "-Wno-deprecated-declarations", "-isystem", os.path.join(torch_dir, "include"),
+          "-isystem", "/opt/rocm/include", "-isystem", sysconfig.get_paths()["include"],
+          os.path.join(CSRC, "torch_calls.cpp"), "-o", TORCH_CALLS, "-L", os.path.join(torch_dir, "lib"), "-ltorch_python",
+          "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip", "-L/opt/rocm/lib", "-lamdhip64"])
+    return TORCH_CALLS
+
+
 def build_cli():
     """msd_compare: host-only golden-file comparison tool (no HIP, no GPU)."""
     nn_dir = os.path.join(CSRC, "nn")
@@ -97,6 +112,7 @@ def build_all(verbose=True):
     nn = build_nn()
     if nn:
         built.append(nn)
+    built.append(build_torch_calls())
     built.append(build_cli())
     if nn:
         built.append(build_layer_check())
