@@ -15,8 +15,16 @@ namespace {
 constexpr int kStreamThreads = 256;
 // GEGLU runs one wavefront per workgroup: with two loads and 21 VALU instructions per element
 // in flight per lane, single-wavefront workgroups start and retire soonest (measured 4.5 %
-// faster over the step's 16 launches than 256-lane workgroups; the plain copy prefers 256).
+// faster over the step's 16 launches than 256-lane workgroups).
 constexpr int kGegluThreads = 64;
+// Lanes of a workgroup of the elementwise kernels: one wavefront when the launch has more of them than the chip holds
+// (32 per CU): it starts as soon as there is room for one and retires by itself, so the launch moves through memory in
+// order.  Shorter launches start sooner in workgroups of four.  us, 256 lanes and 64: fp16 add of 1.3 / 2.6 / 5.2 / 21 / 34 M
+// elements 2.85 / 3.95 / 7.39 / 21.8 / 33.1 and 2.83 / 4.08 / 6.91 / 20.8 / 31.8; fp32 33 M 64.3 and 62.8; copy of 4.2 / 10.5 / 42 /
+// 540 MB 2.83 / 5.09 / 15.8 / 167 and 3.16 / 4.97 / 14.5 / 163 (6.6 TB/s); embedding add at 320 x 64 x 64, batch 2, 3.12 and 3.68.
+inline uint32_t stream_lanes(size_t vecs) {
+    return vecs > 32 * (size_t)kWave * chip_info().cus ? (uint32_t)kWave : (uint32_t)kStreamThreads;
+}
 constexpr int kStreamUnroll = 1;  // vectors per lane of the elementwise kernels
 
 // out[r, c] = proj[r, c] * gelu(proj[r, inner + c]); vectors never straddle a row.
@@ -77,15 +85,16 @@ __global__ __launch_bounds__(kStreamThreads) void act_kernel(const T *x, T *y, u
     constexpr int EPV = Store<T>::EPV;
     const u32x4 *in = reinterpret_cast<const u32x4 *>(x);
     u32x4 *o = reinterpret_cast<u32x4 *>(y);
-    const uint32_t block_base = blockIdx.x * (kStreamThreads * U);
+    const uint32_t nt = blockDim.x;
+    const uint32_t block_base = blockIdx.x * (nt * U);
     const uint32_t base = block_base + threadIdx.x;
-    const bool full = block_base + kStreamThreads * U <= vecs;  // uniform
+    const bool full = block_base + nt * U <= vecs;  // uniform
     if (vecs != 0) {
         u32x4 raw[U];
         uint32_t vs[U];
 #pragma unroll
         for (int u = 0; u < U; u++) {
-            const uint32_t v = base + u * kStreamThreads;
+            const uint32_t v = base + u * nt;
             vs[u] = full ? v : min(v, vecs - 1);
             raw[u] = load_stream(in + vs[u]);
         }
@@ -96,7 +105,7 @@ __global__ __launch_bounds__(kStreamThreads) void act_kernel(const T *x, T *y, u
 #pragma unroll
             for (int e = 0; e < EPV; e++) f[e] = OP::apply(f[e]);
             const u32x4 packed = Store<T>::pack(f);
-            if (full || base + u * kStreamThreads < vecs) store_stream(o + vs[u], packed);
+            if (full || base + u * nt < vecs) store_stream(o + vs[u], packed);
         }
     }
     // ragged tail (n % EPV elements) by the first lanes of block 0
@@ -119,7 +128,7 @@ template <typename T>
 __global__ __launch_bounds__(kStreamThreads) void add_kernel(const T *a, const T *b, T *c,
                                                              uint32_t vecs, FastDiv chunk_vecs) {
     constexpr int EPV = Store<T>::EPV;
-    const uint32_t v = blockIdx.x * kStreamThreads + threadIdx.x;
+    const uint32_t v = blockIdx.x * blockDim.x + threadIdx.x;
     if (v >= vecs) return;
     float fa[EPV], fb[EPV];
     Store<T>::unpack(load_stream(reinterpret_cast<const u32x4 *>(a) + v), fa);
@@ -200,11 +209,6 @@ __global__ __launch_bounds__(256) void timestep_embedding_kernel(
 }
 
 // ---- streaming dispatch ----------------------------------------------------
-inline uint32_t stream_blocks(size_t vecs, int unroll) {
-    const size_t per_block = (size_t)kStreamThreads * unroll;
-    return (uint32_t)((vecs + per_block - 1) / per_block);
-}
-
 }  // namespace
 
 template <typename T>
@@ -251,15 +255,16 @@ int act_launch(const void *xv, void *yv, size_t n, hipStream_t stream) {
     if (aligned16(x) && aligned16(y) && vecs < 0x7FFFFFFFull) {
         const int tune_vectors = g_tuning.act_vectors.load(std::memory_order_relaxed);
         const int unroll = tune_vectors ? tune_vectors : kStreamUnroll;
-        const uint32_t blocks = vecs ? stream_blocks(vecs, unroll) : 1u;
+        const uint32_t lanes = stream_lanes(vecs);
+        const uint32_t blocks = vecs ? (uint32_t)((vecs + (size_t)lanes * unroll - 1) / ((size_t)lanes * unroll)) : 1u;
         if (unroll == 4)
-            launch((act_kernel<T, OP, 4>), dim3(blocks), dim3(kStreamThreads), 0, stream, x, y,
+            launch((act_kernel<T, OP, 4>), dim3(blocks), dim3(lanes), 0, stream, x, y,
                                (uint32_t)vecs, n);
         else if (unroll == 2)
-            launch((act_kernel<T, OP, 2>), dim3(blocks), dim3(kStreamThreads), 0, stream, x, y,
+            launch((act_kernel<T, OP, 2>), dim3(blocks), dim3(lanes), 0, stream, x, y,
                                (uint32_t)vecs, n);
         else
-            launch((act_kernel<T, OP, 1>), dim3(blocks), dim3(kStreamThreads), 0, stream, x, y,
+            launch((act_kernel<T, OP, 1>), dim3(blocks), dim3(lanes), 0, stream, x, y,
                                (uint32_t)vecs, n);
     } else {
         const size_t want = (n + kStreamThreads - 1) / kStreamThreads;
@@ -287,8 +292,8 @@ int add_dispatch(const void *av, const void *bv, void *cv, size_t n, size_t chun
         const uint32_t vecs = (uint32_t)(n / EPV);
         FastDiv fd = make_fast_div((uint32_t)(chunk_size / EPV));
         if (chunk_size == 0) fd.d = 0;
-        launch((add_kernel<T>), dim3((vecs + kStreamThreads - 1) / kStreamThreads),
-                           dim3(kStreamThreads), 0, stream, a, b, c, vecs, fd);
+        const uint32_t lanes = stream_lanes(vecs);
+        launch((add_kernel<T>), dim3((vecs + lanes - 1) / lanes), dim3(lanes), 0, stream, a, b, c, vecs, fd);
     } else {
         const size_t want = (n + kStreamThreads - 1) / kStreamThreads;
         launch((add_generic_kernel<T>), dim3((uint32_t)(want < 65536 ? want : 65536)),

@@ -535,3 +535,25 @@ def test_fused_argument_checks(msd, cuda):
     x = torch.zeros(32 * 64, device=cuda)
     p = ctypes.c_void_p(x.data_ptr())
     assert lib.msd_groupnorm_tokens(p, p, p, p, 1, 32, 64, 32, 1e-6, 0, None) == 1  # y must not be x
+
+
+@pytest.mark.parametrize("half", [False, True], ids=["f32", "f16"])
+@pytest.mark.parametrize("extra", [-1, 0, 1, 65])
+def test_elementwise_launches_around_a_full_chip(msd, cuda, extra, half):
+    """Vectors on both sides of as many as the chip's wavefronts hold (256 CUs), from where on a workgroup is one wavefront, with
+    elements left over: the bits of short launches."""
+    import torch
+    dtype, epv = (torch.float16, 8) if half else (torch.float32, 4)
+    vecs, left = 32 * 64 * 256 + extra, epv - 1
+    g = torch.Generator(device=cuda).manual_seed(extra + 7)
+    x, y = (torch.randn(vecs * epv + left, device=cuda, generator=g).to(dtype) for _ in range(2))
+    for op in (msd.silu, msd.gelu, msd.quick_gelu):
+        got = op(x)
+        for a, b in ((0, 4096), (x.numel() // 2 // 64 * 64, x.numel() // 2 // 64 * 64 + 4096), (x.numel() // 64 * 64 - 4096, x.numel())):
+            assert torch.equal(got[a:b], op(x[a:b].clone()))
+    whole = slice(0, vecs * epv)
+    assert torch.equal(msd.elemwise_add(x[whole], y[whole]), x[whole] + y[whole])
+    assert torch.equal(msd.elemwise_add(x, y), x + y)
+    chunk = vecs * epv // 4 if vecs % 4 == 0 else vecs * epv  # (whole vectors per chunk)
+    addend = torch.randn(vecs * epv // chunk, device=cuda, generator=g).to(dtype)
+    assert torch.equal(msd.chunkwise_add(x[whole], addend, chunk), (x[whole].view(-1, chunk) + addend[:, None]).view(-1))
