@@ -471,6 +471,25 @@ def test_layernorm_mid_size_launches_with_ragged_ends(msd, orc, cuda, rows, dim,
     check(got.float().cpu().numpy(), orc.layernorm64(s.astype(np.float32), g, b, 1e-5), "add + ln mid-size")
 
 
+@pytest.mark.parametrize("half", [False, True], ids=["f32", "f16"])
+@pytest.mark.parametrize("rows,dim", [(1025, 768), (1921, 1280), (2049, 768), (2967, 1024), (4097, 640), (20483, 320)])
+def test_layernorm_between_full_loads_of_wavefronts(msd, orc, cuda, rows, dim, half):
+    # one to four wavefronts per SIMD, the last of them on some SIMDs only: the workgroup's size is chosen by that, and a
+    # row's arithmetic does not depend on it
+    import torch
+    x, r = (orc.normal((rows, dim), seed=rows + dim + i, sigma=1.5, mean=0.5) for i in range(2))
+    g, b = (_to_dev(v, cuda) for v in _affine(orc, dim, dim))
+    xd, rd = _to_dev(x, cuda, half), _to_dev(r, cuda, half)
+    got = (msd.layernorm(xd, g, b),) + msd.add_layernorm(xd, rd, g, b)
+    lib = msd.load_library()
+    try:
+        assert lib.msd_set_tuning(msd.TUNE_LN_THREADS, 256) == 0
+        expected = (msd.layernorm(xd, g, b),) + msd.add_layernorm(xd, rd, g, b)
+    finally:
+        lib.msd_set_tuning(msd.TUNE_LN_THREADS, 0)
+    assert all(torch.equal(a, e) for a, e in zip(got, expected))
+
+
 @pytest.mark.parametrize("chunk,threads", [(8, 0), (16, 0), (8, 64), (16, 512), (0, 128)])
 def test_layernorm_forced_chunk_width(msd, orc, cuda, chunk, threads):
     lib = msd.load_library()
