@@ -17,13 +17,16 @@ constexpr int kStreamThreads = 256;
 // in flight per lane, single-wavefront workgroups start and retire soonest (measured 4.5 %
 // faster over the step's 16 launches than 256-lane workgroups).
 constexpr int kGegluThreads = 64;
-// Lanes of a workgroup of the elementwise kernels: one wavefront when the launch has more of them than the chip holds
-// (32 per CU): it starts as soon as there is room for one and retires by itself, so the launch moves through memory in
-// order.  Shorter launches start sooner in workgroups of four.  us, 256 lanes and 64: fp16 add of 1.3 / 2.6 / 5.2 / 21 / 34 M
-// elements 2.85 / 3.95 / 7.39 / 21.8 / 33.1 and 2.83 / 4.08 / 6.91 / 20.8 / 31.8; fp32 33 M 64.3 and 62.8; copy of 4.2 / 10.5 / 42 /
-// 540 MB 2.83 / 5.09 / 15.8 / 167 and 3.16 / 4.97 / 14.5 / 163 (6.6 TB/s); embedding add at 320 x 64 x 64, batch 2, 3.12 and 3.68.
-inline uint32_t stream_lanes(size_t vecs) {
-    return vecs > 32 * (size_t)kWave * chip_info().cus ? (uint32_t)kWave : (uint32_t)kStreamThreads;
+// Lanes of a workgroup of the elementwise kernels: one wavefront in launches with more wavefronts than the chip has room for
+// (32 per CU), where a wavefront that starts and retires by itself keeps the launch moving through memory in order.  Shorter launches
+// start sooner in workgroups of four.  Sums of two tensors gain from 22 wavefronts per CU on, where workgroups of four leave some
+// CUs one more than others; passes over one tensor from 48.  us, 256 lanes and 64, at 5200 / 6144 / 9216 / 11264 / 14336
+// wavefronts: fp16 add 4.16 / 4.95 / 6.37 / 7.87 / 9.23 and 4.15 / 4.62 / 6.00 / 7.31 / 8.71, copy 3.03 / 3.24 / 4.59 / 5.71 / 6.88 and
+// 3.60 / 3.80 / 4.69 / 5.82 / 6.62, fp32 SiLU 3.04 / 3.24 / 4.64 / 5.87 / 6.98 and 3.66 / 3.88 / 4.84 / 5.86 / 6.76; fp16 add of 34 M
+// elements 33.1 and 31.8, copy of 42 / 540 MB 15.8 / 167 and 14.5 / 163 (6.6 TB/s).
+inline uint32_t stream_lanes(size_t vecs, bool two_tensors) {
+    const size_t most = (two_tensors ? 22 : 48) * (size_t)kWave * chip_info().cus;
+    return vecs > most ? (uint32_t)kWave : (uint32_t)kStreamThreads;
 }
 constexpr int kStreamUnroll = 1;  // vectors per lane of the elementwise kernels
 
@@ -79,22 +82,20 @@ __global__ __launch_bounds__(kStreamThreads) void geglu_generic_kernel(
 
 // y[i] = OP(x[i]); y may alias x: a lane reads its vectors before it writes them,
 // and in the ragged last block the duplicated reads are never written back.
-template <typename T, typename OP, int U>
-__global__ __launch_bounds__(kStreamThreads) void act_kernel(const T *x, T *y, uint32_t vecs,
-                                                             size_t n) {
+template <typename T, typename OP, int U, int NT>
+__global__ __launch_bounds__(NT) void act_kernel(const T *x, T *y, uint32_t vecs, size_t n) {
     constexpr int EPV = Store<T>::EPV;
     const u32x4 *in = reinterpret_cast<const u32x4 *>(x);
     u32x4 *o = reinterpret_cast<u32x4 *>(y);
-    const uint32_t nt = blockDim.x;
-    const uint32_t block_base = blockIdx.x * (nt * U);
+    const uint32_t block_base = blockIdx.x * (NT * U);
     const uint32_t base = block_base + threadIdx.x;
-    const bool full = block_base + nt * U <= vecs;  // uniform
+    const bool full = block_base + NT * U <= vecs;  // uniform
     if (vecs != 0) {
         u32x4 raw[U];
         uint32_t vs[U];
 #pragma unroll
         for (int u = 0; u < U; u++) {
-            const uint32_t v = base + u * nt;
+            const uint32_t v = base + u * NT;
             vs[u] = full ? v : min(v, vecs - 1);
             raw[u] = load_stream(in + vs[u]);
         }
@@ -105,7 +106,7 @@ __global__ __launch_bounds__(kStreamThreads) void act_kernel(const T *x, T *y, u
 #pragma unroll
             for (int e = 0; e < EPV; e++) f[e] = OP::apply(f[e]);
             const u32x4 packed = Store<T>::pack(f);
-            if (full || base + u * nt < vecs) store_stream(o + vs[u], packed);
+            if (full || base + u * NT < vecs) store_stream(o + vs[u], packed);
         }
     }
     // ragged tail (n % EPV elements) by the first lanes of block 0
@@ -124,11 +125,10 @@ __global__ __launch_bounds__(kStreamThreads) void act_generic_kernel(const T *x,
 
 // c[i] = a[i] + b[i]  (chunk_vecs == 0), or c[i] = a[i] + b[i / chunk] with one b value per
 // chunk of `chunk_vecs` vectors (the per-channel broadcast add).  c may alias a or b.
-template <typename T>
-__global__ __launch_bounds__(kStreamThreads) void add_kernel(const T *a, const T *b, T *c,
-                                                             uint32_t vecs, FastDiv chunk_vecs) {
+template <typename T, int NT>
+__global__ __launch_bounds__(NT) void add_kernel(const T *a, const T *b, T *c, uint32_t vecs, FastDiv chunk_vecs) {
     constexpr int EPV = Store<T>::EPV;
-    const uint32_t v = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t v = blockIdx.x * NT + threadIdx.x;
     if (v >= vecs) return;
     float fa[EPV], fb[EPV];
     Store<T>::unpack(load_stream(reinterpret_cast<const u32x4 *>(a) + v), fa);
@@ -245,6 +245,15 @@ int geglu_dispatch(const void *pv, void *ov, size_t rows, size_t inner, hipStrea
 
 namespace {
 
+template <typename T, typename OP, int NT>
+void act_vectors_launch(int unroll, const T *x, T *y, uint32_t vecs, size_t n, hipStream_t stream) {
+    const size_t per_block = (size_t)NT * unroll;
+    const dim3 blocks(vecs ? (uint32_t)((vecs + per_block - 1) / per_block) : 1u);
+    if (unroll == 4) launch((act_kernel<T, OP, 4, NT>), blocks, dim3(NT), 0, stream, x, y, vecs, n);
+    else if (unroll == 2) launch((act_kernel<T, OP, 2, NT>), blocks, dim3(NT), 0, stream, x, y, vecs, n);
+    else launch((act_kernel<T, OP, 1, NT>), blocks, dim3(NT), 0, stream, x, y, vecs, n);
+}
+
 template <typename T, typename OP>
 int act_launch(const void *xv, void *yv, size_t n, hipStream_t stream) {
     constexpr int EPV = Store<T>::EPV;
@@ -255,17 +264,8 @@ int act_launch(const void *xv, void *yv, size_t n, hipStream_t stream) {
     if (aligned16(x) && aligned16(y) && vecs < 0x7FFFFFFFull) {
         const int tune_vectors = g_tuning.act_vectors.load(std::memory_order_relaxed);
         const int unroll = tune_vectors ? tune_vectors : kStreamUnroll;
-        const uint32_t lanes = stream_lanes(vecs);
-        const uint32_t blocks = vecs ? (uint32_t)((vecs + (size_t)lanes * unroll - 1) / ((size_t)lanes * unroll)) : 1u;
-        if (unroll == 4)
-            launch((act_kernel<T, OP, 4>), dim3(blocks), dim3(lanes), 0, stream, x, y,
-                               (uint32_t)vecs, n);
-        else if (unroll == 2)
-            launch((act_kernel<T, OP, 2>), dim3(blocks), dim3(lanes), 0, stream, x, y,
-                               (uint32_t)vecs, n);
-        else
-            launch((act_kernel<T, OP, 1>), dim3(blocks), dim3(lanes), 0, stream, x, y,
-                               (uint32_t)vecs, n);
+        if (stream_lanes(vecs, false) == kWave) act_vectors_launch<T, OP, kWave>(unroll, x, y, (uint32_t)vecs, n, stream);
+        else act_vectors_launch<T, OP, kStreamThreads>(unroll, x, y, (uint32_t)vecs, n, stream);
     } else {
         const size_t want = (n + kStreamThreads - 1) / kStreamThreads;
         launch((act_generic_kernel<T, OP>),
@@ -292,8 +292,9 @@ int add_dispatch(const void *av, const void *bv, void *cv, size_t n, size_t chun
         const uint32_t vecs = (uint32_t)(n / EPV);
         FastDiv fd = make_fast_div((uint32_t)(chunk_size / EPV));
         if (chunk_size == 0) fd.d = 0;
-        const uint32_t lanes = stream_lanes(vecs);
-        launch((add_kernel<T>), dim3((vecs + lanes - 1) / lanes), dim3(lanes), 0, stream, a, b, c, vecs, fd);
+        const uint32_t lanes = stream_lanes(vecs, chunk_size == 0);
+        auto *kernel = lanes == kWave ? add_kernel<T, kWave> : add_kernel<T, kStreamThreads>;
+        launch(kernel, dim3((vecs + lanes - 1) / lanes), dim3(lanes), 0, stream, a, b, c, vecs, fd);
     } else {
         const size_t want = (n + kStreamThreads - 1) / kStreamThreads;
         launch((add_generic_kernel<T>), dim3((uint32_t)(want < 65536 ? want : 65536)),

@@ -539,12 +539,13 @@ def test_fused_argument_checks(msd, cuda):
 
 @pytest.mark.parametrize("half", [False, True], ids=["f32", "f16"])
 @pytest.mark.parametrize("extra", [-1, 0, 1, 65])
-def test_elementwise_launches_around_a_full_chip(msd, cuda, extra, half):
-    """Vectors on both sides of as many as the chip's wavefronts hold (256 CUs), from where on a workgroup is one wavefront, with
-    elements left over: the bits of short launches."""
+@pytest.mark.parametrize("waves", [22, 48])
+def test_elementwise_launches_around_a_full_chip(msd, cuda, waves, extra, half):
+    """Vectors on both sides of 22 and 48 wavefronts per CU (256 CUs), from where on a workgroup is one wavefront, with elements
+    left over: the bits of short launches."""
     import torch
     dtype, epv = (torch.float16, 8) if half else (torch.float32, 4)
-    vecs, left = 32 * 64 * 256 + extra, epv - 1
+    vecs, left = waves * 64 * 256 + extra, epv - 1
     g = torch.Generator(device=cuda).manual_seed(extra + 7)
     x, y = (torch.randn(vecs * epv + left, device=cuda, generator=g).to(dtype) for _ in range(2))
     for op in (msd.silu, msd.gelu, msd.quick_gelu):
