@@ -374,10 +374,13 @@ int ln_dispatch(const void *xv, const void *resv, void *sumv, void *yv, const fl
             uint32_t tl = kWave;
             while ((d / n16) % tl != 0) tl /= 2;
             prefer8 = tl < kWave && (d / tl) > 16;
-            // ... unless 16-byte chunks still give every SIMD of the chip a wavefront: then the
-            // wider accesses win (8192 x 320: 3.7 against 3.9 us, with the residual 5.0 against 5.8)
-            const size_t waves16 = (rows + kWave / tl - 1) / (kWave / tl);
-            if (waves16 >= 1024) prefer8 = false;
+            // ... unless 16-byte chunks still give nearly every SIMD of the chip a wavefront: then the wider accesses win,
+            // and 8-byte ones would give some SIMDs a second wavefront.  us, 8-byte against 16-byte chunks at 900 / 970 / 1000
+            // / 1020 wavefronts of the latter, 320 columns, 1024 SIMDs: 3.85 3.98 4.04 4.02 against 3.44 3.52 3.54 3.58, with the
+            // residual 4.55 5.23 5.12 5.01 against 4.63 4.82 4.84 4.90.  (One rule for both: the chunks decide the order of
+            // the sums, and the fused add has the bits of the two calls.)
+            const size_t waves16 = (rows + kWave / tl - 1) / (kWave / tl), simds = 4 * (size_t)chip_info().cus;
+            if (16 * waves16 >= 15 * simds) prefer8 = false;
         }
         const int tune_chunk = g_tuning.ln_chunk.load(std::memory_order_relaxed);
         if (tune_chunk == 8) prefer8 = true;

@@ -472,10 +472,11 @@ def test_layernorm_mid_size_launches_with_ragged_ends(msd, orc, cuda, rows, dim,
 
 
 @pytest.mark.parametrize("half", [False, True], ids=["f32", "f16"])
-@pytest.mark.parametrize("rows,dim", [(1025, 768), (1921, 1280), (2049, 768), (2967, 1024), (4097, 640), (20483, 320)])
+@pytest.mark.parametrize("rows,dim", [(1025, 768), (1921, 1280), (1925, 1280), (2049, 768), (2967, 1024), (4097, 640),
+                                      (7673, 320), (7687, 320), (20483, 320)])
 def test_layernorm_between_full_loads_of_wavefronts(msd, orc, cuda, rows, dim, half):
-    # one to four wavefronts per SIMD, the last of them on some SIMDs only: the workgroup's size is chosen by that, and a
-    # row's arithmetic does not depend on it
+    # one to four wavefronts per SIMD, the last of them on some SIMDs only, and both sides of the change from 8- to 16-byte
+    # chunks: the workgroup's size is chosen by that, and a row's arithmetic does not depend on it
     import torch
     x, r = (orc.normal((rows, dim), seed=rows + dim + i, sigma=1.5, mean=0.5) for i in range(2))
     g, b = (_to_dev(v, cuda) for v in _affine(orc, dim, dim))
@@ -488,6 +489,7 @@ def test_layernorm_between_full_loads_of_wavefronts(msd, orc, cuda, rows, dim, h
     finally:
         lib.msd_set_tuning(msd.TUNE_LN_THREADS, 0)
     assert all(torch.equal(a, e) for a, e in zip(got, expected))
+    assert torch.equal(msd.layernorm(got[1], g, b), got[2])  # (the fused add: the bits of the two calls)
 
 
 @pytest.mark.parametrize("chunk,threads", [(8, 0), (16, 0), (8, 64), (16, 512), (0, 128)])
