@@ -254,10 +254,10 @@ __global__ __launch_bounds__(kLnThreads) void ln_generic_kernel(
 }
 
 // ---- LayerNorm dispatch ----------------------------------------------------
-// Lanes per workgroup of a launch of fewer than four wavefronts per SIMD.  All of its workgroups are resident at once, so the
-// CU that holds the most rows ends last: workgroups of four wavefronts put one on each SIMD of a CU, and a launch of 1.1
-// wavefronts per SIMD leaves some CUs twice the rows of the others.  Single wavefronts spread evenly, four of them at a time
-// over the chip's CUs.  us, four wavefronts / two / one:
+// Lanes per workgroup.  Up to four wavefronts per SIMD all workgroups of a launch are resident at once, and the CU that holds
+// the most rows ends last: workgroups of four wavefronts put one on each SIMD of a CU, and a launch of 1.1 wavefronts per
+// SIMD leaves some CUs twice the rows of the others.  Single wavefronts spread evenly, four of them at a time over the
+// chip's CUs.  us, four wavefronts / two / one:
 //   fp16 with the residual, 8320 x 320 (1040 wavefronts)   7.11 6.00 5.35     fp32 1232 x 768 (1232)   5.02 3.98 3.81
 //                           20480 x 320 (2560)             11.5 10.3 10.2     fp32 1232 x 1024         5.75 5.17 4.52
 //                           29568 x 320 (3696)             14.9 14.9 14.1     fp16 3080 x 768 (3080)   5.84 4.63 4.46
@@ -266,8 +266,17 @@ __global__ __launch_bounds__(kLnThreads) void ln_generic_kernel(
 // workgroup, which costs single wavefronts more than it gives when the row is long: rows of 1024 and more take two wavefronts with
 // the residual (2464 x 1024 fp32 9.11 8.22 8.34, 2560 x 1024 fp16 5.74 4.93 5.37), four without (fp16 3.73 3.78 4.07); so do
 // fp32 rows of 768 (2849 rows 4.84 against 5.01 with one).
-uint32_t ln_short_lanes(uint32_t wavefronts, uint32_t simds, bool residual, uint32_t dim, uint32_t elt) {
+// From four up to ten per SIMD two wavefronts (3 - 19 % faster there than four, 1 - 7 % slower from ten on), and up to about
+// five one when the row is short: 320 columns, two / one wavefronts, at 4096 / 4608 / 5120 / 5632 / 6144 of them fp16 8.48 9.69
+// 10.9 11.8 12.7 / 8.08 8.84 9.66 11.1 12.3, with the residual 15.0 17.3 19.2 20.8 22.5 / 15.3 17.0 19.0 21.2 22.8; 640
+// columns the same either way.
+uint32_t ln_lanes(uint32_t wavefronts, uint32_t simds, bool residual, uint32_t dim, uint32_t elt) {
     if (wavefronts <= simds) return kLnThreads;
+    if (wavefronts >= 4 * simds) {
+        const bool few = residual ? wavefronts > 4 * simds && wavefronts < 5 * simds : 2 * wavefronts < 11 * simds;
+        if (few && dim <= 320) return kLnThreads;
+        return wavefronts < 10 * simds ? 128 : 256;
+    }
     const uint32_t last = wavefronts % simds;
     if (last == 0 || 8 * last > 7 * simds) return 256;
     if (wavefronts < 2 * simds) return kLnThreads;
@@ -281,9 +290,8 @@ void ln_launch(const T *x, const T *res, T *sum, T *y, const float *gamma, const
     // Up to one wavefront per SIMD of the chip (four SIMDs per CU) the launch is bound by its own latency chain:
     // one wavefront per workgroup (1 - 5 % faster than four), gamma / beta requested together with
     // the row.  From two wavefronts per SIMD on throughput counts: gamma / beta through LDS (fewer
-    // load instructions and registers per wavefront), and from four up to ten wavefronts per SIMD
-    // two wavefronts per workgroup (3 - 19 % faster there, 1 - 7 % slower from ten on).  Measured,
-    // us per launch, with the row / LDS x 64, 128, 256 lanes:
+    // load instructions and registers per wavefront).  Measured, us per launch, with the row / LDS x
+    // 64, 128, 256 lanes:
     //   fp16 8192 x 320 (1024 wavefronts)   3.54 3.71 3.59 / 3.57 3.88 3.57
     //   fp16 16384 x 320 (2048)             5.12 5.19 5.22 / 4.94 4.78 4.94
     //   fp32 8192 x 320 (2048)              5.28 5.29 5.17 / 4.90 4.71 4.99
@@ -296,10 +304,8 @@ void ln_launch(const T *x, const T *res, T *sum, T *y, const float *gamma, const
     const bool early = wavefronts < 2 * simds;
     const int tune_threads = g_tuning.ln_threads.load(std::memory_order_relaxed);
     const uint32_t threads = tune_threads ? (uint32_t)tune_threads
-                             : wavefronts < 4 * simds
-                                 ? ln_short_lanes(wavefronts, simds, res != nullptr,
-                                                  VPL * TL * (NW * 4 / (uint32_t)sizeof(T)), sizeof(T))
-                                 : (wavefronts < 10 * simds ? 128u : 256u);
+                                          : ln_lanes(wavefronts, simds, res != nullptr,
+                                                     VPL * TL * (NW * 4 / (uint32_t)sizeof(T)), sizeof(T));
     const uint32_t rows_per_block = (kWave / TL) * (threads / kWave);
     const uint32_t blocks = (rows + rows_per_block - 1) / rows_per_block;
     if (early)

@@ -473,7 +473,7 @@ def test_layernorm_mid_size_launches_with_ragged_ends(msd, orc, cuda, rows, dim,
 
 @pytest.mark.parametrize("half", [False, True], ids=["f32", "f16"])
 @pytest.mark.parametrize("rows,dim", [(1025, 768), (1921, 1280), (1925, 1280), (2049, 768), (2967, 1024), (4097, 640),
-                                      (7673, 320), (7687, 320), (20483, 320)])
+                                      (7673, 320), (7687, 320), (20483, 320), (33001, 320)])
 def test_layernorm_between_full_loads_of_wavefronts(msd, orc, cuda, rows, dim, half):
     # one to four wavefronts per SIMD, the last of them on some SIMDs only, and both sides of the change from 8- to 16-byte
     # chunks: the workgroup's size is chosen by that, and a row's arithmetic does not depend on it
