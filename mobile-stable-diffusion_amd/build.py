@@ -77,11 +77,14 @@ def build_nn():
 
 
 def build_torch_calls():
-    """msd_torch_calls.so: host C++ against the headers and libraries of the torch that will import it."""
+    """msd_torch_calls.so: host C++ against the headers and libraries of the torch that will import it.  NDEBUG, as torch
+    itself is built: without it pybind11's headers give the library a thread-local counter that nothing here reads, and glibc
+    takes the slow path of every thread-local access of a process (torch's and the runtime's among them) until the thread has
+    touched those of the library loaded last (torch.empty 1.26 us against 1.00)."""
     import importlib.util
     import sysconfig
     torch_dir = importlib.util.find_spec("torch").submodule_search_locations[0]
-    _run([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__",
+    _run([os.environ.get("CXX", "g++"), "-O2", "-DNDEBUG", "-std=c++17", "-fPIC", "-shared", "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__",
           "-Wall", "-Wno-deprecated-declarations", "-isystem", os.path.join(torch_dir, "include"),
           "-isystem", "/opt/rocm/include", "-isystem", sysconfig.get_paths()["include"],
           os.path.join(CSRC, "torch_calls.cpp"), "-o", TORCH_CALLS, "-L", os.path.join(torch_dir, "lib"), "-ltorch_python",

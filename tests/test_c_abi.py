@@ -195,3 +195,14 @@ def test_stream_per_thread_is_refused_for_every_groupnorm_that_may_use_the_strea
 def test_missing_library_fails_loudly(msd):
     with pytest.raises(msd.MsdError):
         msd.load_library(os.path.join(REPO, "does_not_exist.so"))
+
+
+def test_the_torch_extension_has_no_thread_local_storage_of_its_own(msd):
+    """Such a segment, loaded last and never touched, sends every thread-local access of the process down glibc's slow path."""
+    import struct
+    with open(msd.TORCH_CALLS_PATH, "rb") as f:
+        elf = f.read()
+    phoff, = struct.unpack_from("<Q", elf, 32)
+    phentsize, phnum = struct.unpack_from("<HH", elf, 54)
+    kinds = [struct.unpack_from("<I", elf, phoff + i * phentsize)[0] for i in range(phnum)]
+    assert 1 in kinds and 7 not in kinds  # PT_LOAD, PT_TLS
