@@ -450,7 +450,7 @@ __global__ __launch_bounds__(kSmThreads) void softmax_team_kernel(const T *x, T 
 // (softmax_block_launch).  A wavefront per row with 8 - 16 vectors a lane and workgroups of 8 a lane, both as many
 // as fit, before, and so; us, TB/s: fp16 65536 x 4096 170 -> 167 (6.4), 102400 x 6400 437 -> 420 (6.2), 123904 x 7744
 // 661 -> 630 (6.1), 135168 x 8448 796 -> 748 (6.1), 147456 x 9216 917 -> 899 (6.0); fp32 65536 x 4096 351 -> 335 (6.4),
-// 102400 x 6400 905 -> 862 (6.1), 73728 x 9216 967 -> 906 (6.0).  A copy takes 6.4 to 6.5.
+// 102400 x 6400 905 -> 862 (6.1), 73728 x 9216 967 -> 906 (6.0).  A copy takes 6.4 to 6.6.
 // x and y may be the same buffer: a lane stores only what it loaded itself.
 constexpr int kSmBlockMaxThreads = 1024;
 constexpr int kSmBlockMaxVpl = 8;
@@ -722,8 +722,9 @@ bool linear_takes_tiles(size_t m, size_t k) {
 
 template <typename T, int VPL, int TL, bool RAGGED>
 void softmax_team_launch(const T *x, T *y, uint32_t rows, uint32_t cols, int stable, hipStream_t stream) {
-    // long rows (a wavefront per row, 8 or 16 vectors per lane) run as single-wavefront
-    // workgroups: 3 % faster at 65536 x 4096; the shorter ones keep 256 lanes
+    // long rows (a wavefront per row, 8 or 16 vectors per lane) run as single-wavefront workgroups, the shorter
+    // ones in workgroups of four (us, four wavefronts / two / one: fp16 5120 x 576 3.83 3.95 4.61, 24576 x 144 5.01 4.89 5.51,
+    // fp32 20480 x 64 3.16 3.24 3.69, 49152 x 64 5.96 6.07 5.87)
     constexpr uint32_t threads = (TL == kWave && VPL >= 8) ? kWave : kSmThreads;
     constexpr uint32_t rows_per_block = (threads / kWave) * (kWave / TL);
     launch((softmax_team_kernel<T, VPL, TL, RAGGED>), dim3((rows + rows_per_block - 1) / rows_per_block),
