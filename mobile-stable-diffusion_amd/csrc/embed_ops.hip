@@ -8,6 +8,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 namespace msd {
 namespace {
@@ -125,140 +126,45 @@ __global__ __launch_bounds__(kWave) void linear_rows_grouped_kernel(const T *__r
                                 g.n[p], kvecs, act_in, act_out, (blockIdx.x - g.first_block[p]) * CPW);
 }
 
-// The same for m = 3 ... 8 rows of 2-byte elements, on the matrix cores.  A column or a few per wavefront read the rows of x
-// once per column or few, 3 to 8 times the bytes of the weights; here a workgroup of four wavefronts owns 16 columns, its
-// wavefronts a quarter of k each, in runs of 128 bytes per weight row that are all requested before the first is used
-// (k = 1280: five runs), and a 16 x 16 product takes the columns against the rows.  It has room for 16 rows: lanes
-// 8 ... 15 of every 16 hold the other half of a run for the same rows, so that each piece of x is loaded and activated
-// by one lane.  Sums as exact as before: halves are multiplied into float32 accumulators, and an activated x, which is a
-// float32, goes in as the sum of two halves (hi + lo / 2048, 22 bits).  Weights by plain loads: a run is fetched by two
-// instructions, half a line each, and the second finds it in the cache (without: 52 MB of weights 14.5 instead of 12.2 us).
-// The 22 projections of a step, 20160 columns of k = 1280, us: 3 and 4 rows 21.6 -> 13.4, 5 to 8 rows 42.4 -> 14.8
-// (1 row, a column per wavefront: 10.5); a single 1280-column layer, 8 rows 5.2 -> 3.9, with SiLU 7.4 -> 4.5.
-constexpr int kLinTileCols = 16, kLinTileWaves = 4;
-constexpr int kLinTileThreads = kLinTileWaves * kWave;
-constexpr int kLinTileRuns = 5;  // runs in flight per wavefront
-constexpr float kLoScale = 2048.0f;
-
-typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+// The same for m = 3 ... 8 rows of 2-byte elements, on the matrix cores and bit for bit.  A column or a few per wavefront read
+// the rows of x once per column or few, 3 to 8 times the bytes of the weights; here a workgroup of four wavefronts owns 4 CQ
+// columns and reads them once for all.  The 64 lanes among which linear_rows_body deals the pieces of a row are the 16 blocks
+// of four lanes of each of the four wavefronts: v_mfma_f32_4x4x1 multiplies, in every block by itself, one element of four
+// columns (one a lane) with one of four rows of x (one a lane), a float32 fused multiply-add into each of the 16 sums.  So a sum
+// meets the same products in the same order, of float32 values (an activated x has no fewer bits here), and the same tree
+// adds the blocks.  Halves go in as the float32 they are: products of halves by a 16-bit matrix instruction, whose sums over
+// 32 products are rounded in its own way, were up to 1.35 times as far from the sums in 64 bits (k = 5120).
+// R pieces of every row are requested before the first is used.  Bound by the weights' bytes for three and four rows, from
+// five on by conversions, SiLU and products too.  The 22 projections of a
+// step, 20160 columns of k = 1280, us, a column or two per wavefront and so: 3 and 4 rows 20 / 22 with SiLU -> 12.4 / 12.8, 8 rows
+// 41.5 / 42.4 -> 14.0 / 15.8 (1 row: 9.9); a single 1280-column layer, 8 rows 5.5 / 7.5 -> 4.5 / 4.7.
+constexpr int kLinWgWaves = 4;
+constexpr int kLinWgThreads = kLinWgWaves * kWave;
+constexpr int kLinBlock = 4;                       // lanes, columns and rows of a block
+constexpr int kLinBlocks = kWave / kLinBlock;      // blocks of a wavefront
 constexpr int kDppRowRor8 = 0x128;  // lane i <- lane (i + 8) mod 16 inside each 16
 
-__device__ __forceinline__ u32x4 from_other_eight(const u32x4 &v) {
-    u32x4 r;
-#pragma unroll
-    for (int i = 0; i < 4; i++) r[i] = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v[i], kDppRowRor8, 0xF, 0xF, true);
-    return r;
-}
-
-__device__ __forceinline__ f32x4 mfma_16x16x32(const u32x4 &w, const u32x4 &x, const f32x4 &c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, w), __builtin_bit_cast(half8_t, x), c, 0, 0, 0);
-}
-
-__device__ __forceinline__ void linear_tile_body(const __half *__restrict__ x, const __half *__restrict__ w,
-                                                 const float *__restrict__ bias, __half *__restrict__ y, uint32_t m,
-                                                 uint32_t n, uint32_t kvecs, int act_in, int act_out, uint32_t col0) {
-    __shared__ f32x4 parts[kLinTileWaves][kWave];
-    const uint32_t lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-    const uint32_t r = lane & 15, g = lane >> 4;
-    const uint32_t half_run = r & 8 ? 4 : 0;  // which half of a run this lane's piece of x lies in
-    // (columns past the last and rows past m repeat the last one and are not stored)
-    const u32x4 *wrow = reinterpret_cast<const u32x4 *>(w) + (size_t)min(col0 + r, n - 1) * kvecs;
-    const u32x4 *xrow = reinterpret_cast<const u32x4 *>(x) + (size_t)min(r & 7, m - 1) * kvecs;
-    const uint32_t runs = (kvecs + 7) / 8;
-    const bool whole = kvecs % 8 == 0;
-    f32x4 bias_of = {0, 0, 0, 0};
-    if (wave == 0 && bias != nullptr) {
-#pragma unroll
-        for (int i = 0; i < 4; i++) bias_of[i] = bias[min(col0 + 4 * g + i, n - 1)];
-    }
-    f32x4 hi = {0, 0, 0, 0}, lo = {0, 0, 0, 0};  // row r of x against columns 4 g ... 4 g + 3
-    for (uint32_t first = wave; first < runs; first += kLinTileWaves * kLinTileRuns) {
-        u32x4 w0[kLinTileRuns], w1[kLinTileRuns], xs[kLinTileRuns];
-#pragma unroll
-        for (int j = 0; j < kLinTileRuns; j++) {
-            const uint32_t piece = min(first + j * kLinTileWaves, runs - 1) * 8 + g;
-            xs[j] = xrow[min(piece + half_run, kvecs - 1)];
-            w0[j] = wrow[min(piece, kvecs - 1)];
-            w1[j] = wrow[min(piece + 4, kvecs - 1)];
-        }
-#pragma unroll
-        for (int j = 0; j < kLinTileRuns; j++) {
-            const uint32_t run = first + j * kLinTileWaves;
-            if (run >= runs) break;  // uniform over the wavefront
-            if (!whole) {            // pieces past the row's end count as zeros, on both sides
-                const uint32_t piece = run * 8 + g;
-                const u32x4 zero = {0, 0, 0, 0};
-                w0[j] = piece < kvecs ? w0[j] : zero;
-                w1[j] = piece + 4 < kvecs ? w1[j] : zero;
-                xs[j] = piece + half_run < kvecs ? xs[j] : zero;
-            }
-            u32x4 top = xs[j];
-            if (act_in) {
-                float f[8], h[8];
-                Store<__half>::unpack(top, f);
-#pragma unroll
-                for (int e = 0; e < 8; e++) f[e] = silu_f(f[e]);
-                top = Store<__half>::pack(f);
-                Store<__half>::unpack(top, h);
-#pragma unroll
-                for (int e = 0; e < 8; e++) f[e] = fabsf(h[e]) == __builtin_huge_valf() ? 0.0f : (f[e] - h[e]) * kLoScale;
-                const u32x4 rest = Store<__half>::pack(f);
-                lo = mfma_16x16x32(w0[j], rest, lo);
-                lo = mfma_16x16x32(w1[j], from_other_eight(rest), lo);
-            }
-            hi = mfma_16x16x32(w0[j], top, hi);
-            hi = mfma_16x16x32(w1[j], from_other_eight(top), hi);
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < 4; i++)  // (what is not finite in lo came from a weight or an x that hi has met too)
-        hi[i] = fabsf(lo[i]) < __builtin_huge_valf() ? fmaf(lo[i], 1.0f / kLoScale, hi[i]) : hi[i];
-    parts[wave][lane] = hi;
-    __syncthreads();
-    if (wave != 0 || r >= m) return;
-    const f32x4 total = (parts[0][lane] + parts[1][lane]) + (parts[2][lane] + parts[3][lane]);
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const uint32_t col = col0 + 4 * g + i;
-        if (col >= n) break;
-        float v = total[i] + bias_of[i];
-        if (act_out) v = silu_f(v);
-        Store<__half>::store1(y + (size_t)r * n + col, v);
+// The value of lane ^ (1 << bit).
+__device__ __forceinline__ float lane_partner(float f, int bit) {
+    const int i = __float_as_int(f);
+    switch (bit) {
+        case 0: return dpp_move<kDppXor1>(f);
+        case 1: return dpp_move<kDppXor2>(f);
+        case 2: return __int_as_float(__builtin_amdgcn_ds_swizzle(i, 0x101F));
+        case 3: return dpp_move<kDppRowRor8>(f);
+        case 4: return __int_as_float(__builtin_amdgcn_ds_swizzle(i, 0x401F));
+        default: return __shfl_xor(f, 32);
     }
 }
 
-__global__ __launch_bounds__(kLinTileThreads) void linear_tile_kernel(
-    const __half *__restrict__ x, const __half *__restrict__ w, const float *__restrict__ bias, __half *__restrict__ y,
-    uint32_t m, uint32_t n, uint32_t kvecs, int act_in, int act_out) {
-    linear_tile_body(x, w, bias, y, m, n, kvecs, act_in, act_out, blockIdx.x * kLinTileCols);
-}
-
-__global__ __launch_bounds__(kLinTileThreads) void linear_tile_grouped_kernel(const __half *__restrict__ x, LinearGroup g,
-                                                                              uint32_t m, uint32_t kvecs, int act_in,
-                                                                              int act_out) {
-    uint32_t p = 0;
-    while (p + 1 < g.count && blockIdx.x >= g.first_block[p + 1]) p++;  // uniform: scalar loop
-    linear_tile_body(x, static_cast<const __half *>(g.w[p]), g.bias[p], static_cast<__half *>(g.y[p]), m, g.n[p], kvecs,
-                     act_in, act_out, (blockIdx.x - g.first_block[p]) * kLinTileCols);
-}
-
-// Sums over a wavefront of NV values at once: on return lane l holds the sum of value l % NV (NV a power of two, at most
-// 32).  Each step makes the additions of wave_sum, but keeps half as many values: bit for bit the same sums.
-template <int NV>
-__device__ __forceinline__ float wave_sums(float (&v)[NV]) {
+// Sums of NV values (a power of two) over the lanes that differ in bits FIRST ... FIRST + BITS - 1.  Each step makes the
+// additions of team_sum, but keeps half as many values: bit for bit the same sums.  On return v[j] of a lane is the sum of
+// value (j << BITS) + those bits of the lane, of fewer values than 2^BITS that of the bits modulo NV.
+template <int FIRST, int BITS, int NV>
+__device__ __forceinline__ void scatter_sums(float (&v)[NV]) {
     const uint32_t lane = threadIdx.x;
-    auto partner = [](float f, int bit) {
-        const int i = __float_as_int(f);
-        switch (bit) {
-            case 0: return dpp_move<kDppXor1>(f);
-            case 1: return dpp_move<kDppXor2>(f);
-            case 2: return __int_as_float(__builtin_amdgcn_ds_swizzle(i, 0x101F));
-            case 3: return dpp_move<kDppRowRor8>(f);
-            default: return __int_as_float(__builtin_amdgcn_ds_swizzle(i, 0x401F));
-        }
-    };
 #pragma unroll
-    for (int bit = 0, n = NV; bit < 5; bit++) {
+    for (int bit = FIRST, n = NV; bit < FIRST + BITS; bit++) {
         if (n > 1) {
             n /= 2;
             const bool upper = (lane >> bit) & 1;
@@ -266,14 +172,111 @@ __device__ __forceinline__ float wave_sums(float (&v)[NV]) {
             for (int i = 0; i < NV / 2; i++) {
                 if (i < n) {
                     const float mine = upper ? v[2 * i + 1] : v[2 * i], other = upper ? v[2 * i] : v[2 * i + 1];
-                    v[i] = mine + partner(other, bit);
+                    v[i] = mine + lane_partner(other, bit);
                 }
             }
         } else {
-            v[0] += partner(v[0], bit);
+            v[0] += lane_partner(v[0], bit);
         }
     }
-    return v[0] + __shfl_xor(v[0], 32);
+}
+
+template <int MQ, int CQ, int R, bool ACT>
+__device__ __forceinline__ void linear_quads_body(const __half *__restrict__ x, const __half *__restrict__ w,
+                                                  const float *__restrict__ bias, __half *__restrict__ y, uint32_t m,
+                                                  uint32_t n, uint32_t kvecs, int act_out, uint32_t col0) {
+    constexpr int NV = CQ * MQ * kLinBlock;  // sums a lane takes part in
+    __shared__ float parts[kLinWgWaves][NV * kLinBlock];
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const uint32_t block = (threadIdx.x & (kWave - 1)) / kLinBlock, i = threadIdx.x % kLinBlock;
+    const u32x4 *xin = reinterpret_cast<const u32x4 *>(x), *win = reinterpret_cast<const u32x4 *>(w);
+    // what this lane stores in the end
+    const uint32_t t = threadIdx.x, quads = t / (kLinBlock * kLinBlock);
+    const uint32_t row = kLinBlock * (quads % MQ) + i, col = col0 + kLinBlock * (quads / MQ) + t / kLinBlock % kLinBlock;
+    const float b = bias != nullptr ? bias[min(col, n - 1)] : 0.0f;
+    f32x4 acc[CQ][MQ];
+#pragma unroll
+    for (int q = 0; q < CQ; q++)
+#pragma unroll
+        for (int r = 0; r < MQ; r++) acc[q][r] = f32x4{0, 0, 0, 0};
+    for (uint32_t base = kLinBlocks * wave; base < kvecs; base += kWave * R) {
+        u32x4 wraw[CQ][R], xraw[MQ][R];
+#pragma unroll
+        for (int u = 0; u < R; u++) {  // (columns past the last and rows past m repeat the last one and are not stored)
+            const uint32_t piece = min(base + u * kWave + block, kvecs - 1);
+#pragma unroll
+            for (int r = 0; r < MQ; r++) xraw[r][u] = xin[(size_t)min(kLinBlock * r + i, m - 1) * kvecs + piece];
+#pragma unroll
+            for (int q = 0; q < CQ; q++)
+                wraw[q][u] = load_stream(win + (size_t)min(col0 + kLinBlock * q + i, n - 1) * kvecs + piece);
+        }
+        asm volatile("" ::: "memory");  // the loads stay in front of the branches below
+#pragma unroll
+        for (int u = 0; u < R; u++) {
+            const uint32_t first = base + u * kWave;  // (uniform over the wavefront)
+            if (first >= kvecs) break;
+            if (first + kLinBlocks > kvecs) {  // a piece past the row's end counts as zeros, on both sides
+                const bool have = first + block < kvecs;
+                const u32x4 zero = {0, 0, 0, 0};
+#pragma unroll
+                for (int r = 0; r < MQ; r++) xraw[r][u] = have ? xraw[r][u] : zero;
+#pragma unroll
+                for (int q = 0; q < CQ; q++) wraw[q][u] = have ? wraw[q][u] : zero;
+            }
+            float xf[MQ][8], wf[CQ][8];
+#pragma unroll
+            for (int r = 0; r < MQ; r++) {
+                Store<__half>::unpack(xraw[r][u], xf[r]);
+                if (ACT) {
+#pragma unroll
+                    for (int e = 0; e < 8; e++) xf[r][e] = silu_f(xf[r][e]);
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < CQ; q++) Store<__half>::unpack(wraw[q][u], wf[q]);
+#pragma unroll
+            for (int e = 0; e < 8; e++)
+#pragma unroll
+                for (int q = 0; q < CQ; q++)
+#pragma unroll
+                    for (int r = 0; r < MQ; r++)
+                        acc[q][r] = __builtin_amdgcn_mfma_f32_4x4x1f32(wf[q][e], xf[r][e], acc[q][r], 0, 0, 0);
+        }
+    }
+    float v[NV];  // value (q, r, j): column 4 q + j against row 4 r + i
+#pragma unroll
+    for (int q = 0; q < CQ; q++)
+#pragma unroll
+        for (int r = 0; r < MQ; r++)
+#pragma unroll
+            for (int j = 0; j < kLinBlock; j++) v[(q * MQ + r) * kLinBlock + j] = acc[q][r][j];
+    scatter_sums<2, 4>(v);
+#pragma unroll
+    for (int j = 0; j < (NV + kLinBlocks - 1) / kLinBlocks; j++) {
+        const uint32_t value = j * kLinBlocks + block;
+        if (value < NV) parts[wave][value * kLinBlock + i] = v[j];
+    }
+    __syncthreads();
+    if (t >= NV * kLinBlock || row >= m || col >= n) return;
+    float total = (parts[0][t] + parts[1][t]) + (parts[2][t] + parts[3][t]) + b;
+    if (act_out) total = silu_f(total);
+    Store<__half>::store1(y + (size_t)row * n + col, total);
+}
+
+template <int MQ, int CQ, int R, bool ACT>
+__global__ __launch_bounds__(kLinWgThreads, 4) void linear_quads_kernel(
+    const __half *__restrict__ x, const __half *__restrict__ w, const float *__restrict__ bias, __half *__restrict__ y,
+    uint32_t m, uint32_t n, uint32_t kvecs, int act_out) {
+    linear_quads_body<MQ, CQ, R, ACT>(x, w, bias, y, m, n, kvecs, act_out, blockIdx.x * (kLinBlock * CQ));
+}
+
+template <int MQ, int CQ, int R, bool ACT>
+__global__ __launch_bounds__(kLinWgThreads, 4) void linear_quads_grouped_kernel(const __half *__restrict__ x, LinearGroup g,
+                                                                                uint32_t m, uint32_t kvecs, int act_out) {
+    uint32_t p = 0;
+    while (p + 1 < g.count && blockIdx.x >= g.first_block[p + 1]) p++;  // uniform: scalar loop
+    linear_quads_body<MQ, CQ, R, ACT>(x, static_cast<const __half *>(g.w[p]), g.bias[p], static_cast<__half *>(g.y[p]), m,
+                                      g.n[p], kvecs, act_out, (blockIdx.x - g.first_block[p]) * (kLinBlock * CQ));
 }
 
 // Large groups of 4-byte elements, 2 ... 8 rows: four wavefronts share the rows of x, activated once, in LDS, and each takes
@@ -282,7 +285,7 @@ __device__ __forceinline__ float wave_sums(float (&v)[NV]) {
 // weights, us, before with two columns per wavefront and so: 2 rows 21 - 24 -> 20, 4 rows 34 - 43 -> 24.5, 8 rows
 // 53 - 59 -> 29 (1 row: 18).  Two columns instead of four 33 at 8 rows, float32 matrix products 28, with other sums.
 template <int M, int C, int ROUND>
-__global__ __launch_bounds__(kLinTileThreads) void linear_shared_grouped_kernel(const float *__restrict__ x, LinearGroup group,
+__global__ __launch_bounds__(kLinWgThreads) void linear_shared_grouped_kernel(const float *__restrict__ x, LinearGroup group,
                                                                                 uint32_t m, uint32_t kvecs, int act_in,
                                                                                 int act_out) {
     constexpr uint32_t kChunk = ROUND * kWave;  // pieces of a row of x in LDS at a time
@@ -294,7 +297,7 @@ __global__ __launch_bounds__(kLinTileThreads) void linear_shared_grouped_kernel(
     float *y = static_cast<float *>(group.y[p]);
     const uint32_t n = group.n[p];
     const uint32_t lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-    const uint32_t col0 = ((blockIdx.x - group.first_block[p]) * kLinTileWaves + wave) * C;
+    const uint32_t col0 = ((blockIdx.x - group.first_block[p]) * kLinWgWaves + wave) * C;
     const uint32_t out_col = col0 + (lane % (C * M)) / M, out_row = lane % M;  // what this lane stores
     const float b = bias != nullptr ? bias[min(out_col, n - 1)] : 0.0f;
     float acc[C * M];
@@ -310,7 +313,7 @@ __global__ __launch_bounds__(kLinTileThreads) void linear_shared_grouped_kernel(
         const uint32_t here = min(kvecs - base, kChunk);
         if (base != 0) __syncthreads();
         for (uint32_t row = 0; row < m; row++)  // (rows from m on hold anything: their sums are not stored)
-            for (uint32_t i = threadIdx.x; i < here; i += kLinTileThreads) {
+            for (uint32_t i = threadIdx.x; i < here; i += kLinWgThreads) {
                 f32x4 v = reinterpret_cast<const f32x4 *>(x)[(size_t)row * kvecs + base + i];
                 if (act_in) {
 #pragma unroll
@@ -333,7 +336,8 @@ __global__ __launch_bounds__(kLinTileThreads) void linear_shared_grouped_kernel(
             }
         }
     }
-    float r = wave_sums<C * M>(acc);
+    scatter_sums<0, 5>(acc);  // (at most 32 values: one a lane)
+    float r = acc[0] + __shfl_xor(acc[0], 32);
     if (lane < C * M && out_row < m && out_col < n) {
         r += b;
         if (act_out) r = silu_f(r);
@@ -711,15 +715,35 @@ void linear_launch(const T *x, const T *w, const float *bias, T *y, uint32_t m, 
                            k / EPV, act_in, act_out);
 }
 
-// Rows of x on the matrix cores: from three rows of 2-byte elements on, and not for short k, which a quarter of
-// is too little for a wavefront to hide its steps behind (us, column per wavefront and tile, 3 / 4 / 8 rows: k = 320
-// 3.1 3.1 4.0 and 3.6 3.6 3.7, k = 1280 3.7 3.7 5.2 and 3.7 3.7 3.9, with SiLU 4.8 4.8 7.4 and 4.3 4.3 4.5).  One rule for
-// single layers and groups, whose sums are the same bits.
+// Three to eight rows of 2-byte elements on the matrix cores, with the bits of a column or two per wavefront: always where x is
+// activated, once for four wavefronts instead of in each (us, column per wavefront and so: 64 columns of k = 320 2.97 / 2.89,
+// 1280 of 320 3.52 / 3.13, 1280 of 1280 3 rows 4.92 / 3.55, 8 rows 7.60 / 4.37); else from as many columns on as fill the
+// chip anyway (3 rows, k = 1280: 640 columns 3.33 / 3.51, 1280 3.95 / 3.53, 5120 6.64 / 5.57; 8 rows, 320 columns 3.78 / 3.94, 640
+// 4.30 / 4.11, 1280 5.53 / 4.10, 5120 11.4 / 6.92).
 template <typename T>
-bool linear_takes_tiles(size_t m, size_t k) {
-    return sizeof(T) == 2 && m >= 3 && k >= 640;
+bool linear_takes_quads(size_t m, size_t n, int act_in) {
+    return sizeof(T) == 2 && m >= 3 && (act_in || n >= (m <= 4 ? 1280u : 640u));
 }
 
+// Column quads of a workgroup: two, with three pieces of each row in flight, while the launch is short; four, with one
+// piece and less of x to read and activate per column, when it lasts (us, two and four, k = 1280, with SiLU: 8192 columns 3 rows
+// 7.62 / 9.24, 8 rows 9.64 / 10.8; 10240 8.39 / 9.05 and 11.1 / 11.3; 20160 13.0 / 12.8 and 18.1 / 15.8).
+constexpr int linear_column_quads(size_t n) { return n >= 12288 ? 4 : 2; }
+
+// Calls `f` with an instance's parameters: row quads, column quads, pieces in flight, SiLU on the input.
+template <typename F>
+void linear_quads(size_t m, size_t n, int act_in, F f) {
+    auto with_rows = [&](auto cols, auto round) {
+        auto with_act = [&](auto rows) {
+            if (act_in) f(rows, cols, round, std::true_type{});
+            else f(rows, cols, round, std::false_type{});
+        };
+        if (m <= 4) with_act(std::integral_constant<int, 1>{});
+        else with_act(std::integral_constant<int, 2>{});
+    };
+    if (linear_column_quads(n) == 4) with_rows(std::integral_constant<int, 4>{}, std::integral_constant<int, 1>{});
+    else with_rows(std::integral_constant<int, 2>{}, std::integral_constant<int, 3>{});
+}
 template <typename T, int VPL, int TL, bool RAGGED>
 void softmax_team_launch(const T *x, T *y, uint32_t rows, uint32_t cols, int stable, hipStream_t stream) {
     // long rows (a wavefront per row, 8 or 16 vectors per lane) run as single-wavefront workgroups, the shorter
@@ -788,10 +812,12 @@ int linear_rows_dispatch(const void *xv, const void *wv, const float *bias, void
     if (m > 8 || n > 0x7FFFFFFFull || k > 0x7FFFFFFFull) return MSD_ERR_INVALID_VALUE;
     const uint32_t m_pad = m <= 1 ? 1 : m <= 2 ? 2 : m <= 4 ? 4 : 8;
     const bool vectors = k != 0 && k % EPV == 0 && aligned16(x) && aligned16(w);
-    if (vectors && linear_takes_tiles<T>(m, k)) {
-        launch(linear_tile_kernel, dim3((uint32_t)((n + kLinTileCols - 1) / kLinTileCols)), dim3(kLinTileThreads), 0, stream,
-               static_cast<const __half *>(xv), static_cast<const __half *>(wv), bias, static_cast<__half *>(yv), (uint32_t)m,
-               (uint32_t)n, (uint32_t)(k / EPV), act_in, act_out);
+    if (vectors && linear_takes_quads<T>(m, n, act_in)) {
+        linear_quads(m, n, act_in, [&](auto rows, auto quads, auto round, auto act) {
+            launch((linear_quads_kernel<rows, quads, round, act>), dim3((uint32_t)((n + kLinBlock * quads - 1) / (kLinBlock * quads))),
+                   dim3(kLinWgThreads), 0, stream, static_cast<const __half *>(xv), static_cast<const __half *>(wv), bias,
+                   static_cast<__half *>(yv), (uint32_t)m, (uint32_t)n, (uint32_t)(k / EPV), act_out);
+        });
     } else if (vectors) {
         switch (m_pad) {
             case 1: linear_launch<T, 1>(x, w, bias, y, (uint32_t)m, (uint32_t)n, (uint32_t)k, act_in, act_out, stream); break;
@@ -861,10 +887,10 @@ int linear_rows_grouped_dispatch(const void *xv, const void *const *ws, const fl
     // out of registers).  The sums do not depend on it.
     size_t total_n = 0;
     for (size_t i = 0; i < count; i++) total_n += ns[i];
-    const bool tiles = linear_takes_tiles<T>(m, k);
+    const bool quads = linear_takes_quads<T>(m, total_n, act_in);
     const bool shared = sizeof(T) == 4 && m >= 2 && total_n >= 8192;  // (fewer columns leave it too few workgroups)
     constexpr int kSharedCols = 4;
-    const int cpw = tiles ? kLinTileCols : shared ? kLinTileWaves * kSharedCols  // (columns of a workgroup)
+    const int cpw = quads ? kLinBlock * linear_column_quads(total_n) : shared ? kLinWgWaves * kSharedCols  // (columns of a workgroup)
                     : (sizeof(T) == 2 && m_pad <= 2 && total_n >= 8192) ? 4 : act_in ? 2 : 1;
     for (size_t base = 0; base < count; base += kLinGroupMax) {
         LinearGroup g;
@@ -883,12 +909,14 @@ int linear_rows_grouped_dispatch(const void *xv, const void *const *ws, const fl
         if (g.count == 0) continue;
         g.first_block[g.count] = blocks;
         auto rows_in_lds = [&](auto *kernel) {
-            launch(kernel, dim3(blocks), dim3(kLinTileThreads), 0, stream, static_cast<const float *>(xv), g, (uint32_t)m,
+            launch(kernel, dim3(blocks), dim3(kLinWgThreads), 0, stream, static_cast<const float *>(xv), g, (uint32_t)m,
                    (uint32_t)(k / EPV), act_in, act_out);
         };
-        if (tiles)
-            launch(linear_tile_grouped_kernel, dim3(blocks), dim3(kLinTileThreads), 0, stream, static_cast<const __half *>(xv), g,
-                   (uint32_t)m, (uint32_t)(k / EPV), act_in, act_out);
+        if (quads)
+            linear_quads(m, total_n, act_in, [&](auto rows, auto cols, auto round, auto act) {
+                launch((linear_quads_grouped_kernel<rows, cols, round, act>), dim3(blocks), dim3(kLinWgThreads), 0, stream,
+                       static_cast<const __half *>(xv), g, (uint32_t)m, (uint32_t)(k / EPV), act_out);
+            });
         else if (shared && m_pad == 2) rows_in_lds(linear_shared_grouped_kernel<2, kSharedCols, 5>);
         else if (shared && m_pad == 4) rows_in_lds(linear_shared_grouped_kernel<4, kSharedCols, 5>);
         else if (shared) rows_in_lds(linear_shared_grouped_kernel<8, kSharedCols, 5>);

@@ -127,8 +127,7 @@ def test_grouped_linear_runs_the_22_resblock_projections_in_one_launch(msd, orc,
 @pytest.mark.parametrize("m", [3, 4, 5, 8])
 @pytest.mark.parametrize("n,k", [(1, 640), (16, 648), (17, 704), (33, 1280), (15, 2568), (130, 4096), (7, 632)])
 def test_linear_several_half_rows_on_the_matrix_cores(msd, orc, cuda, m, n, k):
-    """Tiles of 16 columns with columns and rows left over; k of whole runs, of runs cut after each number of
-    pieces, of more than one round; the last k is the longest that goes a column per wavefront."""
+    """Blocks of columns and rows with some left over; k of whole rounds of pieces, of cut ones, of more than one."""
     torch = _torch()
     for act_in, act_out, bias in ((0, 1, True), (1, 0, False), (1, 1, True)):
         _linear_case(msd, orc, cuda, m, n, k, 7950 + m + n + k, True, act_in, act_out, bias)
@@ -170,6 +169,78 @@ def test_linear_matrix_core_rows_with_infinities_nan_and_subnormals(msd, cuda):
     half_sum = 640 * 512 * (tiny / (1 + np.exp(-tiny)))
     assert float((msd.linear_rows(xs, ws, act_in=msd.ACT_SILU).double() - half_sum).abs().max()) <= half_sum * (2.0 ** -11 + 1e-5)
     assert float((msd.linear_rows(ws[:4], xs[:1]).double() - 640 * tiny * 512).abs().max()) <= 640 * tiny * 512 * 2.0 ** -11
+
+
+@pytest.mark.parametrize("m", [3, 8])
+@pytest.mark.parametrize("k", [640, 1288])
+def test_linear_matrix_core_rows_keep_small_activated_values(msd, cuda, m, k):
+    """What SiLU leaves of a row goes into the sum as a float32, however small it is: below the smallest half, and down to
+    2^-38 at x = -30, against weights that bring the sum back into the range of halves."""
+    torch = _torch()
+    g = torch.Generator(device=cuda).manual_seed(31 + m + k)
+
+    def check(x, w):
+        x, w = x.to(torch.float16), w.to(torch.float16)
+        got = msd.linear_rows(x, w, act_in=msd.ACT_SILU).double().cpu()
+        xd = x.double().cpu()
+        want = (xd / (1 + torch.exp(-xd))) @ w.double().cpu().t()
+        assert float(want.abs().min()) > 2.0 ** -14  # (a normal half)
+        # half an ulp of the result; SiLU's 2^x (1.2e-7 (1 + 1.45 |x|)) and float32 sums of k values of one sign
+        assert float(((got - want) / want).abs().max()) <= 2.0 ** -11 + 2e-5
+        grouped = msd.linear_rows_grouped(x, [w, w[:3]], act_in=msd.ACT_SILU)
+        assert torch.equal(grouped[0].double().cpu(), got) and torch.equal(grouped[1].double().cpu(), got[:, :3])
+
+    def uniform(rows, low, high):
+        return torch.rand((rows, k), device=cuda, generator=g) * (high - low) + low
+
+    for low, weight in ((-16.0, 100.0), (-20.0, 4e3), (-25.0, 6e4), (-27.0, 6e4), (-30.0, 6e4)):
+        check(torch.full((m, k), low, device=cuda), torch.full((19, k), weight, device=cuda))
+        check(uniform(m, low, low + 1), uniform(19, weight / 2, weight))
+    for top in (-14, -18, -22):  # random magnitudes below 2^top, of both signs: SiLU halves them
+        magnitude = uniform(m, 0.25, 1.0) * 2.0 ** top
+        check(magnitude, uniform(19, 3e4, 6e4))
+        check(-magnitude, uniform(19, 3e4, 6e4))
+    # an infinite weight: a product with anything but zero is infinite, if its half would round to zero too
+    for v in (-19.0, -21.0, -25.0, -40.0, -60.0, 2.0 ** -24, -2.0 ** -24):
+        x = torch.full((m, k), v, device=cuda, dtype=torch.float16)
+        w = torch.full((19, k), 0.5, device=cuda, dtype=torch.float16)
+        w[0, 0], w[7, k - 1], w[18, k // 2] = float("inf"), -float("inf"), float("inf")
+        got = msd.linear_rows(x, w, act_in=msd.ACT_SILU)
+        sign = 1.0 if v > 0 else -1.0
+        for col, inf in ((0, sign), (7, -sign), (18, sign)):
+            assert bool((got[:, col] == inf * float("inf")).all()), v
+        assert bool(torch.isfinite(got[:, [c for c in range(19) if c not in (0, 7, 18)]]).all())
+
+
+@pytest.mark.parametrize("act_in", [0, 1])
+@pytest.mark.parametrize("n,k", [(1, 8), (3, 120), (8, 128), (9, 136), (70, 512), (640, 504), (1283, 640), (1280, 1280),
+                                 (33, 1288), (1281, 1544), (2563, 2568), (12289, 200), (12300, 1280)])
+def test_linear_a_row_has_its_bits_alone_and_among_others(msd, cuda, n, k, act_in):
+    """The sums of three to eight rows at once (four columns, and four or eight rows, per block of lanes; column quads, pieces
+    and rounds left over) are those of a row by itself, a column or two per wavefront: the same products in the same order,
+    with infinities, NaN and values of every size among them."""
+    torch = _torch()
+    g = torch.Generator(device=cuda).manual_seed(n + k)
+    x = torch.randn((8, k), device=cuda, generator=g) * torch.logspace(-7, 4, 8, device=cuda)[:, None]
+    x[3] = -torch.rand((k,), device=cuda, generator=g) * 100  # (SiLU leaves float32 values of 2^-143 and more)
+    w = torch.randn((n, k), device=cuda, generator=g) * torch.logspace(-5, 3, n, device=cuda)[:, None]
+    if n > 8:
+        w[n - 1, k // 2], w[5, 0], x[6, k - 1] = float("inf"), -float("inf"), float("nan")
+        x[1, 0], w[2, :8] = 0.0, 0.0
+    x, w = x.to(torch.float16), w.to(torch.float16)
+    bias = torch.randn((n,), device=cuda, generator=g)
+
+    def bits(t):
+        t = t.clone()
+        t[t.isnan()] = float("nan")
+        return t.view(torch.int16)
+
+    for act_out in (0, 1):
+        alone = torch.cat([msd.linear_rows(x[i:i + 1], w, bias, act_in=act_in, act_out=act_out) for i in range(8)])
+        for m in (2, 3, 4, 5, 8):
+            assert torch.equal(bits(msd.linear_rows(x[:m], w, bias, act_in=act_in, act_out=act_out)), bits(alone[:m]))
+            grouped = msd.linear_rows_grouped(x[:m], [w[:1], w], [None, bias], act_in=act_in, act_out=act_out)[1]
+            assert torch.equal(bits(grouped), bits(alone[:m]))
 
 
 @pytest.mark.parametrize("m", [2, 3, 4, 5, 8])
