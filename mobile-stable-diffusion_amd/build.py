@@ -8,9 +8,11 @@
 
 Run as a script (`python build.py`) or call build_all().
 """
+import importlib.util
 import os
 import subprocess
 import sys
+import sysconfig
 
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(PKG_DIR, "csrc")
@@ -76,14 +78,22 @@ def build_nn():
     return LIB_NN
 
 
+def torch_with_hip_headers():
+    """The folder of the installed torch, or None where there is none or it has no HIP headers.  (Does not import it.)"""
+    spec = importlib.util.find_spec("torch")
+    torch_dir = spec.submodule_search_locations[0] if spec is not None and spec.submodule_search_locations else None
+    return torch_dir if torch_dir and os.path.isdir(os.path.join(torch_dir, "include", "ATen", "hip")) else None
+
+
 def build_torch_calls():
-    """msd_torch_calls.so: host C++ against the headers and libraries of the torch that will import it.  NDEBUG, as torch
-    itself is built: without it pybind11's headers give the library a thread-local counter that nothing here reads, and glibc
-    takes the slow path of every thread-local access of a process (torch's and the runtime's among them) until the thread has
-    touched those of the library loaded last (torch.empty 1.26 us against 1.00)."""
-    import importlib.util
-    import sysconfig
-    torch_dir = importlib.util.find_spec("torch").submodule_search_locations[0]
+    """msd_torch_calls.so: host C++ against the headers and libraries of the torch that will import it; None where there is no
+    such torch, which nothing else here needs.  NDEBUG, as torch itself is built: without it pybind11's headers give the library
+    a thread-local counter that nothing here reads, and glibc takes the slow path of every thread-local access of a process
+    (torch's and the runtime's among them) until the thread has touched those of the library loaded last (torch.empty 1.26 us
+    against 1.00)."""
+    torch_dir = torch_with_hip_headers()
+    if torch_dir is None:
+        return None
     _run([os.environ.get("CXX", "g++"), "-O2", "-DNDEBUG", "-std=c++17", "-fPIC", "-shared", "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__",
           "-Wall", "-Wno-deprecated-declarations", "-isystem", os.path.join(torch_dir, "include"),
           "-isystem", "/opt/rocm/include", "-isystem", sysconfig.get_paths()["include"],
@@ -115,13 +125,17 @@ def build_all(verbose=True):
     nn = build_nn()
     if nn:
         built.append(nn)
-    built.append(build_torch_calls())
     built.append(build_cli())
     if nn:
         built.append(build_layer_check())
+    torch_calls = build_torch_calls()
+    if torch_calls:
+        built.append(torch_calls)
     if verbose:
         for b in built:
             print("built", b)
+        if not torch_calls:
+            print("skipped", TORCH_CALLS, "(no torch with HIP headers here)")
     return built
 
 

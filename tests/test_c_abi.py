@@ -2,6 +2,7 @@
 symbol include/msd_hip.h declares, and its host-only entry points behave.  No
 compute call is made here (there is no GPU in the CPU test environment)."""
 import ctypes
+import importlib
 import os
 import re
 
@@ -206,3 +207,19 @@ def test_the_torch_extension_has_no_thread_local_storage_of_its_own(msd):
     phentsize, phnum = struct.unpack_from("<HH", elf, 54)
     kinds = [struct.unpack_from("<I", elf, phoff + i * phentsize)[0] for i in range(phnum)]
     assert 1 in kinds and 7 not in kinds  # PT_LOAD, PT_TLS
+
+
+def test_without_torch_everything_but_its_extension_is_built(tmp_path, monkeypatch, capsys):
+    """C and C++ callers need no torch: none, or one without HIP headers, ends no build."""
+    build = importlib.import_module("mobile-stable-diffusion_amd.build")
+    made = []
+    for name in ("build_hip", "build_nn", "build_cli", "build_layer_check"):
+        monkeypatch.setattr(build, name, lambda name=name: made.append(name) or name)
+    monkeypatch.setattr(build, "_run", lambda cmd: pytest.fail("nothing to compile"))
+    (tmp_path / "torch" / "include" / "ATen").mkdir(parents=True)
+    headless = type("Spec", (), {"submodule_search_locations": [str(tmp_path / "torch")]})
+    for spec in (None, headless):
+        made.clear()
+        monkeypatch.setattr("importlib.util.find_spec", lambda name: spec)
+        assert build.build_all() == made == ["build_hip", "build_nn", "build_cli", "build_layer_check"]
+        assert "skipped" in capsys.readouterr().out
