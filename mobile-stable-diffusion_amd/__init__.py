@@ -10,6 +10,8 @@ the loader raises.
 import ctypes
 import importlib.util
 import os
+import sys
+import warnings
 
 _PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 CSRC_DIR = os.path.join(_PKG_DIR, "csrc")
@@ -117,6 +119,19 @@ class _Unbound:
         return getattr(_bind_native(), name)
 
 
+class _NoNative:
+    """Stands for the native calls where there are none: every call takes its general path."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+    def names(self):
+        return []
+
+    def bind(self, addresses, check):
+        pass
+
+
 _native = _Unbound()
 
 
@@ -124,16 +139,35 @@ def _bind_addresses(native):
     native.bind({name: ctypes.cast(getattr(_lib, name), ctypes.c_void_p).value for name in native.names()}, check)
 
 
+def _running(torch):
+    """The Python and the torch at hand, as build.py names those that the extension is compiled for."""
+    return "Python %d.%d, torch %s (%s)" % (sys.version_info[:2] + (torch.version.__version__, torch.version.git_version))
+
+
+def _load_native(torch):
+    """The extension, or what stands for it where it is not built or was built for another torch: the C ABI takes tensors of
+    any torch, but the extension reads them as its own torch lays them out."""
+    spec = importlib.util.spec_from_file_location("msd_torch_calls", TORCH_CALLS_PATH)
+    try:
+        native = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(native)
+        built_for = getattr(native, "built_for", "another torch")
+        if built_for == _running(torch):
+            return native
+        why = "was built for %s, this is %s" % (built_for, _running(torch))
+    except ImportError as e:  # (no such file, or symbols that this torch does not have)
+        why = "does not load: %s" % e
+    warnings.warn("%s %s; a call takes about 2.5 us longer without it (run __graft_entry__.build())" % (TORCH_CALLS_PATH, why),
+                  RuntimeWarning, stacklevel=4)
+    return _NoNative()
+
+
 def _bind_native():
     global _native
     load_library()
-    _bind_torch()  # the extension's symbols are torch's
+    torch = _bind_torch()  # the extension's symbols are torch's
     if isinstance(_native, _Unbound):
-        if not os.path.exists(TORCH_CALLS_PATH):
-            raise MsdError("native library %s is missing: run __graft_entry__.build()" % TORCH_CALLS_PATH)
-        spec = importlib.util.spec_from_file_location("msd_torch_calls", TORCH_CALLS_PATH)
-        native = importlib.util.module_from_spec(spec)
-        spec.loader.exec_module(native)
+        native = _load_native(torch)
         _bind_addresses(native)
         _native = native
     return _native

@@ -85,6 +85,14 @@ def torch_with_hip_headers():
     return torch_dir if torch_dir and os.path.isdir(os.path.join(torch_dir, "include", "ATen", "hip")) else None
 
 
+def _runs_with(torch_dir):
+    """The Python and the torch that torch_calls.cpp is compiled for, as the package asks for them (_running in __init__.py)."""
+    spec = importlib.util.spec_from_file_location("torch_version", os.path.join(torch_dir, "version.py"))
+    version = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(version)
+    return "Python %d.%d, torch %s (%s)" % (sys.version_info[:2] + (version.__version__, version.git_version))
+
+
 def build_torch_calls():
     """msd_torch_calls.so: host C++ against the headers and libraries of the torch that will import it; None where there is no
     such torch, which nothing else here needs.  NDEBUG, as torch itself is built: without it pybind11's headers give the library
@@ -95,6 +103,7 @@ def build_torch_calls():
     if torch_dir is None:
         return None
     _run([os.environ.get("CXX", "g++"), "-O2", "-DNDEBUG", "-std=c++17", "-fPIC", "-shared", "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__",
+          '-DMSD_BUILT_FOR="%s"' % _runs_with(torch_dir),
           "-Wall", "-Wno-deprecated-declarations", "-isystem", os.path.join(torch_dir, "include"),
           "-isystem", "/opt/rocm/include", "-isystem", sysconfig.get_paths()["include"],
           os.path.join(CSRC, "torch_calls.cpp"), "-o", TORCH_CALLS, "-L", os.path.join(torch_dir, "lib"), "-ltorch_python",

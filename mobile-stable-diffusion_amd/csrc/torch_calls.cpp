@@ -6,6 +6,9 @@
 // or None where the call is not a plain one: an argument that is no dense contiguous device tensor of torch's own
 // types, that does not fit the others, a call under a tensor or function mode or a transform.  The package then takes the
 // call through its general path, which makes the same call or says what is wrong with it.
+//
+// Tensors are read through inline accessors, so the extension is good for the one Python and torch it was compiled for:
+// `built_for` names them, and the package asks before it makes any other call here.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -592,4 +595,8 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "msd_torch_calls", nullptr, -1, met
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit_msd_torch_calls(void) { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit_msd_torch_calls(void) {
+    PyObject *m = PyModule_Create(&module);
+    if (m != nullptr && PyModule_AddStringConstant(m, "built_for", MSD_BUILT_FOR) != 0) Py_CLEAR(m);
+    return m;
+}

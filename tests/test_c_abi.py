@@ -223,3 +223,29 @@ def test_without_torch_everything_but_its_extension_is_built(tmp_path, monkeypat
         monkeypatch.setattr("importlib.util.find_spec", lambda name: spec)
         assert build.build_all() == made == ["build_hip", "build_nn", "build_cli", "build_layer_check"]
         assert "skipped" in capsys.readouterr().out
+
+
+def test_the_torch_extension_serves_only_the_torch_it_was_built_for(msd, tmp_path, monkeypatch):
+    """Under another torch, or where it does not load, every call takes the general path, and a warning says so once."""
+    torch = pytest.importorskip("torch")
+    native = msd._load_native(torch)
+    assert native.built_for == msd._running(torch) and "msd_layernorm" in native.names()
+
+    def general_path():
+        monkeypatch.setattr(msd, "_native", msd._Unbound())
+        with pytest.warns(RuntimeWarning) as warned:
+            assert msd._native.layernorm(None, None, None, 1e-5, None) is None  # not a plain call
+            assert isinstance(msd._native, msd._NoNative) and msd._native.linear_rows_grouped(1, 2, 3) is None
+            with pytest.raises(msd.MsdError):  # what the general path says of tensors that are on no device
+                msd.silu(torch.ones(4))
+        assert len(warned) == 1
+        msd.load_library(msd.LIB_HIP_PATH)  # binds again: nothing to bind here
+        return str(warned[0].message)
+
+    with monkeypatch.context() as m:
+        m.setattr(torch.version, "git_version", "0" * 40)
+        assert native.built_for in general_path()
+    monkeypatch.setattr(msd, "TORCH_CALLS_PATH", str(tmp_path / "msd_torch_calls.so"))
+    assert "does not load" in general_path()
+    (tmp_path / "msd_torch_calls.so").write_bytes(b"no library")
+    assert "does not load" in general_path()
