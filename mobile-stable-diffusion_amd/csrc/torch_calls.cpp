@@ -20,6 +20,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <algorithm>
 #include <vector>
 
 #include "../../include/msd_hip.h"
@@ -133,6 +134,16 @@ at::Tensor new_tensor(at::IntArrayRef shape, at::ScalarType type, const at::Tens
     return at::Tensor(at::detail::empty_cuda(shape, type, like.device(), std::nullopt));
 }
 
+// Whether a contiguous tensor has the strides that a new one of its shape gets.  Those of axes of length one can be any
+// (channels last with one position per channel), and torch.empty_like keeps them.
+bool plain_strides(const at::Tensor &t) {
+    const at::IntArrayRef sizes = t.sizes(), strides = t.strides();
+    int64_t stride = 1;
+    for (size_t i = sizes.size(); i-- > 0; stride *= std::max<int64_t>(sizes[i], 1))
+        if (strides[i] != stride) return false;
+    return true;
+}
+
 // An output: the caller's tensor, or a new one.
 struct Out {
     PyObject *object = nullptr;  // the caller's
@@ -142,6 +153,10 @@ struct Out {
     void take(Call &c, PyObject *o, const at::Tensor &like) {  // like `like`, or what the caller gave
         if (!c.ok) return;
         if (o == Py_None) {
+            if (!plain_strides(like)) {
+                c.ok = false;
+                return;
+            }
             make(new_tensor(like.sizes(), like.scalar_type(), like));
         } else if (const at::Tensor *t = c.same(o, like, like.numel())) {
             object = o;

@@ -121,6 +121,29 @@ def test_native_calls_take_the_plain_call_and_leave_the_others(msd, cuda):
     assert torch.equal(recorded, msd.layernorm(x, g, b))
 
 
+def test_new_outputs_have_the_strides_of_the_general_path(msd, cuda, monkeypatch):
+    """torch.empty_like keeps the strides of axes of length one, which a contiguous tensor may have any of."""
+    import torch
+    gamma, beta = torch.ones(64, device=cuda), torch.zeros(64, device=cuda)
+    planes = torch.randn(2, 64, 1, 1, device=cuda).to(memory_format=torch.channels_last)
+    one = torch.randn(3, 5, 64, device=cuda)[:1, 2:3]
+    none = torch.randn(2, 64, 3, 0, device=cuda).to(memory_format=torch.channels_last)
+    odd = [planes, one, torch.randn(4, 64, device=cuda).as_strided((1, 64), (7, 1)), none, torch.randn(2, 64, 1, 8, device=cuda)]
+    assert planes.is_contiguous() and planes.stride(1) == 1 and one.is_contiguous() and one.stride(0) == 320
+    calls = [(msd.silu, x) for x in odd] + [(msd.gelu, x) for x in odd] + [(lambda x: msd.elemwise_add(x, x), x) for x in odd] + \
+        [(lambda x: msd.groupnorm(x, gamma, beta, 8), planes), (lambda x: msd.groupnorm(x, gamma, beta, 8), odd[-1]),
+         (lambda x: msd.layernorm(x, gamma, beta), one), (lambda x: msd.add_layernorm(x, x, gamma, beta)[1], one),
+         (lambda x: msd.chunk_add_groupnorm(x, x, gamma, beta, 8), planes), (msd.softmax, one),
+         (lambda x: msd.ddim_update(x, x, 0.5, 0.6, 0.7), one), (lambda x: msd.chunkwise_add(x, x, 1), planes)]
+    for i, (f, x) in enumerate(calls):
+        native = f(x)
+        with monkeypatch.context() as m:
+            m.setattr(msd, "_native", _General())
+            general = f(x)
+        assert native.stride() == general.stride() == torch.empty_like(x).stride(), i
+        assert torch.equal(native, general), i
+
+
 def test_native_calls_use_the_threads_stream(msd, cuda):
     """Threads on streams of their own: what a call reads was written on its stream just before."""
     import torch
