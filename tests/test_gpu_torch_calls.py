@@ -162,3 +162,71 @@ def test_native_calls_use_the_threads_stream(msd, cuda):
     [t.start() for t in threads]
     [t.join() for t in threads]
     assert not wrong
+
+
+# Which calls of _cases are plain: the extension makes them, or refuses them with the library's code, and leaves the others.
+_PLAIN = {
+    "groupnorm": {0, 1, 2, 3, 4, 11, 17, 19}, "chunk_add_groupnorm": {0, 2, 3}, "groupnorm_tokens": {0, 1, 2},
+    "permute_0_2_1": {0, 3}, "layernorm": {0, 1, 5}, "add_layernorm": {0, 2}, "elemwise_add": {0, 2}, "chunkwise_add": {0, 3},
+    "geglu": {0, 1, 3, 4}, "silu": {0, 1}, "gelu": {0}, "quick_gelu": {0}, "timestep_embedding": {0, 1, 2, 5},
+    "linear_rows": {0, 1, 2, 7, 8}, "linear_rows_grouped": {0, 1, 5, 6, 7}, "softmax": {0, 1, 3}, "ddim_update": {0, 1, 2},
+}
+
+
+class _Recorder:
+    """Passes calls on to the extension and notes whether it made them."""
+
+    def __init__(self, native):
+        self.native, self.made = native, []
+
+    def __getattr__(self, name):
+        def call(*args):
+            self.made.append((name, True))  # (so it stands if the extension raises)
+            done = getattr(self.native, name)(*args)
+            self.made[-1] = name, done is not None
+            return done
+        return call
+
+
+@pytest.mark.parametrize("half", [False, True], ids=["f32", "f16"])
+def test_every_plain_call_is_made_by_the_extension_and_no_other(msd, cuda, half, monkeypatch):
+    import torch
+    cases = _cases(torch, msd, cuda, half)
+    native = msd._bind_native()
+    entries = {n for n in dir(native) if not n.startswith("__")} - {"bind", "names", "built_for"}
+    assert set(cases) == set(_PLAIN) == entries
+    recorder = _Recorder(native)
+    monkeypatch.setattr(msd, "_native", recorder)
+    for name, calls in cases.items():
+        for i, args in enumerate(calls):
+            recorder.made.clear()
+            _outcome(torch, getattr(msd, name), args)
+            assert (name, True) in recorder.made if i in _PLAIN[name] else recorder.made in ([], [(name, False)]), (name, i)
+
+
+def test_native_calls_wait_for_what_is_on_the_threads_stream(msd, cuda):
+    """The operand is written behind work that takes far longer than the host needs to reach the call's launch: on any other
+    stream the call would read what was there before."""
+    import torch
+    wrong = []
+
+    def work(i):
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            big, x = torch.empty(1 << 28, device=cuda), torch.full((64, 256), -1.0, device=cuda)  # (1 GiB)
+            for k in range(4):
+                x.fill_(-1.0)
+                stream.synchronize()
+                for _ in range(16):  # (some 3 ms)
+                    big.fill_(float(k))
+                x.fill_(float(i + k))
+                waits = not stream.query()
+                y = msd.elemwise_add(x, x)
+                if not waits or not bool((y == 2.0 * (i + k)).all()):
+                    wrong.append((i, k, waits))
+
+    for i in range(4):  # one after the other: threads that wait for the interpreter could let the work end before the call
+        thread = threading.Thread(target=work, args=(i,))
+        thread.start()
+        thread.join()
+    assert not wrong
