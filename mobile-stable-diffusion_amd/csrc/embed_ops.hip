@@ -280,14 +280,17 @@ __global__ __launch_bounds__(kLinWgThreads, 4) void linear_quads_grouped_kernel(
 }
 
 // Large groups of 4-byte elements, 2 ... 8 rows: four wavefronts share the rows of x, activated once, in LDS, and each takes
-// C columns against them.  The order of every sum is that of linear_rows_body.  Bound by the latency of its three steps
+// four columns against them.  The order of every sum is that of linear_rows_body.  Bound by the latency of its three steps
 // (x to LDS, barrier, products) and, from five rows on, by the products.  The 22 projections of a step, 103 MB of
 // weights, us, before with two columns per wavefront and so: 2 rows 21 - 24 -> 20, 4 rows 34 - 43 -> 24.5, 8 rows
 // 53 - 59 -> 29 (1 row: 18).  Two columns instead of four 33 at 8 rows, float32 matrix products 28, with other sums.
-template <int M, int C, int ROUND>
+constexpr int kSharedCols = 4;
+
+template <int M>
 __global__ __launch_bounds__(kLinWgThreads) void linear_shared_grouped_kernel(const float *__restrict__ x, LinearGroup group,
-                                                                                uint32_t m, uint32_t kvecs, int act_in,
-                                                                                int act_out) {
+                                                                              uint32_t m, uint32_t kvecs, int act_in,
+                                                                              int act_out) {
+    constexpr int C = kSharedCols, ROUND = 5;
     constexpr uint32_t kChunk = ROUND * kWave;  // pieces of a row of x in LDS at a time
     __shared__ f32x4 xs[M][kChunk];
     uint32_t p = 0;
@@ -744,6 +747,7 @@ void linear_quads(size_t m, size_t n, int act_in, F f) {
     if (linear_column_quads(n) == 4) with_rows(std::integral_constant<int, 4>{}, std::integral_constant<int, 1>{});
     else with_rows(std::integral_constant<int, 2>{}, std::integral_constant<int, 3>{});
 }
+
 template <typename T, int VPL, int TL, bool RAGGED>
 void softmax_team_launch(const T *x, T *y, uint32_t rows, uint32_t cols, int stable, hipStream_t stream) {
     // long rows (a wavefront per row, 8 or 16 vectors per lane) run as single-wavefront workgroups, the shorter
@@ -889,7 +893,6 @@ int linear_rows_grouped_dispatch(const void *xv, const void *const *ws, const fl
     for (size_t i = 0; i < count; i++) total_n += ns[i];
     const bool quads = linear_takes_quads<T>(m, total_n, act_in);
     const bool shared = sizeof(T) == 4 && m >= 2 && total_n >= 8192;  // (fewer columns leave it too few workgroups)
-    constexpr int kSharedCols = 4;
     const int cpw = quads ? kLinBlock * linear_column_quads(total_n) : shared ? kLinWgWaves * kSharedCols  // (columns of a workgroup)
                     : (sizeof(T) == 2 && m_pad <= 2 && total_n >= 8192) ? 4 : act_in ? 2 : 1;
     for (size_t base = 0; base < count; base += kLinGroupMax) {
@@ -917,9 +920,9 @@ int linear_rows_grouped_dispatch(const void *xv, const void *const *ws, const fl
                 launch((linear_quads_grouped_kernel<rows, cols, round, act>), dim3(blocks), dim3(kLinWgThreads), 0, stream,
                        static_cast<const __half *>(xv), g, (uint32_t)m, (uint32_t)(k / EPV), act_out);
             });
-        else if (shared && m_pad == 2) rows_in_lds(linear_shared_grouped_kernel<2, kSharedCols, 5>);
-        else if (shared && m_pad == 4) rows_in_lds(linear_shared_grouped_kernel<4, kSharedCols, 5>);
-        else if (shared) rows_in_lds(linear_shared_grouped_kernel<8, kSharedCols, 5>);
+        else if (shared && m_pad == 2) rows_in_lds(linear_shared_grouped_kernel<2>);
+        else if (shared && m_pad == 4) rows_in_lds(linear_shared_grouped_kernel<4>);
+        else if (shared) rows_in_lds(linear_shared_grouped_kernel<8>);
         else switch (m_pad) {
             case 1: linear_grouped_launch<T, 1>(x, g, (uint32_t)m, (uint32_t)k, act_in, act_out, cpw, stream); break;
             case 2: linear_grouped_launch<T, 2>(x, g, (uint32_t)m, (uint32_t)k, act_in, act_out, cpw, stream); break;

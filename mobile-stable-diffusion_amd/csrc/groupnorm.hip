@@ -1111,22 +1111,16 @@ GnTokUnitPlan gn_tokens_unit_plan(const Chip &chip, size_t units, size_t cpg, si
     uint32_t w = tune_writers > 0 ? (uint32_t)tune_writers : 1;
     if (tune_writers == 0 && may_share)
         while (w < 8 && units * w * 2 <= chip.cus) w *= 2;
-    for (bool more = true; more; w *= 2) {
-        pl.writers = w;
-        const size_t vecs = (hw / EPV + w - 1) / w;  // per channel and part
-        pl.part_pos = (uint32_t)(pl.ragged ? (hw + w - 1) / w : vecs * EPV);
+    auto cut = [&](uint32_t parts) {
+        const size_t vecs = (hw / EPV + parts - 1) / parts;  // per channel and part
+        pl.writers = parts;
+        pl.part_pos = (uint32_t)(pl.ragged ? (hw + parts - 1) / parts : vecs * EPV);
         pl.pitch = (uint32_t)(pl.ragged ? hw : vecs * EPV + EPV);
         pl.lds = (cpg * pl.pitch * sizeof(T) + 15) / 16 * 16;
-        // (a part more where one is too much for the LDS)
-        more = !pl.ragged && tune_writers == 0 && may_share && pl.lds > kGnTokMaxLds && w < 8;
-    }
-    while (pl.writers > 1 && (size_t)(pl.writers - 1) * pl.part_pos >= hw) {  // no empty part
-        pl.writers /= 2;
-        const size_t vecs = (hw / EPV + pl.writers - 1) / pl.writers;
-        pl.part_pos = (uint32_t)(pl.ragged ? (hw + pl.writers - 1) / pl.writers : vecs * EPV);
-        if (!pl.ragged) pl.pitch = (uint32_t)(vecs * EPV + EPV);
-        pl.lds = (cpg * pl.pitch * sizeof(T) + 15) / 16 * 16;
-    }
+    };
+    cut(w);
+    while (!pl.ragged && tune_writers == 0 && may_share && pl.lds > kGnTokMaxLds && pl.writers < 8) cut(pl.writers * 2);
+    while (pl.writers > 1 && (size_t)(pl.writers - 1) * pl.part_pos >= hw) cut(pl.writers / 2);  // no empty part
     if (pl.lds > kGnTokMaxLds) return pl;
     const uint32_t max_k = sizeof(T) == 4 ? 10 : kGnMaxRaggedK;
     // (writers that a knob asks for get the lanes of a launch with a workgroup per CU)
