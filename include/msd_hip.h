@@ -290,7 +290,8 @@ int msd_ddim_timesteps(int ddim_num_steps, int *out, int cap);
  *                            (M/nn/ResBlock.cpp:173-183)
  * The reference adds the k products in ascending order into one accumulator; here each of
  * 64 lanes adds its share in ascending order and a fixed tree adds the lanes (agreement
- * within float32 summation error, see the tests).  y must not overlap x
+ * within float32 summation error, see the tests), with the same products and the same order
+ * for every m: a row has the same bits whatever rows come with it.  y must not overlap x
  * (M/nn/Linear.cpp:78-81).
  */
 #define MSD_ACT_NONE 0

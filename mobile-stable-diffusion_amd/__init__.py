@@ -110,8 +110,8 @@ def check(code):
 # 3.5 us of the runtime's launch), so plain calls (dense device tensors that fit each other, no mode or transform around
 # them) go through csrc/torch_calls.cpp, which checks them, makes the outputs and calls the C ABI; it returns None for any
 # other, which the general path below it then makes or refuses.  Eager passes, us, from Python and so: four calls of a
-# sampler's tick 24.8 -> 16.4, the 49 of a text encoder 322 -> 237, 22 grouped projections 53 -> 19.5, the 8 of a
-# 640-channel transformer block 53.5 -> 38.
+# sampler's tick 25.0 -> 14.4, the 49 of a text encoder 325 -> 198 (to 222), 22 grouped projections 53 -> 15.3, the 8 of a
+# 640-channel transformer block 55.6 -> 35.8.
 class _Unbound:
     """Stands for the native calls until the first one."""
 

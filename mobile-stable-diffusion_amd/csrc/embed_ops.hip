@@ -451,11 +451,10 @@ __global__ __launch_bounds__(kSmThreads) void softmax_team_kernel(const T *x, T 
 
 // Rows of more than 256 vectors: the row lives in the registers of a workgroup, VPL 16-byte vectors per lane,
 // one read and one write per element; the wavefronts' maxima and sums meet in LDS.  Bound by HBM, and by how many
-// rows are open at once: what the CUs hold between a row's read and its write is a window on memory that moves
-// through x and y, and beyond about 48 KB a CU a wider window only costs (rows scattered over more pages, reads among
-// writes).  The launch therefore asks for LDS it does not use, which is what keeps workgroups off a CU
-// (softmax_block_launch).  A wavefront per row with 8 - 16 vectors a lane and workgroups of 8 a lane, both as many
-// as fit, before, and so; us, TB/s: fp16 65536 x 4096 170 -> 167 (6.4), 102400 x 6400 437 -> 420 (6.2), 123904 x 7744
+// rows are open at once: beyond about 48 KB of them a CU, read and not yet written, more only cost time (the
+// figures are at softmax_block_launch; the cause was not measured).  The launch therefore asks for LDS it does not use,
+// which is what keeps workgroups off a CU.  A wavefront per row with 8 - 16 vectors a lane and workgroups of 8 a lane, both as many
+// as fit, before, and so; us, TB/s: fp16 65536 x 4096 169.4 -> 168.3 (6.4), 102400 x 6400 437 -> 420 (6.2), 123904 x 7744
 // 661 -> 630 (6.1), 135168 x 8448 796 -> 748 (6.1), 147456 x 9216 917 -> 899 (6.0); fp32 65536 x 4096 351 -> 335 (6.4),
 // 102400 x 6400 905 -> 862 (6.1), 73728 x 9216 967 -> 906 (6.0).  A copy takes 6.4 to 6.6.
 // x and y may be the same buffer: a lane stores only what it loaded itself.
@@ -795,7 +794,9 @@ void softmax_block_launch(const T *x, T *y, uint32_t rows, uint32_t row_vecs, in
 // A row of 257 vectors up to what a wavefront's registers hold (512 of 2-byte storage, whose floats take twice the
 // room, 1024 of 4-byte): a workgroup per row where the rows leave CUs idle or fill the chip many times, a wavefront per
 // row between.  us, wavefront and workgroup: fp16 16 x 3072 2.67 / 2.38, 256 x 4096 3.20 / 2.91, 1024 x 3072 stable 4.15 /
-// 4.32, 4096 x 2304 stable 8.88 / 9.32, 8192 x 4096 23.5 / 22.8, 49152 x 3072 97.2 / 94.4; fp32 16 x 3072 2.58 / 2.03,
+// 4.32, 4096 x 2304 stable 8.88 / 9.32, 8192 x 4096 23.3 / 22.6, 36864 x 2304 55.7 / 53.4, 49152 x 3072 95.8 / 93.6, 65536 x 4096
+// 169.4 / 168.3 (8192 to 131072 fp16 rows of 2056 to 4096, 192 launches: 0.96 up to 2304 columns, 0.98 - 0.99 from 3584 on, none
+// slower by more than two runs differ); fp32 16 x 3072 2.58 / 2.03,
 // 2048 x 4096 11.2 / 12.7, 2048 x 2304 7.14 / 8.4, 3072 x 3072 14.6 / 13.9, 8192 x 4096 44.8 / 42.1.
 template <typename T>
 bool softmax_wave_per_row(uint32_t rows, uint32_t row_vecs) {

@@ -715,8 +715,9 @@ __global__ __launch_bounds__(kGnMaxThreads) void gn_tokens_kernel(
 // in gn_slice_kernel<..., SHARED>, nothing is exchanged).  What a part needs goes to LDS as it was loaded, before the
 // statistics are there, so one barrier covers both; it is normalised on the way out, by lanes that keep to their channels.
 // An XCD takes units_per_xcd units in a row: what the writers of a unit load meets in its L2, and so do the pieces of an
-// output line (ch_per_group elements each) that neighbouring groups store; with units dealt to the XCDs in turn every line
-// was put together in memory from several.
+// output line (ch_per_group elements each) that neighbouring groups store; with units dealt to the XCDs in turn a line
+// went to memory in several.  KiB written (WRITE_SIZE), units in turn and so, which is the output's size: fp16 batch 2, 640
+// channels at 32 x 32 4096 / 2560, at 36 x 28 4048 / 2520, 1280 at 16 x 16 1536 / 1280; fp32 640 at 32 x 32 6144 / 5120.
 // RAGGED: hw is no whole number of vectors, a vector may cross from one channel into the next; LDS then holds the whole unit
 // as it lies in memory.
 struct GnTokUnitParams {
@@ -1190,8 +1191,8 @@ void gn_tokens_launch(uint32_t blocks, uint32_t threads, size_t lds_bytes, hipSt
 // 24 x 24 batch 2 6.4 / 5.0; fp32 640 at 32 x 32 batch 2 6.5 / 5.7, 16 24.3 / 22.6, 1280 at 18 x 14 batch 2 7.8 / 4.4.
 // Above the limits (ratio of this one to the others over 8000 random shapes, by KB a unit): up to half a unit per CU 128: 0.96,
 // 136: 1.01, 152: 1.03; up to one 104: 0.83, 112: 0.88, 120: 1.1 - 1.3; more 64: 0.95, 72: 1.0, 80: 1.0, 88: 1.1.
-// Ragged planes: the 2-byte ones whose rows are whole halves of a vector (others keep the two launches, though 2 x 1280 x 63
-// would take 2.7 us instead of 5.1), short runs of many units not (128 channels at 5732 batch 10 13.9 / 18.6).
+// Ragged planes: the 2-byte ones whose rows are whole halves of a vector.  The others keep the two launches: 2 x 1280 x 63
+// takes 5.1 us in them and would take 2.7 in one, but for which odd planes that holds has not been measured.  Short runs of many units not (128 channels at 5732 batch 10 13.9 / 18.6).
 inline bool gn_tokens_stays_whole(const Chip &chip, size_t elt, size_t units, size_t unit_size, size_t cpg, size_t hw) {
     if (hw * elt % 16 != 0 && (elt != 2 || hw % 4 != 0 || (cpg * elt < 40 && units > chip.cus))) return false;
     const size_t limit = units * 2 <= chip.cus ? 128 : units <= chip.cus ? 112 : 72;
