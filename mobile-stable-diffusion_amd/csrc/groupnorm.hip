@@ -42,13 +42,16 @@ namespace {
 
 constexpr uint32_t kGnSpinLimit = 2048;  // default poll limit: about half a microsecond per poll
 constexpr int kGenericThreads = 256;
+constexpr int kGnRedRow = 16;                // partial sums of a workgroup, one per wavefront: a row of lanes
+constexpr int kGnRedSlots = 3 * kGnRedRow;   // sums, sums of squares, sums about the mean
+static_assert(kGnMaxThreads / kWave <= kGnRedRow, "a row of lanes holds the wavefronts' partial sums");
 
 struct GnParams {
     uint32_t vec_per_unit;   // 16-byte vectors per unit
     uint32_t vec_per_slice;  // vectors per workgroup (the last slice may be shorter)
     uint32_t split;          // workgroups per unit, power of two <= kGnMaxSplit
     uint32_t split_shift;    // log2(split)
-    uint32_t groups;
+    FastDiv groups;          // per sample
     uint32_t ch_per_group;
     FastDiv hw_vec;          // vectors per channel (RAGGED: elements per channel)
     float eps;
@@ -245,30 +248,35 @@ constexpr float kGnFoldMean = 16.0f;
 // mean is large against the spread (or the slice is constant) a second pass over the registers
 // sums (x - mean)^2 instead, so the result is as accurate as a two-pass variance either way.
 // The choice is the same in every wavefront: they all hold bit-identical sums.
+// Between the last load's return and the first store this is the launch's critical path: the two sums
+// are reduced together (one value per lane after the first half of the steps), a wavefront's pair takes one LDS access each way,
+// the at most 16 partial sums meet in one row of lanes, and the mean is a product with the reciprocal of the count, which
+// is there before the loads return, and one correction (correctly rounded, as the division it stands for).  us per launch at
+// batch 2, six LDS swizzles one after the other and a division, and so: fp16 320 channels at 64 x 64 5.19 -> 4.94, in place 5.93 ->
+// 5.76, 640 at 32 x 32 3.92 -> 3.74, in place 4.76 -> 4.59, 1280 at 8 x 8 2.65 -> 2.50; fp32 640 at 32 x 32 in place 5.58 -> 5.29.
 template <typename T, int K, bool FULL>
-__device__ __forceinline__ void gn_slice_stats(u32x4 (&raw)[K], uint32_t n_valid, float *red_a,
-                                               float *red_b, float *red_c, float &slice_mean,
+__device__ __forceinline__ void gn_slice_stats(u32x4 (&raw)[K], uint32_t n_valid, float *red, float &slice_mean,
                                                float &slice_m2) {
     constexpr int EPV = Store<T>::EPV;
     const uint32_t tid = threadIdx.x;
     const uint32_t nt = blockDim.x;
     const uint32_t lane = tid & (kWave - 1);
     const uint32_t nw = nt / kWave;
+    const float count = (float)(n_valid * EPV);
+    float inv = 1.0f / count;
+    asm volatile("" : "+v"(inv));  // (computed here, while the loads are in flight)
     float s[2] = {0.0f, 0.0f}, q[2] = {0.0f, 0.0f};
 #pragma unroll
     for (int k = 0; k < K; k++) Moments<T>::add(raw[k], s, q);
-    const float wave_s = wave_sum(s[0] + s[1]);
-    const float wave_q = wave_sum(q[0] + q[1]);
-    if (lane == 0) {
-        red_a[tid / kWave] = wave_s;
-        red_b[tid / kWave] = wave_q;
-    }
+    const float wave_sums = wave_sum_of_two(s[0] + s[1], q[0] + q[1]);
+    if (lane % kGnRedRow == 0 && lane < 2 * kGnRedRow) red[lane + tid / kWave] = wave_sums;
     __syncthreads();
-    const bool entry = lane < nw;
-    const float sum_x = wave_sum(entry ? red_a[lane] : 0.0f);
-    const float sum_xx = wave_sum(entry ? red_b[lane] : 0.0f);
-    const float count = (float)(n_valid * EPV);
-    slice_mean = sum_x / count;
+    const bool entry = lane % kGnRedRow < nw;
+    const float sums = team_sum<kGnRedRow>(entry ? red[lane % (2 * kGnRedRow)] : 0.0f);
+    const float sum_x = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(sums), 0));
+    const float sum_xx = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(sums), kGnRedRow));
+    const float quotient = sum_x * inv;
+    slice_mean = fmaf(fmaf(-quotient, count, sum_x), inv, quotient);
     slice_m2 = sum_xx - sum_x * slice_mean;
     // n mean^2 <= kappa M2; false also for a negative or NaN M2
     if (!(sum_x * slice_mean <= kGnFastMoments * slice_m2)) {  // uniform over the workgroup
@@ -290,9 +298,10 @@ __device__ __forceinline__ void gn_slice_stats(u32x4 (&raw)[K], uint32_t n_valid
             __builtin_amdgcn_sched_barrier(0);
         }
         const float wave_c = wave_sum(c);
+        float *red_c = red + 2 * kGnRedRow;
         if (lane == 0) red_c[tid / kWave] = wave_c;
         __syncthreads();
-        slice_m2 = wave_sum(entry ? red_c[lane] : 0.0f);
+        slice_m2 = wave_sum(lane < nw ? red_c[lane] : 0.0f);
     }
 }
 
@@ -321,8 +330,8 @@ __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
                                         const float *__restrict__ gamma,
                                         const float *__restrict__ beta, const GnScratch &scratch,
                                         const GnParams &p, uint32_t unit, uint32_t slice, uint32_t part,
-                                        uint32_t v_begin, uint32_t v_end, float *red_a,
-                                        float *red_b, float *red_c, float *stats, float2 *aff) {
+                                        uint32_t v_begin, uint32_t v_end, float *red, float *stats,
+                                        float2 *aff) {
     constexpr int EPV = Store<T>::EPV;
     const uint32_t tid = threadIdx.x;
     const uint32_t nt = blockDim.x;
@@ -360,19 +369,21 @@ __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
     };
 #pragma unroll
     for (int k = 0; k < K; k++) raw[k] = load_stream(at(xin, k, tid));
-    const uint32_t ch0 = (unit % p.groups) * p.ch_per_group;
+    const uint32_t ch0 = (unit - fast_div(unit, p.groups) * p.groups.d) * p.ch_per_group;
+    // the addends of the unit's channels
+    auto unit_chunk = [&]() { return chunk + (size_t)unit * p.ch_per_group; };
     // v plus its channels' addends, rounded to the storage type
     auto with_chunk = [&](const u32x4 &raw_v, uint32_t v, const T *cb) {
         float f[EPV];
         Store<T>::unpack(raw_v, f);
         if (RAGGED) {
             const GnStraddle at_v = gn_straddle<EPV>(v, p.hw_vec);
-            const float c0 = Store<T>::load1(cb + ch0 + at_v.channel);
-            const float c1 = Store<T>::load1(cb + ch0 + min(at_v.channel + 1, p.ch_per_group - 1));
+            const float c0 = Store<T>::load1(cb + at_v.channel);
+            const float c1 = Store<T>::load1(cb + min(at_v.channel + 1, p.ch_per_group - 1));
 #pragma unroll
             for (int e = 0; e < EPV; e++) f[e] += (uint32_t)e < at_v.first ? c0 : c1;
         } else {
-            const float cv = Store<T>::load1(cb + ch0 + fast_div(v, p.hw_vec));
+            const float cv = Store<T>::load1(cb + fast_div(v, p.hw_vec));
 #pragma unroll
             for (int e = 0; e < EPV; e++) f[e] += cv;
         }
@@ -382,7 +393,7 @@ __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
     // chunkwise_add pass): the sum replaces the slice in registers, rounded to the storage
     // type exactly as a separate add kernel would have stored it
     if (chunk != nullptr) {  // uniform
-        const T *cb = chunk + (size_t)(unit / p.groups) * (p.groups * p.ch_per_group);
+        const T *cb = unit_chunk();
 #pragma unroll
         for (int k = 0; k < K; k++) raw[k] = with_chunk(raw[k], vidx(k, tid), cb);
     }
@@ -414,7 +425,7 @@ __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
     }
 
     float slice_mean, slice_m2;
-    gn_slice_stats<T, K, FULL>(raw, v_end - v_begin, red_a, red_b, red_c, slice_mean, slice_m2);
+    gn_slice_stats<T, K, FULL>(raw, v_end - v_begin, red, slice_mean, slice_m2);
 
     float mean, rstd;
     uint32_t arrived_before = 0;
@@ -427,7 +438,7 @@ __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
             const uint32_t v = l * p.vec_per_slice + i;
             u32x4 r = xin[v];
             if (chunk != nullptr) {
-                r = with_chunk(r, v, chunk + (size_t)(unit / p.groups) * (p.groups * p.ch_per_group));
+                r = with_chunk(r, v, unit_chunk());
             }
             return r;
         };
@@ -522,9 +533,7 @@ template <typename T, int K, bool SILU, bool SHARED, bool RAGGED>
 __global__ __launch_bounds__(kGnMaxThreads, (K <= (sizeof(T) == 2 ? 5 : 4) ? 8 : 4)) void gn_slice_kernel(
     const T *x, const T *chunk, T *y, const float *__restrict__ gamma,
     const float *__restrict__ beta, GnScratch scratch, GnParams p) {
-    __shared__ float red_a[kGnMaxThreads / kWave];
-    __shared__ float red_b[kGnMaxThreads / kWave];
-    __shared__ float red_c[kGnMaxThreads / kWave];
+    __shared__ float red[kGnRedSlots];
     __shared__ float stats[2];
     __shared__ float2 aff[!RAGGED && K <= kGnPrefetchAffineK ? 1 : kGnLdsChannels];  // (gamma, beta) of the group's channels
     uint32_t unit, slice, part;
@@ -543,10 +552,10 @@ __global__ __launch_bounds__(kGnMaxThreads, (K <= (sizeof(T) == 2 ? 5 : 4) ? 8 :
     // uniform over the workgroup; the largest K is only launched on slices it fits exactly
     if (K == kGnMaxK || v_end - v_begin == K * blockDim.x)
         gn_body<T, K, SILU, true, SHARED, RAGGED>(x, chunk, y, gamma, beta, scratch, p, unit, slice, part, v_begin, v_end,
-                                          red_a, red_b, red_c, stats, aff);
+                                          red, stats, aff);
     else
         gn_body<T, K, SILU, false, SHARED, RAGGED>(x, chunk, y, gamma, beta, scratch, p, unit, slice, part, v_begin, v_end,
-                                           red_a, red_b, red_c, stats, aff);
+                                           red, stats, aff);
 }
 
 // Any shape or alignment (units that are no whole number of vectors, channels of less than a vector, many
@@ -611,9 +620,7 @@ __global__ __launch_bounds__(kGnMaxThreads) void gn_tokens_kernel(
     const float *__restrict__ beta, GnScratch scratch, GnTokParams q) {
     constexpr int EPV = Store<T>::EPV;
     extern __shared__ u32x4 lds_vec[];
-    __shared__ float red_a[kGnMaxThreads / kWave];
-    __shared__ float red_b[kGnMaxThreads / kWave];
-    __shared__ float red_c[kGnMaxThreads / kWave];
+    __shared__ float red[kGnRedSlots];
     __shared__ float stats[2];
     const GnParams &p = q.base;
     const uint32_t tid = threadIdx.x;
@@ -625,7 +632,8 @@ __global__ __launch_bounds__(kGnMaxThreads) void gn_tokens_kernel(
     // the slices of a unit stay adjacent
     const uint32_t group = fast_div(blockIdx.x, q.combos);
     const uint32_t combo = blockIdx.x - group * q.combos.d;
-    const uint32_t unit = (combo >> p.split_shift) * p.groups + group;
+    const uint32_t sample = combo >> p.split_shift;
+    const uint32_t unit = sample * p.groups.d + group;
     const uint32_t slice = combo & (p.split - 1);
     const uint32_t nvec = p.vec_per_slice;
     const uint32_t pvs = q.pos_vecs.d;
@@ -648,10 +656,10 @@ __global__ __launch_bounds__(kGnMaxThreads) void gn_tokens_kernel(
 #pragma unroll
         for (int i = 0; i < 4; i++) raw[k][i] = have ? raw[k][i] : 0u;
     }
-    const uint32_t ch0 = (unit % p.groups) * p.ch_per_group;
+    const uint32_t ch0 = group * p.ch_per_group;
 
     float slice_mean, slice_m2;
-    gn_slice_stats<T, K, false>(raw, nvec, red_a, red_b, red_c, slice_mean, slice_m2);
+    gn_slice_stats<T, K, false>(raw, nvec, red, slice_mean, slice_m2);
 
     float mean, rstd;
     if (p.split == 1) {
@@ -690,7 +698,6 @@ __global__ __launch_bounds__(kGnMaxThreads) void gn_tokens_kernel(
     // ---- token-major store: for each position of the slice one run of ch_per_group values
     const uint32_t rows = pvs * EPV;                         // positions in the slice
     const uint32_t words = rows * q.row_dwords.d;            // 4-byte words to write
-    const uint32_t sample = unit / p.groups;
     const size_t first = ((size_t)sample * q.hw + (size_t)slice * rows) * q.channels + ch0;
     uint32_t *out = reinterpret_cast<uint32_t *>(y + first);
     const uint32_t row_stride = q.channels * sizeof(T) / 4;  // words between positions
@@ -722,7 +729,8 @@ __global__ __launch_bounds__(kGnMaxThreads) void gn_tokens_kernel(
 // as it lies in memory.
 struct GnTokUnitParams {
     uint32_t vec_per_unit;
-    uint32_t groups, ch_per_group, channels, hw;
+    FastDiv groups;          // per sample
+    uint32_t ch_per_group, channels, hw;
     uint32_t writers, writers_shift, xcd_shift;
     uint32_t units_per_xcd;  // units >> xcd_shift
     uint32_t part_pos;       // positions of a part; of the last one what is left
@@ -741,14 +749,15 @@ __device__ __forceinline__ void gn_tokens_store(const T *lds, T *y, uint32_t uni
     constexpr int N = 4 / (int)sizeof(T);  // channels per store
     const uint32_t row0 = fast_div(threadIdx.x, q.row_dwords), c0 = (threadIdx.x - row0 * q.row_dwords.d) * N;
     if (row0 >= q.row_step) return;
-    const uint32_t ch0 = (unit % q.groups) * q.ch_per_group + c0;
+    const uint32_t sample = fast_div(unit, q.groups);
+    const uint32_t ch0 = (unit - sample * q.groups.d) * q.ch_per_group + c0;
     float a[N], b[N];
 #pragma unroll
     for (int i = 0; i < N; i++) {
         a[i] = rstd * gamma[ch0 + i];
         b[i] = beta[ch0 + i];
     }
-    T *out = y + ((size_t)(unit / q.groups) * q.hw + pos0) * q.channels + ch0;
+    T *out = y + ((size_t)sample * q.hw + pos0) * q.channels + ch0;
     const T *in = lds + c0 * q.pitch;
 #pragma unroll 4
     for (uint32_t r = row0; r < rows; r += q.row_step) {
@@ -772,9 +781,7 @@ __global__ __launch_bounds__(kGnMaxThreads) void gn_tokens_unit_kernel(
     GnTokUnitParams q) {
     constexpr int EPV = Store<T>::EPV;
     extern __shared__ u32x4 lds_vec[];
-    __shared__ float red_a[kGnMaxThreads / kWave];
-    __shared__ float red_b[kGnMaxThreads / kWave];
-    __shared__ float red_c[kGnMaxThreads / kWave];
+    __shared__ float red[kGnRedSlots];
     const uint32_t tid = threadIdx.x, nt = blockDim.x;
     const uint32_t of_xcd = blockIdx.x >> q.xcd_shift;
     const uint32_t part = of_xcd & (q.writers - 1);
@@ -800,7 +807,7 @@ __global__ __launch_bounds__(kGnMaxThreads) void gn_tokens_unit_kernel(
         for (int i = 0; i < 4; i++) raw[k][i] = have ? raw[k][i] : 0u;  // (the statistics rely on it)
     }
     float mean, m2;
-    gn_slice_stats<T, K, false>(raw, nvec, red_a, red_b, red_c, mean, m2);  // (its barrier covers the tile)
+    gn_slice_stats<T, K, false>(raw, nvec, red, mean, m2);  // (its barrier covers the tile)
     const float rstd = __builtin_amdgcn_rsqf(m2 * q.inv_count + q.eps);
     gn_tokens_store<T>(RAGGED ? lds + pos0 : lds, y, unit, pos0, rows, mean, rstd, gamma, beta, q);
 }
@@ -856,7 +863,8 @@ template <typename T>
 __global__ __launch_bounds__(kStatsThreads) void gn_stats_kernel(const T *__restrict__ x, float2 *__restrict__ partials,
                                                                  GnStatsParams p) {
     constexpr int EPV = Store<T>::EPV;
-    __shared__ float red_a[kStatsThreads / kWave], red_b[kStatsThreads / kWave], red_c[kStatsThreads / kWave];
+    __shared__ float2 red[kStatsThreads / kWave];
+    __shared__ float red_c[kStatsThreads / kWave];
     const uint32_t unit = fast_div(blockIdx.x, p.slices);
     const uint32_t slice = blockIdx.x - unit * p.slices.d;
     const uint32_t begin = slice * p.vec_per_slice;
@@ -876,17 +884,15 @@ __global__ __launch_bounds__(kStatsThreads) void gn_stats_kernel(const T *__rest
     float s[2] = {0.0f, 0.0f}, q[2] = {0.0f, 0.0f};
     for_each(u32x4{0, 0, 0, 0}, [&](const u32x4 &v) { Moments<T>::add(v, s, q); });
     const uint32_t lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-    auto total = [&](float v, float *slots) {
-        const float w = wave_sum(v);
-        if (lane == 0) slots[wave] = w;
-        __syncthreads();
-        float t = 0.0f;
+    const float sums = wave_sum_of_two(s[0] + s[1], q[0] + q[1]);
+    if (lane % kGnRedRow == 0 && lane < 2 * kGnRedRow) reinterpret_cast<float *>(&red[wave])[lane / kGnRedRow] = sums;
+    __syncthreads();
+    float sum_x = 0.0f, sum_xx = 0.0f;
 #pragma unroll
-        for (int i = 0; i < kStatsThreads / kWave; i++) t += slots[i];
-        return t;
-    };
-    const float sum_x = total(s[0] + s[1], red_a);
-    const float sum_xx = total(q[0] + q[1], red_b);
+    for (int i = 0; i < kStatsThreads / kWave; i++) {
+        sum_x += red[i].x;
+        sum_xx += red[i].y;
+    }
     const float mean = sum_x / (float)(n * EPV);
     float m2 = sum_xx - sum_x * mean;
     // as in gn_slice_stats: when the mean is large against the spread, a second pass about the mean
@@ -901,7 +907,12 @@ __global__ __launch_bounds__(kStatsThreads) void gn_stats_kernel(const T *__rest
                 c = fmaf(d, d, c);
             }
         }
-        m2 = total(c, red_c);
+        const float wave_c = wave_sum(c);
+        if (lane == 0) red_c[wave] = wave_c;
+        __syncthreads();
+        m2 = 0.0f;
+#pragma unroll
+        for (int i = 0; i < kStatsThreads / kWave; i++) m2 += red_c[i];
     }
     if (threadIdx.x == 0) partials[(size_t)unit * kGnStatSlices + slice] = make_float2(mean, m2);
 }
@@ -1060,7 +1071,7 @@ int gn_dispatch(const void *xv, const void *chunkv, void *yv, const float *gamma
     p.vec_per_slice = d.vec_per_slice;
     p.split = split;
     p.split_shift = (uint32_t)__builtin_ctz(split);
-    p.groups = (uint32_t)groups;
+    p.groups = make_fast_div((uint32_t)groups);
     p.ch_per_group = (uint32_t)cpg;
     p.hw_vec = make_fast_div((uint32_t)(ragged ? hw : hw / EPV));
     p.eps = eps;
@@ -1146,7 +1157,7 @@ int gn_tokens_unit(const GnTokUnitPlan &pl, const Chip &chip, const T *x, T *y, 
     const size_t cpg = channels / groups, unit_size = cpg * hw;
     GnTokUnitParams q;
     q.vec_per_unit = (uint32_t)(unit_size / EPV);
-    q.groups = (uint32_t)groups;
+    q.groups = make_fast_div((uint32_t)groups);
     q.ch_per_group = (uint32_t)cpg;
     q.channels = (uint32_t)channels;
     q.hw = (uint32_t)hw;
@@ -1354,7 +1365,7 @@ int gn_tokens_dispatch(const void *xv, void *yv, const float *gamma, const float
     q.base.writers_shift = 0;
     q.base.part_vecs = (uint32_t)nvec;
     q.base.xcd_shift = 0;
-    q.base.groups = (uint32_t)groups;
+    q.base.groups = make_fast_div((uint32_t)groups);
     q.base.ch_per_group = (uint32_t)cpg;
     q.base.hw_vec = make_fast_div((uint32_t)hw_vec);
     q.base.eps = eps;

@@ -120,7 +120,7 @@ __device__ __forceinline__ uint32_t fast_div(uint32_t n, const FastDiv &fd) {
 }
 
 // ---------------------------------------------------------------------------
-// Wavefront reductions with DPP (no LDS traffic for the first four steps).
+// Wavefront reductions with DPP and lane swaps (no LDS traffic).
 // ---------------------------------------------------------------------------
 template <int CTRL>
 __device__ __forceinline__ float dpp_move(float v) {
@@ -133,6 +133,19 @@ constexpr int kDppXor2 = 0x4E;        // quad_perm [2,3,0,1]
 constexpr int kDppHalfMirror = 0x141; // lane i <-> 7-i inside each 8
 constexpr int kDppRowMirror = 0x140;  // lane i <-> 15-i inside each 16
 
+// Sums of every lane's value and that of the lane 16 (32) away: v_permlane16_swap (v_permlane32_swap) of a value with
+// itself leaves one lane's value in one register and its partner's in the other.  Vector instructions of a few cycles, where
+// ds_swizzle is a round trip through LDS (over a hundred cycles, which these short launches wait for) and v_readlane
+// one through scalar registers; the same two values are added either way.
+__device__ __forceinline__ float row_pair_sum(float v) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float half_pair_sum(float v) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
 // Sum over aligned teams of TL lanes (TL = 4, 8, 16, 32 or 64); every lane of a
 // team ends with the team total, added in the same order in every lane pair.
 template <int TL>
@@ -142,17 +155,22 @@ __device__ __forceinline__ float team_sum(float v) {
     v += dpp_move<kDppXor2>(v);
     if (TL >= 8) v += dpp_move<kDppHalfMirror>(v);
     if (TL >= 16) v += dpp_move<kDppRowMirror>(v);
-    if (TL >= 32)  // swap 16-lane rows inside each 32: ds_swizzle bit mode, xor 0x10
-        v += __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), 0x401F));
-    if (TL >= 64) {
-        const float lo = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 0));
-        const float hi = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 32));
-        v = lo + hi;
-    }
+    if (TL >= 32) v = row_pair_sum(v);
+    if (TL >= 64) v = half_pair_sum(v);
     return v;
 }
 
 __device__ __forceinline__ float wave_sum(float v) { return team_sum<64>(v); }
+
+// wave_sum of two values at once, the additions of each the same: lanes 0 - 15 and 32 - 47 end with the sum of `a`, the
+// others with that of `b`.
+__device__ __forceinline__ float wave_sum_of_two(float a, float b) {
+    a = team_sum<16>(a);
+    b = team_sum<16>(b);
+    // the odd rows of `a` for the even rows of `b`: the rows are then a0 b0 a2 b2 and a1 b1 a3 b3
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return half_pair_sum(__uint_as_float(r[0]) + __uint_as_float(r[1]));
+}
 
 // Maximum over aligned teams of TL lanes, same exchange pattern as team_sum.
 template <int TL>
@@ -162,11 +180,13 @@ __device__ __forceinline__ float team_max(float v) {
     v = fmaxf(v, dpp_move<kDppXor2>(v));
     if (TL >= 8) v = fmaxf(v, dpp_move<kDppHalfMirror>(v));
     if (TL >= 16) v = fmaxf(v, dpp_move<kDppRowMirror>(v));
-    if (TL >= 32) v = fmaxf(v, __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), 0x401F)));
+    if (TL >= 32) {
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        v = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    }
     if (TL >= 64) {
-        const float lo = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 0));
-        const float hi = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 32));
-        v = fmaxf(lo, hi);
+        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        v = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
     }
     return v;
 }
