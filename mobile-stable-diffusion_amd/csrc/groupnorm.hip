@@ -741,39 +741,53 @@ struct GnTokUnitParams {
     float eps, inv_count;
 };
 
+// What a lane stores: always the same 4 bytes of an output run (its channels), of every row_step-th position.  gamma and beta
+// of those channels are requested behind the data and have arrived when the sums have (us per launch, requested behind the
+// sums and so, fp16 batch 2: 1280 channels at 8 x 8 2.70 -> 2.51, at 16 x 16 3.56 -> 3.27, 640 at 32 x 32 4.28 -> 4.18).
 // Stores of 4 bytes: 8 and 16 bytes at a time read LDS with more bank conflicts (us with 16 / 8 / 4 bytes, fp16 batch 2: 1280
 // channels at 16 x 16 4.2 / - / 3.7, 640 at 32 x 32 - / 4.9 / 4.7).
 template <typename T>
-__device__ __forceinline__ void gn_tokens_store(const T *lds, T *y, uint32_t unit, uint32_t pos0, uint32_t rows, float mean,
-                                                float rstd, const float *gamma, const float *beta, const GnTokUnitParams &q) {
-    constexpr int N = 4 / (int)sizeof(T);  // channels per store
-    const uint32_t row0 = fast_div(threadIdx.x, q.row_dwords), c0 = (threadIdx.x - row0 * q.row_dwords.d) * N;
-    if (row0 >= q.row_step) return;
-    const uint32_t sample = fast_div(unit, q.groups);
-    const uint32_t ch0 = (unit - sample * q.groups.d) * q.ch_per_group + c0;
-    float a[N], b[N];
+struct GnTokStore {
+    static constexpr int N = 4 / (int)sizeof(T);  // channels per store
+    uint32_t row0, c0, ch0, sample;
+    float g[N], b[N];
+
+    __device__ __forceinline__ GnTokStore(uint32_t unit, const float *gamma, const float *beta, const GnTokUnitParams &q) {
+        row0 = fast_div(threadIdx.x, q.row_dwords);
+        c0 = (threadIdx.x - row0 * q.row_dwords.d) * N;
+        sample = fast_div(unit, q.groups);
+        ch0 = (unit - sample * q.groups.d) * q.ch_per_group + c0;
 #pragma unroll
-    for (int i = 0; i < N; i++) {
-        a[i] = rstd * gamma[ch0 + i];
-        b[i] = beta[ch0 + i];
-    }
-    T *out = y + ((size_t)sample * q.hw + pos0) * q.channels + ch0;
-    const T *in = lds + c0 * q.pitch;
-#pragma unroll 4
-    for (uint32_t r = row0; r < rows; r += q.row_step) {
-        float f[N];
-#pragma unroll
-        for (int i = 0; i < N; i++) f[i] = fmaf(Store<T>::load1(in + i * q.pitch + r) - mean, a[i], b[i]);
-        uint32_t w;
-        if constexpr (sizeof(T) == 2) {
-            const __half2 h = __floats2half2_rn(f[0], f[N - 1]);
-            w = *reinterpret_cast<const uint32_t *>(&h);
-        } else {
-            w = __float_as_uint(f[0]);
+        for (int i = 0; i < N; i++) {
+            g[i] = gamma[ch0 + i];
+            b[i] = beta[ch0 + i];
         }
-        *reinterpret_cast<uint32_t *>(out + (size_t)r * q.channels) = w;
     }
-}
+
+    __device__ __forceinline__ void operator()(const T *lds, T *y, uint32_t pos0, uint32_t rows, float mean, float rstd,
+                                               const GnTokUnitParams &q) const {
+        if (row0 >= q.row_step) return;
+        float a[N];
+#pragma unroll
+        for (int i = 0; i < N; i++) a[i] = rstd * g[i];
+        T *out = y + ((size_t)sample * q.hw + pos0) * q.channels + ch0;
+        const T *in = lds + c0 * q.pitch;
+#pragma unroll 4
+        for (uint32_t r = row0; r < rows; r += q.row_step) {
+            float f[N];
+#pragma unroll
+            for (int i = 0; i < N; i++) f[i] = fmaf(Store<T>::load1(in + i * q.pitch + r) - mean, a[i], b[i]);
+            uint32_t w;
+            if constexpr (sizeof(T) == 2) {
+                const __half2 h = __floats2half2_rn(f[0], f[N - 1]);
+                w = *reinterpret_cast<const uint32_t *>(&h);
+            } else {
+                w = __float_as_uint(f[0]);
+            }
+            *reinterpret_cast<uint32_t *>(out + (size_t)r * q.channels) = w;
+        }
+    }
+};
 
 template <typename T, int K, bool RAGGED>
 __global__ __launch_bounds__(kGnMaxThreads) void gn_tokens_unit_kernel(
@@ -793,6 +807,9 @@ __global__ __launch_bounds__(kGnMaxThreads) void gn_tokens_unit_kernel(
     u32x4 raw[K];
 #pragma unroll
     for (int k = 0; k < K; k++) raw[k] = load_stream(xin + min(k * nt + tid, nvec - 1));  // ragged tail: the last vector again
+    __builtin_amdgcn_sched_barrier(0);  // (loads return in order: the data does not wait for gamma and beta)
+    const GnTokStore<T> store(unit, gamma, beta, q);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int k = 0; k < K; k++) {
         const uint32_t v = k * nt + tid;
@@ -809,7 +826,7 @@ __global__ __launch_bounds__(kGnMaxThreads) void gn_tokens_unit_kernel(
     float mean, m2;
     gn_slice_stats<T, K, false>(raw, nvec, red, mean, m2);  // (its barrier covers the tile)
     const float rstd = __builtin_amdgcn_rsqf(m2 * q.inv_count + q.eps);
-    gn_tokens_store<T>(RAGGED ? lds + pos0 : lds, y, unit, pos0, rows, mean, rstd, gamma, beta, q);
+    store(RAGGED ? lds + pos0 : lds, y, pos0, rows, mean, rstd, q);
 }
 
 // Any shape: one workgroup per unit, three passes, element-wise scattered stores.
