@@ -10,10 +10,10 @@
 //      over the packed registers (DPP wavefront reduction, one LDS slot per wavefront), with
 //      a second, centred pass when the mean is large against the spread;
 //   3. split > 1: slices publish (mean, M2) as two tagged 64-bit words, poll
-//      their siblings' words, and merge with Chan's formula.  The tag is the
-//      unit's launch count, read at kernel start; the last slice to finish
-//      advances it, so nothing is reset between launches and a replayed graph
-//      works.  All traffic is relaxed agent-scope atomics: no cache flushes.
+//      their siblings' words, and merge with Chan's formula.  The tag is one
+//      more than that of the slice's own word, read at kernel start, so nothing
+//      is reset between launches and a replayed graph works.  All traffic is
+//      relaxed agent-scope atomics: no cache flushes.
 //   4. y = fma(x - mean, rstd * gamma[c], beta[c]) (the mean folded into the offset when it
 //      is small), optional SiLU, packed store.
 //
@@ -81,22 +81,28 @@ __device__ __forceinline__ unsigned long long tagged(uint32_t tag, float v) {
     return ((unsigned long long)tag << 32) | (unsigned long long)__float_as_uint(v);
 }
 
+// The tag of the last launch on this unit: its own first word, which only this slice writes in this launch.
+__device__ __forceinline__ uint32_t gn_exchange_last_tag(const GnScratch &scratch, uint32_t unit, uint32_t slice) {
+    return (uint32_t)(__hip_atomic_load(scratch.slot_mean + (size_t)unit * kGnMaxSplit + slice, __ATOMIC_RELAXED,
+                                        __HIP_MEMORY_SCOPE_AGENT) >> 32);
+}
+
 // Merges the slices of one unit.  Called by every lane of the workgroup with the slice's
-// (mean, M2); `epoch` is the unit's launch count as lane 0 read it at kernel start.  On return
+// (mean, M2); `last_tag` is what lane 0 read with gn_exchange_last_tag at kernel start.  On return
 // stats[0] = mean and stats[1] = 1/sqrt(var + eps) of the whole unit, in LDS, after a barrier.
 // Slice l covers vectors [l * vec_per_slice, min(vec_per_unit, (l + 1) * vec_per_slice)).
 // `read(l, i)` returns vector i of slice l as the statistics see it (after the optional addend);
 // it is only used when slice l has not published within the poll limit.
 template <typename T, typename Reader>
 __device__ __forceinline__ void gn_exchange(const GnScratch &scratch, const GnParams &p, uint32_t unit,
-                                            uint32_t slice, uint32_t epoch, float slice_mean,
+                                            uint32_t slice, uint32_t last_tag, float slice_mean,
                                             float slice_m2, float *stats, Reader read) {
     constexpr int EPV = Store<T>::EPV;
     const uint32_t tid = threadIdx.x;
     unsigned long long *slot_mean = scratch.slot_mean + (size_t)unit * kGnMaxSplit;
     unsigned long long *slot_m2 = scratch.slot_m2 + (size_t)unit * kGnMaxSplit;
-    if (tid < kWave) {  // wavefront 0 owns the exchange; lane 0 holds the epoch
-        const uint32_t tag = (uint32_t)__builtin_amdgcn_readfirstlane((int)epoch) + 1u;
+    if (tid < kWave) {  // wavefront 0 owns the exchange; lane 0 holds the last tag
+        const uint32_t tag = (uint32_t)__builtin_amdgcn_readfirstlane((int)last_tag) + 1u;
         if (tid == 0) {
             __hip_atomic_store(slot_mean + slice, tagged(tag, slice_mean), __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_AGENT);
@@ -184,22 +190,18 @@ __device__ __forceinline__ void gn_exchange(const GnScratch &scratch, const GnPa
     __syncthreads();
 }
 
-// This slice has consumed its siblings' words: it counts itself done.  Called by lane 0 of the
-// workgroup after the barrier that ends gn_exchange, so that no wavefront waits for the
-// counter's old value, which comes back a memory round trip later; gn_exchange_close uses it
-// at the end of the kernel.
-__device__ __forceinline__ uint32_t gn_exchange_arrive(const GnScratch &scratch, uint32_t unit) {
-    return __hip_atomic_fetch_add(scratch.done + unit, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// The last slice to arrive closes the launch: the counter goes back to zero and the unit's
-// launch count advances (both visible to the next launch, which starts after this kernel).
-__device__ __forceinline__ void gn_exchange_close(const GnScratch &scratch, const GnParams &p, uint32_t unit,
-                                                  uint32_t epoch, uint32_t arrived_before) {
-    if (arrived_before == p.split - 1) {
-        __hip_atomic_store(scratch.done + unit, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(scratch.epoch + unit, epoch + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+// Behind the barrier that ends gn_exchange, by wavefront 0: the first words that no slice of this launch uses get its tag
+// too, slot l from slice l % split, so that all slots of a unit carry the same one between launches, whatever the next
+// launch's split.  Nothing waits for these stores.  (A launch count per unit that the last slice advances, found with an
+// atomic counter, ended the kernel a memory round trip later.  us per launch, so and with the tags, in place, four slices: fp16
+// 320 channels at 64 x 64 batch 2 5.76 -> 5.20, with the addend 5.97 -> 5.62, fp32 batch 1 5.58 -> 5.24.)
+__device__ __forceinline__ void gn_exchange_advance(const GnScratch &scratch, const GnParams &p, uint32_t unit, uint32_t slice,
+                                                    uint32_t last_tag) {
+    const uint32_t tag = (uint32_t)__builtin_amdgcn_readfirstlane((int)last_tag) + 1u;
+    const uint32_t l = slice + (threadIdx.x + 1) * p.split;
+    if (l < kGnMaxSplit)
+        __hip_atomic_store(scratch.slot_mean + (size_t)unit * kGnMaxSplit + l, tagged(tag, 0.0f), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Sum and sum of squares of a packed vector, accumulated in float32.  Half storage uses
@@ -338,10 +340,8 @@ __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
     const u32x4 *xin = reinterpret_cast<const u32x4 *>(x) + (size_t)unit * p.vec_per_unit;
     u32x4 *yout = reinterpret_cast<u32x4 *>(y) + (size_t)unit * p.vec_per_unit;
 
-    // launch count of this unit: the tag of this launch's exchange (latency hidden by the loads)
-    uint32_t epoch = 0;
-    if (!SHARED && p.split > 1 && tid == 0)
-        epoch = __hip_atomic_load(scratch.epoch + unit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    uint32_t last_tag = 0;  // (its latency is hidden by the loads)
+    if (!SHARED && p.split > 1 && tid == 0) last_tag = gn_exchange_last_tag(scratch, unit, slice);
 
     // ---- the slice goes into registers.  Lanes past the end of a ragged slice re-read its
     // last vector (a valid address) and are masked later: no load sits behind a branch.
@@ -428,7 +428,6 @@ __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
     gn_slice_stats<T, K, FULL>(raw, v_end - v_begin, red, slice_mean, slice_m2);
 
     float mean, rstd;
-    uint32_t arrived_before = 0;
     if (SHARED || p.split == 1) {
         mean = slice_mean;
         rstd = __builtin_amdgcn_rsqf(slice_m2 * p.inv_count + p.eps);
@@ -442,10 +441,10 @@ __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
             }
             return r;
         };
-        gn_exchange<T>(scratch, p, unit, slice, epoch, slice_mean, slice_m2, stats, read);
+        gn_exchange<T>(scratch, p, unit, slice, last_tag, slice_mean, slice_m2, stats, read);
         mean = stats[0];
         rstd = stats[1];
-        if (tid == 0) arrived_before = gn_exchange_arrive(scratch, unit);
+        if (tid < kWave) gn_exchange_advance(scratch, p, unit, slice, last_tag);
     }
 
     // ---- normalise from registers, per-channel affine, optional SiLU.  When the unit's mean is
@@ -523,7 +522,6 @@ __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
         epilogue(std::true_type{});
     else
         epilogue(std::false_type{});
-    if (!SHARED && p.split > 1 && tid == 0) gn_exchange_close(scratch, p, unit, epoch, arrived_before);
 }
 
 // Up to five vectors per lane (four for float storage) the kernel fits 64 registers: eight
@@ -639,9 +637,8 @@ __global__ __launch_bounds__(kGnMaxThreads) void gn_tokens_kernel(
     const uint32_t pvs = q.pos_vecs.d;
     const u32x4 *xin = reinterpret_cast<const u32x4 *>(x) + (size_t)unit * p.vec_per_unit;
 
-    uint32_t epoch = 0;
-    if (p.split > 1 && tid == 0)
-        epoch = __hip_atomic_load(scratch.epoch + unit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    uint32_t last_tag = 0;
+    if (p.split > 1 && tid == 0) last_tag = gn_exchange_last_tag(scratch, unit, slice);
 
     // lane-local vector -> (channel of the group, position vector of the slice)
     u32x4 raw[K];
@@ -671,9 +668,10 @@ __global__ __launch_bounds__(kGnMaxThreads) void gn_tokens_kernel(
             const uint32_t c = fast_div(i, q.pos_vecs);
             return xin[(size_t)c * p.hw_vec.d + l * pvs + (i - c * pvs)];
         };
-        gn_exchange<T>(scratch, p, unit, slice, epoch, slice_mean, slice_m2, stats, read);
+        gn_exchange<T>(scratch, p, unit, slice, last_tag, slice_mean, slice_m2, stats, read);
         mean = stats[0];
         rstd = stats[1];
+        if (tid < kWave) gn_exchange_advance(scratch, p, unit, slice, last_tag);
     }
 
     // ---- normalise into LDS as [channel][position]
@@ -691,9 +689,6 @@ __global__ __launch_bounds__(kGnMaxThreads) void gn_tokens_kernel(
         }
     }
     __syncthreads();
-    // the slice counts itself done here, behind the last barrier: nothing waits for the answer
-    uint32_t arrived_before = 0;
-    if (p.split > 1 && tid == 0) arrived_before = gn_exchange_arrive(scratch, unit);
 
     // ---- token-major store: for each position of the slice one run of ch_per_group values
     const uint32_t rows = pvs * EPV;                         // positions in the slice
@@ -714,7 +709,6 @@ __global__ __launch_bounds__(kGnMaxThreads) void gn_tokens_kernel(
         }
         out[(size_t)r * row_stride + c] = w;
     }
-    if (p.split > 1 && tid == 0) gn_exchange_close(scratch, p, unit, epoch, arrived_before);
 }
 
 // The token-major norm for units that stay whole: `writers` workgroups (one or several) per unit, each of which loads

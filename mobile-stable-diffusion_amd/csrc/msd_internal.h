@@ -58,10 +58,8 @@ constexpr int kGnPrefetchAffineK = 6;   // vectors per lane up to which gamma / 
 constexpr uint32_t kGnLdsChannels = 1024;  // channels per group the LDS copy of gamma / beta has room for
 
 struct GnScratch {
-    unsigned long long *slot_mean;  // [kGnMaxUnits][kGnMaxSplit]  (tag << 32) | float bits
+    unsigned long long *slot_mean;  // [kGnMaxUnits][kGnMaxSplit]  (tag << 32) | float bits; one tag per unit between launches
     unsigned long long *slot_m2;    // [kGnMaxUnits][kGnMaxSplit]
-    uint32_t *epoch;                // [kGnMaxUnits] launches completed on this unit
-    uint32_t *done;                 // [kGnMaxUnits] slices finished in the running launch
     uint32_t *fallbacks;            // [1] slices that stopped waiting and computed a sibling's statistics themselves
     float2 *partials;               // [kGnMaxUnits][kGnStatSlices] (mean, M2) for one pair of launches; null in the fixed scratch
     uint32_t units;                 // units the arrays above have room for

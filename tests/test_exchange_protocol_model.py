@@ -1,7 +1,9 @@
 """CPU model of the exchange between the workgroups ("slices") that share one GroupNorm unit
 (csrc/groupnorm.hip: gn_exchange), run over randomised interleavings.
 
-What the kernel does per slice, and what the model replays one memory operation at a time:
+What a slice does, and what the model replays one memory operation at a time (steps 1 and 6 with a launch count per unit and a
+counter of finished slices; the kernels have neither since the tags are kept in the slots themselves, which
+test_exchange_tags_model.py replays on top of this model):
 
   1. read the unit's launch count `epoch` (once, at kernel start); tag = epoch + 1
   2. publish (tag, mean) and (tag, M2) of its own part as two separate 64-bit words
