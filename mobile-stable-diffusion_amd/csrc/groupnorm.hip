@@ -46,24 +46,37 @@ constexpr int kGnRedRow = 16;                // partial sums of a workgroup, one
 constexpr int kGnRedSlots = 3 * kGnRedRow;   // sums, sums of squares, sums about the mean
 static_assert(kGnMaxThreads / kWave <= kGnRedRow, "a row of lanes holds the wavefronts' partial sums");
 
+// (No field that no kernel reads: what is loaded with its neighbours and not used costs a wait, for its register.)
 struct GnParams {
     uint32_t vec_per_unit;   // 16-byte vectors per unit
     uint32_t vec_per_slice;  // vectors per workgroup (the last slice may be shorter)
     uint32_t split;          // workgroups per unit, power of two <= kGnMaxSplit
-    uint32_t split_shift;    // log2(split)
+    uint32_t spin_limit;     // polls before a slice stops waiting for a sibling's words
     FastDiv groups;          // per sample
     uint32_t ch_per_group;
     FastDiv hw_vec;          // vectors per channel (RAGGED: elements per channel)
     float eps;
     float inv_count;         // 1 / elements per unit
-    uint32_t spin_limit;     // polls before a slice stops waiting for a sibling's words
-    // gn_slice_kernel<..., SHARED>: `writers` workgroups per whole unit; each loads and reduces the
+    // gn_slice_kernel<..., SHARED>: several workgroups per whole unit; each loads and reduces the
     // whole unit and normalises and stores one part of it
-    uint32_t writers;        // power of two
-    uint32_t writers_shift;  // log2(writers)
     uint32_t part_vecs;      // vectors per part, a multiple of 64 (a wavefront is inside one part or outside)
-    uint32_t xcd_shift;      // the writers of a unit have block ids (1 << xcd_shift) apart: with that many XCDs they
-                             // share one XCD and its L2 (units in whole rows of that many); 0: adjacent ids
+};
+
+// The arguments that a wavefront needs before it can ask for its data are the kernels' first ones, plain values that arrive
+// in scalar registers (build.py); the rest, loaded from memory, is needed when the data is on its way.  One word holds the
+// logarithms of the launch's shape and its lanes.  us, structures and so: recorded steps of 512 x 512 fp16 batch 2 752 -> 739, fp32
+// batch 1 762 -> 750; per launch, fp16 batch 2, in place, 640 channels at 32 x 32 4.55 -> 4.45, 1280 at 16 x 16 3.37 -> 3.22, token
+// norm of those 3.29 -> 3.02 (an argument from memory in a step: 620 cycles).
+// xcd_shift: the writers of a unit have block ids (1 << xcd_shift) apart: with that many XCDs they share one XCD and its L2
+// (units in whole rows of that many); 0: adjacent ids.
+inline uint32_t gn_shape_word(uint32_t split_shift, uint32_t writers_shift, uint32_t xcd_shift,
+                                                  uint32_t threads) {
+    return split_shift | writers_shift << 4 | xcd_shift << 8 | threads << 16;
+}
+struct GnShape {
+    uint32_t split_shift, writers_shift, xcd_shift, threads;
+    __device__ __forceinline__ explicit GnShape(uint32_t word)
+        : split_shift(word & 15u), writers_shift(word >> 4 & 15u), xcd_shift(word >> 8 & 255u), threads(word >> 16) {}
 };
 
 // Sum over the workgroup (blockDim.x / 64 wavefronts); one barrier.
@@ -83,8 +96,8 @@ __device__ __forceinline__ unsigned long long tagged(uint32_t tag, float v) {
 
 // The tag of the last launch on this unit: its own first word, which only this slice writes in this launch.
 __device__ __forceinline__ uint32_t gn_exchange_last_tag(const GnScratch &scratch, uint32_t unit, uint32_t slice) {
-    return (uint32_t)(__hip_atomic_load(scratch.slot_mean + (size_t)unit * kGnMaxSplit + slice, __ATOMIC_RELAXED,
-                                        __HIP_MEMORY_SCOPE_AGENT) >> 32);
+    const unsigned long long *own = scratch.slot_mean + (size_t)unit * kGnMaxSplit + slice;
+    return __hip_atomic_load(reinterpret_cast<const uint32_t *>(own) + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Merges the slices of one unit.  Called by every lane of the workgroup with the slice's
@@ -243,7 +256,7 @@ constexpr float kGnFastMoments = 4.0f;
 constexpr float kGnFoldMean = 16.0f;
 
 // Mean and M2 = sum (x - mean)^2 of the workgroup's slice, held as K packed vectors per lane
-// (vector k of lane t is element k * blockDim.x + t of the slice; the first n_valid count, the
+// (vector k of lane t is element k * nt + t of the slice, nt the workgroup's lanes; the first n_valid count, the
 // registers of the others hold zeros).  One pass gives sum and sum of squares (wavefront
 // reduction by DPP, the wavefronts' partial sums meet once in LDS, every wavefront adds them
 // in the same order).  M2 = sum x^2 - n mean^2 is kept when it is well conditioned; when the
@@ -257,11 +270,10 @@ constexpr float kGnFoldMean = 16.0f;
 // batch 2, six LDS swizzles one after the other and a division, and so: fp16 320 channels at 64 x 64 5.19 -> 4.94, in place 5.93 ->
 // 5.76, 640 at 32 x 32 3.92 -> 3.74, in place 4.76 -> 4.59, 1280 at 8 x 8 2.65 -> 2.50; fp32 640 at 32 x 32 in place 5.58 -> 5.29.
 template <typename T, int K, bool FULL>
-__device__ __forceinline__ void gn_slice_stats(u32x4 (&raw)[K], uint32_t n_valid, float *red, float &slice_mean,
-                                               float &slice_m2) {
+__device__ __forceinline__ void gn_slice_stats(u32x4 (&raw)[K], uint32_t n_valid, uint32_t nt, float *red,
+                                               float &slice_mean, float &slice_m2) {
     constexpr int EPV = Store<T>::EPV;
     const uint32_t tid = threadIdx.x;
-    const uint32_t nt = blockDim.x;
     const uint32_t lane = tid & (kWave - 1);
     const uint32_t nw = nt / kWave;
     const float count = (float)(n_valid * EPV);
@@ -331,17 +343,13 @@ template <typename T, int K, bool SILU, bool FULL, bool SHARED, bool RAGGED>
 __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
                                         const float *__restrict__ gamma,
                                         const float *__restrict__ beta, const GnScratch &scratch,
-                                        const GnParams &p, uint32_t unit, uint32_t slice, uint32_t part,
-                                        uint32_t v_begin, uint32_t v_end, float *red, float *stats,
+                                        const GnParams &p, uint32_t nt, uint32_t vec_per_unit, uint32_t unit, uint32_t slice,
+                                        uint32_t part, uint32_t v_begin, uint32_t v_end, float *red, float *stats,
                                         float2 *aff) {
     constexpr int EPV = Store<T>::EPV;
     const uint32_t tid = threadIdx.x;
-    const uint32_t nt = blockDim.x;
-    const u32x4 *xin = reinterpret_cast<const u32x4 *>(x) + (size_t)unit * p.vec_per_unit;
-    u32x4 *yout = reinterpret_cast<u32x4 *>(y) + (size_t)unit * p.vec_per_unit;
-
-    uint32_t last_tag = 0;  // (its latency is hidden by the loads)
-    if (!SHARED && p.split > 1 && tid == 0) last_tag = gn_exchange_last_tag(scratch, unit, slice);
+    const u32x4 *xin = reinterpret_cast<const u32x4 *>(x) + (size_t)unit * vec_per_unit;
+    u32x4 *yout = reinterpret_cast<u32x4 *>(y) + (size_t)unit * vec_per_unit;
 
     // ---- the slice goes into registers.  Lanes past the end of a ragged slice re-read its
     // last vector (a valid address) and are masked later: no load sits behind a branch.
@@ -369,6 +377,12 @@ __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
     };
 #pragma unroll
     for (int k = 0; k < K; k++) raw[k] = load_stream(at(xin, k, tid));
+    // What follows waits for the arguments in memory: the compiler neither moves it up nor, as new values to it, shares it
+    // with another branch in front of the loads.
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" : "+s"(unit), "+s"(part));
+    uint32_t last_tag = 0;  // (arrives right behind the data)
+    if (!SHARED && p.split > 1 && tid == 0) last_tag = gn_exchange_last_tag(scratch, unit, slice);
     const uint32_t ch0 = (unit - fast_div(unit, p.groups) * p.groups.d) * p.ch_per_group;
     // the addends of the unit's channels
     auto unit_chunk = [&]() { return chunk + (size_t)unit * p.ch_per_group; };
@@ -425,7 +439,7 @@ __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
     }
 
     float slice_mean, slice_m2;
-    gn_slice_stats<T, K, FULL>(raw, v_end - v_begin, red, slice_mean, slice_m2);
+    gn_slice_stats<T, K, FULL>(raw, v_end - v_begin, nt, red, slice_mean, slice_m2);
 
     float mean, rstd;
     if (SHARED || p.split == 1) {
@@ -529,31 +543,32 @@ __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
 // computes (what large batches need).
 template <typename T, int K, bool SILU, bool SHARED, bool RAGGED>
 __global__ __launch_bounds__(kGnMaxThreads, (K <= (sizeof(T) == 2 ? 5 : 4) ? 8 : 4)) void gn_slice_kernel(
-    const T *x, const T *chunk, T *y, const float *__restrict__ gamma,
-    const float *__restrict__ beta, GnScratch scratch, GnParams p) {
+    const T *x, uint32_t vec_per_unit, uint32_t vec_per_slice, uint32_t shape, const T *chunk, T *y,
+    const float *__restrict__ gamma, const float *__restrict__ beta, GnScratch scratch, GnParams p) {
     __shared__ float red[kGnRedSlots];
     __shared__ float stats[2];
     __shared__ float2 aff[!RAGGED && K <= kGnPrefetchAffineK ? 1 : kGnLdsChannels];  // (gamma, beta) of the group's channels
+    const GnShape of(shape);
     uint32_t unit, slice, part;
     if (SHARED) {  // whole units, `writers` workgroups each
-        const uint32_t j = blockIdx.x >> p.xcd_shift;
-        part = j & (p.writers - 1);
-        unit = ((j >> p.writers_shift) << p.xcd_shift) + (blockIdx.x & ((1u << p.xcd_shift) - 1u));
+        const uint32_t j = blockIdx.x >> of.xcd_shift;
+        part = j & ((1u << of.writers_shift) - 1u);
+        unit = ((j >> of.writers_shift) << of.xcd_shift) + (blockIdx.x & ((1u << of.xcd_shift) - 1u));
         slice = 0;
     } else {
-        unit = blockIdx.x >> p.split_shift;
-        slice = blockIdx.x & (p.split - 1);
+        unit = blockIdx.x >> of.split_shift;
+        slice = blockIdx.x & ((1u << of.split_shift) - 1u);
         part = 0;
     }
-    const uint32_t v_begin = slice * p.vec_per_slice;
-    const uint32_t v_end = min(p.vec_per_unit, v_begin + p.vec_per_slice);
+    const uint32_t v_begin = slice * vec_per_slice;
+    const uint32_t v_end = min(vec_per_unit, v_begin + vec_per_slice);
     // uniform over the workgroup; the largest K is only launched on slices it fits exactly
-    if (K == kGnMaxK || v_end - v_begin == K * blockDim.x)
-        gn_body<T, K, SILU, true, SHARED, RAGGED>(x, chunk, y, gamma, beta, scratch, p, unit, slice, part, v_begin, v_end,
-                                          red, stats, aff);
+    if (K == kGnMaxK || v_end - v_begin == K * of.threads)
+        gn_body<T, K, SILU, true, SHARED, RAGGED>(x, chunk, y, gamma, beta, scratch, p, of.threads, vec_per_unit, unit, slice, part,
+                                          v_begin, v_end, red, stats, aff);
     else
-        gn_body<T, K, SILU, false, SHARED, RAGGED>(x, chunk, y, gamma, beta, scratch, p, unit, slice, part, v_begin, v_end,
-                                           red, stats, aff);
+        gn_body<T, K, SILU, false, SHARED, RAGGED>(x, chunk, y, gamma, beta, scratch, p, of.threads, vec_per_unit, unit, slice, part,
+                                           v_begin, v_end, red, stats, aff);
 }
 
 // Any shape or alignment (units that are no whole number of vectors, channels of less than a vector, many
@@ -603,42 +618,38 @@ __global__ __launch_bounds__(kGenericThreads) void gn_generic_kernel(
 // runs.  Statistics and the exchange between slices are those of gn_slice_kernel.
 // ---------------------------------------------------------------------------
 struct GnTokParams {
-    GnParams base;        // vec_per_slice = ch_per_group * pos_vecs.d ; vec_per_unit = that * split
-    FastDiv pos_vecs;     // position vectors per slice (hw_vec / split)
+    GnParams base;        // vec_per_slice = ch_per_group * position vectors per slice; vec_per_unit = that * split
     FastDiv row_dwords;   // 4-byte words per output run: ch_per_group * sizeof(T) / 4
     uint32_t hw;          // positions per sample
     uint32_t channels;
     uint32_t pitch;       // LDS elements between channels: positions per slice + 16 bytes
-    FastDiv combos;       // batch * split: (sample, slice) pairs, the fastest part of the block id
 };
 
 template <typename T, int K>
 __global__ __launch_bounds__(kGnMaxThreads) void gn_tokens_kernel(
-    const T *__restrict__ x, T *__restrict__ y, const float *__restrict__ gamma,
-    const float *__restrict__ beta, GnScratch scratch, GnTokParams q) {
+    const T *__restrict__ x, uint32_t vec_per_unit, uint32_t nvec, uint32_t pos_mul, uint32_t pos_shift, uint32_t pvs,
+    uint32_t hw_vec, uint32_t combos_mul, uint32_t combos_shift, uint32_t combos, uint32_t groups, uint32_t shape,
+    T *__restrict__ y, const float *__restrict__ gamma, const float *__restrict__ beta, GnScratch scratch, GnTokParams q) {
     constexpr int EPV = Store<T>::EPV;
     extern __shared__ u32x4 lds_vec[];
     __shared__ float red[kGnRedSlots];
     __shared__ float stats[2];
     const GnParams &p = q.base;
+    const GnShape of(shape);
+    const FastDiv pos_vecs{pos_mul, pos_shift, pvs};
     const uint32_t tid = threadIdx.x;
-    const uint32_t nt = blockDim.x;
+    const uint32_t nt = of.threads;
     // block id = group * (batch * split) + sample * split + slice: the workgroups that write
     // pieces of the same output lines (all groups of one sample and position range) have ids
     // that differ by multiples of batch * split, so with workgroups dealt round-robin to the
     // 8 XCDs they meet in one L2 when that product is a multiple of 8 (batch 2 x 4 slices);
     // the slices of a unit stay adjacent
-    const uint32_t group = fast_div(blockIdx.x, q.combos);
-    const uint32_t combo = blockIdx.x - group * q.combos.d;
-    const uint32_t sample = combo >> p.split_shift;
-    const uint32_t unit = sample * p.groups.d + group;
-    const uint32_t slice = combo & (p.split - 1);
-    const uint32_t nvec = p.vec_per_slice;
-    const uint32_t pvs = q.pos_vecs.d;
-    const u32x4 *xin = reinterpret_cast<const u32x4 *>(x) + (size_t)unit * p.vec_per_unit;
-
-    uint32_t last_tag = 0;
-    if (p.split > 1 && tid == 0) last_tag = gn_exchange_last_tag(scratch, unit, slice);
+    const uint32_t group = fast_div(blockIdx.x, FastDiv{combos_mul, combos_shift, combos});
+    const uint32_t combo = blockIdx.x - group * combos;
+    const uint32_t sample = combo >> of.split_shift;
+    const uint32_t unit = sample * groups + group;
+    const uint32_t slice = combo & ((1u << of.split_shift) - 1u);
+    const u32x4 *xin = reinterpret_cast<const u32x4 *>(x) + (size_t)unit * vec_per_unit;
 
     // lane-local vector -> (channel of the group, position vector of the slice)
     u32x4 raw[K];
@@ -646,17 +657,20 @@ __global__ __launch_bounds__(kGnMaxThreads) void gn_tokens_kernel(
 #pragma unroll
     for (int k = 0; k < K; k++) {
         const uint32_t vl = min(k * nt + tid, nvec - 1);  // ragged tail re-reads the last vector
-        cl[k] = fast_div(vl, q.pos_vecs);
+        cl[k] = fast_div(vl, pos_vecs);
         pv[k] = vl - cl[k] * pvs;
-        raw[k] = load_stream(xin + (size_t)cl[k] * p.hw_vec.d + slice * pvs + pv[k]);
+        raw[k] = load_stream(xin + (size_t)cl[k] * hw_vec + slice * pvs + pv[k]);
         const bool have = k * nt + tid < nvec;  // lanes past the end hold zeros (the statistics rely on it)
 #pragma unroll
         for (int i = 0; i < 4; i++) raw[k][i] = have ? raw[k][i] : 0u;
     }
+    __builtin_amdgcn_sched_barrier(0);  // (what follows waits for the arguments in memory)
+    uint32_t last_tag = 0;
+    if (p.split > 1 && tid == 0) last_tag = gn_exchange_last_tag(scratch, unit, slice);
     const uint32_t ch0 = group * p.ch_per_group;
 
     float slice_mean, slice_m2;
-    gn_slice_stats<T, K, false>(raw, nvec, red, slice_mean, slice_m2);
+    gn_slice_stats<T, K, false>(raw, nvec, nt, red, slice_mean, slice_m2);
 
     float mean, rstd;
     if (p.split == 1) {
@@ -665,8 +679,8 @@ __global__ __launch_bounds__(kGnMaxThreads) void gn_tokens_kernel(
     } else {
         // vector i of slice l: channel i / pos_vecs of the group, position vector i % pos_vecs
         auto read = [&](uint32_t l, uint32_t i) {
-            const uint32_t c = fast_div(i, q.pos_vecs);
-            return xin[(size_t)c * p.hw_vec.d + l * pvs + (i - c * pvs)];
+            const uint32_t c = fast_div(i, pos_vecs);
+            return xin[(size_t)c * hw_vec + l * pvs + (i - c * pvs)];
         };
         gn_exchange<T>(scratch, p, unit, slice, last_tag, slice_mean, slice_m2, stats, read);
         mean = stats[0];
@@ -722,11 +736,8 @@ __global__ __launch_bounds__(kGnMaxThreads) void gn_tokens_kernel(
 // RAGGED: hw is no whole number of vectors, a vector may cross from one channel into the next; LDS then holds the whole unit
 // as it lies in memory.
 struct GnTokUnitParams {
-    uint32_t vec_per_unit;
     FastDiv groups;          // per sample
     uint32_t ch_per_group, channels, hw;
-    uint32_t writers, writers_shift, xcd_shift;
-    uint32_t units_per_xcd;  // units >> xcd_shift
     uint32_t part_pos;       // positions of a part; of the last one what is left
     uint32_t pitch;          // LDS elements between channels
     uint32_t row_step;       // positions that the workgroup stores at a time
@@ -785,23 +796,23 @@ struct GnTokStore {
 
 template <typename T, int K, bool RAGGED>
 __global__ __launch_bounds__(kGnMaxThreads) void gn_tokens_unit_kernel(
-    const T *__restrict__ x, T *__restrict__ y, const float *__restrict__ gamma, const float *__restrict__ beta,
-    GnTokUnitParams q) {
+    const T *__restrict__ x, uint32_t nvec, uint32_t units_per_xcd, uint32_t shape, T *__restrict__ y,
+    const float *__restrict__ gamma, const float *__restrict__ beta, GnTokUnitParams q) {
     constexpr int EPV = Store<T>::EPV;
     extern __shared__ u32x4 lds_vec[];
     __shared__ float red[kGnRedSlots];
-    const uint32_t tid = threadIdx.x, nt = blockDim.x;
-    const uint32_t of_xcd = blockIdx.x >> q.xcd_shift;
-    const uint32_t part = of_xcd & (q.writers - 1);
-    const uint32_t unit = (blockIdx.x & ((1u << q.xcd_shift) - 1u)) * q.units_per_xcd + (of_xcd >> q.writers_shift);
-    const uint32_t nvec = q.vec_per_unit;
-    const uint32_t pos0 = part * q.part_pos, rows = min(q.part_pos, q.hw - pos0);
+    const GnShape of(shape);
+    const uint32_t tid = threadIdx.x, nt = of.threads;
+    const uint32_t of_xcd = blockIdx.x >> of.xcd_shift;
+    const uint32_t part = of_xcd & ((1u << of.writers_shift) - 1u);
+    const uint32_t unit = (blockIdx.x & ((1u << of.xcd_shift) - 1u)) * units_per_xcd + (of_xcd >> of.writers_shift);
     const u32x4 *xin = reinterpret_cast<const u32x4 *>(x) + (size_t)unit * nvec;
     T *lds = reinterpret_cast<T *>(lds_vec);
     u32x4 raw[K];
 #pragma unroll
     for (int k = 0; k < K; k++) raw[k] = load_stream(xin + min(k * nt + tid, nvec - 1));  // ragged tail: the last vector again
     __builtin_amdgcn_sched_barrier(0);  // (loads return in order: the data does not wait for gamma and beta)
+    const uint32_t pos0 = part * q.part_pos, rows = min(q.part_pos, q.hw - pos0);
     const GnTokStore<T> store(unit, gamma, beta, q);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -818,7 +829,7 @@ __global__ __launch_bounds__(kGnMaxThreads) void gn_tokens_unit_kernel(
         for (int i = 0; i < 4; i++) raw[k][i] = have ? raw[k][i] : 0u;  // (the statistics rely on it)
     }
     float mean, m2;
-    gn_slice_stats<T, K, false>(raw, nvec, red, mean, m2);  // (its barrier covers the tile)
+    gn_slice_stats<T, K, false>(raw, nvec, nt, red, mean, m2);  // (its barrier covers the tile)
     const float rstd = __builtin_amdgcn_rsqf(m2 * q.inv_count + q.eps);
     store(RAGGED ? lds + pos0 : lds, y, pos0, rows, mean, rstd, q);
 }
@@ -862,25 +873,21 @@ __global__ __launch_bounds__(kGenericThreads) void gn_tokens_generic_kernel(
 constexpr int kStatsThreads = 256;
 constexpr int kStatsUnroll = 4;  // vectors per lane in flight
 
-struct GnStatsParams {
-    uint32_t vec_per_unit;
-    uint32_t vec_per_slice;
-    FastDiv slices;  // per unit, at most kGnStatSlices
-};
-
 // (mean, M2) of one slice per workgroup.  Bound by the read of x.  Plain loads: the next launch wants
 // the lines in the caches.
 template <typename T>
-__global__ __launch_bounds__(kStatsThreads) void gn_stats_kernel(const T *__restrict__ x, float2 *__restrict__ partials,
-                                                                 GnStatsParams p) {
+__global__ __launch_bounds__(kStatsThreads) void gn_stats_kernel(const T *__restrict__ x, uint32_t vec_per_unit,
+                                                                 uint32_t vec_per_slice, uint32_t slices_mul,
+                                                                 uint32_t slices_shift, uint32_t slices,
+                                                                 float2 *__restrict__ partials) {
     constexpr int EPV = Store<T>::EPV;
     __shared__ float2 red[kStatsThreads / kWave];
     __shared__ float red_c[kStatsThreads / kWave];
-    const uint32_t unit = fast_div(blockIdx.x, p.slices);
-    const uint32_t slice = blockIdx.x - unit * p.slices.d;
-    const uint32_t begin = slice * p.vec_per_slice;
-    const uint32_t n = min(p.vec_per_unit, begin + p.vec_per_slice) - begin;
-    const u32x4 *in = reinterpret_cast<const u32x4 *>(x) + (size_t)unit * p.vec_per_unit + begin;
+    const uint32_t unit = fast_div(blockIdx.x, FastDiv{slices_mul, slices_shift, slices});
+    const uint32_t slice = blockIdx.x - unit * slices;
+    const uint32_t begin = slice * vec_per_slice;
+    const uint32_t n = min(vec_per_unit, begin + vec_per_slice) - begin;
+    const u32x4 *in = reinterpret_cast<const u32x4 *>(x) + (size_t)unit * vec_per_unit + begin;
     // every vector of the slice that is this lane's, kStatsUnroll requested at a time; what lies past
     // the end re-reads the last vector and counts as `past`
     auto for_each = [&](const u32x4 &past, auto use) {
@@ -928,40 +935,41 @@ __global__ __launch_bounds__(kStatsThreads) void gn_stats_kernel(const T *__rest
     if (threadIdx.x == 0) partials[(size_t)unit * kGnStatSlices + slice] = make_float2(mean, m2);
 }
 
+// (no field that the kernel does not read: see GnParams)
 struct GnApplyParams {
-    GnStatsParams stats;
-    FastDiv ch_per_group;
-    uint32_t groups, channels, hw;
+    uint32_t vec_per_unit, vec_per_slice, slices;  // of the statistics
+    uint32_t cpg_mul, cpg_shift;                   // division by the channels of a group
+    uint32_t groups;
     float eps, inv_count;
 };
 
 // JFAST, RAGGED: as in permute_021_words_kernel.
 template <typename T, bool JFAST, bool RAGGED>
 __global__ __launch_bounds__(kTileThreads) void gn_tokens_apply_kernel(
-    const T *__restrict__ x, T *__restrict__ y, const float *__restrict__ gamma, const float *__restrict__ beta,
-    const float2 *__restrict__ partials, GnApplyParams p) {
+    const T *__restrict__ x, uint32_t channels, uint32_t hw, const float *__restrict__ gamma, const float *__restrict__ beta,
+    T *__restrict__ y, const float2 *__restrict__ partials, GnApplyParams p) {
     constexpr int ES = (int)sizeof(T), EPV = Store<T>::EPV;
     constexpr uint32_t kTeam = kTileThreads / kTile;  // lanes that merge one channel's statistics
     __shared__ u32x4 tile4[tile_lds_words<ES>()];
     __shared__ float4 affine[kTile];  // (mean, rstd * gamma, beta) of the tile's channels
     const uint32_t k0 = (JFAST ? blockIdx.y : blockIdx.x) * kTile, j0 = (JFAST ? blockIdx.x : blockIdx.y) * kTile;
-    const size_t plane = (size_t)blockIdx.z * p.channels * p.hw;
+    const size_t plane = (size_t)blockIdx.z * channels * hw;
     // Chan's formula over the unit's slices, by the four lanes of a channel
     auto ready = [&]() {
         const uint32_t j = threadIdx.x / kTeam, lane = threadIdx.x % kTeam;
-        const uint32_t c = min(j0 + j, p.channels - 1);
+        const uint32_t c = min(j0 + j, channels - 1);
         const float g = gamma[c], b = beta[c];
-        const float2 *of_unit = partials + (size_t)(blockIdx.z * p.groups + fast_div(c, p.ch_per_group)) * kGnStatSlices;
+        const float2 *of_unit = partials + (size_t)(blockIdx.z * p.groups + fast_div(c, FastDiv{p.cpg_mul, p.cpg_shift, 0})) * kGnStatSlices;
         float n_l[kGnStatSlices / kTeam];
         float2 part[kGnStatSlices / kTeam];
         float weighted = 0.0f;
 #pragma unroll
         for (uint32_t i = 0; i < kGnStatSlices / kTeam; i++) {
             const uint32_t l = lane + i * kTeam;
-            const bool have = l < p.stats.slices.d;
+            const bool have = l < p.slices;
             part[i] = of_unit[have ? l : 0];
-            const uint32_t begin = l * p.stats.vec_per_slice;
-            n_l[i] = have ? (float)((min(p.stats.vec_per_unit, begin + p.stats.vec_per_slice) - begin) * EPV) : 0.0f;
+            const uint32_t begin = l * p.vec_per_slice;
+            n_l[i] = have ? (float)((min(p.vec_per_unit, begin + p.vec_per_slice) - begin) * EPV) : 0.0f;
             weighted = have ? fmaf(part[i].x, n_l[i], weighted) : weighted;
         }
         const float mean = team_sum<kTeam>(weighted) * p.inv_count;
@@ -969,7 +977,7 @@ __global__ __launch_bounds__(kTileThreads) void gn_tokens_apply_kernel(
 #pragma unroll
         for (uint32_t i = 0; i < kGnStatSlices / kTeam; i++) {
             const float d = part[i].x - mean;
-            if (lane + i * kTeam < p.stats.slices.d) m2 += fmaf(n_l[i] * d, d, part[i].y);
+            if (lane + i * kTeam < p.slices) m2 += fmaf(n_l[i] * d, d, part[i].y);
         }
         const float rstd = __builtin_amdgcn_rsqf(team_sum<kTeam>(m2) * p.inv_count + p.eps);
         if (lane == 0) affine[j] = make_float4(mean, rstd * g, b, 0.0f);
@@ -983,8 +991,8 @@ __global__ __launch_bounds__(kTileThreads) void gn_tokens_apply_kernel(
         for (int e = 0; e < EPV; e++) f[e] = fmaf(f[e] - a.x, a.y, a.z);
         return Store<T>::pack(f);
     };
-    transpose_tile<ES, RAGGED>(reinterpret_cast<const char *>(x + plane), reinterpret_cast<char *>(y + plane), p.channels,
-                               p.hw, j0, k0, tile4, ready, normalise);
+    transpose_tile<ES, RAGGED>(reinterpret_cast<const char *>(x + plane), reinterpret_cast<char *>(y + plane), channels,
+                               hw, j0, k0, tile4, ready, normalise);
 }
 
 // ---------------------------------------------------------------------------
@@ -999,34 +1007,34 @@ inline uint32_t gn_xcd_shift(const Chip &chip, bool shared, size_t units) {
 }
 
 template <typename T, int K, bool RAGGED>
-void gn_launch_k(bool silu, bool shared, uint32_t blocks, uint32_t threads, hipStream_t stream, const T *x,
+void gn_launch_k(bool silu, bool shared, uint32_t blocks, uint32_t threads, uint32_t shape, hipStream_t stream, const T *x,
                  const T *chunk, T *y, const float *gamma, const float *beta, const GnScratch &sc,
                  const GnParams &p) {
     if (K <= kGnSharedMaxK && shared) {
         constexpr int KS = K <= kGnSharedMaxK ? K : 1;  // (larger K never get here: no such instances)
         launch((silu ? gn_slice_kernel<T, KS, true, true, RAGGED> : gn_slice_kernel<T, KS, false, true, RAGGED>),
-               dim3(blocks), dim3(threads), 0, stream, x, chunk, y, gamma, beta, sc, p);
+               dim3(blocks), dim3(threads), 0, stream, x, p.vec_per_unit, p.vec_per_slice, shape, chunk, y, gamma, beta, sc, p);
     } else {
         launch((silu ? gn_slice_kernel<T, K, true, false, RAGGED> : gn_slice_kernel<T, K, false, false, RAGGED>),
-               dim3(blocks), dim3(threads), 0, stream, x, chunk, y, gamma, beta, sc, p);
+               dim3(blocks), dim3(threads), 0, stream, x, p.vec_per_unit, p.vec_per_slice, shape, chunk, y, gamma, beta, sc, p);
     }
 }
 
 template <typename T, bool RAGGED>
-int gn_launch(uint32_t k, bool silu, bool shared, uint32_t blocks, uint32_t threads, hipStream_t stream, const T *x,
+int gn_launch(uint32_t k, bool silu, bool shared, uint32_t blocks, uint32_t threads, uint32_t shape, hipStream_t stream, const T *x,
               const T *chunk, T *y, const float *gamma, const float *beta, const GnScratch &sc, const GnParams &p) {
     switch (k) {
-        case 1: gn_launch_k<T, 1, RAGGED>(silu, shared, blocks, threads, stream, x, chunk, y, gamma, beta, sc, p); break;
-        case 2: gn_launch_k<T, 2, RAGGED>(silu, shared, blocks, threads, stream, x, chunk, y, gamma, beta, sc, p); break;
-        case 3: gn_launch_k<T, 3, RAGGED>(silu, shared, blocks, threads, stream, x, chunk, y, gamma, beta, sc, p); break;
-        case 4: gn_launch_k<T, 4, RAGGED>(silu, shared, blocks, threads, stream, x, chunk, y, gamma, beta, sc, p); break;
-        case 5: gn_launch_k<T, 5, RAGGED>(silu, shared, blocks, threads, stream, x, chunk, y, gamma, beta, sc, p); break;
-        case 6: gn_launch_k<T, 6, RAGGED>(silu, shared, blocks, threads, stream, x, chunk, y, gamma, beta, sc, p); break;
-        case 8: gn_launch_k<T, 8, RAGGED>(silu, shared, blocks, threads, stream, x, chunk, y, gamma, beta, sc, p); break;
-        case 10: gn_launch_k<T, 10, RAGGED>(silu, shared, blocks, threads, stream, x, chunk, y, gamma, beta, sc, p); break;
-        case 12: gn_launch_k<T, 12, RAGGED>(silu, shared, blocks, threads, stream, x, chunk, y, gamma, beta, sc, p); break;
-        case 16: gn_launch_k<T, 16, RAGGED>(silu, shared, blocks, threads, stream, x, chunk, y, gamma, beta, sc, p); break;
-        case 20: gn_launch_k<T, 20, RAGGED>(silu, shared, blocks, threads, stream, x, chunk, y, gamma, beta, sc, p); break;
+        case 1: gn_launch_k<T, 1, RAGGED>(silu, shared, blocks, threads, shape, stream, x, chunk, y, gamma, beta, sc, p); break;
+        case 2: gn_launch_k<T, 2, RAGGED>(silu, shared, blocks, threads, shape, stream, x, chunk, y, gamma, beta, sc, p); break;
+        case 3: gn_launch_k<T, 3, RAGGED>(silu, shared, blocks, threads, shape, stream, x, chunk, y, gamma, beta, sc, p); break;
+        case 4: gn_launch_k<T, 4, RAGGED>(silu, shared, blocks, threads, shape, stream, x, chunk, y, gamma, beta, sc, p); break;
+        case 5: gn_launch_k<T, 5, RAGGED>(silu, shared, blocks, threads, shape, stream, x, chunk, y, gamma, beta, sc, p); break;
+        case 6: gn_launch_k<T, 6, RAGGED>(silu, shared, blocks, threads, shape, stream, x, chunk, y, gamma, beta, sc, p); break;
+        case 8: gn_launch_k<T, 8, RAGGED>(silu, shared, blocks, threads, shape, stream, x, chunk, y, gamma, beta, sc, p); break;
+        case 10: gn_launch_k<T, 10, RAGGED>(silu, shared, blocks, threads, shape, stream, x, chunk, y, gamma, beta, sc, p); break;
+        case 12: gn_launch_k<T, 12, RAGGED>(silu, shared, blocks, threads, shape, stream, x, chunk, y, gamma, beta, sc, p); break;
+        case 16: gn_launch_k<T, 16, RAGGED>(silu, shared, blocks, threads, shape, stream, x, chunk, y, gamma, beta, sc, p); break;
+        case 20: gn_launch_k<T, 20, RAGGED>(silu, shared, blocks, threads, shape, stream, x, chunk, y, gamma, beta, sc, p); break;
         default: return MSD_ERR_INVALID_VALUE;  // not a K the kernels are built for: a planning error
     }
     return launch_status();
@@ -1081,7 +1089,6 @@ int gn_dispatch(const void *xv, const void *chunkv, void *yv, const float *gamma
     p.vec_per_unit = (uint32_t)(unit_size / EPV);
     p.vec_per_slice = d.vec_per_slice;
     p.split = split;
-    p.split_shift = (uint32_t)__builtin_ctz(split);
     p.groups = make_fast_div((uint32_t)groups);
     p.ch_per_group = (uint32_t)cpg;
     p.hw_vec = make_fast_div((uint32_t)(ragged ? hw : hw / EPV));
@@ -1089,10 +1096,9 @@ int gn_dispatch(const void *xv, const void *chunkv, void *yv, const float *gamma
     p.inv_count = 1.0f / (float)unit_size;
     p.spin_limit = tune_spin > 0 ? (uint32_t)tune_spin : kGnSpinLimit;
     const bool shared = d.writers > 1;
-    p.writers = d.writers;
-    p.writers_shift = (uint32_t)__builtin_ctz(d.writers);
     p.part_vecs = (uint32_t)((((p.vec_per_unit + d.writers - 1) / d.writers + kWave - 1) / kWave) * kWave);
-    p.xcd_shift = gn_xcd_shift(chip_info(), shared, units);
+    const uint32_t shape = gn_shape_word((uint32_t)__builtin_ctz(split), (uint32_t)__builtin_ctz(d.writers),
+                                         gn_xcd_shift(chip_info(), shared, units), d.threads);
 
     if (fixed != nullptr) {
         sc = *fixed;
@@ -1102,8 +1108,8 @@ int gn_dispatch(const void *xv, const void *chunkv, void *yv, const float *gamma
     }
     const uint32_t blocks = (uint32_t)(units * split * d.writers);
     if (ragged)
-        return gn_launch<T, true>(d.k, silu, shared, blocks, d.threads, stream, x, chunk, y, gamma, beta, sc, p);
-    return gn_launch<T, false>(d.k, silu, shared, blocks, d.threads, stream, x, chunk, y, gamma, beta, sc, p);
+        return gn_launch<T, true>(d.k, silu, shared, blocks, d.threads, shape, stream, x, chunk, y, gamma, beta, sc, p);
+    return gn_launch<T, false>(d.k, silu, shared, blocks, d.threads, shape, stream, x, chunk, y, gamma, beta, sc, p);
 }
 
 template int gn_dispatch<float>(const void *, const void *, void *, const float *, const float *,
@@ -1155,10 +1161,12 @@ GnTokUnitPlan gn_tokens_unit_plan(const Chip &chip, size_t units, size_t cpg, si
 }
 
 template <typename T, int K>
-void gn_tokens_unit_launch(const GnTokUnitPlan &pl, uint32_t blocks, hipStream_t stream, const T *x, T *y, const float *gamma,
-                           const float *beta, const GnTokUnitParams &q) {
+void gn_tokens_unit_launch(const GnTokUnitPlan &pl, uint32_t xcd_shift, uint32_t units, uint32_t vec_per_unit, hipStream_t stream,
+                           const T *x, T *y, const float *gamma, const float *beta, const GnTokUnitParams &q) {
+    const uint32_t blocks = units * pl.writers, units_per_xcd = units >> xcd_shift;
     launch((pl.ragged ? gn_tokens_unit_kernel<T, K, true> : gn_tokens_unit_kernel<T, K, false>), dim3(blocks),
-           dim3(pl.threads), pl.lds, stream, x, y, gamma, beta, q);
+           dim3(pl.threads), pl.lds, stream, x, vec_per_unit, units_per_xcd,
+           gn_shape_word(0, (uint32_t)__builtin_ctz(pl.writers), xcd_shift, pl.threads), y, gamma, beta, q);
 }
 
 template <typename T>
@@ -1166,16 +1174,12 @@ int gn_tokens_unit(const GnTokUnitPlan &pl, const Chip &chip, const T *x, T *y, 
                    size_t units, size_t channels, size_t hw, size_t groups, float eps, hipStream_t stream) {
     constexpr uint32_t EPV = Store<T>::EPV;
     const size_t cpg = channels / groups, unit_size = cpg * hw;
+    const uint32_t vec_per_unit = (uint32_t)(unit_size / EPV), xcd_shift = gn_xcd_shift(chip, true, units);
     GnTokUnitParams q;
-    q.vec_per_unit = (uint32_t)(unit_size / EPV);
     q.groups = make_fast_div((uint32_t)groups);
     q.ch_per_group = (uint32_t)cpg;
     q.channels = (uint32_t)channels;
     q.hw = (uint32_t)hw;
-    q.writers = pl.writers;
-    q.writers_shift = (uint32_t)__builtin_ctz(pl.writers);
-    q.xcd_shift = gn_xcd_shift(chip, true, units);
-    q.units_per_xcd = (uint32_t)(units >> q.xcd_shift);
     q.part_pos = pl.part_pos;
     q.pitch = pl.pitch;
     q.hw_vec = make_fast_div(pl.ragged ? 1u : (uint32_t)hw / EPV);
@@ -1183,18 +1187,17 @@ int gn_tokens_unit(const GnTokUnitPlan &pl, const Chip &chip, const T *x, T *y, 
     q.row_step = pl.threads / q.row_dwords.d;
     q.eps = eps;
     q.inv_count = 1.0f / (float)unit_size;
-    const uint32_t blocks = (uint32_t)(units * pl.writers);
     switch (pl.k) {
-        case 1: gn_tokens_unit_launch<T, 1>(pl, blocks, stream, x, y, gamma, beta, q); break;
-        case 2: gn_tokens_unit_launch<T, 2>(pl, blocks, stream, x, y, gamma, beta, q); break;
-        case 3: gn_tokens_unit_launch<T, 3>(pl, blocks, stream, x, y, gamma, beta, q); break;
-        case 4: gn_tokens_unit_launch<T, 4>(pl, blocks, stream, x, y, gamma, beta, q); break;
-        case 5: gn_tokens_unit_launch<T, 5>(pl, blocks, stream, x, y, gamma, beta, q); break;
-        case 6: gn_tokens_unit_launch<T, 6>(pl, blocks, stream, x, y, gamma, beta, q); break;
-        case 8: gn_tokens_unit_launch<T, 8>(pl, blocks, stream, x, y, gamma, beta, q); break;
-        case 10: gn_tokens_unit_launch<T, 10>(pl, blocks, stream, x, y, gamma, beta, q); break;
-        case 12: gn_tokens_unit_launch<T, 12>(pl, blocks, stream, x, y, gamma, beta, q); break;
-        default: gn_tokens_unit_launch<T, 16>(pl, blocks, stream, x, y, gamma, beta, q); break;
+        case 1: gn_tokens_unit_launch<T, 1>(pl, xcd_shift, (uint32_t)units, vec_per_unit, stream, x, y, gamma, beta, q); break;
+        case 2: gn_tokens_unit_launch<T, 2>(pl, xcd_shift, (uint32_t)units, vec_per_unit, stream, x, y, gamma, beta, q); break;
+        case 3: gn_tokens_unit_launch<T, 3>(pl, xcd_shift, (uint32_t)units, vec_per_unit, stream, x, y, gamma, beta, q); break;
+        case 4: gn_tokens_unit_launch<T, 4>(pl, xcd_shift, (uint32_t)units, vec_per_unit, stream, x, y, gamma, beta, q); break;
+        case 5: gn_tokens_unit_launch<T, 5>(pl, xcd_shift, (uint32_t)units, vec_per_unit, stream, x, y, gamma, beta, q); break;
+        case 6: gn_tokens_unit_launch<T, 6>(pl, xcd_shift, (uint32_t)units, vec_per_unit, stream, x, y, gamma, beta, q); break;
+        case 8: gn_tokens_unit_launch<T, 8>(pl, xcd_shift, (uint32_t)units, vec_per_unit, stream, x, y, gamma, beta, q); break;
+        case 10: gn_tokens_unit_launch<T, 10>(pl, xcd_shift, (uint32_t)units, vec_per_unit, stream, x, y, gamma, beta, q); break;
+        case 12: gn_tokens_unit_launch<T, 12>(pl, xcd_shift, (uint32_t)units, vec_per_unit, stream, x, y, gamma, beta, q); break;
+        default: gn_tokens_unit_launch<T, 16>(pl, xcd_shift, (uint32_t)units, vec_per_unit, stream, x, y, gamma, beta, q); break;
     }
     return launch_status();
 }
@@ -1202,8 +1205,11 @@ int gn_tokens_unit(const GnTokUnitPlan &pl, const Chip &chip, const T *x, T *y, 
 template <typename T, int K>
 void gn_tokens_launch(uint32_t blocks, uint32_t threads, size_t lds_bytes, hipStream_t stream,
                       const T *x, T *y, const float *gamma, const float *beta, const GnScratch &sc,
-                      const GnTokParams &q) {
-    launch((gn_tokens_kernel<T, K>), dim3(blocks), dim3(threads), lds_bytes, stream, x, y, gamma, beta, sc, q);
+                      const GnTokParams &q, const FastDiv &pos_vecs, const FastDiv &combos) {
+    const GnParams &p = q.base;
+    launch((gn_tokens_kernel<T, K>), dim3(blocks), dim3(threads), lds_bytes, stream, x, p.vec_per_unit, p.vec_per_slice,
+           pos_vecs.mul, pos_vecs.shift, pos_vecs.d, p.hw_vec.d, combos.mul, combos.shift, combos.d, p.groups.d,
+           gn_shape_word((uint32_t)__builtin_ctz(p.split), 0, 0, threads), y, gamma, beta, sc, q);
 }
 
 // Whether gn_tokens_unit_kernel is the better one launch for a shape it can take: its units are loaded once per writer and
@@ -1270,30 +1276,31 @@ bool gn_tokens_two_launches(const T *x, T *y, const float *gamma, const float *b
         lock = std::unique_lock<std::mutex>(partials_lock(sc));
     }
     GnApplyParams p;
-    p.stats.vec_per_unit = (uint32_t)(unit_size / EPV);
+    p.vec_per_unit = (uint32_t)(unit_size / EPV);
     const Chip chip = chip_info();
     // slices of at most 2048 vectors, shorter (two per lane at least) while the chip has less than two
     // workgroups per CU
     uint32_t slices = 1;
-    while (slices < kGnStatSlices && ((units * slices < 2 * (size_t)chip.cus && p.stats.vec_per_unit >= slices * 2 * kStatsThreads) ||
-                                      p.stats.vec_per_unit > slices * 2048))
+    while (slices < kGnStatSlices && ((units * slices < 2 * (size_t)chip.cus && p.vec_per_unit >= slices * 2 * kStatsThreads) ||
+                                      p.vec_per_unit > slices * 2048))
         slices *= 2;
-    p.stats.vec_per_slice = (p.stats.vec_per_unit + slices - 1) / slices;
-    slices = (p.stats.vec_per_unit + p.stats.vec_per_slice - 1) / p.stats.vec_per_slice;  // (no empty slice)
-    p.stats.slices = make_fast_div(slices);
-    p.ch_per_group = make_fast_div((uint32_t)cpg);
+    p.vec_per_slice = (p.vec_per_unit + slices - 1) / slices;
+    slices = (p.vec_per_unit + p.vec_per_slice - 1) / p.vec_per_slice;  // (no empty slice)
+    p.slices = slices;
+    const FastDiv by_slices = make_fast_div(slices), by_cpg = make_fast_div((uint32_t)cpg);
+    p.cpg_mul = by_cpg.mul;
+    p.cpg_shift = by_cpg.shift;
     p.groups = (uint32_t)groups;
-    p.channels = (uint32_t)channels;
-    p.hw = (uint32_t)hw;
     p.eps = eps;
     p.inv_count = 1.0f / (float)unit_size;
     const bool ragged = channels % EPV != 0 || hw % EPV != 0 || !aligned16(y);
     const bool jfast = (channels < hw && tiles.x <= 65535) || tiles.y > 65535;
     auto *apply = jfast ? (ragged ? gn_tokens_apply_kernel<T, true, true> : gn_tokens_apply_kernel<T, true, false>)
                         : (ragged ? gn_tokens_apply_kernel<T, false, true> : gn_tokens_apply_kernel<T, false, false>);
-    launch((gn_stats_kernel<T>), dim3((uint32_t)(units * slices)), dim3(kStatsThreads), 0, stream, x, partials, p.stats);
-    launch(apply, jfast ? dim3(tiles.y, tiles.x, tiles.z) : tiles, dim3(kTileThreads), 0, stream, x, y, gamma, beta,
-           partials, p);
+    launch((gn_stats_kernel<T>), dim3((uint32_t)(units * slices)), dim3(kStatsThreads), 0, stream, x, p.vec_per_unit,
+           p.vec_per_slice, by_slices.mul, by_slices.shift, slices, partials);
+    launch(apply, jfast ? dim3(tiles.y, tiles.x, tiles.z) : tiles, dim3(kTileThreads), 0, stream, x, (uint32_t)channels,
+           (uint32_t)hw, gamma, beta, y, partials, p);
     *status = launch_status();
     return true;
 }
@@ -1371,23 +1378,18 @@ int gn_tokens_dispatch(const void *xv, void *yv, const float *gamma, const float
     q.base.vec_per_unit = (uint32_t)(cpg * hw_vec);
     q.base.vec_per_slice = (uint32_t)nvec;
     q.base.split = split;
-    q.base.split_shift = (uint32_t)__builtin_ctz(split);
-    q.base.writers = 1;
-    q.base.writers_shift = 0;
     q.base.part_vecs = (uint32_t)nvec;
-    q.base.xcd_shift = 0;
     q.base.groups = make_fast_div((uint32_t)groups);
     q.base.ch_per_group = (uint32_t)cpg;
     q.base.hw_vec = make_fast_div((uint32_t)hw_vec);
     q.base.eps = eps;
     q.base.inv_count = 1.0f / (float)unit_size;
     q.base.spin_limit = tune_spin > 0 ? (uint32_t)tune_spin : kGnSpinLimit;
-    q.pos_vecs = make_fast_div((uint32_t)pvs);
+    const FastDiv pos_vecs = make_fast_div((uint32_t)pvs), combos = make_fast_div((uint32_t)(batch * split));  // ((sample, slice) pairs)
     q.row_dwords = make_fast_div((uint32_t)(cpg * sizeof(T) / 4));
     q.hw = (uint32_t)hw;
     q.channels = (uint32_t)channels;
     q.pitch = (uint32_t)(pvs * EPV + 16 / sizeof(T));
-    q.combos = make_fast_div((uint32_t)(batch * split));
     const size_t lds_bytes = cpg * q.pitch * sizeof(T);
     const GnThreads pl = gn_threads_for(chip, sizeof(T), (uint32_t)nvec, split, units * split, kMaxK, false, false);
     if (pl.k == 0) return whole ? in_one() : generic();
@@ -1405,16 +1407,16 @@ int gn_tokens_dispatch(const void *xv, void *yv, const float *gamma, const float
     }
     const uint32_t threads = pl.threads;
     switch (pl.k) {
-        case 1: gn_tokens_launch<T, 1>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q); break;
-        case 2: gn_tokens_launch<T, 2>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q); break;
-        case 3: gn_tokens_launch<T, 3>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q); break;
-        case 4: gn_tokens_launch<T, 4>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q); break;
-        case 5: gn_tokens_launch<T, 5>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q); break;
-        case 6: gn_tokens_launch<T, 6>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q); break;
-        case 8: gn_tokens_launch<T, 8>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q); break;
-        case 10: gn_tokens_launch<T, 10>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q); break;
-        case 12: gn_tokens_launch<T, 12>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q); break;
-        default: gn_tokens_launch<T, 16>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q); break;
+        case 1: gn_tokens_launch<T, 1>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, pos_vecs, combos); break;
+        case 2: gn_tokens_launch<T, 2>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, pos_vecs, combos); break;
+        case 3: gn_tokens_launch<T, 3>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, pos_vecs, combos); break;
+        case 4: gn_tokens_launch<T, 4>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, pos_vecs, combos); break;
+        case 5: gn_tokens_launch<T, 5>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, pos_vecs, combos); break;
+        case 6: gn_tokens_launch<T, 6>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, pos_vecs, combos); break;
+        case 8: gn_tokens_launch<T, 8>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, pos_vecs, combos); break;
+        case 10: gn_tokens_launch<T, 10>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, pos_vecs, combos); break;
+        case 12: gn_tokens_launch<T, 12>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, pos_vecs, combos); break;
+        default: gn_tokens_launch<T, 16>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, pos_vecs, combos); break;
     }
     return launch_status();
 }
