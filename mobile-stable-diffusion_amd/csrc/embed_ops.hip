@@ -391,13 +391,18 @@ constexpr float kNegInf = -__builtin_huge_valf();
 // by element are eight loads and stores a lane (and three passes beyond 512 columns); softmax_dispatch says from how
 // many rows on that is slower.  fp16, us, element by element and so: 16128 x 252 6.63 -> 4.66, 32256 x 252
 // 10.9 -> 7.1, 65536 x 140 17.9 -> 10.2, 4000 x 1023 9.5 -> 5.2; 16128 x 256, whole vectors, takes 4.1.
+// Lanes of a workgroup: long rows (a wavefront per row, 8 or 16 vectors per lane) run as single-wavefront workgroups, the shorter
+// ones in workgroups of four (us, four wavefronts / two / one: fp16 5120 x 576 3.83 3.95 4.61, 24576 x 144 5.01 4.89 5.51,
+// fp32 20480 x 64 3.16 3.24 3.69, 49152 x 64 5.96 6.07 5.87)
+constexpr uint32_t softmax_team_lanes(int vpl, int tl) { return (tl == kWave && vpl >= 8) ? kWave : kSmThreads; }
+
 template <typename T, int VPL, int TL, bool RAGGED>
 __global__ __launch_bounds__(kSmThreads) void softmax_team_kernel(const T *x, T *y, uint32_t rows, uint32_t cols,
                                                                   int stable) {
     constexpr int EPV = Store<T>::EPV, ES = (int)sizeof(T);
     constexpr int RPW = kWave / TL;
     const uint32_t lane = threadIdx.x & (kWave - 1);
-    const uint32_t wave = blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave;
+    const uint32_t wave = blockIdx.x * (softmax_team_lanes(VPL, TL) / kWave) + threadIdx.x / kWave;
     const uint32_t row = wave * RPW + lane / TL;
     const uint32_t j = lane % TL;
     const bool live = row < rows;
@@ -463,10 +468,10 @@ constexpr int kSmBlockMaxVpl = 8;
 
 template <typename T, int VPL>
 __global__ __launch_bounds__(kSmBlockMaxThreads, 4) void softmax_block_kernel(const T *x, T *y, uint32_t row_vecs,
-                                                                            int stable) {
+                                                                            int stable, uint32_t nt) {
     constexpr int EPV = Store<T>::EPV;
     __shared__ float slots_max[kSmBlockMaxThreads / kWave], slots_sum[kSmBlockMaxThreads / kWave];
-    const uint32_t tid = threadIdx.x, nt = blockDim.x;
+    const uint32_t tid = threadIdx.x;
     const uint32_t lane = tid & (kWave - 1), wave = tid / kWave, waves = nt / kWave;
     const size_t row_base = (size_t)blockIdx.x * row_vecs;
     const u32x4 *in = reinterpret_cast<const u32x4 *>(x) + row_base;
@@ -682,10 +687,10 @@ __device__ __forceinline__ float ddim_one(float x, float e, const DdimCoef &c) {
 }
 
 template <typename T>
-__global__ __launch_bounds__(kDdimThreads) void ddim_update_kernel(const T *x, const T *e_t, T *x_prev,
-                                                                   size_t n, int vectors, DdimCoef c) {
+__global__ __launch_bounds__(kDdimThreads) void ddim_update_kernel(const T *x, const T *e_t, T *x_prev, size_t n,
+                                                                   int vectors, uint32_t blocks, DdimCoef c) {
     constexpr int EPV = Store<T>::EPV;
-    const size_t stride = (size_t)gridDim.x * kDdimThreads;
+    const size_t stride = (size_t)blocks * kDdimThreads;
     const size_t first = (size_t)blockIdx.x * kDdimThreads + threadIdx.x;
     if (vectors) {
         const size_t vecs = n / EPV;
@@ -749,10 +754,7 @@ void linear_quads(size_t m, size_t n, int act_in, F f) {
 
 template <typename T, int VPL, int TL, bool RAGGED>
 void softmax_team_launch(const T *x, T *y, uint32_t rows, uint32_t cols, int stable, hipStream_t stream) {
-    // long rows (a wavefront per row, 8 or 16 vectors per lane) run as single-wavefront workgroups, the shorter
-    // ones in workgroups of four (us, four wavefronts / two / one: fp16 5120 x 576 3.83 3.95 4.61, 24576 x 144 5.01 4.89 5.51,
-    // fp32 20480 x 64 3.16 3.24 3.69, 49152 x 64 5.96 6.07 5.87)
-    constexpr uint32_t threads = (TL == kWave && VPL >= 8) ? kWave : kSmThreads;
+    constexpr uint32_t threads = softmax_team_lanes(VPL, TL);
     constexpr uint32_t rows_per_block = (threads / kWave) * (kWave / TL);
     launch((softmax_team_kernel<T, VPL, TL, RAGGED>), dim3((rows + rows_per_block - 1) / rows_per_block),
                        dim3(threads), 0, stream, x, y, rows, cols, stable);
@@ -786,7 +788,7 @@ void softmax_block_launch(const T *x, T *y, uint32_t rows, uint32_t row_vecs, in
         const dim3 grid(min(rows - done, kMostRows));
         const T *xs = x + (size_t)done * row_vecs * Store<T>::EPV;
         T *ys = y + (size_t)done * row_vecs * Store<T>::EPV;
-        launch(kernel, grid, block, lds, stream, xs, ys, row_vecs, stable);
+        launch(kernel, grid, block, lds, stream, xs, ys, row_vecs, stable, block.x);
         if (rows - done <= kMostRows) break;
     }
 }
@@ -1037,9 +1039,9 @@ int ddim_update_dispatch(const void *xv, const void *ev, void *yv, size_t n, flo
     c.sqrt_aprev = sqrtf(a_prev);
     const int vectors = aligned16(xv) && aligned16(ev) && aligned16(yv);
     const size_t want = (n / Store<T>::EPV + kDdimThreads) / kDdimThreads;
-    launch((ddim_update_kernel<T>), dim3((uint32_t)(want < 4096 ? want : 4096)),
-                       dim3(kDdimThreads), 0, stream, static_cast<const T *>(xv),
-                       static_cast<const T *>(ev), static_cast<T *>(yv), n, vectors, c);
+    const uint32_t blocks = (uint32_t)(want < 4096 ? want : 4096);
+    launch((ddim_update_kernel<T>), dim3(blocks), dim3(kDdimThreads), 0, stream, static_cast<const T *>(xv),
+           static_cast<const T *>(ev), static_cast<T *>(yv), n, vectors, blocks, c);
     return launch_status();
 }
 

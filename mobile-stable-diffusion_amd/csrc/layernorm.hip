@@ -99,10 +99,13 @@ constexpr float kLnFastMoments = 4.0f;
 // reads its columns from there: fetching them from the cache per row costs four times the
 // row's own bytes in load instructions (measured at 131072 x 320 fp16: 31.2 us from global
 // memory, 29.7 us from LDS, 29.4 us with no affine at all).
+// What the loads need comes first among the arguments, the lanes of the workgroup too (asked from the launch they are an
+// argument in memory): the leading ones come in scalar registers (build.py).  fp16 8192 x 320 3.51 -> 3.44 us, 2048 x 640 2.66 -> 2.63;
+// in a recorded step, where the arguments are in no cache, more (GEGLU's note in stream_ops.hip).
 template <typename T, int NW, int VPL, int TL, bool EARLY>
 __global__ __launch_bounds__(kLnMaxThreads) void ln_team_kernel(
-    const T *x, const T *res, T *sum, T *y, const float *__restrict__ gamma,
-    const float *__restrict__ beta, uint32_t rows, float eps, float inv_dim) {
+    const T *x, const T *res, const float *__restrict__ gamma, const float *__restrict__ beta, uint32_t rows,
+    uint32_t threads, T *sum, T *y, float eps, float inv_dim) {
     typedef Chunk<T, NW> C;
     typedef typename C::vec_t vec_t;
     constexpr int N = C::N;
@@ -110,7 +113,7 @@ __global__ __launch_bounds__(kLnMaxThreads) void ln_team_kernel(
     constexpr int DIM = VPL * TL * N;
     extern __shared__ f32x4 ln_lds[];  // !EARLY: gamma[DIM] then beta[DIM]
     const uint32_t lane = threadIdx.x & (kWave - 1);
-    const uint32_t wave = blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave;
+    const uint32_t wave = blockIdx.x * (threads / kWave) + threadIdx.x / kWave;
     const uint32_t row = wave * RPW + lane / TL;
     const uint32_t j = lane % TL;
     const bool live = row < rows;
@@ -142,7 +145,7 @@ __global__ __launch_bounds__(kLnMaxThreads) void ln_team_kernel(
         }
     }
     if (!EARLY) {  // the whole workgroup, rows past the end included, fills the LDS copy
-        for (uint32_t i = threadIdx.x; i < DIM / 4; i += blockDim.x) {
+        for (uint32_t i = threadIdx.x; i < DIM / 4; i += threads) {
             ln_lds[i] = reinterpret_cast<const f32x4 *>(gamma)[i];
             ln_lds[DIM / 4 + i] = reinterpret_cast<const f32x4 *>(beta)[i];
         }
@@ -310,11 +313,11 @@ void ln_launch(const T *x, const T *res, T *sum, T *y, const float *gamma, const
     const uint32_t blocks = (rows + rows_per_block - 1) / rows_per_block;
     if (early)
         launch((ln_team_kernel<T, NW, VPL, TL, true>), dim3(blocks), dim3(threads), 0, stream, x,
-                           res, sum, y, gamma, beta, rows, eps, inv_dim);
+                           res, gamma, beta, rows, threads, sum, y, eps, inv_dim);
     else
         launch((ln_team_kernel<T, NW, VPL, TL, false>), dim3(blocks), dim3(threads),
-                           2 * sizeof(float) * VPL * TL * (NW * 4 / sizeof(T)), stream, x, res, sum, y, gamma, beta,
-                           rows, eps, inv_dim);
+                           2 * sizeof(float) * VPL * TL * (NW * 4 / sizeof(T)), stream, x, res, gamma, beta, rows,
+                           threads, sum, y, eps, inv_dim);
 }
 
 template <typename T, int NW, int TL>
