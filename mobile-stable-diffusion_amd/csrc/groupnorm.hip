@@ -53,13 +53,12 @@ struct GnParams {
     uint32_t split;          // workgroups per unit, power of two <= kGnMaxSplit
     uint32_t spin_limit;     // polls before a slice stops waiting for a sibling's words
     FastDiv groups;          // per sample
-    uint32_t ch_per_group;
-    FastDiv hw_vec;          // vectors per channel (RAGGED: elements per channel)
     float eps;
     float inv_count;         // 1 / elements per unit
     // gn_slice_kernel<..., SHARED>: several workgroups per whole unit; each loads and reduces the
     // whole unit and normalises and stores one part of it
     uint32_t part_vecs;      // vectors per part, a multiple of 64 (a wavefront is inside one part or outside)
+    uint32_t hw;             // RAGGED: elements per channel
 };
 
 // The arguments that a wavefront needs before it can ask for its data are the kernels' first ones, plain values that arrive
@@ -344,12 +343,11 @@ __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
                                         const float *__restrict__ gamma,
                                         const float *__restrict__ beta, const GnScratch &scratch,
                                         const GnParams &p, uint32_t nt, uint32_t vec_per_unit, uint32_t unit, uint32_t slice,
-                                        uint32_t part, uint32_t v_begin, uint32_t v_end, float *red, float *stats,
-                                        float2 *aff) {
+                                        uint32_t part, uint32_t v_begin, uint32_t v_end, uint32_t ch_per_group,
+                                        const FastDiv &hw_vec, float *red, float *stats, float2 *aff) {
     constexpr int EPV = Store<T>::EPV;
     const uint32_t tid = threadIdx.x;
     const u32x4 *xin = reinterpret_cast<const u32x4 *>(x) + (size_t)unit * vec_per_unit;
-    u32x4 *yout = reinterpret_cast<u32x4 *>(y) + (size_t)unit * vec_per_unit;
 
     // ---- the slice goes into registers.  Lanes past the end of a ragged slice re-read its
     // last vector (a valid address) and are masked later: no load sits behind a branch.
@@ -377,39 +375,69 @@ __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
     };
 #pragma unroll
     for (int k = 0; k < K; k++) raw[k] = load_stream(at(xin, k, tid));
+    // optional per-(sample, channel) addend applied before the statistics (the reference's
+    // chunkwise_add pass): the sum replaces the slice in registers, rounded to the storage
+    // type exactly as a separate add kernel would have stored it
+    struct Addend {
+        T first, second;  // of a vector's channel, RAGGED of the two it may hold
+    };
+    auto addend_of = [&](uint32_t v) {
+        const T *cb = chunk + (size_t)unit * ch_per_group;  // the unit's channels
+        if (!RAGGED) {
+            const T c = cb[fast_div(v, hw_vec)];
+            return Addend{c, c};
+        }
+        const uint32_t c = gn_straddle<EPV>(v, hw_vec).channel;
+        return Addend{cb[c], cb[min(c + 1, ch_per_group - 1)]};
+    };
+    auto plus = [&](const u32x4 &raw_v, uint32_t v, const Addend &addend) {
+        const float c0 = Store<T>::load1(&addend.first), c1 = Store<T>::load1(&addend.second);
+        const uint32_t first = RAGGED ? gn_straddle<EPV>(v, hw_vec).first : EPV;
+        float f[EPV];
+        Store<T>::unpack(raw_v, f);
+#pragma unroll
+        for (int e = 0; e < EPV; e++) f[e] += !RAGGED || (uint32_t)e < first ? c0 : c1;
+        return Store<T>::pack(f);
+    };
+    // Everything is requested before anything is waited for, in the order in which it is needed (loads return in order): data,
+    // addends, then gamma and beta (us per launch with addends, fp16 batch 2, one after the other and so: 640 channels at 32 x 32
+    // 4.63 -> 4.47, 1280 at 16 x 16 3.51 -> 3.40; recorded step of 512 x 512 727 -> 721).  Long slices request
+    // their addends when they have the data: K more registers, and their launches are long enough to hide it (fp32 128
+    // channels at 512 x 512, three passes of a decoder block 152.7 us, with everything early 153.5).
+    constexpr bool kPrefetchAffine = !RAGGED && K <= kGnPrefetchAffineK, kAddendEarly = kPrefetchAffine;
+    Addend addend[kAddendEarly ? K : 1];
+    if (kAddendEarly && chunk != nullptr) {  // uniform
+#pragma unroll
+        for (int k = 0; k < K; k++) addend[kAddendEarly ? k : 0] = addend_of(vidx(k, tid));
+    }
     // What follows waits for the arguments in memory: the compiler neither moves it up nor, as new values to it, shares it
     // with another branch in front of the loads.
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("" : "+s"(unit), "+s"(part));
+    u32x4 *yout = reinterpret_cast<u32x4 *>(y) + (size_t)unit * vec_per_unit;
     uint32_t last_tag = 0;  // (arrives right behind the data)
     if (!SHARED && p.split > 1 && tid == 0) last_tag = gn_exchange_last_tag(scratch, unit, slice);
-    const uint32_t ch0 = (unit - fast_div(unit, p.groups) * p.groups.d) * p.ch_per_group;
-    // the addends of the unit's channels
-    auto unit_chunk = [&]() { return chunk + (size_t)unit * p.ch_per_group; };
-    // v plus its channels' addends, rounded to the storage type
-    auto with_chunk = [&](const u32x4 &raw_v, uint32_t v, const T *cb) {
-        float f[EPV];
-        Store<T>::unpack(raw_v, f);
-        if (RAGGED) {
-            const GnStraddle at_v = gn_straddle<EPV>(v, p.hw_vec);
-            const float c0 = Store<T>::load1(cb + at_v.channel);
-            const float c1 = Store<T>::load1(cb + min(at_v.channel + 1, p.ch_per_group - 1));
+    const uint32_t ch0 = (unit - fast_div(unit, p.groups) * p.groups.d) * ch_per_group;
+    // per-vector channel affine.  Up to six vectors per lane: fetched into registers up front,
+    // while the data is in flight.  More: the group's gamma and beta go to LDS once (they are
+    // there after the barrier of the statistics) and the epilogue reads each vector's pair one
+    // vector ahead, so a lane's registers hold little besides its packed slice.
+    float ga[kPrefetchAffine ? K : 1], be[kPrefetchAffine ? K : 1];
+    if (kPrefetchAffine) {
 #pragma unroll
-            for (int e = 0; e < EPV; e++) f[e] += (uint32_t)e < at_v.first ? c0 : c1;
-        } else {
-            const float cv = Store<T>::load1(cb + fast_div(v, p.hw_vec));
-#pragma unroll
-            for (int e = 0; e < EPV; e++) f[e] += cv;
+        for (int k = 0; k < K; k++) {
+            const uint32_t c = ch0 + fast_div(vidx(k, tid), hw_vec);
+            ga[kPrefetchAffine ? k : 0] = gamma[c];
+            be[kPrefetchAffine ? k : 0] = beta[c];
         }
-        return Store<T>::pack(f);
-    };
-    // optional per-(sample, channel) addend applied before the statistics (the reference's
-    // chunkwise_add pass): the sum replaces the slice in registers, rounded to the storage
-    // type exactly as a separate add kernel would have stored it
+        __builtin_amdgcn_sched_barrier(0);
+    }
     if (chunk != nullptr) {  // uniform
-        const T *cb = unit_chunk();
 #pragma unroll
-        for (int k = 0; k < K; k++) raw[k] = with_chunk(raw[k], vidx(k, tid), cb);
+        for (int k = 0; k < K; k++) {
+            const uint32_t v = vidx(k, tid);
+            raw[k] = plus(raw[k], v, kAddendEarly ? addend[kAddendEarly ? k : 0] : addend_of(v));
+        }
     }
     if (!FULL) {  // registers of lanes past the end of a ragged slice hold zeros from here on
 #pragma unroll
@@ -419,21 +447,8 @@ __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
             for (int i = 0; i < 4; i++) raw[k][i] = mine ? raw[k][i] : 0u;
         }
     }
-    // per-vector channel affine.  Up to six vectors per lane: fetched into registers up front,
-    // while the data is in flight.  More: the group's gamma and beta go to LDS once (they are
-    // there after the barrier of the statistics) and the epilogue reads each vector's pair one
-    // vector ahead, so a lane's registers hold little besides its packed slice.
-    constexpr bool kPrefetchAffine = !RAGGED && K <= kGnPrefetchAffineK;
-    float ga[kPrefetchAffine ? K : 1], be[kPrefetchAffine ? K : 1];
-    if (kPrefetchAffine) {
-#pragma unroll
-        for (int k = 0; k < K; k++) {
-            const uint32_t c = ch0 + fast_div(vidx(k, tid), p.hw_vec);
-            ga[kPrefetchAffine ? k : 0] = gamma[c];
-            be[kPrefetchAffine ? k : 0] = beta[c];
-        }
-    } else {
-        for (uint32_t c = tid; c < p.ch_per_group; c += nt) {  // ch_per_group <= kGnLdsChannels (host)
+    if (!kPrefetchAffine) {
+        for (uint32_t c = tid; c < ch_per_group; c += nt) {  // ch_per_group <= kGnLdsChannels (host)
             aff[c] = make_float2(gamma[ch0 + c], beta[ch0 + c]);
         }
     }
@@ -450,9 +465,7 @@ __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
         auto read = [&](uint32_t l, uint32_t i) {
             const uint32_t v = l * p.vec_per_slice + i;
             u32x4 r = xin[v];
-            if (chunk != nullptr) {
-                r = with_chunk(r, v, unit_chunk());
-            }
+            if (chunk != nullptr) r = plus(r, v, addend_of(v));
             return r;
         };
         gn_exchange<T>(scratch, p, unit, slice, last_tag, slice_mean, slice_m2, stats, read);
@@ -469,7 +482,7 @@ __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
         constexpr bool kFold = decltype(fold_tag)::value;
         float g_next = 0.0f, b_next = 0.0f;
         if (!kPrefetchAffine && !RAGGED) {
-            const uint32_t c = fast_div(vidx(0, lane_again()), p.hw_vec);
+            const uint32_t c = fast_div(vidx(0, lane_again()), hw_vec);
             const float2 gb = aff[c];  // one 8-byte LDS read
             g_next = gb.x;
             b_next = gb.y;
@@ -486,7 +499,7 @@ __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
                 g_k = g_next;
                 b_k = b_next;
                 if (k + 1 < K) {  // the next vector's pair: its LDS latency passes under this vector's work
-                    const uint32_t c = fast_div(vidx(k + 1, lane_again()), p.hw_vec);
+                    const uint32_t c = fast_div(vidx(k + 1, lane_again()), hw_vec);
                     const float2 gb = aff[c];
                     g_next = gb.x;
                     b_next = gb.y;
@@ -500,9 +513,9 @@ __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
             }
             float f[EPV];
             if (RAGGED) {
-                const GnStraddle at_v = gn_straddle<EPV>(vidx(k, lane_again()), p.hw_vec);
+                const GnStraddle at_v = gn_straddle<EPV>(vidx(k, lane_again()), hw_vec);
                 const float2 gb0 = aff[at_v.channel];
-                const float2 gb1 = aff[min(at_v.channel + 1, p.ch_per_group - 1)];
+                const float2 gb1 = aff[min(at_v.channel + 1, ch_per_group - 1)];
                 const float a0 = rstd * gb0.x, a1 = rstd * gb1.x;
                 const float b0 = kFold ? fmaf(-mean, a0, gb0.y) : gb0.y, b1 = kFold ? fmaf(-mean, a1, gb1.y) : gb1.y;
                 forget(raw[k]);  // unpack here, one vector at a time
@@ -543,12 +556,14 @@ __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
 // computes (what large batches need).
 template <typename T, int K, bool SILU, bool SHARED, bool RAGGED>
 __global__ __launch_bounds__(kGnMaxThreads, (K <= (sizeof(T) == 2 ? 5 : 4) ? 8 : 4)) void gn_slice_kernel(
-    const T *x, uint32_t vec_per_unit, uint32_t vec_per_slice, uint32_t shape, const T *chunk, T *y,
-    const float *__restrict__ gamma, const float *__restrict__ beta, GnScratch scratch, GnParams p) {
+    const T *x, uint32_t vec_per_unit, uint32_t vec_per_slice, uint32_t shape, const T *chunk, uint32_t hw_mul,
+    uint32_t hw_shift, uint32_t ch_per_group, const float *__restrict__ gamma, const float *__restrict__ beta, T *y,
+    GnScratch scratch, GnParams p) {
     __shared__ float red[kGnRedSlots];
     __shared__ float stats[2];
     __shared__ float2 aff[!RAGGED && K <= kGnPrefetchAffineK ? 1 : kGnLdsChannels];  // (gamma, beta) of the group's channels
     const GnShape of(shape);
+    const FastDiv hw_vec{hw_mul, hw_shift, RAGGED ? p.hw : 0};
     uint32_t unit, slice, part;
     if (SHARED) {  // whole units, `writers` workgroups each
         const uint32_t j = blockIdx.x >> of.xcd_shift;
@@ -565,10 +580,10 @@ __global__ __launch_bounds__(kGnMaxThreads, (K <= (sizeof(T) == 2 ? 5 : 4) ? 8 :
     // uniform over the workgroup; the largest K is only launched on slices it fits exactly
     if (K == kGnMaxK || v_end - v_begin == K * of.threads)
         gn_body<T, K, SILU, true, SHARED, RAGGED>(x, chunk, y, gamma, beta, scratch, p, of.threads, vec_per_unit, unit, slice, part,
-                                          v_begin, v_end, red, stats, aff);
+                                          v_begin, v_end, ch_per_group, hw_vec, red, stats, aff);
     else
         gn_body<T, K, SILU, false, SHARED, RAGGED>(x, chunk, y, gamma, beta, scratch, p, of.threads, vec_per_unit, unit, slice, part,
-                                           v_begin, v_end, red, stats, aff);
+                                           v_begin, v_end, ch_per_group, hw_vec, red, stats, aff);
 }
 
 // Any shape or alignment (units that are no whole number of vectors, channels of less than a vector, many
@@ -618,6 +633,7 @@ __global__ __launch_bounds__(kGenericThreads) void gn_generic_kernel(
 // runs.  Statistics and the exchange between slices are those of gn_slice_kernel.
 // ---------------------------------------------------------------------------
 struct GnTokParams {
+    uint32_t ch_per_group;
     GnParams base;        // vec_per_slice = ch_per_group * position vectors per slice; vec_per_unit = that * split
     FastDiv row_dwords;   // 4-byte words per output run: ch_per_group * sizeof(T) / 4
     uint32_t hw;          // positions per sample
@@ -667,7 +683,7 @@ __global__ __launch_bounds__(kGnMaxThreads) void gn_tokens_kernel(
     __builtin_amdgcn_sched_barrier(0);  // (what follows waits for the arguments in memory)
     uint32_t last_tag = 0;
     if (p.split > 1 && tid == 0) last_tag = gn_exchange_last_tag(scratch, unit, slice);
-    const uint32_t ch0 = group * p.ch_per_group;
+    const uint32_t ch0 = group * q.ch_per_group;
 
     float slice_mean, slice_m2;
     gn_slice_stats<T, K, false>(raw, nvec, nt, red, slice_mean, slice_m2);
@@ -1006,35 +1022,43 @@ inline uint32_t gn_xcd_shift(const Chip &chip, bool shared, size_t units) {
     return (uint32_t)__builtin_ctz(chip.xcds);
 }
 
+// The leading plain arguments of gn_slice_kernel beside those of GnParams.
+struct GnGeometry {
+    uint32_t blocks, threads, shape, ch_per_group;
+    FastDiv hw;  // vectors per channel (RAGGED: elements per channel)
+};
+
 template <typename T, int K, bool RAGGED>
-void gn_launch_k(bool silu, bool shared, uint32_t blocks, uint32_t threads, uint32_t shape, hipStream_t stream, const T *x,
+void gn_launch_k(bool silu, bool shared, const GnGeometry &g, hipStream_t stream, const T *x,
                  const T *chunk, T *y, const float *gamma, const float *beta, const GnScratch &sc,
                  const GnParams &p) {
     if (K <= kGnSharedMaxK && shared) {
         constexpr int KS = K <= kGnSharedMaxK ? K : 1;  // (larger K never get here: no such instances)
         launch((silu ? gn_slice_kernel<T, KS, true, true, RAGGED> : gn_slice_kernel<T, KS, false, true, RAGGED>),
-               dim3(blocks), dim3(threads), 0, stream, x, p.vec_per_unit, p.vec_per_slice, shape, chunk, y, gamma, beta, sc, p);
+               dim3(g.blocks), dim3(g.threads), 0, stream, x, p.vec_per_unit, p.vec_per_slice, g.shape, chunk, g.hw.mul,
+               g.hw.shift, g.ch_per_group, gamma, beta, y, sc, p);
     } else {
         launch((silu ? gn_slice_kernel<T, K, true, false, RAGGED> : gn_slice_kernel<T, K, false, false, RAGGED>),
-               dim3(blocks), dim3(threads), 0, stream, x, p.vec_per_unit, p.vec_per_slice, shape, chunk, y, gamma, beta, sc, p);
+               dim3(g.blocks), dim3(g.threads), 0, stream, x, p.vec_per_unit, p.vec_per_slice, g.shape, chunk, g.hw.mul,
+               g.hw.shift, g.ch_per_group, gamma, beta, y, sc, p);
     }
 }
 
 template <typename T, bool RAGGED>
-int gn_launch(uint32_t k, bool silu, bool shared, uint32_t blocks, uint32_t threads, uint32_t shape, hipStream_t stream, const T *x,
+int gn_launch(uint32_t k, bool silu, bool shared, const GnGeometry &g, hipStream_t stream, const T *x,
               const T *chunk, T *y, const float *gamma, const float *beta, const GnScratch &sc, const GnParams &p) {
     switch (k) {
-        case 1: gn_launch_k<T, 1, RAGGED>(silu, shared, blocks, threads, shape, stream, x, chunk, y, gamma, beta, sc, p); break;
-        case 2: gn_launch_k<T, 2, RAGGED>(silu, shared, blocks, threads, shape, stream, x, chunk, y, gamma, beta, sc, p); break;
-        case 3: gn_launch_k<T, 3, RAGGED>(silu, shared, blocks, threads, shape, stream, x, chunk, y, gamma, beta, sc, p); break;
-        case 4: gn_launch_k<T, 4, RAGGED>(silu, shared, blocks, threads, shape, stream, x, chunk, y, gamma, beta, sc, p); break;
-        case 5: gn_launch_k<T, 5, RAGGED>(silu, shared, blocks, threads, shape, stream, x, chunk, y, gamma, beta, sc, p); break;
-        case 6: gn_launch_k<T, 6, RAGGED>(silu, shared, blocks, threads, shape, stream, x, chunk, y, gamma, beta, sc, p); break;
-        case 8: gn_launch_k<T, 8, RAGGED>(silu, shared, blocks, threads, shape, stream, x, chunk, y, gamma, beta, sc, p); break;
-        case 10: gn_launch_k<T, 10, RAGGED>(silu, shared, blocks, threads, shape, stream, x, chunk, y, gamma, beta, sc, p); break;
-        case 12: gn_launch_k<T, 12, RAGGED>(silu, shared, blocks, threads, shape, stream, x, chunk, y, gamma, beta, sc, p); break;
-        case 16: gn_launch_k<T, 16, RAGGED>(silu, shared, blocks, threads, shape, stream, x, chunk, y, gamma, beta, sc, p); break;
-        case 20: gn_launch_k<T, 20, RAGGED>(silu, shared, blocks, threads, shape, stream, x, chunk, y, gamma, beta, sc, p); break;
+        case 1: gn_launch_k<T, 1, RAGGED>(silu, shared, g, stream, x, chunk, y, gamma, beta, sc, p); break;
+        case 2: gn_launch_k<T, 2, RAGGED>(silu, shared, g, stream, x, chunk, y, gamma, beta, sc, p); break;
+        case 3: gn_launch_k<T, 3, RAGGED>(silu, shared, g, stream, x, chunk, y, gamma, beta, sc, p); break;
+        case 4: gn_launch_k<T, 4, RAGGED>(silu, shared, g, stream, x, chunk, y, gamma, beta, sc, p); break;
+        case 5: gn_launch_k<T, 5, RAGGED>(silu, shared, g, stream, x, chunk, y, gamma, beta, sc, p); break;
+        case 6: gn_launch_k<T, 6, RAGGED>(silu, shared, g, stream, x, chunk, y, gamma, beta, sc, p); break;
+        case 8: gn_launch_k<T, 8, RAGGED>(silu, shared, g, stream, x, chunk, y, gamma, beta, sc, p); break;
+        case 10: gn_launch_k<T, 10, RAGGED>(silu, shared, g, stream, x, chunk, y, gamma, beta, sc, p); break;
+        case 12: gn_launch_k<T, 12, RAGGED>(silu, shared, g, stream, x, chunk, y, gamma, beta, sc, p); break;
+        case 16: gn_launch_k<T, 16, RAGGED>(silu, shared, g, stream, x, chunk, y, gamma, beta, sc, p); break;
+        case 20: gn_launch_k<T, 20, RAGGED>(silu, shared, g, stream, x, chunk, y, gamma, beta, sc, p); break;
         default: return MSD_ERR_INVALID_VALUE;  // not a K the kernels are built for: a planning error
     }
     return launch_status();
@@ -1090,15 +1114,16 @@ int gn_dispatch(const void *xv, const void *chunkv, void *yv, const float *gamma
     p.vec_per_slice = d.vec_per_slice;
     p.split = split;
     p.groups = make_fast_div((uint32_t)groups);
-    p.ch_per_group = (uint32_t)cpg;
-    p.hw_vec = make_fast_div((uint32_t)(ragged ? hw : hw / EPV));
+    p.hw = (uint32_t)hw;
     p.eps = eps;
     p.inv_count = 1.0f / (float)unit_size;
     p.spin_limit = tune_spin > 0 ? (uint32_t)tune_spin : kGnSpinLimit;
     const bool shared = d.writers > 1;
     p.part_vecs = (uint32_t)((((p.vec_per_unit + d.writers - 1) / d.writers + kWave - 1) / kWave) * kWave);
-    const uint32_t shape = gn_shape_word((uint32_t)__builtin_ctz(split), (uint32_t)__builtin_ctz(d.writers),
-                                         gn_xcd_shift(chip_info(), shared, units), d.threads);
+    const GnGeometry g{(uint32_t)(units * split * d.writers), d.threads,
+                       gn_shape_word((uint32_t)__builtin_ctz(split), (uint32_t)__builtin_ctz(d.writers),
+                                     gn_xcd_shift(chip_info(), shared, units), d.threads),
+                       (uint32_t)cpg, make_fast_div((uint32_t)(ragged ? hw : hw / EPV))};
 
     if (fixed != nullptr) {
         sc = *fixed;
@@ -1106,10 +1131,9 @@ int gn_dispatch(const void *xv, const void *chunkv, void *yv, const float *gamma
         const hipError_t err = get_scratch(stream, &sc);
         if (err != hipSuccess) return (int)err;
     }
-    const uint32_t blocks = (uint32_t)(units * split * d.writers);
     if (ragged)
-        return gn_launch<T, true>(d.k, silu, shared, blocks, d.threads, shape, stream, x, chunk, y, gamma, beta, sc, p);
-    return gn_launch<T, false>(d.k, silu, shared, blocks, d.threads, shape, stream, x, chunk, y, gamma, beta, sc, p);
+        return gn_launch<T, true>(d.k, silu, shared, g, stream, x, chunk, y, gamma, beta, sc, p);
+    return gn_launch<T, false>(d.k, silu, shared, g, stream, x, chunk, y, gamma, beta, sc, p);
 }
 
 template int gn_dispatch<float>(const void *, const void *, void *, const float *, const float *,
@@ -1205,10 +1229,10 @@ int gn_tokens_unit(const GnTokUnitPlan &pl, const Chip &chip, const T *x, T *y, 
 template <typename T, int K>
 void gn_tokens_launch(uint32_t blocks, uint32_t threads, size_t lds_bytes, hipStream_t stream,
                       const T *x, T *y, const float *gamma, const float *beta, const GnScratch &sc,
-                      const GnTokParams &q, const FastDiv &pos_vecs, const FastDiv &combos) {
+                      const GnTokParams &q, uint32_t hw_vec, const FastDiv &pos_vecs, const FastDiv &combos) {
     const GnParams &p = q.base;
     launch((gn_tokens_kernel<T, K>), dim3(blocks), dim3(threads), lds_bytes, stream, x, p.vec_per_unit, p.vec_per_slice,
-           pos_vecs.mul, pos_vecs.shift, pos_vecs.d, p.hw_vec.d, combos.mul, combos.shift, combos.d, p.groups.d,
+           pos_vecs.mul, pos_vecs.shift, pos_vecs.d, hw_vec, combos.mul, combos.shift, combos.d, p.groups.d,
            gn_shape_word((uint32_t)__builtin_ctz(p.split), 0, 0, threads), y, gamma, beta, sc, q);
 }
 
@@ -1380,8 +1404,7 @@ int gn_tokens_dispatch(const void *xv, void *yv, const float *gamma, const float
     q.base.split = split;
     q.base.part_vecs = (uint32_t)nvec;
     q.base.groups = make_fast_div((uint32_t)groups);
-    q.base.ch_per_group = (uint32_t)cpg;
-    q.base.hw_vec = make_fast_div((uint32_t)hw_vec);
+    q.ch_per_group = (uint32_t)cpg;
     q.base.eps = eps;
     q.base.inv_count = 1.0f / (float)unit_size;
     q.base.spin_limit = tune_spin > 0 ? (uint32_t)tune_spin : kGnSpinLimit;
@@ -1407,16 +1430,16 @@ int gn_tokens_dispatch(const void *xv, void *yv, const float *gamma, const float
     }
     const uint32_t threads = pl.threads;
     switch (pl.k) {
-        case 1: gn_tokens_launch<T, 1>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, pos_vecs, combos); break;
-        case 2: gn_tokens_launch<T, 2>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, pos_vecs, combos); break;
-        case 3: gn_tokens_launch<T, 3>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, pos_vecs, combos); break;
-        case 4: gn_tokens_launch<T, 4>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, pos_vecs, combos); break;
-        case 5: gn_tokens_launch<T, 5>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, pos_vecs, combos); break;
-        case 6: gn_tokens_launch<T, 6>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, pos_vecs, combos); break;
-        case 8: gn_tokens_launch<T, 8>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, pos_vecs, combos); break;
-        case 10: gn_tokens_launch<T, 10>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, pos_vecs, combos); break;
-        case 12: gn_tokens_launch<T, 12>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, pos_vecs, combos); break;
-        default: gn_tokens_launch<T, 16>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, pos_vecs, combos); break;
+        case 1: gn_tokens_launch<T, 1>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, (uint32_t)hw_vec, pos_vecs, combos); break;
+        case 2: gn_tokens_launch<T, 2>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, (uint32_t)hw_vec, pos_vecs, combos); break;
+        case 3: gn_tokens_launch<T, 3>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, (uint32_t)hw_vec, pos_vecs, combos); break;
+        case 4: gn_tokens_launch<T, 4>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, (uint32_t)hw_vec, pos_vecs, combos); break;
+        case 5: gn_tokens_launch<T, 5>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, (uint32_t)hw_vec, pos_vecs, combos); break;
+        case 6: gn_tokens_launch<T, 6>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, (uint32_t)hw_vec, pos_vecs, combos); break;
+        case 8: gn_tokens_launch<T, 8>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, (uint32_t)hw_vec, pos_vecs, combos); break;
+        case 10: gn_tokens_launch<T, 10>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, (uint32_t)hw_vec, pos_vecs, combos); break;
+        case 12: gn_tokens_launch<T, 12>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, (uint32_t)hw_vec, pos_vecs, combos); break;
+        default: gn_tokens_launch<T, 16>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, (uint32_t)hw_vec, pos_vecs, combos); break;
     }
     return launch_status();
 }
