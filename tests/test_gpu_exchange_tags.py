@@ -1,0 +1,68 @@
+"""Launches of cut units one after the other on one stream's scratch, in changing numbers of slices (csrc/groupnorm.hip:
+gn_exchange): every launch finds its slices agreed on the tag, so none of them gives up waiting, and each result is that of
+the first launch with its number of slices, bit for bit, eagerly and from a replayed graph.  The tokens' kernel shares the
+words."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+SPLITS = [2, 64, 4, 8, 2, 16, 32, 4, 64, 2]
+
+
+@pytest.mark.parametrize("batch,channels,side", [(1, 320, 64), (2, 64, 64)])
+@pytest.mark.parametrize("half", [False, True], ids=["f32", "f16"])
+def test_launches_in_changing_slices_agree_on_the_tag(msd, orc, cuda, half, batch, channels, side):
+    import torch
+    lib = msd.load_library()
+    x = torch.from_numpy(orc.normal((batch, channels, side, side), seed=channels, sigma=2.0)).to(cuda)
+    x = x.half() if half else x
+    gamma, beta = (torch.from_numpy(orc.normal((channels,), seed=s)).to(cuda) for s in (1, 2))
+    out = [torch.empty_like(x) for _ in SPLITS]
+
+    def launches():
+        for split, y in zip(SPLITS, out):
+            torch.add(x, 0, out=y)
+            assert lib.msd_set_tuning(msd.TUNE_GN_SPLIT, split) == 0
+            msd.groupnorm(y, gamma, beta, 32, 1e-5, True, out=y)
+
+    try:
+        assert lib.msd_set_tuning(msd.TUNE_GN_WRITERS, 1) == 0
+        stream = torch.cuda.Stream()
+        stream.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(stream):
+            msd.init()
+            msd.gn_fallbacks(reset=True)
+            launches()
+            assert lib.msd_set_tuning(msd.TUNE_GN_SPLIT, 4) == 0
+            tokens = msd.groupnorm_tokens(x, gamma, beta, 32, 1e-5)
+            first = [y.clone() for y in out]
+            launches()
+        torch.cuda.synchronize()
+        of = {}
+        for split, a, b in zip(SPLITS, first, out):
+            assert torch.equal(a, b) and torch.equal(of.setdefault(split, a), a), split
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            launches()
+        assert lib.msd_set_tuning(msd.TUNE_GN_SPLIT, 4) == 0
+        for _ in range(3):
+            for y in out:
+                y.zero_()
+            torch.cuda.synchronize()
+            with torch.cuda.stream(stream):
+                graph.replay()
+                launches_between = msd.groupnorm_tokens(x, gamma, beta, 32, 1e-5)
+            torch.cuda.synchronize()
+            assert all(torch.equal(a, b) for a, b in zip(first, out)) and torch.equal(tokens, launches_between)
+        with torch.cuda.stream(stream):
+            assert msd.gn_fallbacks() == 0
+    finally:
+        lib.msd_set_tuning(msd.TUNE_GN_SPLIT, 0)
+        lib.msd_set_tuning(msd.TUNE_GN_WRITERS, 0)
+    # against the oracle, within what another order of the sums gives (tests of the kernel itself: test_gpu_parity.py)
+    xin = x.float().cpu().numpy()
+    ref = orc.groupnorm(xin, gamma.cpu().numpy(), beta.cpu().numpy(), 32, 1e-5, silu=True)
+    got = first[0].float().cpu().numpy()
+    bound = (2.0 ** -10 if half else 0.0) * np.abs(ref) + 1e-5 * np.maximum(1.0, np.abs(ref))  # a last bit of fp16, and 1e-5
+    assert np.all(np.abs(got - ref) <= bound)
