@@ -132,13 +132,12 @@ int msd_groupnorm(const void *x, void *y, const float *gamma, const float *beta,
  * loops, harnesses that forbid hipMalloc): same arguments, same kernels, same result bit for
  * bit (while msd_gn_fallbacks() stays 0, see msd_groupnorm; hw of no whole 16-byte vectors: as
  * msd_groupnorm outside a capture, inside one too), but the workgroups' exchange area is a fixed
- * 1 MiB array inside the library's code object instead of a per-stream allocation, so the call never allocates or frees (its first
+ * array of 1.1 MiB inside the library's code object instead of a per-stream allocation, so the call never allocates or frees (its first
  * call on a device looks the array's address up; msd_init does that ahead of time).  Limit:
  * batch * groups <= 1024, otherwise MSD_ERR_SCRATCH_LIMIT.  Every stream of a device shares
- * the one array: calls that overlap in time on one GPU race (their results are undefined, and
- * later calls may take a millisecond: the array's words then no longer agree on the launch, and
- * workgroups give up waiting for each other, see msd_gn_fallbacks);
- * calls ordered by a stream or by events are fine, and nothing needs clearing between them.
+ * the one array: calls that overlap in time on one GPU race (their results are undefined);
+ * calls ordered by a stream or by events are fine, those after an overlap too, and nothing
+ * needs clearing between them.
  * Each GPU holds its array until the process ends.  No counterpart in the reference.
  */
 int msd_groupnorm_noalloc(const void *x, void *y, const float *gamma, const float *beta,

@@ -25,25 +25,27 @@ std::mutex g_scratch_mutex;
 std::unordered_map<ScratchKey, GnScratch, ScratchKeyHash> g_scratch;
 
 // Scratch for `units` (sample, group) pairs, carved out of one block:
-// [slot_mean | slot_m2 | fallbacks] and, in an allocated one, [partials], every part 256-byte aligned.
+// [slot_mean | slot_m2 | counts | fallbacks] and, in an allocated one, [partials], every part 256-byte aligned.
 constexpr size_t slot_bytes(size_t units) { return sizeof(unsigned long long) * units * kGnMaxSplit; }
 constexpr size_t partial_bytes(size_t units) { return sizeof(float2) * units * kGnStatSlices; }
-constexpr size_t exchange_bytes(size_t units) { return 2 * slot_bytes(units) + 256; }
+constexpr size_t count_bytes(size_t units) { return sizeof(unsigned long long) * units * kGnCountStride; }
+constexpr size_t exchange_bytes(size_t units) { return 2 * slot_bytes(units) + count_bytes(units) + 256; }
 constexpr size_t kAllocatedBytes = exchange_bytes(kGnMaxUnits) + partial_bytes(kGnMaxUnits);
 
 GnScratch carve(char *base, size_t units, bool with_partials) {
     GnScratch s;
     s.slot_mean = reinterpret_cast<unsigned long long *>(base);
     s.slot_m2 = reinterpret_cast<unsigned long long *>(base + slot_bytes(units));
-    s.fallbacks = reinterpret_cast<uint32_t *>(base + 2 * slot_bytes(units));
+    s.counts = reinterpret_cast<unsigned long long *>(base + 2 * slot_bytes(units));
+    s.fallbacks = reinterpret_cast<uint32_t *>(base + 2 * slot_bytes(units) + count_bytes(units));
     s.partials = with_partials ? reinterpret_cast<float2 *>(base + exchange_bytes(units)) : nullptr;
     s.units = (uint32_t)units;
     return s;
 }
 
 // Scratch of the entry point that allocates nothing: part of the code object, one copy per
-// device, zero when the module is loaded (tags and the counter start at zero and
-// are never reset: see groupnorm.hip).  In host code this name is only a handle for
+// device, zero when the module is loaded (tags, counts and the counter start at zero
+// and are never reset: see groupnorm.hip).  In host code this name is only a handle for
 // hipGetSymbolAddress; kernels get the device address that call returns.
 constexpr uint32_t kStaticUnits = 1024;
 static __device__ __align__(256) unsigned char scratch[exchange_bytes(kStaticUnits)];
@@ -71,7 +73,7 @@ hipError_t get_scratch(hipStream_t stream, GnScratch *out, bool clear_on_stream)
     char *base = nullptr;
     err = hipMalloc(reinterpret_cast<void **>(&base), kAllocatedBytes);
     if (err != hipSuccess) return err;
-    // tags and the counter start at zero
+    // tags, counts and the counter start at zero
     if (clear_on_stream) {
         err = hipMemsetAsync(base, 0, kAllocatedBytes, stream);
     } else {

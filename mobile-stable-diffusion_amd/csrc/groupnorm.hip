@@ -10,9 +10,9 @@
 //      over the packed registers (DPP wavefront reduction, one LDS slot per wavefront), with
 //      a second, centred pass when the mean is large against the spread;
 //   3. split > 1: slices publish (mean, M2) as two tagged 64-bit words, poll
-//      their siblings' words, and merge with Chan's formula.  The tag is one
-//      more than that of the slice's own word, read at kernel start, so nothing
-//      is reset between launches and a replayed graph works.  All traffic is
+//      their siblings' words, and merge with Chan's formula.  The tag comes from
+//      a count per unit that every slice advances by its share, so nothing is
+//      reset between launches and a replayed graph works.  All traffic is
 //      relaxed agent-scope atomics: no cache flushes.
 //   4. y = fma(x - mean, rstd * gamma[c], beta[c]) (the mean folded into the offset when it
 //      is small), optional SiLU, packed store.
@@ -93,28 +93,40 @@ __device__ __forceinline__ unsigned long long tagged(uint32_t tag, float v) {
     return ((unsigned long long)tag << 32) | (unsigned long long)__float_as_uint(v);
 }
 
-// The tag of the last launch on this unit: its own first word, which only this slice writes in this launch.
-__device__ __forceinline__ uint32_t gn_exchange_last_tag(const GnScratch &scratch, uint32_t unit, uint32_t slice) {
-    const unsigned long long *own = scratch.slot_mean + (size_t)unit * kGnMaxSplit + slice;
-    return __hip_atomic_load(reinterpret_cast<const uint32_t *>(own) + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// What a launch's tag on a unit comes from, the same for all its slices: by one lane at kernel start each slice adds its share of
+// kGnMaxSplit to the unit's count, and what it finds there, divided by kGnMaxSplit, is the number of launches before.  The shares
+// of a launch sum to exactly kGnMaxSplit, whatever its split, and a slice that has not added its own finds less than that on top,
+// however late it starts; nothing is left to do at the end.  After launches that overlapped on one scratch, which the rules
+// forbid, the count is a multiple of kGnMaxSplit again and no tag that they left in the slots is above its launches: those
+// that follow in order are not affected.
+// (The index is a vector register to the compiler, which otherwise adds for all lanes at once and waits for the answer on the spot;
+// and the answer stays whole until the statistics are there: with one half of it unused the next loads waited for its register.)
+// us per launch, in place, a launch count that the last slice to finish advances / a tag per slice kept in its own slot, which
+// an overlap could set apart for good / so: fp16 320 channels at 64 x 64 batch 2 5.97 / 4.91 / 4.92, 640 7.12 / 6.37 / 6.35, fp32 320
+// batch 1 5.83 / 5.01 / 5.02, 960 batch 2 11.72 / 10.79 / 10.82; sixteen units' counts in a line: fp16 960 batch 1 5.70 -> 6.25.
+__device__ __forceinline__ unsigned long long gn_exchange_enter(const GnExchange &scratch, const GnParams &p, uint32_t unit) {
+    uint32_t index = unit * kGnCountStride;
+    asm volatile("" : "+v"(index));
+    const unsigned long long share = kGnMaxSplit >> __builtin_ctz(p.split);
+    return __hip_atomic_fetch_add(scratch.counts + index, share, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Merges the slices of one unit.  Called by every lane of the workgroup with the slice's
-// (mean, M2); `last_tag` is what lane 0 read with gn_exchange_last_tag at kernel start.  On return
+// (mean, M2); `count` is what lane 0 got from gn_exchange_enter at kernel start.  On return
 // stats[0] = mean and stats[1] = 1/sqrt(var + eps) of the whole unit, in LDS, after a barrier.
 // Slice l covers vectors [l * vec_per_slice, min(vec_per_unit, (l + 1) * vec_per_slice)).
 // `read(l, i)` returns vector i of slice l as the statistics see it (after the optional addend);
 // it is only used when slice l has not published within the poll limit.
 template <typename T, typename Reader>
-__device__ __forceinline__ void gn_exchange(const GnScratch &scratch, const GnParams &p, uint32_t unit,
-                                            uint32_t slice, uint32_t last_tag, float slice_mean,
+__device__ __forceinline__ void gn_exchange(const GnExchange &scratch, const GnParams &p, uint32_t unit,
+                                            uint32_t slice, unsigned long long count, float slice_mean,
                                             float slice_m2, float *stats, Reader read) {
     constexpr int EPV = Store<T>::EPV;
     const uint32_t tid = threadIdx.x;
     unsigned long long *slot_mean = scratch.slot_mean + (size_t)unit * kGnMaxSplit;
     unsigned long long *slot_m2 = scratch.slot_m2 + (size_t)unit * kGnMaxSplit;
-    if (tid < kWave) {  // wavefront 0 owns the exchange; lane 0 holds the last tag
-        const uint32_t tag = (uint32_t)__builtin_amdgcn_readfirstlane((int)last_tag) + 1u;
+    if (tid < kWave) {  // wavefront 0 owns the exchange; lane 0 holds the count
+        const uint32_t tag = (uint32_t)__builtin_amdgcn_readfirstlane((int)(count / kGnMaxSplit)) + 1u;
         if (tid == 0) {
             __hip_atomic_store(slot_mean + slice, tagged(tag, slice_mean), __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_AGENT);
@@ -200,20 +212,6 @@ __device__ __forceinline__ void gn_exchange(const GnScratch &scratch, const GnPa
         }
     }
     __syncthreads();
-}
-
-// Behind the barrier that ends gn_exchange, by wavefront 0: the first words that no slice of this launch uses get its tag
-// too, slot l from slice l % split, so that all slots of a unit carry the same one between launches, whatever the next
-// launch's split.  Nothing waits for these stores.  (A launch count per unit that the last slice advances, found with an
-// atomic counter, ended the kernel a memory round trip later.  us per launch, so and with the tags, in place, four slices: fp16
-// 320 channels at 64 x 64 batch 2 5.76 -> 5.20, with the addend 5.97 -> 5.62, fp32 batch 1 5.58 -> 5.24.)
-__device__ __forceinline__ void gn_exchange_advance(const GnScratch &scratch, const GnParams &p, uint32_t unit, uint32_t slice,
-                                                    uint32_t last_tag) {
-    const uint32_t tag = (uint32_t)__builtin_amdgcn_readfirstlane((int)last_tag) + 1u;
-    const uint32_t l = slice + (threadIdx.x + 1) * p.split;
-    if (l < kGnMaxSplit)
-        __hip_atomic_store(scratch.slot_mean + (size_t)unit * kGnMaxSplit + l, tagged(tag, 0.0f), __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Sum and sum of squares of a packed vector, accumulated in float32.  Half storage uses
@@ -341,7 +339,7 @@ __device__ __forceinline__ GnStraddle gn_straddle(uint32_t v, const FastDiv &hw)
 template <typename T, int K, bool SILU, bool FULL, bool SHARED, bool RAGGED>
 __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
                                         const float *__restrict__ gamma,
-                                        const float *__restrict__ beta, const GnScratch &scratch,
+                                        const float *__restrict__ beta, const GnExchange &scratch,
                                         const GnParams &p, uint32_t nt, uint32_t vec_per_unit, uint32_t unit, uint32_t slice,
                                         uint32_t part, uint32_t v_begin, uint32_t v_end, uint32_t ch_per_group,
                                         const FastDiv &hw_vec, float *red, float *stats, float2 *aff) {
@@ -415,8 +413,8 @@ __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("" : "+s"(unit), "+s"(part));
     u32x4 *yout = reinterpret_cast<u32x4 *>(y) + (size_t)unit * vec_per_unit;
-    uint32_t last_tag = 0;  // (arrives right behind the data)
-    if (!SHARED && p.split > 1 && tid == 0) last_tag = gn_exchange_last_tag(scratch, unit, slice);
+    unsigned long long count = 0;  // (arrives right behind the data)
+    if (!SHARED && p.split > 1 && tid == 0) count = gn_exchange_enter(scratch, p, unit);
     const uint32_t ch0 = (unit - fast_div(unit, p.groups) * p.groups.d) * ch_per_group;
     // per-vector channel affine.  Up to six vectors per lane: fetched into registers up front,
     // while the data is in flight.  More: the group's gamma and beta go to LDS once (they are
@@ -468,10 +466,9 @@ __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
             if (chunk != nullptr) r = plus(r, v, addend_of(v));
             return r;
         };
-        gn_exchange<T>(scratch, p, unit, slice, last_tag, slice_mean, slice_m2, stats, read);
+        gn_exchange<T>(scratch, p, unit, slice, count, slice_mean, slice_m2, stats, read);
         mean = stats[0];
         rstd = stats[1];
-        if (tid < kWave) gn_exchange_advance(scratch, p, unit, slice, last_tag);
     }
 
     // ---- normalise from registers, per-channel affine, optional SiLU.  When the unit's mean is
@@ -558,7 +555,7 @@ template <typename T, int K, bool SILU, bool SHARED, bool RAGGED>
 __global__ __launch_bounds__(kGnMaxThreads, (K <= (sizeof(T) == 2 ? 5 : 4) ? 8 : 4)) void gn_slice_kernel(
     const T *x, uint32_t vec_per_unit, uint32_t vec_per_slice, uint32_t shape, const T *chunk, uint32_t hw_mul,
     uint32_t hw_shift, uint32_t ch_per_group, const float *__restrict__ gamma, const float *__restrict__ beta, T *y,
-    GnScratch scratch, GnParams p) {
+    GnExchange scratch, GnParams p) {
     __shared__ float red[kGnRedSlots];
     __shared__ float stats[2];
     __shared__ float2 aff[!RAGGED && K <= kGnPrefetchAffineK ? 1 : kGnLdsChannels];  // (gamma, beta) of the group's channels
@@ -645,7 +642,7 @@ template <typename T, int K>
 __global__ __launch_bounds__(kGnMaxThreads) void gn_tokens_kernel(
     const T *__restrict__ x, uint32_t vec_per_unit, uint32_t nvec, uint32_t pos_mul, uint32_t pos_shift, uint32_t pvs,
     uint32_t hw_vec, uint32_t combos_mul, uint32_t combos_shift, uint32_t combos, uint32_t groups, uint32_t shape,
-    T *__restrict__ y, const float *__restrict__ gamma, const float *__restrict__ beta, GnScratch scratch, GnTokParams q) {
+    T *__restrict__ y, const float *__restrict__ gamma, const float *__restrict__ beta, GnExchange scratch, GnTokParams q) {
     constexpr int EPV = Store<T>::EPV;
     extern __shared__ u32x4 lds_vec[];
     __shared__ float red[kGnRedSlots];
@@ -681,8 +678,8 @@ __global__ __launch_bounds__(kGnMaxThreads) void gn_tokens_kernel(
         for (int i = 0; i < 4; i++) raw[k][i] = have ? raw[k][i] : 0u;
     }
     __builtin_amdgcn_sched_barrier(0);  // (what follows waits for the arguments in memory)
-    uint32_t last_tag = 0;
-    if (p.split > 1 && tid == 0) last_tag = gn_exchange_last_tag(scratch, unit, slice);
+    unsigned long long count = 0;
+    if (p.split > 1 && tid == 0) count = gn_exchange_enter(scratch, p, unit);
     const uint32_t ch0 = group * q.ch_per_group;
 
     float slice_mean, slice_m2;
@@ -698,10 +695,9 @@ __global__ __launch_bounds__(kGnMaxThreads) void gn_tokens_kernel(
             const uint32_t c = fast_div(i, pos_vecs);
             return xin[(size_t)c * hw_vec + l * pvs + (i - c * pvs)];
         };
-        gn_exchange<T>(scratch, p, unit, slice, last_tag, slice_mean, slice_m2, stats, read);
+        gn_exchange<T>(scratch, p, unit, slice, count, slice_mean, slice_m2, stats, read);
         mean = stats[0];
         rstd = stats[1];
-        if (tid < kWave) gn_exchange_advance(scratch, p, unit, slice, last_tag);
     }
 
     // ---- normalise into LDS as [channel][position]

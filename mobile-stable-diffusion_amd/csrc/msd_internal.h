@@ -46,6 +46,7 @@ inline int launch_status() {
 
 // ---- GroupNorm scratch: what workgroups sharing one (sample, group) exchange ----
 constexpr uint32_t kGnMaxSplit = 64;    // workgroups per unit (one wavefront reads all slots)
+constexpr uint32_t kGnCountStride = 16; // 64-bit words from one unit's count to the next: a cache line each
 constexpr uint32_t kGnMaxUnits = 8192;  // units that own scratch slots; larger launches never split
 constexpr uint32_t kGnStatSlices = 16;  // slices per unit of the token-major norm's statistics launch
 
@@ -57,10 +58,13 @@ constexpr int kGnSharedMaxK = 10;       // kernels with several writers per unit
 constexpr int kGnPrefetchAffineK = 6;   // vectors per lane up to which gamma / beta are kept in registers
 constexpr uint32_t kGnLdsChannels = 1024;  // channels per group the LDS copy of gamma / beta has room for
 
-struct GnScratch {
-    unsigned long long *slot_mean;  // [kGnMaxUnits][kGnMaxSplit]  (tag << 32) | float bits; one tag per unit between launches
+struct GnExchange {  // (what kernels are given)
+    unsigned long long *slot_mean;  // [kGnMaxUnits][kGnMaxSplit]  (tag << 32) | float bits
     unsigned long long *slot_m2;    // [kGnMaxUnits][kGnMaxSplit]
+    unsigned long long *counts;     // [kGnMaxUnits][kGnCountStride] kGnMaxSplit for every launch that cut the unit
     uint32_t *fallbacks;            // [1] slices that stopped waiting and computed a sibling's statistics themselves
+};
+struct GnScratch : GnExchange {
     float2 *partials;               // [kGnMaxUnits][kGnStatSlices] (mean, M2) for one pair of launches; null in the fixed scratch
     uint32_t units;                 // units the arrays above have room for
 };

@@ -1,20 +1,16 @@
 """CPU model of the exchange between the workgroups ("slices") that share one GroupNorm unit
 (csrc/groupnorm.hip: gn_exchange), run over randomised interleavings.
 
-What a slice does, and what the model replays one memory operation at a time (steps 1 and 6 with a launch count per unit and a
-counter of finished slices; the kernels have neither since the tags are kept in the slots themselves, which
-test_exchange_tags_model.py replays on top of this model):
+What a slice does, and what the model replays one memory operation at a time:
 
-  1. read the unit's launch count `epoch` (once, at kernel start); tag = epoch + 1
+  1. add its share, MAX_SPLIT / split, to the unit's count (once, at kernel start); tag = what it found / MAX_SPLIT + 1
   2. publish (tag, mean) and (tag, M2) of its own part as two separate 64-bit words
   3. lane l polls slice l's two words until both carry the tag, at most `spin_limit` times -
      without limit for the slice's OWN words, which arrive without anybody's help; a sibling
      that has not published by then is computed from the sibling's part of the INPUT (two
      passes, all of whose loads have returned before the next step), after which its words are
      read once more and win if they have arrived
-  4. merge all slices (Chan), then fetch_add(done) (its old value is used in step 6)
-  5. only now store the output over its own part (the call may be in place)
-  6. the slice whose fetch_add returned split - 1 stores done = 0, epoch = tag
+  4. merge all slices (Chan); only now store the output over its own part (the call may be in place)
 
 All of it is relaxed atomics: stores become visible to the other slices after arbitrary delays
 and in any order across addresses.  One thing the protocol leans on is modelled as a fact of
@@ -25,7 +21,7 @@ issues its output stores only after it has read both words back.
 Checked over many random schedules, several consecutive launches per unit and changing split
 factors: a word of an earlier launch is never accepted, every slice ends up with the statistics
 of exactly this launch's data whichever way it obtained them, an overwritten input is never
-used, and the counters return to their rest state.  The reference has no counterpart (it runs
+used, and the count has advanced by exactly MAX_SPLIT.  The reference has no counterpart (it runs
 three ordered kernels, M/nn/GroupNorm.cpp:105-145).
 """
 import random
@@ -41,8 +37,7 @@ class Unit:
     def __init__(self):
         self.slot_mean = [(0, None)] * MAX_SPLIT  # (tag, value)
         self.slot_m2 = [(0, None)] * MAX_SPLIT
-        self.epoch = 0
-        self.done = 0
+        self.count = 0
         self.fallbacks = 0
 
 
@@ -67,10 +62,6 @@ class Launch:
             u.slot_mean[index] = value
         elif kind == "m2":
             u.slot_m2[index] = value
-        elif kind == "done":
-            u.done = value
-        elif kind == "epoch":
-            u.epoch = value
         elif kind == "output":
             self.overwritten[index] = True
 
@@ -88,9 +79,9 @@ class Launch:
     def slice_program(self, s):
         """Generator: one yield per memory operation of slice s."""
         u = self.unit
-        epoch = u.epoch                       # 1. (all stores of earlier launches are visible)
+        tag = u.count // MAX_SPLIT + 1        # 1. an atomic at memory: immediate
+        u.count += MAX_SPLIT // self.split
         yield
-        tag = epoch + 1
         mean, m2 = self.truth[s]
         self.store(s, "mean", s, (tag, mean))  # 2.
         yield
@@ -122,16 +113,8 @@ class Launch:
                     u.fallbacks += 1
                 waiting.remove(l)
         self.accepted[s] = got
-        old = u.done                          # 4. fetch_add is atomic at memory: immediate
-        u.done = old + 1
+        self.store(s, "output", s, True)      # 4.
         yield
-        self.store(s, "output", s, True)      # 5.
-        yield
-        if old == self.split - 1:             # 6.
-            self.store(s, "done", 0, 0)
-            yield
-            self.store(s, "epoch", 0, tag)
-            yield
         self.finished[s] = True
 
     def run(self, starve=None):
@@ -167,7 +150,7 @@ def test_random_interleavings_never_accept_a_stale_word(seed):
     rng = random.Random(seed)
     unit = Unit()
     launch_id = 0
-    expected_epoch = 0
+    launches = 0
     for _ in range(12):  # consecutive launches on the same unit (same stream: ordered)
         split = rng.choice([1, 2, 2, 4, 4, 8, 16, 64])
         launch_id += 1
@@ -176,11 +159,9 @@ def test_random_interleavings_never_accept_a_stale_word(seed):
         spin_limit = rng.choice([1, 1, 2, 5, 50, 10 ** 9])
         starve = rng.randrange(split) if rng.random() < 0.5 and spin_limit < 10 ** 9 else None
         Launch(unit, split, launch_id, rng, spin_limit).run(starve)
-        expected_epoch += 1
+        launches += 1
         # rest state: nothing left to reset before the next launch (a replayed graph relies on it)
-        assert unit.done == 0
-        assert unit.epoch == expected_epoch
-    assert unit.epoch == expected_epoch
+        assert unit.count == launches * MAX_SPLIT
 
 
 def test_patient_slices_never_fall_back_and_impatient_ones_do():
@@ -204,4 +185,4 @@ def test_a_different_split_on_the_same_unit_sees_only_its_own_tags():
     Launch(unit, 2, 2, rng, 3).run()
     assert [t for t, _ in unit.slot_mean[:8]] == [2, 2, 1, 1, 1, 1, 1, 1]
     Launch(unit, 8, 3, rng, 2).run(starve=5)
-    assert unit.epoch == 3 and unit.done == 0
+    assert unit.count == 3 * MAX_SPLIT

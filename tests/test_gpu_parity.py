@@ -658,7 +658,7 @@ def test_config5_timesteps_feed_embedding_bit_exact_integers(msd, orc, cuda):
 
 # ----------------------------------------------------------------- launch machinery
 def test_groupnorm_graph_replay_matches_eager(msd, orc, cuda):
-    """The cross-workgroup exchange keeps per-unit launch counts in device memory, so a
+    """The cross-workgroup exchange keeps a count per unit in device memory, so a
     captured graph must give on every replay what the eager launch gives."""
     torch = _torch()
     stream = torch.cuda.Stream()
