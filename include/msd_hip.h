@@ -48,7 +48,8 @@ const char *msd_error_string(int code);
  * stream capture.  A graph captured on a stream keeps using that stream's
  * scratch: GroupNorm launches that share scratch must not run concurrently
  * (do not replay such a graph on a second stream while the first is busy with
- * GroupNorms, nor two graphs captured on one stream at the same time).  Channels of no
+ * GroupNorms, nor two graphs captured on one stream at the same time: their results are
+ * undefined; those of launches that follow in order are not).  Channels of no
  * whole 16-byte vectors are recorded without it: such a GroupNorm works on whole units then,
  * or through the general kernel, and may differ from the same call outside a capture in the
  * last bit, as it may where no scratch can be allocated.  Also looks up the device address of

@@ -23,7 +23,7 @@
 // placed on) and does step 4 for its own part of the unit.  No step 3, nothing waits.
 //
 // Workgroups of one unit have adjacent block ids, so a waiter's siblings are
-// normally dispatched together with it.  Nothing depends on that: a wait is
+// normally dispatched together with it.  Nothing depends on that: every wait is
 // bounded (about a millisecond of polls), and a slice whose sibling has not
 // published by then computes that sibling's statistics itself from the
 // sibling's part of the input, which no workgroup overwrites before it has
@@ -41,6 +41,10 @@ namespace msd {
 namespace {
 
 constexpr uint32_t kGnSpinLimit = 2048;  // default poll limit: about half a microsecond per poll
+// Polls that a slice waits for its own words, however short the limit for its siblings' is: some 30 ms, far more than its stores
+// take.  Only another launch that overlaps this one on the same scratch, against the rules, can write over them before they are
+// read; the slice then gives up on them as on a sibling's, and the kernel ends.
+constexpr uint32_t kGnOwnSpinLimit = 65536;
 constexpr int kGenericThreads = 256;
 constexpr int kGnRedRow = 16;                // partial sums of a workgroup, one per wavefront: a row of lanes
 constexpr int kGnRedSlots = 3 * kGnRedRow;   // sums, sums of squares, sums about the mean
@@ -139,9 +143,9 @@ __device__ __forceinline__ void gn_exchange(const GnExchange &scratch, const GnP
         if (tid < p.split) {
             unsigned long long wm, wq;
             uint32_t polls = 0;
-            // A slice never gives up on its own words: they arrive without anybody's help, and
+            // A slice does not give up on its own words: they arrive without anybody's help, and
             // having read them back is what lets it store output (see below).
-            const uint32_t limit = tid == slice ? 0xFFFFFFFFu : p.spin_limit;
+            const uint32_t limit = tid == slice ? max(kGnOwnSpinLimit, p.spin_limit) : p.spin_limit;
             do {
                 wm = __hip_atomic_load(slot_mean + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 wq = __hip_atomic_load(slot_m2 + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

@@ -6,8 +6,8 @@ What a slice does, and what the model replays one memory operation at a time:
   1. add its share, MAX_SPLIT / split, to the unit's count (once, at kernel start); tag = what it found / MAX_SPLIT + 1
   2. publish (tag, mean) and (tag, M2) of its own part as two separate 64-bit words
   3. lane l polls slice l's two words until both carry the tag, at most `spin_limit` times -
-     without limit for the slice's OWN words, which arrive without anybody's help; a sibling
-     that has not published by then is computed from the sibling's part of the INPUT (two
+     `own_limit` times, far longer than its stores take, for the slice's OWN words, which arrive
+     without anybody's help; a sibling that has not published by then is computed from the sibling's part of the INPUT (two
      passes, all of whose loads have returned before the next step), after which its words are
      read once more and win if they have arrived
   4. merge all slices (Chan); only now store the output over its own part (the call may be in place)
@@ -21,10 +21,14 @@ issues its output stores only after it has read both words back.
 Checked over many random schedules, several consecutive launches per unit and changing split
 factors: a word of an earlier launch is never accepted, every slice ends up with the statistics
 of exactly this launch's data whichever way it obtained them, an overwritten input is never
-used, and the count has advanced by exactly MAX_SPLIT.  The reference has no counterpart (it runs
+used, and the count has advanced by exactly MAX_SPLIT.  And for launches that overlap on one unit,
+which the header forbids and which may compute anything: all of them end, and what follows them in
+order is right again.  The reference has no counterpart (it runs
 three ordered kernels, M/nn/GroupNorm.cpp:105-145).
 """
+import os
 import random
+import re
 
 import pytest
 
@@ -42,8 +46,10 @@ class Unit:
 
 
 class Launch:
-    def __init__(self, unit, split, launch_id, rng, spin_limit):
+    def __init__(self, unit, split, launch_id, rng, spin_limit, own_limit=10 ** 9, alone=True):
         self.unit, self.split, self.rng, self.spin_limit = unit, split, rng, spin_limit
+        self.own_limit = own_limit
+        self.alone = alone                      # no other launch on this unit: the results are promised
         # this launch's data: the true (mean, M2) of every slice, unlike any other launch's
         self.truth = [(launch_id * 1000 + s + 0.25, launch_id * 1000 + s + 0.75) for s in range(split)]
         self.overwritten = [False] * split      # slice s has stored output over its input
@@ -99,7 +105,8 @@ class Launch:
                 waiting.remove(l)
                 continue
             polls[l] += 1
-            if l != s and polls[l] >= self.spin_limit:   # give up on sibling l: compute it from its input
+            if polls[l] >= (max(self.own_limit, self.spin_limit) if l == s else self.spin_limit):
+                # give up on slice l: compute it from its input
                 clean = not self.overwritten[l]
                 yield                         # (the two passes over the sibling's input)
                 clean = clean and not self.overwritten[l]
@@ -108,7 +115,7 @@ class Launch:
                 if wm[0] == tag and wq[0] == tag:
                     got[l] = (wm[1], wq[1], "published late")
                 else:
-                    assert clean, "slice %d used input of slice %d that was already overwritten" % (s, l)
+                    assert clean or not self.alone, "slice %d used input of slice %d that was already overwritten" % (s, l)
                     got[l] = (self.truth[l][0], self.truth[l][1], "recomputed")
                     u.fallbacks += 1
                 waiting.remove(l)
@@ -120,29 +127,36 @@ class Launch:
     def run(self, starve=None):
         """Random schedule.  `starve`: a slice that is not dispatched until all others are stuck
         waiting or finished (what another stream filling the GPU can do)."""
-        programs = {s: self.slice_program(s) for s in range(self.split)}
-        steps = 0
-        while programs or self.pending:
-            steps += 1
-            assert steps < 200000, "schedule does not terminate"
-            runnable = [s for s in programs if s != starve]
-            if starve in programs and (not runnable or self.rng.random() < 0.002):
-                runnable.append(starve)  # dispatched at last (or by chance)
-            can_commit = self.committable()
-            if can_commit and (not runnable or self.rng.random() < 0.4):
-                self.commit_one(self.rng.choice(can_commit))
-                continue
-            s = self.rng.choice(runnable)
-            try:
-                next(programs[s])
-            except StopIteration:
-                del programs[s]
+        run_together([self], self.rng, starve)
         # every slice holds this launch's statistics of every sibling
         for s in range(self.split):
             assert set(self.accepted[s]) == set(range(self.split))
             for l, (mean, m2, how) in self.accepted[s].items():
                 assert (mean, m2) == self.truth[l], "slice %d took %r for slice %d (%s)" % (s, (mean, m2), l, how)
         assert all(self.finished) and all(self.overwritten)
+
+
+def run_together(launches, rng, starve=None):
+    """The slices of all `launches` in one random schedule (`starve`: a slice of the first)."""
+    programs = {(i, s): launch.slice_program(s) for i, launch in enumerate(launches) for s in range(launch.split)}
+    late = (0, starve)
+    steps = 0
+    while programs or any(launch.pending for launch in launches):
+        steps += 1
+        assert steps < 200000, "schedule does not terminate"
+        runnable = [key for key in programs if key != late]
+        if late in programs and (not runnable or rng.random() < 0.002):
+            runnable.append(late)  # dispatched at last (or by chance)
+        can_commit = [(launch, i) for launch in launches for i in launch.committable()]
+        if can_commit and (not runnable or rng.random() < 0.4):
+            launch, i = rng.choice(can_commit)
+            launch.commit_one(i)
+            continue
+        key = rng.choice(runnable)
+        try:
+            next(programs[key])
+        except StopIteration:
+            del programs[key]
 
 
 @pytest.mark.parametrize("seed", range(40))
@@ -186,3 +200,31 @@ def test_a_different_split_on_the_same_unit_sees_only_its_own_tags():
     assert [t for t, _ in unit.slot_mean[:8]] == [2, 2, 1, 1, 1, 1, 1, 1]
     Launch(unit, 8, 3, rng, 2).run(starve=5)
     assert unit.count == 3 * MAX_SPLIT
+
+
+@pytest.mark.parametrize("splits", [(2, 2), (4, 4), (4, 2), (2, 8), (4, 4, 4), (64, 2)])
+@pytest.mark.parametrize("seed", range(15))
+def test_overlapping_launches_end_and_leave_nothing_behind(seed, splits):
+    """Words are written over by another launch before their own slice has read them, siblings of one launch find different
+    counts: whatever they compute, every slice ends, and launches that follow in order are right."""
+    rng = random.Random(seed)
+    unit = Unit()
+    Launch(unit, splits[0], 1, rng, 10 ** 9).run()
+    run_together([Launch(unit, split, 2 + i, rng, spin_limit=20, own_limit=100, alone=False) for i, split in enumerate(splits)], rng)
+    assert unit.count == (1 + len(splits)) * MAX_SPLIT
+    gave_up = unit.fallbacks
+    for launch in range(10, 16):
+        Launch(unit, rng.choice(splits), launch, rng, 10 ** 9).run()  # asserts the statistics of every slice
+    assert unit.fallbacks == gave_up
+
+
+def test_every_wait_of_the_kernels_is_bounded():
+    """The limits as csrc/groupnorm.hip has them: half a microsecond a poll, and the wait of a slice for its own words is
+    longer than that for its siblings' and well below a second."""
+    with open(os.path.join(os.path.dirname(__file__), os.pardir, "mobile-stable-diffusion_amd", "csrc", "groupnorm.hip")) as f:
+        source = f.read()
+    limits = {name: int(value) for name, value in re.findall(r"constexpr uint32_t (kGn\w*SpinLimit) = (\w+);", source)}
+    assert set(limits) == {"kGnSpinLimit", "kGnOwnSpinLimit"}
+    assert limits["kGnSpinLimit"] < limits["kGnOwnSpinLimit"] <= 2 ** 18
+    assert "0xFFFFFFFF" not in source
+    assert "limit = tid == slice ? max(kGnOwnSpinLimit, p.spin_limit) : p.spin_limit;" in source
