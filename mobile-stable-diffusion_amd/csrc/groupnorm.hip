@@ -403,14 +403,17 @@ __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
     };
     // Everything is requested before anything is waited for, in the order in which it is needed (loads return in order): data,
     // addends, then gamma and beta (us per launch with addends, fp16 batch 2, one after the other and so: 640 channels at 32 x 32
-    // 4.63 -> 4.47, 1280 at 16 x 16 3.51 -> 3.40; recorded step of 512 x 512 727 -> 721).  Long slices request
+    // 4.63 -> 4.47, 1280 at 16 x 16 3.51 -> 3.40; recorded step of 512 x 512 727 -> 721).  Six vectors per lane request addends,
+    // gamma and beta when the data is there: only launches of several workgroups per CU have that many, and twelve more requests a
+    // lane in front of the other wavefronts' data cost them 10 % (us, everything early and so: fp16 640 channels at 600 positions
+    // batch 32, no SiLU, 9.64 -> 8.70, fp32 at 300 9.81 -> 8.88, 320 at 9216 batch 3 13.0 -> 12.1, batch 2 8.98 -> 9.11).  Long slices request
     // their addends when they have the data: K more registers, and their launches are long enough to hide it (fp32 128
     // channels at 512 x 512, three passes of a decoder block 152.7 us, with everything early 153.5).
-    constexpr bool kPrefetchAffine = !RAGGED && K <= kGnPrefetchAffineK, kAddendEarly = kPrefetchAffine;
-    Addend addend[kAddendEarly ? K : 1];
-    if (kAddendEarly && chunk != nullptr) {  // uniform
+    constexpr bool kPrefetchAffine = !RAGGED && K <= kGnPrefetchAffineK, kEarly = kPrefetchAffine && K <= kGnEarlyK;
+    Addend addend[kEarly ? K : 1];
+    if (kEarly && chunk != nullptr) {  // uniform
 #pragma unroll
-        for (int k = 0; k < K; k++) addend[kAddendEarly ? k : 0] = addend_of(vidx(k, tid));
+        for (int k = 0; k < K; k++) addend[kEarly ? k : 0] = addend_of(vidx(k, tid));
     }
     // What follows waits for the arguments in memory: the compiler neither moves it up nor, as new values to it, shares it
     // with another branch in front of the loads.
@@ -425,20 +428,23 @@ __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
     // there after the barrier of the statistics) and the epilogue reads each vector's pair one
     // vector ahead, so a lane's registers hold little besides its packed slice.
     float ga[kPrefetchAffine ? K : 1], be[kPrefetchAffine ? K : 1];
-    if (kPrefetchAffine) {
+    auto fetch_affine = [&]() {
 #pragma unroll
         for (int k = 0; k < K; k++) {
             const uint32_t c = ch0 + fast_div(vidx(k, tid), hw_vec);
             ga[kPrefetchAffine ? k : 0] = gamma[c];
             be[kPrefetchAffine ? k : 0] = beta[c];
         }
+    };
+    if (kEarly) {
+        fetch_affine();
         __builtin_amdgcn_sched_barrier(0);
     }
     if (chunk != nullptr) {  // uniform
 #pragma unroll
         for (int k = 0; k < K; k++) {
             const uint32_t v = vidx(k, tid);
-            raw[k] = plus(raw[k], v, kAddendEarly ? addend[kAddendEarly ? k : 0] : addend_of(v));
+            raw[k] = plus(raw[k], v, kEarly ? addend[kEarly ? k : 0] : addend_of(v));
         }
     }
     if (!FULL) {  // registers of lanes past the end of a ragged slice hold zeros from here on
@@ -449,6 +455,7 @@ __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
             for (int i = 0; i < 4; i++) raw[k][i] = mine ? raw[k][i] : 0u;
         }
     }
+    if (kPrefetchAffine && !kEarly) fetch_affine();
     if (!kPrefetchAffine) {
         for (uint32_t c = tid; c < ch_per_group; c += nt) {  // ch_per_group <= kGnLdsChannels (host)
             aff[c] = make_float2(gamma[ch0 + c], beta[ch0 + c]);

@@ -41,6 +41,25 @@ def test_add_kernels(msd, orc, cuda, n, chunk, half):
         assert np.array_equal(got, ref)
 
 
+@pytest.mark.parametrize("half,shape", [(True, (32, 640, 600)), (True, (24, 256, 1536)), (False, (32, 640, 300)), (False, (24, 128, 1536))])
+def test_chunk_add_groupnorm_of_six_vectors_per_lane(msd, orc, cuda, half, shape):
+    """Slices that fill six vectors of every lane and slices that do not; launches of several workgroups per CU."""
+    import torch
+    batch, channels, hw = shape
+    assert msd.groupnorm_plan(batch, channels, hw, 32, msd.DTYPE_F16 if half else msd.DTYPE_F32)[1:3] == (256, 6)
+    x = orc.normal(shape, seed=hw, sigma=1.5, mean=0.3)
+    emb = orc.normal((batch, channels), seed=hw + 1, sigma=0.7)
+    g, b = _affine(orc, channels, 9)
+    x, emb = (orc.round_to_half(x), orc.round_to_half(emb)) if half else (x, emb)
+    xd, ed, gd, bd = _dev(x, cuda, half), _dev(emb, cuda, half), _dev(g, cuda), _dev(b, cuda)
+    for silu in (True, False):
+        tmp = msd.chunkwise_add(xd, ed, hw)
+        two = msd.groupnorm(tmp, gd, bd, 32, 1e-5, silu)
+        assert torch.equal(msd.chunk_add_groupnorm(xd, ed, gd, bd, 32, 1e-5, silu), two)
+        ref = orc.groupnorm64(tmp.float().cpu().numpy(), g, b, 32, 1e-5, silu).astype(np.float32).reshape(shape)
+        (assert_close_f16 if half else assert_close_f32)(two.float().cpu().numpy(), ref, what="six vectors per lane")
+
+
 @pytest.mark.parametrize("half", [False, True], ids=["f32", "f16"])
 @pytest.mark.parametrize("shape,groups", [((2, 320, 64, 64), 32), ((2, 640, 32, 32), 32), ((2, 1280, 8, 8), 32),
                                           ((1, 96, 24, 24), 32), ((3, 64, 5, 7), 8), ((1, 8, 128, 128), 1)])
