@@ -769,9 +769,7 @@ struct GnTokUnitParams {
     float eps, inv_count;
 };
 
-// What a lane stores: always the same 4 bytes of an output run (its channels), of every row_step-th position.  gamma and beta
-// of those channels are requested behind the data and have arrived when the sums have (us per launch, requested behind the
-// sums and so, fp16 batch 2: 1280 channels at 8 x 8 2.70 -> 2.51, at 16 x 16 3.56 -> 3.27, 640 at 32 x 32 4.28 -> 4.18).
+// What a lane stores: always the same 4 bytes of an output run (its channels), of every row_step-th position.
 // Stores of 4 bytes: 8 and 16 bytes at a time read LDS with more bank conflicts (us with 16 / 8 / 4 bytes, fp16 batch 2: 1280
 // channels at 16 x 16 4.2 / - / 3.7, 640 at 32 x 32 - / 4.9 / 4.7).
 template <typename T>
@@ -780,11 +778,14 @@ struct GnTokStore {
     uint32_t row0, c0, ch0, sample;
     float g[N], b[N];
 
-    __device__ __forceinline__ GnTokStore(uint32_t unit, const float *gamma, const float *beta, const GnTokUnitParams &q) {
+    __device__ __forceinline__ GnTokStore(uint32_t unit, const GnTokUnitParams &q) {
         row0 = fast_div(threadIdx.x, q.row_dwords);
         c0 = (threadIdx.x - row0 * q.row_dwords.d) * N;
         sample = fast_div(unit, q.groups);
         ch0 = (unit - sample * q.groups.d) * q.ch_per_group + c0;
+    }
+
+    __device__ __forceinline__ void fetch(const float *gamma, const float *beta) {
 #pragma unroll
         for (int i = 0; i < N; i++) {
             g[i] = gamma[ch0 + i];
@@ -817,7 +818,7 @@ struct GnTokStore {
     }
 };
 
-template <typename T, int K, bool RAGGED>
+template <typename T, int K, bool RAGGED, bool EARLY>
 __global__ __launch_bounds__(kGnMaxThreads) void gn_tokens_unit_kernel(
     const T *__restrict__ x, uint32_t nvec, uint32_t units_per_xcd, uint32_t shape, T *__restrict__ y,
     const float *__restrict__ gamma, const float *__restrict__ beta, GnTokUnitParams q) {
@@ -836,7 +837,8 @@ __global__ __launch_bounds__(kGnMaxThreads) void gn_tokens_unit_kernel(
     for (int k = 0; k < K; k++) raw[k] = load_stream(xin + min(k * nt + tid, nvec - 1));  // ragged tail: the last vector again
     __builtin_amdgcn_sched_barrier(0);  // (loads return in order: the data does not wait for gamma and beta)
     const uint32_t pos0 = part * q.part_pos, rows = min(q.part_pos, q.hw - pos0);
-    const GnTokStore<T> store(unit, gamma, beta, q);
+    GnTokStore<T> store(unit, q);
+    if (EARLY) store.fetch(gamma, beta);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int k = 0; k < K; k++) {
@@ -854,6 +856,7 @@ __global__ __launch_bounds__(kGnMaxThreads) void gn_tokens_unit_kernel(
     float mean, m2;
     gn_slice_stats<T, K, false>(raw, nvec, nt, red, mean, m2);  // (its barrier covers the tile)
     const float rstd = __builtin_amdgcn_rsqf(m2 * q.inv_count + q.eps);
+    if (!EARLY) store.fetch(gamma, beta);
     store(RAGGED ? lds + pos0 : lds, y, pos0, rows, mean, rstd, q);
 }
 
@@ -1164,15 +1167,27 @@ struct GnTokUnitPlan {
     bool ragged;
     uint32_t part_pos, pitch;
     size_t lds;
+    bool early;
 };
 
 constexpr size_t kGnTokMaxLds = 60 * 1024;
+
+// When gn_tokens_unit_kernel requests gamma and beta (EARLY): with the data, so that they have arrived when the sums have, except in large
+// launches of many workgroups or of several writers per unit.  There the time is the memory's, and stores that start that much
+// earlier, while other workgroups still load, cost more than the wait (us, behind the sums / with the data: fp16 batch 2 1280
+// channels at 8 x 8 2.70 / 2.51, at 16 x 16 3.56 / 3.27, batch 16 2560 at 320 positions 13.2 / 12.7; fp32 512 at 784 batch 24
+// 13.9 / 17.6, 640 at 784 batch 12, two writers, 10.9 / 13.4, fp16 1280 at 324 batch 48 19.6 / 23.2, 2560 at 380 batch 24
+// 26.1 / 24.4.  With the data over behind the sums, means over 110 random shapes: up to 2.5 workgroups per CU, one writer, 0.98,
+// more of them and 16 MB or more 1.04, below that 0.99).
+inline bool gn_tokens_early_affine(const Chip &chip, size_t bytes, size_t blocks, uint32_t writers) {
+    return bytes < (size_t)16 << 20 || (writers == 1 && blocks * 2 <= 5 * (size_t)chip.cus);
+}
 
 template <typename T>
 GnTokUnitPlan gn_tokens_unit_plan(const Chip &chip, size_t units, size_t cpg, size_t hw, int tune_writers) {
     constexpr size_t EPV = Store<T>::EPV;
     const size_t unit_size = cpg * hw, run = cpg * sizeof(T);
-    GnTokUnitPlan pl{1, 0, 0, hw % EPV != 0, 0, 0, 0};
+    GnTokUnitPlan pl{1, 0, 0, hw % EPV != 0, 0, 0, 0, false};
     if (unit_size % EPV != 0 || run % 4 != 0 || units > 0x7FFFFFFFull / 16) return pl;
     // as many writers as give the chip a workgroup per CU; they must share an XCD (gn_auto_writers)
     const bool may_share = (chip.xcds & (chip.xcds - 1)) == 0 && units % chip.xcds == 0;
@@ -1196,6 +1211,7 @@ GnTokUnitPlan gn_tokens_unit_plan(const Chip &chip, size_t units, size_t cpg, si
     const GnThreads t = gn_threads_for(chip, sizeof(T), (uint32_t)(unit_size / EPV), 1, blocks, max_k, false, pl.writers > 1);
     pl.threads = t.threads;
     pl.k = t.threads < run / 4 ? 0 : (uint32_t)t.k;  // (a lane per word of an output run)
+    pl.early = gn_tokens_early_affine(chip, units * unit_size * sizeof(T), units * pl.writers, pl.writers);
     return pl;
 }
 
@@ -1203,8 +1219,9 @@ template <typename T, int K>
 void gn_tokens_unit_launch(const GnTokUnitPlan &pl, uint32_t xcd_shift, uint32_t units, uint32_t vec_per_unit, hipStream_t stream,
                            const T *x, T *y, const float *gamma, const float *beta, const GnTokUnitParams &q) {
     const uint32_t blocks = units * pl.writers, units_per_xcd = units >> xcd_shift;
-    launch((pl.ragged ? gn_tokens_unit_kernel<T, K, true> : gn_tokens_unit_kernel<T, K, false>), dim3(blocks),
-           dim3(pl.threads), pl.lds, stream, x, vec_per_unit, units_per_xcd,
+    auto *kernel = pl.early ? (pl.ragged ? gn_tokens_unit_kernel<T, K, true, true> : gn_tokens_unit_kernel<T, K, false, true>)
+                            : (pl.ragged ? gn_tokens_unit_kernel<T, K, true, false> : gn_tokens_unit_kernel<T, K, false, false>);
+    launch(kernel, dim3(blocks), dim3(pl.threads), pl.lds, stream, x, vec_per_unit, units_per_xcd,
            gn_shape_word(0, (uint32_t)__builtin_ctz(pl.writers), xcd_shift, pl.threads), y, gamma, beta, q);
 }
 

@@ -352,7 +352,9 @@ def test_groupnorm_tokens_in_two_launches(msd, orc, cuda, shape, groups, mean, h
 @pytest.mark.parametrize("shape,half,two", [
     ((39, 1280, 16, 16), True, True), ((38, 1280, 16, 16), True, False),       # 24 MiB; more channels than positions
     ((20, 1280, 16, 16), False, True), ((24, 1280, 16, 16), False, False),     # a whole number of workgroups per CU
-    ((16, 640, 36, 36), False, False)])                                        # positions that leave a tile half empty
+    ((16, 640, 36, 36), False, False),                                         # positions that leave a tile half empty
+    ((48, 1280, 18, 18), True, False), ((24, 512, 28, 28), False, False),      # one launch that asks for gamma and beta behind the sums
+    ((12, 640, 28, 28), False, False), ((40, 320, 20, 16), False, False)])     # (two writers); a small one that does not
 def test_groupnorm_tokens_of_large_tensors(msd, orc, cuda, shape, half, two):
     import torch
     batch, channels, hw = shape[0], shape[1], shape[2] * shape[3]
