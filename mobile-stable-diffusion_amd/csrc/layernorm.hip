@@ -94,7 +94,10 @@ constexpr float kLnFastMoments = 4.0f;
 // second pass sums (x - mean)^2.  The epilogue unpacks one chunk at a time, so the row never
 // sits in registers twice.  gamma / beta of the lane's columns are requested together with
 // the row when EARLY (short launches: one memory latency instead of two on the critical path,
-// at the price of 2 * VPL * N registers).  Otherwise (long launches, bound by throughput) the
+// at the price of 2 * VPL * N registers).  float rows, whose requests for them are as many again as two rows', make
+// them when the row's first chunk is there: right behind the row they stand in the way of the other wavefronts' rows.  us, so
+// and when the first chunk is there: 4096 x 320 3.27 -> 3.16, 4500 x 320 3.66 -> 3.30, 5000 x 320 3.83 -> 3.40, 7000 x 320
+// 4.53 -> 4.01, 12000 x 160 4.11 -> 3.71, 3000 x 320 2.77 -> 2.80; half rows, in a recorded step of 512 x 512, 723 -> 724.  Otherwise (long launches, bound by throughput) the
 // workgroup copies gamma and beta into LDS once while its rows are in flight and every lane
 // reads its columns from there: fetching them from the cache per row costs four times the
 // row's own bytes in load instructions (measured at 131072 x 320 fp16: 31.2 us from global
@@ -174,13 +177,22 @@ __global__ __launch_bounds__(kLnMaxThreads) void ln_team_kernel(
         }
     };
     float g_all[EARLY ? VPL : 1][N], b_all[EARLY ? VPL : 1][N];
-    if (EARLY) {
+    auto fetch_affine = [&]() {
 #pragma unroll
         for (int k = 0; k < VPL; k++) affine(gamma, beta, k, g_all[EARLY ? k : 0], b_all[EARLY ? k : 0]);
-    }
+    };
+    constexpr bool kBehindFirst = EARLY && sizeof(T) == 4;
+    if (EARLY && !kBehindFirst) fetch_affine();
     float s[2] = {0.0f, 0.0f}, q[2] = {0.0f, 0.0f};
 #pragma unroll
-    for (int k = 0; k < VPL; k++) chunk_moments<T, NW>(raw[k], s, q);
+    for (int k = 0; k < VPL; k++) {
+        chunk_moments<T, NW>(raw[k], s, q);
+        if (kBehindFirst && k == 0) {
+            __builtin_amdgcn_sched_barrier(0);
+            fetch_affine();
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
     const float sum_x = team_sum<TL>(s[0] + s[1]);
     const float sum_xx = team_sum<TL>(q[0] + q[1]);
     const float mean = sum_x * inv_dim;
