@@ -108,10 +108,10 @@ __device__ __forceinline__ unsigned long long tagged(uint32_t tag, float v) {
 // us per launch, in place, a launch count that the last slice to finish advances / a tag per slice kept in its own slot, which
 // an overlap could set apart for good / so: fp16 320 channels at 64 x 64 batch 2 5.97 / 4.91 / 4.92, 640 7.12 / 6.37 / 6.35, fp32 320
 // batch 1 5.83 / 5.01 / 5.02, 960 batch 2 11.72 / 10.79 / 10.82; sixteen units' counts in a line: fp16 960 batch 1 5.70 -> 6.25.
-__device__ __forceinline__ unsigned long long gn_exchange_enter(const GnExchange &scratch, const GnParams &p, uint32_t unit) {
+__device__ __forceinline__ unsigned long long gn_exchange_enter(const GnExchange &scratch, uint32_t split, uint32_t unit) {
     uint32_t index = unit * kGnCountStride;
     asm volatile("" : "+v"(index));
-    const unsigned long long share = kGnMaxSplit >> __builtin_ctz(p.split);
+    const unsigned long long share = kGnMaxSplit >> __builtin_ctz(split);
     return __hip_atomic_fetch_add(scratch.counts + index, share, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
@@ -121,8 +121,8 @@ __device__ __forceinline__ unsigned long long gn_exchange_enter(const GnExchange
 // Slice l covers vectors [l * vec_per_slice, min(vec_per_unit, (l + 1) * vec_per_slice)).
 // `read(l, i)` returns vector i of slice l as the statistics see it (after the optional addend);
 // it is only used when slice l has not published within the poll limit.
-template <typename T, typename Reader>
-__device__ __forceinline__ void gn_exchange(const GnExchange &scratch, const GnParams &p, uint32_t unit,
+template <typename T, typename Params, typename Reader>
+__device__ __forceinline__ void gn_exchange(const GnExchange &scratch, const Params &p, uint32_t unit,
                                             uint32_t slice, unsigned long long count, float slice_mean,
                                             float slice_m2, float *stats, Reader read) {
     constexpr int EPV = Store<T>::EPV;
@@ -421,7 +421,7 @@ __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
     asm volatile("" : "+s"(unit), "+s"(part));
     u32x4 *yout = reinterpret_cast<u32x4 *>(y) + (size_t)unit * vec_per_unit;
     unsigned long long count = 0;  // (arrives right behind the data)
-    if (!SHARED && p.split > 1 && tid == 0) count = gn_exchange_enter(scratch, p, unit);
+    if (!SHARED && p.split > 1 && tid == 0) count = gn_exchange_enter(scratch, p.split, unit);
     const uint32_t ch0 = (unit - fast_div(unit, p.groups) * p.groups.d) * ch_per_group;
     // per-vector channel affine.  Up to six vectors per lane: fetched into registers up front,
     // while the data is in flight.  More: the group's gamma and beta go to LDS once (they are
@@ -642,7 +642,9 @@ __global__ __launch_bounds__(kGenericThreads) void gn_generic_kernel(
 // ---------------------------------------------------------------------------
 struct GnTokParams {
     uint32_t ch_per_group;
-    GnParams base;        // vec_per_slice = ch_per_group * position vectors per slice; vec_per_unit = that * split
+    // as in GnParams, for gn_exchange; vec_per_slice = ch_per_group * position vectors per slice, vec_per_unit = that * split
+    uint32_t vec_per_unit, vec_per_slice, split, spin_limit;
+    float eps, inv_count;
     FastDiv row_dwords;   // 4-byte words per output run: ch_per_group * sizeof(T) / 4
     uint32_t hw;          // positions per sample
     uint32_t channels;
@@ -658,7 +660,7 @@ __global__ __launch_bounds__(kGnMaxThreads) void gn_tokens_kernel(
     extern __shared__ u32x4 lds_vec[];
     __shared__ float red[kGnRedSlots];
     __shared__ float stats[2];
-    const GnParams &p = q.base;
+    const GnTokParams &p = q;
     const GnShape of(shape);
     const FastDiv pos_vecs{pos_mul, pos_shift, pvs};
     const uint32_t tid = threadIdx.x;
@@ -690,7 +692,7 @@ __global__ __launch_bounds__(kGnMaxThreads) void gn_tokens_kernel(
     }
     __builtin_amdgcn_sched_barrier(0);  // (what follows waits for the arguments in memory)
     unsigned long long count = 0;
-    if (p.split > 1 && tid == 0) count = gn_exchange_enter(scratch, p, unit);
+    if (p.split > 1 && tid == 0) count = gn_exchange_enter(scratch, p.split, unit);
     const uint32_t ch0 = group * q.ch_per_group;
 
     float slice_mean, slice_m2;
@@ -1252,8 +1254,13 @@ int gn_tokens_unit(const GnTokUnitPlan &pl, const Chip &chip, const T *x, T *y, 
         case 6: gn_tokens_unit_launch<T, 6>(pl, xcd_shift, (uint32_t)units, vec_per_unit, stream, x, y, gamma, beta, q); break;
         case 8: gn_tokens_unit_launch<T, 8>(pl, xcd_shift, (uint32_t)units, vec_per_unit, stream, x, y, gamma, beta, q); break;
         case 10: gn_tokens_unit_launch<T, 10>(pl, xcd_shift, (uint32_t)units, vec_per_unit, stream, x, y, gamma, beta, q); break;
-        case 12: gn_tokens_unit_launch<T, 12>(pl, xcd_shift, (uint32_t)units, vec_per_unit, stream, x, y, gamma, beta, q); break;
-        default: gn_tokens_unit_launch<T, 16>(pl, xcd_shift, (uint32_t)units, vec_per_unit, stream, x, y, gamma, beta, q); break;
+        default:  // (12, 16: 2-byte elements only, see max_k)
+            if constexpr (sizeof(T) == 2) {
+                if (pl.k == 12)
+                    gn_tokens_unit_launch<T, 12>(pl, xcd_shift, (uint32_t)units, vec_per_unit, stream, x, y, gamma, beta, q);
+                else
+                    gn_tokens_unit_launch<T, 16>(pl, xcd_shift, (uint32_t)units, vec_per_unit, stream, x, y, gamma, beta, q);
+            }
     }
     return launch_status();
 }
@@ -1261,11 +1268,10 @@ int gn_tokens_unit(const GnTokUnitPlan &pl, const Chip &chip, const T *x, T *y, 
 template <typename T, int K>
 void gn_tokens_launch(uint32_t blocks, uint32_t threads, size_t lds_bytes, hipStream_t stream,
                       const T *x, T *y, const float *gamma, const float *beta, const GnScratch &sc,
-                      const GnTokParams &q, uint32_t hw_vec, const FastDiv &pos_vecs, const FastDiv &combos) {
-    const GnParams &p = q.base;
-    launch((gn_tokens_kernel<T, K>), dim3(blocks), dim3(threads), lds_bytes, stream, x, p.vec_per_unit, p.vec_per_slice,
-           pos_vecs.mul, pos_vecs.shift, pos_vecs.d, hw_vec, combos.mul, combos.shift, combos.d, p.groups.d,
-           gn_shape_word((uint32_t)__builtin_ctz(p.split), 0, 0, threads), y, gamma, beta, sc, q);
+                      const GnTokParams &q, uint32_t groups, uint32_t hw_vec, const FastDiv &pos_vecs, const FastDiv &combos) {
+    launch((gn_tokens_kernel<T, K>), dim3(blocks), dim3(threads), lds_bytes, stream, x, q.vec_per_unit, q.vec_per_slice,
+           pos_vecs.mul, pos_vecs.shift, pos_vecs.d, hw_vec, combos.mul, combos.shift, combos.d, groups,
+           gn_shape_word((uint32_t)__builtin_ctz(q.split), 0, 0, threads), y, gamma, beta, sc, q);
 }
 
 // Whether gn_tokens_unit_kernel is the better one launch for a shape it can take: its units are loaded once per writer and
@@ -1427,15 +1433,13 @@ int gn_tokens_dispatch(const void *xv, void *yv, const float *gamma, const float
     GnTokParams q;
     const size_t pvs = hw_vec / split;  // position vectors of a slice
     const size_t nvec = cpg * pvs;
-    q.base.vec_per_unit = (uint32_t)(cpg * hw_vec);
-    q.base.vec_per_slice = (uint32_t)nvec;
-    q.base.split = split;
-    q.base.part_vecs = (uint32_t)nvec;
-    q.base.groups = make_fast_div((uint32_t)groups);
     q.ch_per_group = (uint32_t)cpg;
-    q.base.eps = eps;
-    q.base.inv_count = 1.0f / (float)unit_size;
-    q.base.spin_limit = tune_spin > 0 ? (uint32_t)tune_spin : kGnSpinLimit;
+    q.vec_per_unit = (uint32_t)(cpg * hw_vec);
+    q.vec_per_slice = (uint32_t)nvec;
+    q.split = split;
+    q.eps = eps;
+    q.inv_count = 1.0f / (float)unit_size;
+    q.spin_limit = tune_spin > 0 ? (uint32_t)tune_spin : kGnSpinLimit;
     const FastDiv pos_vecs = make_fast_div((uint32_t)pvs), combos = make_fast_div((uint32_t)(batch * split));  // ((sample, slice) pairs)
     q.row_dwords = make_fast_div((uint32_t)(cpg * sizeof(T) / 4));
     q.hw = (uint32_t)hw;
@@ -1458,16 +1462,21 @@ int gn_tokens_dispatch(const void *xv, void *yv, const float *gamma, const float
     }
     const uint32_t threads = pl.threads;
     switch (pl.k) {
-        case 1: gn_tokens_launch<T, 1>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, (uint32_t)hw_vec, pos_vecs, combos); break;
-        case 2: gn_tokens_launch<T, 2>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, (uint32_t)hw_vec, pos_vecs, combos); break;
-        case 3: gn_tokens_launch<T, 3>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, (uint32_t)hw_vec, pos_vecs, combos); break;
-        case 4: gn_tokens_launch<T, 4>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, (uint32_t)hw_vec, pos_vecs, combos); break;
-        case 5: gn_tokens_launch<T, 5>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, (uint32_t)hw_vec, pos_vecs, combos); break;
-        case 6: gn_tokens_launch<T, 6>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, (uint32_t)hw_vec, pos_vecs, combos); break;
-        case 8: gn_tokens_launch<T, 8>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, (uint32_t)hw_vec, pos_vecs, combos); break;
-        case 10: gn_tokens_launch<T, 10>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, (uint32_t)hw_vec, pos_vecs, combos); break;
-        case 12: gn_tokens_launch<T, 12>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, (uint32_t)hw_vec, pos_vecs, combos); break;
-        default: gn_tokens_launch<T, 16>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, (uint32_t)hw_vec, pos_vecs, combos); break;
+        case 1: gn_tokens_launch<T, 1>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, (uint32_t)groups, (uint32_t)hw_vec, pos_vecs, combos); break;
+        case 2: gn_tokens_launch<T, 2>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, (uint32_t)groups, (uint32_t)hw_vec, pos_vecs, combos); break;
+        case 3: gn_tokens_launch<T, 3>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, (uint32_t)groups, (uint32_t)hw_vec, pos_vecs, combos); break;
+        case 4: gn_tokens_launch<T, 4>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, (uint32_t)groups, (uint32_t)hw_vec, pos_vecs, combos); break;
+        case 5: gn_tokens_launch<T, 5>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, (uint32_t)groups, (uint32_t)hw_vec, pos_vecs, combos); break;
+        case 6: gn_tokens_launch<T, 6>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, (uint32_t)groups, (uint32_t)hw_vec, pos_vecs, combos); break;
+        case 8: gn_tokens_launch<T, 8>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, (uint32_t)groups, (uint32_t)hw_vec, pos_vecs, combos); break;
+        case 10: gn_tokens_launch<T, 10>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, (uint32_t)groups, (uint32_t)hw_vec, pos_vecs, combos); break;
+        default:  // (12, 16: 2-byte elements only, see kMaxK)
+            if constexpr (sizeof(T) == 2) {
+                if (pl.k == 12)
+                    gn_tokens_launch<T, 12>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, (uint32_t)groups, (uint32_t)hw_vec, pos_vecs, combos);
+                else
+                    gn_tokens_launch<T, 16>(blocks, threads, lds_bytes, stream, x, y, gamma, beta, sc, q, (uint32_t)groups, (uint32_t)hw_vec, pos_vecs, combos);
+            }
     }
     return launch_status();
 }
