@@ -267,7 +267,8 @@ constexpr float kGnFoldMean = 16.0f;
 // Between the last load's return and the first store this is the launch's critical path: the two sums
 // are reduced together (one value per lane after the first half of the steps), a wavefront's pair takes one LDS access each way,
 // the at most 16 partial sums meet in one row of lanes, and the mean is a product with the reciprocal of the count, which
-// is there before the loads return, and one correction (correctly rounded, as the division it stands for).  us per launch at
+// is there before the loads return, corrected once by the remainder (Markstein's division: the bits of the quotient, but
+// for subnormal ones; NaN instead of an infinity where the sum has overflowed, where the output is NaN with either).  us per launch at
 // batch 2, six LDS swizzles one after the other and a division, and so: fp16 320 channels at 64 x 64 5.19 -> 4.94, in place 5.93 ->
 // 5.76, 640 at 32 x 32 3.92 -> 3.74, in place 4.76 -> 4.59, 1280 at 8 x 8 2.65 -> 2.50; fp32 640 at 32 x 32 in place 5.58 -> 5.29.
 template <typename T, int K, bool FULL>
@@ -403,17 +404,18 @@ __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
     };
     // Everything is requested before anything is waited for, in the order in which it is needed (loads return in order): data,
     // addends, then gamma and beta (us per launch with addends, fp16 batch 2, one after the other and so: 640 channels at 32 x 32
-    // 4.63 -> 4.47, 1280 at 16 x 16 3.51 -> 3.40; recorded step of 512 x 512 727 -> 721).  Six vectors per lane request addends,
+    // 4.63 -> 4.47, 1280 at 16 x 16 3.51 -> 3.40; recorded step of 512 x 512 727 -> 721).  Six vectors per lane request
     // gamma and beta when the data is there: only launches of several workgroups per CU have that many, and twelve more requests a
     // lane in front of the other wavefronts' data cost them 10 % (us, everything early and so: fp16 640 channels at 600 positions
-    // batch 32, no SiLU, 9.64 -> 8.70, fp32 at 300 9.81 -> 8.88, 320 at 9216 batch 3 13.0 -> 12.1, batch 2 8.98 -> 9.11).  Long slices request
+    // batch 32, no SiLU, 9.70 -> 8.71, fp32 at 300 9.84 -> 8.63, 320 at 9216 batch 3 13.1 -> 12.2, batch 2 8.96 -> 9.16; with the
+    // addends late too 960 at 784 batch 12 9.07 -> 9.22).  Long slices request
     // their addends when they have the data: K more registers, and their launches are long enough to hide it (fp32 128
     // channels at 512 x 512, three passes of a decoder block 152.7 us, with everything early 153.5).
     constexpr bool kPrefetchAffine = !RAGGED && K <= kGnPrefetchAffineK, kEarly = kPrefetchAffine && K <= kGnEarlyK;
-    Addend addend[kEarly ? K : 1];
-    if (kEarly && chunk != nullptr) {  // uniform
+    Addend addend[kPrefetchAffine ? K : 1];
+    if (kPrefetchAffine && chunk != nullptr) {  // uniform
 #pragma unroll
-        for (int k = 0; k < K; k++) addend[kEarly ? k : 0] = addend_of(vidx(k, tid));
+        for (int k = 0; k < K; k++) addend[kPrefetchAffine ? k : 0] = addend_of(vidx(k, tid));
     }
     // What follows waits for the arguments in memory: the compiler neither moves it up nor, as new values to it, shares it
     // with another branch in front of the loads.
@@ -444,7 +446,7 @@ __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
 #pragma unroll
         for (int k = 0; k < K; k++) {
             const uint32_t v = vidx(k, tid);
-            raw[k] = plus(raw[k], v, kEarly ? addend[kEarly ? k : 0] : addend_of(v));
+            raw[k] = plus(raw[k], v, kPrefetchAffine ? addend[kPrefetchAffine ? k : 0] : addend_of(v));
         }
     }
     if (!FULL) {  // registers of lanes past the end of a ragged slice hold zeros from here on
@@ -559,11 +561,11 @@ __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
         epilogue(std::false_type{});
 }
 
-// Up to five vectors per lane (four for float storage) the kernel fits 64 registers: eight
+// Up to six vectors per lane (four for float storage) the kernel fits 64 registers: eight
 // wavefronts per SIMD, so two 1024-lane workgroups share a CU and one loads while the other
 // computes (what large batches need).
 template <typename T, int K, bool SILU, bool SHARED, bool RAGGED>
-__global__ __launch_bounds__(kGnMaxThreads, (K <= (sizeof(T) == 2 ? 5 : 4) ? 8 : 4)) void gn_slice_kernel(
+__global__ __launch_bounds__(kGnMaxThreads, (K <= (sizeof(T) == 2 ? 6 : 4) ? 8 : 4)) void gn_slice_kernel(
     const T *x, uint32_t vec_per_unit, uint32_t vec_per_slice, uint32_t shape, const T *chunk, uint32_t hw_mul,
     uint32_t hw_shift, uint32_t ch_per_group, const float *__restrict__ gamma, const float *__restrict__ beta, T *y,
     GnExchange scratch, GnParams p) {

@@ -56,7 +56,7 @@ constexpr int kGnMaxK = 20;             // vectors per lane; the largest only fo
 constexpr int kGnMaxRaggedK = 16;       // the largest with code for a ragged slice
 constexpr int kGnSharedMaxK = 10;       // kernels with several writers per unit exist up to this many vectors per lane
 constexpr int kGnPrefetchAffineK = 6;   // vectors per lane up to which gamma / beta are kept in registers
-constexpr int kGnEarlyK = 5;            // vectors per lane up to which they, and addends, are requested before the data is waited for
+constexpr int kGnEarlyK = 5;            // vectors per lane up to which they are requested before the data is waited for
 constexpr uint32_t kGnLdsChannels = 1024;  // channels per group the LDS copy of gamma / beta has room for
 
 struct GnExchange {  // (what kernels are given)
