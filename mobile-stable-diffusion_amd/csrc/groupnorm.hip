@@ -422,8 +422,6 @@ __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("" : "+s"(unit), "+s"(part));
     u32x4 *yout = reinterpret_cast<u32x4 *>(y) + (size_t)unit * vec_per_unit;
-    unsigned long long count = 0;  // (arrives right behind the data)
-    if (!SHARED && p.split > 1 && tid == 0) count = gn_exchange_enter(scratch, p.split, unit);
     const uint32_t ch0 = (unit - fast_div(unit, p.groups) * p.groups.d) * ch_per_group;
     // per-vector channel affine.  Up to six vectors per lane: fetched into registers up front,
     // while the data is in flight.  More: the group's gamma and beta go to LDS once (they are
@@ -442,6 +440,14 @@ __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
         fetch_affine();
         __builtin_amdgcn_sched_barrier(0);
     }
+    // The count is asked for behind what is waited for first.  Up to five vectors a lane that is everything (recorded step of
+    // 512 x 512, fp32, in front of gamma and beta / so: 728 / 726 us).  Slices of twelve and more put gamma and beta into LDS in front of
+    // the sums and would wait for the count with them; they ask for it after that, and their sums take long enough for it to
+    // arrive (us, in front / so: fp32 128 channels at 512 x 512, 16 vectors, 45.35 / 45.13, fp16 22.61 / 22.41; those of ten would
+    // lose: fp32 320 at 64 x 64 batch 8 13.5 / 13.9).
+    constexpr bool kLong = K >= 12;
+    unsigned long long count = 0;
+    if (!kLong && !SHARED && p.split > 1 && tid == 0) count = gn_exchange_enter(scratch, p.split, unit);
     if (chunk != nullptr) {  // uniform
 #pragma unroll
         for (int k = 0; k < K; k++) {
@@ -463,6 +469,8 @@ __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
             aff[c] = make_float2(gamma[ch0 + c], beta[ch0 + c]);
         }
     }
+
+    if (kLong && !SHARED && p.split > 1 && tid == 0) count = gn_exchange_enter(scratch, p.split, unit);
 
     float slice_mean, slice_m2;
     gn_slice_stats<T, K, FULL>(raw, v_end - v_begin, nt, red, slice_mean, slice_m2);
