@@ -26,8 +26,9 @@ ARCH = "gfx950"
 # values, up to the first structure), loaded by the command processor while it prepares the launch.  Otherwise a wavefront's
 # first act is to load them, and in a step of 200 launches, each with arguments of its own, that is a miss of every cache in
 # front of the launch's first access to its data.  Recorded steps of 512 x 512, us, loaded by the wavefronts and so: fp16
-# batch 2 780 -> 753, fp32 batch 1 788 -> 760.  (A chain of empty launches gets 0.1 us slower per launch, copies of up to
-# 0.6 MB 0.07; from 2 MB on they get 0.04 faster even where the arguments are in a cache.)
+# batch 2 780 -> 753, fp32 batch 1 788 -> 760.  (Launches below 2 us in a row - empty ones, copies, SiLU, DDIM updates of up to
+# 0.6 MB - get 0.05 - 0.15 us slower each: the preload is part of what the next one waits for.  Behind a longer launch the same
+# ones take as much as before or 0.1 less, and from 2 MB on they get 0.04 faster even where the arguments are in a cache.)
 DEVICE_FLAGS = [
     "-O3", "-std=c++17", f"--offload-arch={ARCH}", "-fPIC",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",

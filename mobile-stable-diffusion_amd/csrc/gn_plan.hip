@@ -58,7 +58,8 @@ inline float k_cost(int k) {
 }
 
 // A workgroup normalises about this many elements in the time an exchange between the slices of
-// a unit costs (two round trips through the memory-side coherence point, 1.3 - 2.5 us): units up
+// a unit cost when this was measured (two round trips through the memory-side coherence point, 1.3 - 2.5 us; now
+// about 0.9, and neither this nor the table of measured plans below, with its times, has been measured again): units up
 // to this size stay whole, longer ones are cut into slices of at most this size.  In elements,
 // not bytes: the epilogue's arithmetic per element is what a slice's time is made of.
 constexpr size_t kSliceElements = 20480;
