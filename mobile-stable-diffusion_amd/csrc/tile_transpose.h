@@ -16,6 +16,7 @@
 namespace msd {
 
 constexpr int kTile = 64;
+constexpr size_t kCacheLine = 128;
 constexpr int kTileThreads = 256;
 // Most positions along a side: a grid holds less than 2^32 lanes in a dimension.
 constexpr size_t kTileMaxSide = 0xFFFFFFFFull / kTileThreads * kTile;
@@ -40,8 +41,10 @@ __device__ __forceinline__ void store_any(char *at, W w) {
 
 // The piece (16 / ES elements) at `at` of a row with `left` elements from there on; what lies past the
 // row's end is not read.  RAGGED: pieces may start at any element and may be cut by the row's end.
-template <int ES, bool RAGGED>
+// KEEP: the lines stay in the caches, for the pieces beside this one.
+template <int ES, bool RAGGED, bool KEEP = false>
 __device__ __forceinline__ u32x4 tile_load(const char *at, uint32_t left) {
+    if constexpr (!RAGGED && KEEP) return *reinterpret_cast<const u32x4 *>(at);
     if constexpr (!RAGGED) return load_stream(reinterpret_cast<const u32x4 *>(at));
     if (left >= 16 / ES) return load_any<u32x4>(at);
     uint32_t w0 = 0, w1 = 0, w2 = 0, w3 = 0;
@@ -89,9 +92,9 @@ __device__ __forceinline__ void tile_store(char *at, uint32_t left, const u32x4 
 // in: the [jsize, ksize] plane, out: the [ksize, jsize] plane, ES bytes per element; the tile starts at
 // (j0, k0).  Without RAGGED jsize and ksize are multiples of 16 / ES and both planes are 16-byte
 // aligned (a piece is all inside the tensor or all outside).  ready() runs between the loads and their
-// first use, by every lane; map(row, piece) returns the piece of tile row `row` (channel j0 + row) as
+// first use, by every lane (KEEP: see tile_load); map(row, piece) returns the piece of tile row `row` (channel j0 + row) as
 // it is to be stored.
-template <int ES, bool RAGGED, typename Ready, typename Map>
+template <int ES, bool RAGGED, bool KEEP = false, typename Ready, typename Map>
 __device__ __forceinline__ void transpose_tile(const char *in, char *out, uint32_t jsize, uint32_t ksize, uint32_t j0,
                                                uint32_t k0, u32x4 *tile4, Ready ready, Map map) {
     constexpr uint32_t kWords = kTile * ES / 4;      // 32-bit words per output row of the tile: 32 or 64
@@ -112,7 +115,7 @@ __device__ __forceinline__ void transpose_tile(const char *in, char *out, uint32
             const uint32_t k = k0 + kq + 32 * (pass & 1), j = j0 + jr + 32 * (pass >> 1);
             const bool inside = j < jsize && k < ksize;
             const size_t from = inside ? ((size_t)j * ksize + k) * 4 : 0;
-            v[pass] = tile_load<ES, RAGGED>(in + from, inside ? ksize - k : 0);
+            v[pass] = tile_load<ES, RAGGED, KEEP>(in + from, inside ? ksize - k : 0);
         }
         ready();
 #pragma unroll
@@ -131,10 +134,10 @@ __device__ __forceinline__ void transpose_tile(const char *in, char *out, uint32
         const bool inside = j < jsize && k < ksize;
         u32x4 a = {0, 0, 0, 0}, b = {0, 0, 0, 0};
         if (inside) {
-            a = tile_load<ES, RAGGED>(in + ((size_t)j * ksize + k) * 2, ksize - k);
+            a = tile_load<ES, RAGGED, KEEP>(in + ((size_t)j * ksize + k) * 2, ksize - k);
             // (without RAGGED jsize is even; an odd one's last row pairs with itself)
             const uint32_t second = RAGGED ? min(j + 1, jsize - 1) : j + 1;
-            b = tile_load<ES, RAGGED>(in + ((size_t)second * ksize + k) * 2, ksize - k);
+            b = tile_load<ES, RAGGED, KEEP>(in + ((size_t)second * ksize + k) * 2, ksize - k);
         }
         ready();
         if (inside) {

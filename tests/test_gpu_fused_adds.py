@@ -303,6 +303,8 @@ def _takes_two_launches(msd, xd, gd, bd, groups):
     ((2, 65, 8, 161), 65, True, True), ((2, 65, 10, 129), 65, False, False),   # a group per channel; no whole vectors
     ((1, 8, 300, 300), 1, True, True), ((1, 8, 300, 300), 1, False, True),     # one unit in 16 slices
     ((2, 320, 56, 48), 32, True, True), ((2, 320, 56, 48), 32, False, True),   # short runs, long units
+    ((2, 320, 45, 56), 32, True, True), ((2, 320, 45, 56), 32, False, True),   # ... rows of no whole cache lines, 200 tiles a plane
+    ((3, 320, 41, 56), 32, True, True), ((3, 320, 41, 56), 32, False, True),   # ... 180 tiles: no whole number per XCD
     ((1, 2560, 34, 32), 128, True, True),                                      # ... and more channels than positions
     ((20, 640, 2, 13), 32, False, False), ((40, 640, 2, 13), 32, False, True),  # units of 520: few of them, many
     ((40, 640, 2, 13), 32, True, True), ((60, 640, 1, 22), 32, False, False),   # planes much narrower than a tile
