@@ -94,10 +94,11 @@ constexpr float kLnFastMoments = 4.0f;
 // second pass sums (x - mean)^2.  The epilogue unpacks one chunk at a time, so the row never
 // sits in registers twice.  gamma / beta of the lane's columns are requested together with
 // the row when EARLY (short launches: one memory latency instead of two on the critical path,
-// at the price of 2 * VPL * N registers).  float rows, whose requests for them are as many again as two rows', make
-// them when the row's first chunk is there: right behind the row they stand in the way of the other wavefronts' rows.  us, so
-// and when the first chunk is there: 4096 x 320 3.27 -> 3.16, 4500 x 320 3.66 -> 3.30, 5000 x 320 3.83 -> 3.40, 7000 x 320
-// 4.53 -> 4.01, 12000 x 160 4.11 -> 3.71, 3000 x 320 2.77 -> 2.80; half rows, in a recorded step of 512 x 512, 723 -> 724.  Otherwise (long launches, bound by throughput) the
+// at the price of 2 * VPL * N registers).  float rows and half rows in 8-byte chunks, whose requests for them
+// are as many as two rows' own, make them when the row's first chunk is there: right behind the row they stand in
+// the way of the other wavefronts' rows.  us, so and when the first chunk is there: fp32 4096 x 320 3.27 -> 3.16, 4500 x 320
+// 3.66 -> 3.30, 5000 x 320 3.83 -> 3.40, 7000 x 320 4.53 -> 4.01, 3000 x 320 2.77 -> 2.80; fp16 2500 x 640 3.17 -> 2.93, 5694 x 320
+// 3.34 -> 3.05, 512 x 1280 2.44 -> 2.40; in 16-byte chunks 1608 x 2560 4.38 -> 4.51, 1083 x 512 2.30 -> 2.36.  Otherwise (long launches, bound by throughput) the
 // workgroup copies gamma and beta into LDS once while its rows are in flight and every lane
 // reads its columns from there: fetching them from the cache per row costs four times the
 // row's own bytes in load instructions (measured at 131072 x 320 fp16: 31.2 us from global
@@ -181,7 +182,7 @@ __global__ __launch_bounds__(kLnMaxThreads) void ln_team_kernel(
 #pragma unroll
         for (int k = 0; k < VPL; k++) affine(gamma, beta, k, g_all[EARLY ? k : 0], b_all[EARLY ? k : 0]);
     };
-    constexpr bool kBehindFirst = EARLY && sizeof(T) == 4;
+    constexpr bool kBehindFirst = EARLY && (sizeof(T) == 4 || NW == 2);
     if (EARLY && !kBehindFirst) fetch_affine();
     float s[2] = {0.0f, 0.0f}, q[2] = {0.0f, 0.0f};
 #pragma unroll
