@@ -341,7 +341,7 @@ __device__ __forceinline__ GnStraddle gn_straddle(uint32_t v, const FastDiv &hw)
 // per launch, before and now: fp16 batch 2, 2560 channels at 9 x 7 10.1 -> 2.9, in place 14.1 -> 3.8;
 // 1280 at 18 x 14 17.9 -> 2.9, in place 25.3 -> 4.4; batch 16, 640 at 18 x 14 10.7 -> 4.7; fp32 batch 4,
 // 2560 at 11 x 9 15.9 -> 3.4.
-template <typename T, int K, bool SILU, bool FULL, bool SHARED, bool RAGGED>
+template <typename T, int K, bool SILU, bool FULL, bool SHARED, bool RAGGED, bool EARLY>
 __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
                                         const float *__restrict__ gamma,
                                         const float *__restrict__ beta, const GnExchange &scratch,
@@ -411,7 +411,7 @@ __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
     // addends late too 960 at 784 batch 12 9.07 -> 9.22).  Long slices request
     // their addends when they have the data: K more registers, and their launches are long enough to hide it (fp32 128
     // channels at 512 x 512, three passes of a decoder block 152.7 us, with everything early 153.5).
-    constexpr bool kPrefetchAffine = !RAGGED && K <= kGnPrefetchAffineK, kEarly = kPrefetchAffine && K <= kGnEarlyK;
+    constexpr bool kPrefetchAffine = !RAGGED && K <= kGnPrefetchAffineK, kEarly = kPrefetchAffine && EARLY;
     Addend addend[kPrefetchAffine ? K : 1];
     if (kPrefetchAffine && chunk != nullptr) {  // uniform
 #pragma unroll
@@ -572,7 +572,8 @@ __device__ __forceinline__ void gn_body(const T *x, const T *chunk, T *y,
 // Up to six vectors per lane (four for float storage) the kernel fits 64 registers: eight
 // wavefronts per SIMD, so two 1024-lane workgroups share a CU and one loads while the other
 // computes (what large batches need).
-template <typename T, int K, bool SILU, bool SHARED, bool RAGGED>
+// EARLY: gamma and beta are requested in front of the wait for the data (gn_body).
+template <typename T, int K, bool SILU, bool SHARED, bool RAGGED, bool EARLY = K <= kGnEarlyK>
 __global__ __launch_bounds__(kGnMaxThreads, (K <= (sizeof(T) == 2 ? 6 : 4) ? 8 : 4)) void gn_slice_kernel(
     const T *x, uint32_t vec_per_unit, uint32_t vec_per_slice, uint32_t shape, const T *chunk, uint32_t hw_mul,
     uint32_t hw_shift, uint32_t ch_per_group, const float *__restrict__ gamma, const float *__restrict__ beta, T *y,
@@ -597,10 +598,10 @@ __global__ __launch_bounds__(kGnMaxThreads, (K <= (sizeof(T) == 2 ? 6 : 4) ? 8 :
     const uint32_t v_end = min(vec_per_unit, v_begin + vec_per_slice);
     // uniform over the workgroup; the largest K is only launched on slices it fits exactly
     if (K == kGnMaxK || v_end - v_begin == K * of.threads)
-        gn_body<T, K, SILU, true, SHARED, RAGGED>(x, chunk, y, gamma, beta, scratch, p, of.threads, vec_per_unit, unit, slice, part,
+        gn_body<T, K, SILU, true, SHARED, RAGGED, EARLY>(x, chunk, y, gamma, beta, scratch, p, of.threads, vec_per_unit, unit, slice, part,
                                           v_begin, v_end, ch_per_group, hw_vec, red, stats, aff);
     else
-        gn_body<T, K, SILU, false, SHARED, RAGGED>(x, chunk, y, gamma, beta, scratch, p, of.threads, vec_per_unit, unit, slice, part,
+        gn_body<T, K, SILU, false, SHARED, RAGGED, EARLY>(x, chunk, y, gamma, beta, scratch, p, of.threads, vec_per_unit, unit, slice, part,
                                            v_begin, v_end, ch_per_group, hw_vec, red, stats, aff);
 }
 
@@ -1072,6 +1073,7 @@ inline uint32_t gn_xcd_shift(const Chip &chip, bool shared, size_t units) {
 // The leading plain arguments of gn_slice_kernel beside those of GnParams.
 struct GnGeometry {
     uint32_t blocks, threads, shape, ch_per_group;
+    bool late;   // four workgroups per CU or more
     FastDiv hw;  // vectors per channel (RAGGED: elements per channel)
 };
 
@@ -1085,8 +1087,15 @@ void gn_launch_k(bool silu, bool shared, const GnGeometry &g, hipStream_t stream
                dim3(g.blocks), dim3(g.threads), 0, stream, x, p.vec_per_unit, p.vec_per_slice, g.shape, chunk, g.hw.mul,
                g.hw.shift, g.ch_per_group, gamma, beta, y, sc, p);
     } else {
-        launch((silu ? gn_slice_kernel<T, K, true, false, RAGGED> : gn_slice_kernel<T, K, false, false, RAGGED>),
-               dim3(g.blocks), dim3(g.threads), 0, stream, x, p.vec_per_unit, p.vec_per_slice, g.shape, chunk, g.hw.mul,
+        auto *kernel = silu ? gn_slice_kernel<T, K, true, false, RAGGED> : gn_slice_kernel<T, K, false, false, RAGGED>;
+        if constexpr (sizeof(T) == 4 && K <= kGnEarlyK && !RAGGED) {
+            // Float slices of launches with at least four workgroups per CU ask for gamma and beta behind the data (see gn_body): us,
+            // early / so, 256 channels at 304 positions batch 48 6.41 / 5.92, 512 at 192 batch 60 9.53 / 8.90, 192 at 736
+            // batch 32 7.27 / 6.82, 128 at 920 batch 40 6.90 / 6.96; at three per CU 128 at 680 batch 24 4.29 / 4.39.  (Half slices of as
+            // many: 0.95 to 1.03 of the early ones.)
+            if (g.late) kernel = silu ? gn_slice_kernel<T, K, true, false, RAGGED, false> : gn_slice_kernel<T, K, false, false, RAGGED, false>;
+        }
+        launch(kernel, dim3(g.blocks), dim3(g.threads), 0, stream, x, p.vec_per_unit, p.vec_per_slice, g.shape, chunk, g.hw.mul,
                g.hw.shift, g.ch_per_group, gamma, beta, y, sc, p);
     }
 }
@@ -1167,10 +1176,12 @@ int gn_dispatch(const void *xv, const void *chunkv, void *yv, const float *gamma
     p.spin_limit = tune_spin > 0 ? (uint32_t)tune_spin : kGnSpinLimit;
     const bool shared = d.writers > 1;
     p.part_vecs = (uint32_t)((((p.vec_per_unit + d.writers - 1) / d.writers + kWave - 1) / kWave) * kWave);
-    const GnGeometry g{(uint32_t)(units * split * d.writers), d.threads,
+    const Chip chip = chip_info();
+    const size_t blocks = units * split * d.writers;
+    const GnGeometry g{(uint32_t)blocks, d.threads,
                        gn_shape_word((uint32_t)__builtin_ctz(split), (uint32_t)__builtin_ctz(d.writers),
-                                     gn_xcd_shift(chip_info(), shared, units), d.threads),
-                       (uint32_t)cpg, make_fast_div((uint32_t)(ragged ? hw : hw / EPV))};
+                                     gn_xcd_shift(chip, shared, units), d.threads),
+                       (uint32_t)cpg, blocks >= 4 * (size_t)chip.cus, make_fast_div((uint32_t)(ragged ? hw : hw / EPV))};
 
     if (fixed != nullptr) {
         sc = *fixed;

@@ -41,12 +41,14 @@ def test_add_kernels(msd, orc, cuda, n, chunk, half):
         assert np.array_equal(got, ref)
 
 
-@pytest.mark.parametrize("half,shape", [(True, (32, 640, 600)), (True, (24, 256, 1536)), (False, (32, 640, 300)), (False, (24, 128, 1536))])
-def test_chunk_add_groupnorm_of_six_vectors_per_lane(msd, orc, cuda, half, shape):
-    """Slices that fill six vectors of every lane and slices that do not; launches of several workgroups per CU."""
+@pytest.mark.parametrize("half,shape,vectors", [
+    (True, (32, 640, 600), 6), (True, (24, 256, 1536), 6), (False, (32, 640, 300), 6), (False, (24, 128, 1536), 6),
+    (False, (32, 64, 500), 1), (False, (48, 256, 304), 3), (False, (32, 64, 2560), 5), (False, (60, 512, 192), 3)])  # four per CU and more
+def test_chunk_add_groupnorm_of_several_workgroups_per_cu(msd, orc, cuda, half, shape, vectors):
+    """Slices that fill their vectors in every lane and slices that do not, of launches that ask for gamma and beta behind the data."""
     import torch
     batch, channels, hw = shape
-    assert msd.groupnorm_plan(batch, channels, hw, 32, msd.DTYPE_F16 if half else msd.DTYPE_F32)[1:3] == (256, 6)
+    assert msd.groupnorm_plan(batch, channels, hw, 32, msd.DTYPE_F16 if half else msd.DTYPE_F32)[1:3] == (256, vectors)
     x = orc.normal(shape, seed=hw, sigma=1.5, mean=0.3)
     emb = orc.normal((batch, channels), seed=hw + 1, sigma=0.7)
     g, b = _affine(orc, channels, 9)
@@ -57,7 +59,7 @@ def test_chunk_add_groupnorm_of_six_vectors_per_lane(msd, orc, cuda, half, shape
         two = msd.groupnorm(tmp, gd, bd, 32, 1e-5, silu)
         assert torch.equal(msd.chunk_add_groupnorm(xd, ed, gd, bd, 32, 1e-5, silu), two)
         ref = orc.groupnorm64(tmp.float().cpu().numpy(), g, b, 32, 1e-5, silu).astype(np.float32).reshape(shape)
-        (assert_close_f16 if half else assert_close_f32)(two.float().cpu().numpy(), ref, what="six vectors per lane")
+        (assert_close_f16 if half else assert_close_f32)(two.float().cpu().numpy(), ref, what="several workgroups per CU")
 
 
 @pytest.mark.parametrize("half", [False, True], ids=["f32", "f16"])

@@ -55,7 +55,7 @@ def test_short_groupnorm_slices_leave_room_for_eight_wavefronts_per_simd(kernels
         if m and int(m.group(2)) <= (6 if m.group(1) == "__half" else 5):
             assert registers <= 64, name
             seen += 1
-    assert seen == 8 * (6 + 5)
+    assert seen == 8 * (6 + 5) + 2 * 5  # (float slices exist in two orders of requests)
 
 
 def test_no_kernel_keeps_registers_in_memory(kernels):
