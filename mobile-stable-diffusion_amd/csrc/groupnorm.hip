@@ -1217,10 +1217,11 @@ constexpr size_t kGnTokMaxLds = 60 * 1024;
 // earlier, while other workgroups still load, cost more than the wait (us, behind the sums / with the data: fp16 batch 2 1280
 // channels at 8 x 8 2.70 / 2.51, at 16 x 16 3.56 / 3.27, batch 16 2560 at 320 positions 13.2 / 12.7; fp32 512 at 784 batch 24
 // 13.9 / 17.6, 640 at 784 batch 12, two writers, 10.9 / 13.4, fp16 1280 at 324 batch 48 19.6 / 23.2, 2560 at 380 batch 24
-// 26.1 / 24.4.  With the data over behind the sums, means over 110 random shapes: up to 2.5 workgroups per CU, one writer, 0.98,
-// more of them and 16 MB or more 1.04, below that 0.99).
+// 26.1 / 24.4; just over two workgroups per CU 512 at 792 batch 18 12.1 / 15.2, fp16 960 at 840 batch 19 17.7 / 21.5, fp32 640 at 700
+// batch 19 22.3 / 21.4.  With the data over behind the sums, means over 146 random shapes: up to two workgroups per CU, one
+// writer, 0.98, more of them and 16 MB or more 1.03, below that 0.99).
 inline bool gn_tokens_early_affine(const Chip &chip, size_t bytes, size_t blocks, uint32_t writers) {
-    return bytes < (size_t)16 << 20 || (writers == 1 && blocks * 2 <= 5 * (size_t)chip.cus);
+    return bytes < (size_t)16 << 20 || (writers == 1 && blocks <= 2 * (size_t)chip.cus);
 }
 
 template <typename T>

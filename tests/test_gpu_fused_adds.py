@@ -357,7 +357,7 @@ def test_groupnorm_tokens_in_two_launches(msd, orc, cuda, shape, groups, mean, h
     ((39, 1280, 16, 16), True, True), ((38, 1280, 16, 16), True, False),       # 24 MiB; more channels than positions
     ((20, 1280, 16, 16), False, True), ((24, 1280, 16, 16), False, False),     # a whole number of workgroups per CU
     ((16, 640, 36, 36), False, False),                                         # positions that leave a tile half empty
-    ((48, 1280, 18, 18), True, False), ((24, 512, 28, 28), False, False),      # one launch that asks for gamma and beta behind the sums
+    ((48, 1280, 18, 18), True, False), ((18, 512, 24, 33), False, False),      # one launch that asks for gamma and beta behind the sums
     ((12, 640, 28, 28), False, False), ((40, 320, 20, 16), False, False)])     # (two writers); a small one that does not
 def test_groupnorm_tokens_of_large_tensors(msd, orc, cuda, shape, half, two):
     import torch
