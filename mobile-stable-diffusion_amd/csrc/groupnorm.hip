@@ -1073,7 +1073,7 @@ inline uint32_t gn_xcd_shift(const Chip &chip, bool shared, size_t units) {
 // The leading plain arguments of gn_slice_kernel beside those of GnParams.
 struct GnGeometry {
     uint32_t blocks, threads, shape, ch_per_group;
-    bool late;   // four workgroups per CU or more
+    uint32_t per_cu;  // workgroups, rounded down
     FastDiv hw;  // vectors per channel (RAGGED: elements per channel)
 };
 
@@ -1089,11 +1089,12 @@ void gn_launch_k(bool silu, bool shared, const GnGeometry &g, hipStream_t stream
     } else {
         auto *kernel = silu ? gn_slice_kernel<T, K, true, false, RAGGED> : gn_slice_kernel<T, K, false, false, RAGGED>;
         if constexpr (sizeof(T) == 4 && K <= kGnEarlyK && !RAGGED) {
-            // Float slices of launches with at least four workgroups per CU ask for gamma and beta behind the data (see gn_body): us,
-            // early / so, 256 channels at 304 positions batch 48 6.41 / 5.92, 512 at 192 batch 60 9.53 / 8.90, 192 at 736
-            // batch 32 7.27 / 6.82, 128 at 920 batch 40 6.90 / 6.96; at three per CU 128 at 680 batch 24 4.29 / 4.39.  (Half slices of as
-            // many: 0.95 to 1.03 of the early ones.)
-            if (g.late) kernel = silu ? gn_slice_kernel<T, K, true, false, RAGGED, false> : gn_slice_kernel<T, K, false, false, RAGGED, false>;
+            // Float slices of launches with several workgroups per CU ask for gamma and beta behind the data (see gn_body): us, early /
+            // so, two per CU 192 channels at 752 positions batch 17 (three vectors) 5.68 / 4.95, 256 at 800 batch 16 (four) 5.98 / 5.35, 384
+            // at 704 batch 18 (five) 8.81 / 8.41; six 256 at 304 batch 48 6.41 / 5.92, 512 at 192 batch 60 9.53 / 8.90; against it three
+            // per CU 128 at 568 batch 24 (three) 4.01 / 4.10, two 128 at 824 batch 16 (two) 4.02 / 4.09.  (Half slices of as many: 0.95
+            // to 1.03 of the early ones.)
+            if (g.per_cu >= (K >= 3 ? 2u : 4u)) kernel = silu ? gn_slice_kernel<T, K, true, false, RAGGED, false> : gn_slice_kernel<T, K, false, false, RAGGED, false>;
         }
         launch(kernel, dim3(g.blocks), dim3(g.threads), 0, stream, x, p.vec_per_unit, p.vec_per_slice, g.shape, chunk, g.hw.mul,
                g.hw.shift, g.ch_per_group, gamma, beta, y, sc, p);
@@ -1181,7 +1182,7 @@ int gn_dispatch(const void *xv, const void *chunkv, void *yv, const float *gamma
     const GnGeometry g{(uint32_t)blocks, d.threads,
                        gn_shape_word((uint32_t)__builtin_ctz(split), (uint32_t)__builtin_ctz(d.writers),
                                      gn_xcd_shift(chip, shared, units), d.threads),
-                       (uint32_t)cpg, blocks >= 4 * (size_t)chip.cus, make_fast_div((uint32_t)(ragged ? hw : hw / EPV))};
+                       (uint32_t)cpg, (uint32_t)(blocks / chip.cus), make_fast_div((uint32_t)(ragged ? hw : hw / EPV))};
 
     if (fixed != nullptr) {
         sc = *fixed;
