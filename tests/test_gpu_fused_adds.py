@@ -353,6 +353,27 @@ def test_groupnorm_tokens_in_two_launches(msd, orc, cuda, shape, groups, mean, h
             check(plain, "gn tokens, recorded without scratch")
 
 
+@pytest.mark.parametrize("shape,half", [((3, 320, 41, 56), True), ((3, 320, 41, 56), False), ((2, 1280, 9, 7), True), ((2, 65, 8, 161), True)])
+def test_groupnorm_tokens_in_two_launches_on_other_xcd_counts(msd, orc, cuda, shape, half):
+    """The tiles of planes whose rows are no whole cache lines are dealt out by XCD: every tile once, whatever their number."""
+    import torch
+    lib, groups = msd.load_library(), 65 if shape[1] == 65 else 32
+    xd = torch.empty(shape, dtype=torch.float16 if half else torch.float32, device=cuda).normal_(0.4, 1.5)
+    gd, bd = (_dev(t, cuda) for t in _affine(orc, shape[1], 26))
+    assert _takes_two_launches(msd, xd, gd, bd, groups)
+    want = msd.groupnorm_tokens(xd, gd, bd, groups, 1e-6)
+    try:
+        for xcds in (1, 2, 6, 16, 64):
+            assert lib.msd_set_tuning(msd.TUNE_DEVICE_XCDS, xcds) == 0
+            got = torch.full_like(want, float("nan"))
+            assert lib.msd_groupnorm_tokens(
+                xd.data_ptr(), got.data_ptr(), gd.data_ptr(), bd.data_ptr(), shape[0], shape[1], shape[2] * shape[3], groups, 1e-6,
+                msd.DTYPE_F16 if half else msd.DTYPE_F32, torch.cuda.current_stream().cuda_stream) == 0
+            assert torch.equal(got, want), xcds
+    finally:
+        assert lib.msd_set_tuning(msd.TUNE_DEVICE_XCDS, 0) == 0
+
+
 @pytest.mark.parametrize("shape,half,two", [
     ((39, 1280, 16, 16), True, True), ((38, 1280, 16, 16), True, False),       # 24 MiB; more channels than positions
     ((20, 1280, 16, 16), False, True), ((24, 1280, 16, 16), False, False),     # a whole number of workgroups per CU
